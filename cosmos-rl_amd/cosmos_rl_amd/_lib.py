@@ -54,6 +54,9 @@ SIGNATURES = {
     "cfp8_gemm_grouped_swiglu_quant": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p,
                                                c_int64, c_int64, c_int64, c_int64, c_void_p]),
     "cfp8_generate_permute_indices": (c_int, [c_void_p, c_int, c_int, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "cfp8_route_tokens_workspace_bytes": (c_size_t, [c_int64, c_int, c_int]),
+    "cfp8_route_tokens": (c_int, [c_void_p, c_int, c_void_p, c_int64, c_int, c_int, c_int64, c_int, c_int64, c_void_p, c_void_p, c_void_p, c_void_p,
+                                  c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
     "cfp8_gather_rows": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_void_p]),
     "cfp8_combine_rows": (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int, c_int64, c_int, c_int64, c_int,
                                   c_void_p, c_int64, c_void_p]),

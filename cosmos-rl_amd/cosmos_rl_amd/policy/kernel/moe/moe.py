@@ -30,6 +30,30 @@ class TokenRouting:
     m_offsets: torch.Tensor    # int32 [experts]: their inclusive cumulative sum
 
 
+_ROUTE_MAX_EXPERTS = 1024  # what the tables of cfp8_route_tokens hold
+
+
+def _route_tokens_by_sorting(indices: torch.Tensor, token_mask: Optional[torch.Tensor], n_experts: int, alignment: int,
+                             capacity: int) -> TokenRouting:
+    """``route_tokens`` for more experts than the routing kernel's tables hold, from library calls."""
+    T, K = indices.shape
+    dev = indices.device
+    key = indices.to(torch.int64)
+    if token_mask is not None:
+        key = torch.where(token_mask.to(torch.bool).unsqueeze(-1), key, n_experts)
+    order = torch.argsort(key.reshape(-1), stable=True)
+    counts = torch.zeros(n_experts + 1, dtype=torch.int64, device=dev).scatter_add_(0, key.reshape(-1), torch.ones_like(order))[:n_experts]
+    permuted, m_sizes, m_offsets = generate_permute_indices(counts, n_experts, 1, alignment, max_len=capacity)
+    valid = permuted >= 0
+    pair = order[permuted.clamp_min(0).to(torch.int64)]
+    row_tokens = torch.where(valid, (pair // K).to(torch.int32), -1)
+    row_of = torch.full((T * K + 1,), -1, dtype=torch.int32, device=dev)   # the last entry catches the padding rows
+    row_of.scatter_(0, torch.where(valid, pair, T * K), torch.arange(capacity, dtype=torch.int32, device=dev))
+    slot_order = torch.sort(key, dim=1, stable=True)[1]
+    row_map = torch.gather(row_of[:T * K].view(T, K), 1, slot_order).contiguous()
+    return TokenRouting(row_tokens, row_map, slot_order, m_sizes, m_offsets)
+
+
 def route_tokens(indices: torch.Tensor, token_mask: Optional[torch.Tensor], n_experts: int, alignment: int = 128,
                  max_rows: Optional[int] = None) -> TokenRouting:
     """Expert-grouped layout of the routed (token, slot) pairs: groups in expert order, tokens ascending
@@ -40,24 +64,26 @@ def route_tokens(indices: torch.Tensor, token_mask: Optional[torch.Tensor], n_ex
         raise ValueError("indices must be a [tokens, topk] GPU tensor")
     T, K = indices.shape
     dev = indices.device
-    idx64 = indices.to(torch.int64)
-    if token_mask is not None:
-        idx64 = torch.where(token_mask.to(torch.bool).unsqueeze(-1), idx64, torch.full_like(idx64, n_experts))
-    key = idx64.reshape(-1)                                   # masked slots fall into a bin past the last expert
-    order = torch.argsort(key, stable=True)
-    # (torch.bincount reads its result size back from the device; a scatter-add does not, so this can be graph-captured)
-    counts = torch.zeros(n_experts + 1, dtype=torch.int64, device=dev).scatter_add_(0, key, torch.ones_like(key))[:n_experts]
     capacity = int(max_rows) if max_rows is not None else T * K + n_experts * alignment
-    permuted, m_sizes, m_offsets = generate_permute_indices(counts, n_experts, 1, alignment, max_len=capacity)
-    valid_row = permuted >= 0
-    src_slot = order[permuted.clamp_min(0).to(torch.int64)]  # flat (token, slot) behind every row
-    row_tokens = torch.where(valid_row, (src_slot // K).to(torch.int32), torch.full_like(permuted, -1))
-    row_of_slot = torch.full((T * K + 1,), -1, dtype=torch.int32, device=dev)
-    row_of_slot.scatter_(0, torch.where(valid_row, src_slot, torch.full_like(src_slot, T * K)),
-                         torch.arange(capacity, dtype=torch.int32, device=dev))
-    row_of_slot[T * K:].fill_(-1)                             # the slot that caught the padding rows
-    _, slot_order = torch.sort(idx64, dim=1, stable=True)
-    row_map = torch.gather(row_of_slot[:T * K].view(T, K), 1, slot_order).contiguous()
+    if n_experts > _ROUTE_MAX_EXPERTS:
+        return _route_tokens_by_sorting(indices, token_mask, n_experts, alignment, capacity)
+    if indices.dtype not in (torch.int32, torch.int64):
+        indices = indices.to(torch.int64)
+    indices = indices.contiguous()
+    if token_mask is not None:
+        token_mask = token_mask.to(torch.bool).contiguous()
+    lib = _lib.load()
+    row_tokens = torch.empty(capacity, dtype=torch.int32, device=dev)
+    row_map = torch.empty((T, K), dtype=torch.int32, device=dev)
+    slot_order = torch.empty((T, K), dtype=torch.int64, device=dev)
+    m_sizes = torch.empty(n_experts, dtype=torch.int32, device=dev)
+    m_offsets = torch.empty(n_experts, dtype=torch.int32, device=dev)
+    need = lib.cfp8_route_tokens_workspace_bytes(T, K, n_experts)
+    work = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
+    _lib.check(lib.cfp8_route_tokens(indices.data_ptr(), indices.element_size(), token_mask.data_ptr() if token_mask is not None else None, T, K,
+                                     n_experts, alignment, 1, capacity, row_tokens.data_ptr(), None, row_map.data_ptr(), slot_order.data_ptr(),
+                                     None, _lib.IN_BF16, None, m_sizes.data_ptr(), m_offsets.data_ptr(), work.data_ptr() if need else None, need,
+                                     torch.cuda.current_stream().cuda_stream))
     return TokenRouting(row_tokens, row_map, slot_order, m_sizes, m_offsets)
 
 

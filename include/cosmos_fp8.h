@@ -245,6 +245,23 @@ int cfp8_generate_permute_indices(const int64_t* tokens_per_expert_group, int ex
                                   int64_t capacity, int32_t* m_sizes, int32_t* m_offsets,
                                   int64_t* start_index_values, void* stream);
 
+/* Expert-grouped row layout of routed tokens from their expert indices (int32 or int64 [tokens, topk], index_bytes 4 or
+ * 8): the (token, slot) pairs sorted stably by expert, every group padded to a multiple of `alignment` rows (keep_empty:
+ * an expert without pairs still gets `alignment` rows; else none).  Pairs of a token whose token_mask byte is 0 (null:
+ * none), or whose index is not in [0, experts), go nowhere.  Outputs: row_tokens int32 [capacity] (token behind every
+ * row, -1 for padding and past the end; pairs whose row lies at or past capacity are dropped), row_experts int32
+ * [capacity] (or null: expert of every row of a group, its padding included, -1 past the end), row_map int32 [tokens,
+ * topk] (rows of a token by ascending expert, -1 for a pair that has none), slot_order int64 [tokens, topk] (or null: the
+ * slot behind every entry of row_map), sorted_weights bf16 [tokens, topk] (or null: weights[t, slot_order[t, :]], weights
+ * bf16 or fp32), m_sizes, m_offsets int32 [experts] (padded group sizes, inclusive cumulative sum).  At most 1024 experts.
+ * Workspace: cfp8_route_tokens_workspace_bytes (0 for few pairs).  One or two launches.
+ * Replaces the per-expert torch.where of GroupedExperts.forward, cosmos_rl/policy/kernel/moe/moe.py:240-263. */
+size_t cfp8_route_tokens_workspace_bytes(int64_t tokens, int topk, int experts);
+int cfp8_route_tokens(const void* indices, int index_bytes, const uint8_t* token_mask, int64_t tokens, int topk, int experts,
+                      int64_t alignment, int keep_empty, int64_t capacity, int32_t* row_tokens, int32_t* row_experts,
+                      int32_t* row_map, int64_t* slot_order, const void* weights, int weights_dtype, void* sorted_weights,
+                      int32_t* m_sizes, int32_t* m_offsets, void* workspace, size_t workspace_bytes, void* stream);
+
 /* out[i, :] = x[indices[i], :] for indices[i] >= 0, zeros for -1: the row gather that applies
  * permuted_indices to the token matrix (the reference indexes with torch:
  * cosmos_rl/policy/kernel/moe/moe.py token regrouping before group_gemms.py:152-156).
