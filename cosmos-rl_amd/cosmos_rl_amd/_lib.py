@@ -20,6 +20,9 @@ TENSORWISE_AMAX_SLOTS = 64
 TENSORWISE_STATIC_MAX_TENSORS = 512
 IN_BF16, IN_F16, IN_F32 = 0, 1, 2
 COMBINE_BF16_STEPS, COMBINE_F32 = 0, 1
+ROUTE_KEEP_EMPTY, ROUTE_END_NOT_PADDING = 1, 2
+ROUTE_MAX_EXPERTS = 1024
+SWIGLU_GEMM_MAX_K = 2048 * 64  # what the weight-scale table of the fused gate_up kernel holds
 
 EINVAL, EARCH, ELAUNCH, EWORKSPACE = -1, -2, -3, -4
 
@@ -57,6 +60,9 @@ SIGNATURES = {
     "cfp8_route_tokens_workspace_bytes": (c_size_t, [c_int64, c_int, c_int]),
     "cfp8_route_tokens": (c_int, [c_void_p, c_int, c_void_p, c_int64, c_int, c_int, c_int64, c_int, c_int64, c_void_p, c_void_p, c_void_p, c_void_p,
                                   c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
+    "cfp8_moe_experts_workspace_bytes": (c_size_t, [c_int64, c_int, c_int, c_int64, c_int64]),
+    "cfp8_moe_experts": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p,
+                                 c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_size_t, c_void_p]),
     "cfp8_gather_rows": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_void_p]),
     "cfp8_combine_rows": (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int, c_int64, c_int, c_int64, c_int,
                                   c_void_p, c_int64, c_void_p]),

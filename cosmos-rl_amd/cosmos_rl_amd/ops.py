@@ -637,6 +637,41 @@ def grouped_gemm_swiglu_quant(lhs: Tuple[torch.Tensor, torch.Tensor], rhs_interl
     return q, s
 
 
+def moe_experts(x: torch.Tensor, token_mask: Optional[torch.Tensor], weights: torch.Tensor, indices: torch.Tensor,
+                gate_up_interleaved: Tuple[torch.Tensor, torch.Tensor], down: Tuple[torch.Tensor, torch.Tensor]) -> torch.Tensor:
+    """The experts of one MoE layer on routed tokens in one library call (``GroupedExperts.forward`` on one rank,
+    cosmos_rl/policy/kernel/moe/moe.py:179-285): x bf16 [T, H], token_mask [T] or None, weights and indices [T, topk],
+    gate_up as ``interleave_gate_up`` gives it, down (fp8 [E, H, I], scales [E, H/128, I/128]).  Returns bf16 [T, H]."""
+    gu, gus = gate_up_interleaved
+    dn, dns = down
+    _need_gpu(x, weights, indices, gu, gus, dn, dns)
+    T, H = x.shape
+    E, N2, Kb = gu.shape
+    I = N2 // 2
+    topk = indices.shape[1]
+    if Kb != H or tuple(dn.shape) != (E, H, I) or weights.shape != indices.shape or indices.shape[0] != T:
+        raise ValueError("shape mismatch in MoE experts")
+    if tuple(gus.shape) != (E, N2 // BLOCK, H // BLOCK) or tuple(dns.shape) != (E, H // BLOCK, I // BLOCK):
+        raise ValueError("scale shape mismatch in MoE experts")
+    if indices.dtype not in (torch.int32, torch.int64):
+        indices = indices.to(torch.int64)
+    if weights.dtype not in (torch.bfloat16, torch.float32):
+        weights = weights.to(torch.bfloat16)
+    if token_mask is not None and token_mask.dtype != torch.bool:
+        token_mask = token_mask.to(torch.bool)
+    indices, weights, gu, gus, dn, dns = (t.contiguous() for t in (indices, weights, gu, gus, dn, dns))
+    mask = token_mask.contiguous() if token_mask is not None else None
+    y = torch.empty((T, H), dtype=torch.bfloat16, device=x.device)
+    lib = _lib.load()
+    need = lib.cfp8_moe_experts_workspace_bytes(T, topk, E, H, I)
+    work = torch.empty(max(need, 1), dtype=torch.uint8, device=x.device)
+    _lib.check(lib.cfp8_moe_experts(x.data_ptr(), x.stride(0) if T > 1 else H, T, H, indices.data_ptr(), indices.element_size(), _ptr(mask),
+                                    weights.data_ptr(), _lib.IN_F32 if weights.dtype == torch.float32 else _lib.IN_BF16, topk, E,
+                                    gu.data_ptr(), gus.data_ptr(), dn.data_ptr(), dns.data_ptr(), I, y.data_ptr(), H, work.data_ptr(), need,
+                                    _stream()))
+    return y
+
+
 def create_indices_from_offsets_nosync(m_offsets: torch.Tensor, total: Optional[int] = None,
                                        n_experts: Optional[int] = None) -> torch.Tensor:
     """``dsgemm_utils.create_indices_from_offsets_nosync`` (group_gemms.py:157): expert id per

@@ -147,6 +147,31 @@ class DSGroupGEMM(GroupGEMMStrategy):
         # (rows of row_map at or past `total` would be padding; the scatter form skips rows beyond its output)
         return self._run(permute_quantize_tokens(tokens, row_tokens[:total], row_map), m_indices, total, module, tokens.dtype)
 
+    def forward_experts(self, x, token_mask, weights, indices, module, n_experts):
+        """``grouped_experts_forward`` as one library call, or None where the configuration or the shapes need the
+        general chain: the fused gate_up form, bf16 tokens, sizes in multiples of 128."""
+        if not (self.fuse_gate_up and self.fuse_swiglu and self.fuse_epilogue) or x.dtype != torch.bfloat16 or not x.is_cuda:
+            return None
+        if x.dim() != 2 or indices.dim() != 2 or weights.shape != indices.shape or indices.shape[0] != x.shape[0]:
+            return None
+        inter, hidden = module.get_parameter("gate_proj_weight").shape[1], module.get_parameter("down_proj_weight").shape[1]
+        down_fp8, down_s = module.get_parameter("down_proj_fp8"), module.get_parameter("down_proj_scales")
+        if inter % ops.BLOCK or hidden % ops.BLOCK or hidden != x.shape[1] or indices.shape[1] > 64 or n_experts > _lib.ROUTE_MAX_EXPERTS:
+            return None
+        if x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16 or down_fp8.shape[0] != n_experts or hidden > _lib.SWIGLU_GEMM_MAX_K:
+            return None
+        return ops.moe_experts(x, token_mask, weights, indices, self._interleaved(module), (down_fp8, down_s))
+
+    def _interleaved(self, module):
+        gate_fp8, gate_s = module.get_parameter("gate_proj_fp8"), module.get_parameter("gate_proj_scales")
+        up_fp8, up_s = module.get_parameter("up_proj_fp8"), module.get_parameter("up_proj_scales")
+        key = self._weights_key(gate_fp8, up_fp8, gate_s, up_s)
+        inter = getattr(module, "_gate_up_fp8_interleaved", None)
+        if inter is None or inter[2] != key:
+            inter = (*ops.interleave_gate_up((gate_fp8, gate_s), (up_fp8, up_s)), key)
+            module._gate_up_fp8_interleaved = inter
+        return inter[0], inter[1]
+
     @staticmethod
     def _weights_key(*tensors):
         # address and in-place version of every tensor a fused copy was built from: an in-place update (copy_,
@@ -179,12 +204,7 @@ class DSGroupGEMM(GroupGEMMStrategy):
         # activation reads there is defined
         hidden_quantized = None
         if self.fuse_gate_up and self.fuse_swiglu and self.fuse_epilogue and intermediate_size % 128 == 0 and total % 128 == 0:
-            key = self._weights_key(gate_fp8, up_fp8, gate_s, up_s)
-            inter = getattr(module, "_gate_up_fp8_interleaved", None)
-            if inter is None or inter[2] != key:
-                inter = (*ops.interleave_gate_up((gate_fp8, gate_s), (up_fp8, up_s)), key)
-                module._gate_up_fp8_interleaved = inter
-            hidden_quantized = ops.grouped_gemm_swiglu_quant(gate_up_input, (inter[0], inter[1]), m_indices)
+            hidden_quantized = ops.grouped_gemm_swiglu_quant(gate_up_input, self._interleaved(module), m_indices)
         elif self.fuse_gate_up and intermediate_size % 128 == 0:
             key = self._weights_key(gate_fp8, up_fp8, gate_s, up_s)
             fused = getattr(module, "_gate_up_fp8_fused", None)

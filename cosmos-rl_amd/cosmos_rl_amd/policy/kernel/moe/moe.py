@@ -30,9 +30,6 @@ class TokenRouting:
     m_offsets: torch.Tensor    # int32 [experts]: their inclusive cumulative sum
 
 
-_ROUTE_MAX_EXPERTS = 1024  # what the tables of cfp8_route_tokens hold
-
-
 def _route_tokens_by_sorting(indices: torch.Tensor, token_mask: Optional[torch.Tensor], n_experts: int, alignment: int,
                              capacity: int) -> TokenRouting:
     """``route_tokens`` for more experts than the routing kernel's tables hold, from library calls."""
@@ -65,7 +62,7 @@ def route_tokens(indices: torch.Tensor, token_mask: Optional[torch.Tensor], n_ex
     T, K = indices.shape
     dev = indices.device
     capacity = int(max_rows) if max_rows is not None else T * K + n_experts * alignment
-    if n_experts > _ROUTE_MAX_EXPERTS:
+    if n_experts > _lib.ROUTE_MAX_EXPERTS:
         return _route_tokens_by_sorting(indices, token_mask, n_experts, alignment, capacity)
     if indices.dtype not in (torch.int32, torch.int64):
         indices = indices.to(torch.int64)
@@ -81,7 +78,7 @@ def route_tokens(indices: torch.Tensor, token_mask: Optional[torch.Tensor], n_ex
     need = lib.cfp8_route_tokens_workspace_bytes(T, K, n_experts)
     work = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
     _lib.check(lib.cfp8_route_tokens(indices.data_ptr(), indices.element_size(), token_mask.data_ptr() if token_mask is not None else None, T, K,
-                                     n_experts, alignment, 1, capacity, row_tokens.data_ptr(), None, row_map.data_ptr(), slot_order.data_ptr(),
+                                     n_experts, alignment, _lib.ROUTE_KEEP_EMPTY, capacity, row_tokens.data_ptr(), None, row_map.data_ptr(), slot_order.data_ptr(),
                                      None, _lib.IN_BF16, None, m_sizes.data_ptr(), m_offsets.data_ptr(), work.data_ptr() if need else None, need,
                                      torch.cuda.current_stream().cuda_stream))
     return TokenRouting(row_tokens, row_map, slot_order, m_sizes, m_offsets)
@@ -122,6 +119,10 @@ def grouped_experts_forward(x: torch.Tensor, token_mask: Optional[torch.Tensor],
                             indices: torch.Tensor, strategy, module, n_experts: int, alignment: int = 128) -> torch.Tensor:
     """``GroupedExperts.forward(x, token_mask, weights, indices)`` (moe.py:179-285) on one rank, with the
     experts of ``module`` run by ``strategy`` (a ``GroupGEMMStrategy``) instead of the per-expert loop."""
+    if hasattr(strategy, "forward_experts"):
+        y = strategy.forward_experts(x, token_mask, weights, indices, module, n_experts)
+        if y is not None:
+            return y
     routing = route_tokens(indices, token_mask, n_experts, alignment)
     if hasattr(strategy, "execute_from_tokens") and x.dtype == torch.bfloat16:
         # the FP8 strategy quantises while it gathers: the expert-grouped bf16 copy of the tokens is never built

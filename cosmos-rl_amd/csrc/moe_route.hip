@@ -38,7 +38,7 @@ struct RouteArgs {
     int32_t* m_offsets;       // [experts]
     int64_t pairs, capacity, alignment, chunk;
     int topk, experts, bits;
-    int idx64, w32, keep_empty;
+    int idx64, w32, flags;
 };
 
 // expert of a pair; `experts` for a pair that goes nowhere (masked token, index out of range)
@@ -102,7 +102,7 @@ __global__ __launch_bounds__(kRouteThreads) void route_place_kernel(const RouteA
         int64_t size = 0;
         if (t < E) {
             size = total[t];
-            if (p.keep_empty && size < p.alignment) size = p.alignment;
+            if ((p.flags & CFP8_ROUTE_KEEP_EMPTY) && size < p.alignment) size = p.alignment;
             size = (size + p.alignment - 1) / p.alignment * p.alignment;
         }
         int run = (int)size;
@@ -186,7 +186,7 @@ __global__ __launch_bounds__(kRouteThreads) void route_place_kernel(const RouteA
         }
     }
     for (int64_t r = (int64_t)ends[E - 1] + (int64_t)blockIdx.x * kRouteThreads + t; r < p.capacity; r += (int64_t)gridDim.x * kRouteThreads) {
-        p.row_tokens[r] = -1;
+        p.row_tokens[r] = (p.flags & CFP8_ROUTE_END_NOT_PADDING) ? 0x7FFFFFFF : -1;
         if (p.row_experts) p.row_experts[r] = -1;
     }
 }
@@ -206,7 +206,7 @@ extern "C" size_t cfp8_route_tokens_workspace_bytes(int64_t tokens, int topk, in
 }
 
 extern "C" int cfp8_route_tokens(const void* indices, int index_bytes, const uint8_t* token_mask, int64_t tokens, int topk, int experts,
-                                 int64_t alignment, int keep_empty, int64_t capacity, int32_t* row_tokens, int32_t* row_experts,
+                                 int64_t alignment, int flags, int64_t capacity, int32_t* row_tokens, int32_t* row_experts,
                                  int32_t* row_map, int64_t* slot_order, const void* weights, int weights_dtype, void* sorted_weights,
                                  int32_t* m_sizes, int32_t* m_offsets, void* workspace, size_t workspace_bytes, void* stream) {
     using namespace cfp8;
@@ -244,7 +244,7 @@ extern "C" int cfp8_route_tokens(const void* indices, int index_bytes, const uin
     p.bits = experts > 1 ? 32 - __builtin_clz((unsigned)experts - 1) : 0;
     p.idx64 = index_bytes == 8;
     p.w32 = weights_dtype == CFP8_IN_F32;
-    p.keep_empty = keep_empty;
+    p.flags = flags;
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int64_t blocks = route_blocks(p.pairs);
     const size_t lds = (size_t)kRouteWaves * ((experts + 1) & ~1) * sizeof(uint16_t);

@@ -246,19 +246,22 @@ int cfp8_generate_permute_indices(const int64_t* tokens_per_expert_group, int ex
                                   int64_t* start_index_values, void* stream);
 
 /* Expert-grouped row layout of routed tokens from their expert indices (int32 or int64 [tokens, topk], index_bytes 4 or
- * 8): the (token, slot) pairs sorted stably by expert, every group padded to a multiple of `alignment` rows (keep_empty:
- * an expert without pairs still gets `alignment` rows; else none).  Pairs of a token whose token_mask byte is 0 (null:
- * none), or whose index is not in [0, experts), go nowhere.  Outputs: row_tokens int32 [capacity] (token behind every
- * row, -1 for padding and past the end; pairs whose row lies at or past capacity are dropped), row_experts int32
- * [capacity] (or null: expert of every row of a group, its padding included, -1 past the end), row_map int32 [tokens,
- * topk] (rows of a token by ascending expert, -1 for a pair that has none), slot_order int64 [tokens, topk] (or null: the
- * slot behind every entry of row_map), sorted_weights bf16 [tokens, topk] (or null: weights[t, slot_order[t, :]], weights
- * bf16 or fp32), m_sizes, m_offsets int32 [experts] (padded group sizes, inclusive cumulative sum).  At most 1024 experts.
+ * 8): the (token, slot) pairs sorted stably by expert, every group padded to a multiple of `alignment` rows.  Pairs of a
+ * token whose token_mask byte is 0 (null: none), or whose index is not in [0, experts), go nowhere.  Outputs: row_tokens
+ * int32 [capacity] (token behind every row, -1 for padding and past the end; pairs whose row lies at or past capacity are
+ * dropped), row_experts int32 [capacity] (or null: expert of every row, -1 past the end), row_map int32 [tokens, topk]
+ * (rows of a token by ascending expert, -1 for a pair that has none), slot_order int64 [tokens, topk] (or null: the slot
+ * behind every entry of row_map), sorted_weights bf16 [tokens, topk] (or null: weights[t, slot_order[t, :]], weights bf16
+ * or fp32), m_sizes, m_offsets int32 [experts] (padded group sizes, inclusive cumulative sum).  At most 1024 experts.
+ * Flags: KEEP_EMPTY: an expert without pairs gets `alignment` rows of padding (else none); END_NOT_PADDING: row_tokens is
+ * INT32_MAX past the last group (else -1), so that cfp8_scatter_quant_group128 leaves those rows alone.
  * Workspace: cfp8_route_tokens_workspace_bytes (0 for few pairs).  One or two launches.
  * Replaces the per-expert torch.where of GroupedExperts.forward, cosmos_rl/policy/kernel/moe/moe.py:240-263. */
+#define CFP8_ROUTE_KEEP_EMPTY 1
+#define CFP8_ROUTE_END_NOT_PADDING 2
 size_t cfp8_route_tokens_workspace_bytes(int64_t tokens, int topk, int experts);
 int cfp8_route_tokens(const void* indices, int index_bytes, const uint8_t* token_mask, int64_t tokens, int topk, int experts,
-                      int64_t alignment, int keep_empty, int64_t capacity, int32_t* row_tokens, int32_t* row_experts,
+                      int64_t alignment, int flags, int64_t capacity, int32_t* row_tokens, int32_t* row_experts,
                       int32_t* row_map, int64_t* slot_order, const void* weights, int weights_dtype, void* sorted_weights,
                       int32_t* m_sizes, int32_t* m_offsets, void* workspace, size_t workspace_bytes, void* stream);
 
@@ -287,6 +290,20 @@ int cfp8_gather_rows(const void* x, int64_t ld_x_bytes, const int32_t* indices, 
 int cfp8_combine_rows(const void* rows, int64_t ld_rows, int64_t num_rows, const int32_t* row_map,
                       const void* weights, int weights_dtype, int64_t tokens, int topk, int64_t hidden,
                       int mode, void* out, int64_t ld_out, void* stream);
+
+/* GroupedExperts.forward of one rank as one call (cosmos_rl/policy/kernel/moe/moe.py:179-285 with the experts of
+ * cosmos_rl/policy/kernel/group_gemms.py:121-229): routing (cfp8_route_tokens), 1x128 quantisation of the tokens, gate_up
+ * product with SwiGLU and requantisation, down product, weighted sum in ascending order of experts with bf16 steps.
+ * x bf16 [tokens, hidden] (ld_x), indices and token_mask as cfp8_route_tokens, weights bf16 or fp32 [tokens, topk] (rounded
+ * to bf16), gate_up fp8 [experts, 2 inter, hidden] interleaved with scales [experts, 2 inter / 128, hidden / 128] as
+ * cfp8_gemm_grouped_swiglu_quant takes them, down fp8 [experts, hidden, inter] with scales [experts, hidden / 128,
+ * inter / 128], y bf16 [tokens, hidden] (ld_y): zero rows for tokens that go nowhere.  hidden, inter multiples of 128,
+ * topk <= 64, experts <= 1024.  The workspace is 256-byte aligned and belongs to the call until the stream has run it. */
+size_t cfp8_moe_experts_workspace_bytes(int64_t tokens, int topk, int experts, int64_t hidden, int64_t inter);
+int cfp8_moe_experts(const void* x, int64_t ld_x, int64_t tokens, int64_t hidden, const void* indices, int index_bytes,
+                     const uint8_t* token_mask, const void* weights, int weights_dtype, int topk, int experts,
+                     const void* gate_up, const float* gate_up_scales, const void* down, const float* down_scales, int64_t inter,
+                     void* y, int64_t ld_y, void* workspace, size_t workspace_bytes, void* stream);
 
 /* MXFP4 quantisation of bf16 rows: every block of 32 consecutive elements of a row gets one
  * e8m0 scale byte 2^ceil(log2(amax / 6)) and 32 e2m1 codes (round to nearest, ties away from zero),

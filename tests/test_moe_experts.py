@@ -1,0 +1,54 @@
+"""The one-call MoE experts (cfp8_moe_experts, what grouped_experts_forward runs for the FP8 strategy) against the chain of
+the separate entry points, each of which has its own test against the oracle."""
+import pytest
+import torch
+
+from cosmos_rl_amd import _lib, ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _module(dev, E, H, I, seed):
+    from cosmos_rl_amd.policy.kernel.group_gemms import DSGroupGEMM
+    g = torch.Generator(device=dev).manual_seed(seed)
+    strategy, module = DSGroupGEMM(torch.nn.SiLU(), fuse_gate_up=True), torch.nn.Module()
+    for name, rows, cols in (("gate_proj", I, H), ("up_proj", I, H), ("down_proj", H, I)):
+        w = (torch.randn(E, rows, cols, generator=g, device=dev) * 0.05).to(torch.bfloat16)
+        module.register_parameter(f"{name}_weight", torch.nn.Parameter(strategy.arrange_expert_weights(list(w), name, module), requires_grad=False))
+    return strategy, module
+
+
+def _chain(x, mask, w, idx, strategy, module, E):
+    from cosmos_rl_amd.policy.kernel.moe.moe import combine_expert_outputs, route_tokens
+    r = route_tokens(idx, mask, E)
+    return combine_expert_outputs(strategy.execute_from_tokens(x, r.row_tokens, r.m_sizes, r.m_offsets, module, row_map=r.row_map), r, w)
+
+
+@pytest.mark.parametrize("T,E,topk,H,I", [(1, 8, 2, 256, 128), (5, 4, 4, 128, 256), (40, 16, 8, 384, 128), (700, 7, 3, 1024, 768), (3300, 7, 2, 1152, 1024),
+                                          (200, 3, 1, 4224, 640), (130, 6, 2, 512, 1664),
+                                              (777, 64, 8, 1024, 896)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_one_call_experts(dev, T, E, topk, H, I, masked):
+    from cosmos_rl_amd.policy.kernel.moe.moe import grouped_experts_forward
+    strategy, module = _module(dev, E, H, I, T)
+    g = torch.Generator(device=dev).manual_seed(T + 1)
+    x = torch.randn(T, H, generator=g, device=dev).to(torch.bfloat16)
+    idx = torch.rand(T, E, generator=g, device=dev).topk(topk, dim=1).indices
+    w = torch.rand(T, topk, generator=g, device=dev)
+    mask = (torch.rand(T, generator=g, device=dev) < 0.7) if masked else None
+    for wt, it in ((torch.bfloat16, torch.int64), (torch.float32, torch.int32)):
+        junk = torch.full((64 << 20,), 0x7F, dtype=torch.uint8, device=dev)   # what the workspace holds before is no number
+        del junk
+        y = grouped_experts_forward(x, mask, w.to(wt), idx.to(it), strategy, module, E)
+        want = _chain(x, mask, w.to(torch.bfloat16), idx, strategy, module, E)
+        assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+    if masked:
+        assert not bool(y[~mask].any())
+
+
+def test_one_call_experts_refuses_a_small_workspace(dev):
+    t = torch.zeros(256, 256, device=dev, dtype=torch.bfloat16)
+    need = _lib.load().cfp8_moe_experts_workspace_bytes(4, 2, 2, 256, 128)
+    args = lambda n: _lib.load().cfp8_moe_experts(t.data_ptr(), 256, 4, 256, t.data_ptr(), 8, None, t.data_ptr(), 0, 2, 2, t.data_ptr(), t.data_ptr(),
+                                                  t.data_ptr(), t.data_ptr(), 128, t.data_ptr(), 256, t.data_ptr(), n, None)
+    assert need > 0 and args(need - 1) == _lib.EWORKSPACE

@@ -57,7 +57,7 @@ def test_route_tokens(dev, T, K, E, alignment, distinct, short, keep_empty):
         so = torch.full((T, K), 77, dtype=torch.int64, device=dev)
         sw = torch.zeros(T, K, dtype=torch.bfloat16, device=dev)
         ws = torch.empty(max(need, 1), dtype=torch.uint8, device=dev)
-        _lib.check(lib.cfp8_route_tokens(ind.data_ptr(), ind.element_size(), mk.data_ptr(), T, K, E, alignment, int(keep_empty), capacity, rt.data_ptr(),
+        _lib.check(lib.cfp8_route_tokens(ind.data_ptr(), ind.element_size(), mk.data_ptr(), T, K, E, alignment, _lib.ROUTE_KEEP_EMPTY if keep_empty else 0, capacity, rt.data_ptr(),
                                          re.data_ptr(), rm.data_ptr(), so.data_ptr(), wd.data_ptr(),
                                          _lib.IN_BF16 if wt == torch.bfloat16 else _lib.IN_F32, sw.data_ptr(), ms.data_ptr(), mo.data_ptr(),
                                          ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream))
