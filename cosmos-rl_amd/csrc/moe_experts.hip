@@ -1,27 +1,234 @@
 // The experts of one MoE layer on routed tokens as one call: routing, 1x128 quantisation of the tokens, the gate_up product
 // with SwiGLU, the down product and the weighted sum over each token's experts - launches only, on caller memory.
 //
-// Every expert's rows are padded to tiles of 128 (experts without a row get none), the tokens quantised into that layout
-// (cfp8_scatter_quant_group128) and multiplied by the grouped GEMMs of the training path.  A group's rows of padding are
-// zeros all the way: a walking GEMM carries a row's last products into the first step of its next tile with a scale of
-// zero, so what multiplies there must be finite.  Rows past the last group are not touched, neither by the quantiser nor
-// as a zero-filled output of the down product (at 8192 tokens of 2048, top 8 of 128 experts: 42 us of zeros), and the
-// routing's row experts and sorted weights spare seven launches that derived them: 250 -> 230 us at 777 tokens,
-// 669 -> 577 us at 8192.
+// Two forms, by the mean number of rows an expert gets:
+//
+//   many rows   Every expert's rows are padded to tiles of 128 (experts without a row get none), the tokens quantised into
+//               that layout (cfp8_scatter_quant_group128) and multiplied by the grouped GEMMs of the training path.  A
+//               group's rows of padding are zeros all the way: a walking GEMM carries a row's last products into the first
+//               step of its next tile with a scale of zero, so what multiplies there must be finite.  Rows past the last
+//               group are not touched.
+//   few rows    A decode batch: reading the weights of the experts that have a row is all the time there is, and tiles of
+//               128 rows would hold one or two.  Rows lie one behind the other without padding; a workgroup takes a strip
+//               of ONE expert's weight rows, requests all of its K into registers before anything else, and then walks
+//               the expert's rows in tiles of 16 (few_gate_up_kernel, few_down_kernel).
 #include "cfp8_common.h"
 
 namespace cfp8 {
 
+struct FewArgs {
+    const uint8_t* xq;       // [tokens, hidden] fp8
+    const float* xs;         // [tokens, hidden / 128]
+    const uint8_t* w;        // gate_up [experts, 2 inter, hidden] interleaved, or down [experts, hidden, inter]
+    const float* ws;
+    const int32_t* row_tokens;
+    const int32_t* sizes;    // rows of every expert, and their inclusive cumulative sum
+    const int32_t* ends;
+    uint16_t* h;             // [rows, inter] bf16
+    uint16_t* out;           // [rows, hidden] bf16
+    int experts, hidden, inter;
+};
+
+// The slot-th expert that has rows (-1: there are fewer), and its rows.
+__device__ __forceinline__ int few_expert(const FewArgs& p, int slot, int lane, int& start, int& end) {
+    for (int e0 = 0; e0 < p.experts; e0 += 64) {
+        const int n = e0 + lane < p.experts ? p.sizes[e0 + lane] : 0;
+        const uint64_t has = __ballot(n > 0);
+        const int c = __popcll(has);
+        if (slot < c) {
+            const uint64_t mine = __ballot(n > 0 && __popcll(has & ((1ull << lane) - 1)) == slot);
+            const int bit = __ffsll((unsigned long long)mine) - 1;
+            end = p.ends[e0 + bit];
+            start = end - __builtin_amdgcn_readlane(n, bit);
+            return e0 + bit;
+        }
+        slot -= c;
+    }
+    return -1;
+}
+
+__device__ __forceinline__ i32x8 few_frag(const u32x4& lo, const u32x4& hi) {
+    return i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
+}
+
+// ---------------------------------------------------------------------------
+// gate_up and SwiGLU.  A workgroup of four waves: 16 gate rows and the 16 up rows of the same features (neighbours in the
+// interleaved weight); wave w takes K steps w, w + 4, ... (NI of them), all of whose weights it requests at once.  A lane
+// reads bytes 16 q .. 16 q + 15 and 64 + 16 q .. of a K step (q = lane >> 4) of both operands: which K positions a lane
+// holds is free as long as both operands agree, and this way a load takes 64 contiguous bytes of each of 16 rows.
+// (Cacheable loads: 55 -> 49 us for the 258 MB of 16 tokens' experts against streaming ones, 2048 x 768; with four waves
+// a SIMD 47 us = 5.5 TB/s, 69 us = 5.8 TB/s once every expert has a row.)  The four waves' sums meet in LDS; h = bf16(bf16(silu(gate)) * up) leaves as bf16, since a 1x128 group of it is spread
+// over eight workgroups.
+// ---------------------------------------------------------------------------
+template <int NI>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NI <= 4 ? 4 : 2))) void few_gate_up_kernel(const FewArgs p) {
+    __shared__ __attribute__((aligned(16))) f32x4 red[2][4][2][64];
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int lrow = lane & 15, quarter = lane >> 4;
+    const int KT = p.hidden >> 7, strip = blockIdx.x;
+    int start, end;
+    const int e = few_expert(p, (int)blockIdx.y, lane, start, end);
+    if (e < 0) return;
+    const uint8_t* const wg = p.w + ((int64_t)e * 2 * p.inter + strip * 32 + lrow) * p.hidden + quarter * 16;
+    const uint8_t* const wu = wg + (int64_t)16 * p.hidden;
+    u32x4 w[NI][4];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int kt = wave + 4 * i < KT ? wave + 4 * i : KT - 1;
+        w[i][0] = *reinterpret_cast<const u32x4*>(wg + (kt << 7));
+        w[i][1] = *reinterpret_cast<const u32x4*>(wg + (kt << 7) + 64);
+        w[i][2] = *reinterpret_cast<const u32x4*>(wu + (kt << 7));
+        w[i][3] = *reinterpret_cast<const u32x4*>(wu + (kt << 7) + 64);
+    }
+    float sg[NI], su[NI];
+    const float* const sp = p.ws + ((int64_t)e * (p.inter >> 6) + 2 * (strip >> 3)) * KT;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int kt = wave + 4 * i < KT ? wave + 4 * i : KT - 1;
+        sg[i] = sp[kt];
+        su[i] = sp[KT + kt];
+    }
+    int turn = 0;
+    for (int r0 = start; r0 < end; r0 += 16, turn ^= 1) {
+        const int row = r0 + lrow;
+        const int64_t token = p.row_tokens[row < end ? row : end - 1];
+        const uint8_t* const xp = p.xq + token * p.hidden + quarter * 16;
+        const float* const xsp = p.xs + token * KT;
+        u32x4 x[NI][2];
+        float xs[NI];
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int kt = wave + 4 * i < KT ? wave + 4 * i : KT - 1;
+            x[i][0] = *reinterpret_cast<const u32x4*>(xp + (kt << 7));
+            x[i][1] = *reinterpret_cast<const u32x4*>(xp + (kt << 7) + 64);
+            xs[i] = xsp[kt];
+        }
+        f32x4 g = {0.f, 0.f, 0.f, 0.f}, u = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            if (i == NI - 1 && wave + 4 * i >= KT) continue;
+            const i32x8 xf = few_frag(x[i][0], x[i][1]);
+            const f32x4 pg = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(few_frag(w[i][0], w[i][1]), xf, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
+            const f32x4 pu = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(few_frag(w[i][2], w[i][3]), xf, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
+            const float fg = xs[i] * sg[i], fu = xs[i] * su[i];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                g[k] = __builtin_fmaf(pg[k], fg, g[k]);
+                u[k] = __builtin_fmaf(pu[k], fu, u[k]);
+            }
+        }
+        red[turn][wave][0][lane] = g;
+        red[turn][wave][1][lane] = u;
+        // one barrier a tile: the buffer written two tiles on has been read before its writers pass the next barrier
+        __syncthreads();
+        if (wave == ((r0 - start) >> 4 & 3) && row < end) {
+#pragma unroll
+            for (int v = 1; v < 4; ++v) {
+                const f32x4 og = red[turn][(wave + v) & 3][0][lane], ou = red[turn][(wave + v) & 3][1][lane];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) g[k] += og[k], u[k] += ou[k];
+            }
+            u32 h0, h1;
+            swiglu_quad(pack_bf16x2(g[0], g[1]), pack_bf16x2(g[2], g[3]), pack_bf16x2(u[0], u[1]), pack_bf16x2(u[2], u[3]), h0, h1);
+            *reinterpret_cast<uint2*>(p.h + (int64_t)row * p.inter + strip * 16 + quarter * 4) = make_uint2(h0, h1);
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// down.  A workgroup of eight waves: 128 weight rows, 16 a wave over the whole of K (NI = inter / 128 steps), all requested
+// at once; under those loads the workgroup quantises 16 rows of h (1x128, as the quantiser does) into LDS.  27 us for the
+// 129 MB of 16 tokens' experts (2048 x 768), 39 us for all 201 MB; the grouped GEMM on tiles of 128 rows took 68 us.
+// ---------------------------------------------------------------------------
+template <int NI>
+__global__ __launch_bounds__(512) void few_down_kernel(const FewArgs p) {
+    constexpr int PITCH = NI * 128 + 16;
+    __shared__ __attribute__((aligned(16))) uint8_t q[2][16 * PITCH];
+    __shared__ float qs[2][16][NI];
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int lrow = lane & 15, quarter = lane >> 4;
+    int start, end;
+    const int e = few_expert(p, (int)blockIdx.y, lane, start, end);
+    if (e < 0) return;
+    const int n0 = (int)blockIdx.x * 128 + wave * 16;
+    const uint8_t* const wp = p.w + ((int64_t)e * p.hidden + n0 + lrow) * p.inter + quarter * 16;
+    u32x4 w[NI][2];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        w[i][0] = *reinterpret_cast<const u32x4*>(wp + (i << 7));
+        w[i][1] = *reinterpret_cast<const u32x4*>(wp + (i << 7) + 64);
+    }
+    float sw[NI];
+    const float* const sp = p.ws + ((int64_t)e * (p.hidden >> 7) + blockIdx.x) * NI;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) sw[i] = sp[i];
+    int turn = 0;
+    for (int r0 = start; r0 < end; r0 += 16, turn ^= 1) {
+        const int rows = end - r0 < 16 ? end - r0 : 16;
+        for (int g = t >> 4; g < rows * NI; g += 32) {
+            const int r = g / NI, c = g - r * NI, sub = t & 15;
+            const uint4 v = *reinterpret_cast<const uint4*>(p.h + (int64_t)(r0 + r) * p.inter + c * 128 + sub * 8);
+            const float scale = scale_from_amax(amax_from_bits(row16_max(pk_fold(absmax8(0u, v)))));
+            *reinterpret_cast<uint2*>(&q[turn][r * PITCH + c * 128 + sub * 8]) = cast8(v, Divider(scale));
+            if (sub == 0) qs[turn][r][c] = scale;
+        }
+        __syncthreads();
+        const int rr = lrow < rows ? lrow : rows - 1;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const u32x4 lo = *reinterpret_cast<const u32x4*>(&q[turn][rr * PITCH + i * 128 + quarter * 16]);
+            const u32x4 hi = *reinterpret_cast<const u32x4*>(&q[turn][rr * PITCH + i * 128 + 64 + quarter * 16]);
+            const f32x4 pr = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(few_frag(w[i][0], w[i][1]), few_frag(lo, hi), f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
+            const float f = qs[turn][rr][i] * sw[i];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) acc[k] = __builtin_fmaf(pr[k], f, acc[k]);
+        }
+        if (lrow < rows)
+            *reinterpret_cast<uint2*>(p.out + (int64_t)(r0 + lrow) * p.hidden + n0 + quarter * 4) =
+                make_uint2(pack_bf16x2(acc[0], acc[1]), pack_bf16x2(acc[2], acc[3]));
+    }
+}
+
+template <int NI>
+static void launch_few_gate_up(int ni, dim3 grid, hipStream_t st, const FewArgs& p) {
+    if constexpr (NI > 0) {
+        if (ni == NI) hipLaunchKernelGGL(few_gate_up_kernel<NI>, grid, dim3(256), 0, st, p);
+        else launch_few_gate_up<NI - 1>(ni, grid, st, p);
+    }
+}
+template <int NI>
+static void launch_few_down(int ni, dim3 grid, hipStream_t st, const FewArgs& p) {
+    if constexpr (NI > 0) {
+        if (ni == NI) hipLaunchKernelGGL(few_down_kernel<NI>, grid, dim3(512), 0, st, p);
+        else launch_few_down<NI - 1>(ni, grid, st, p);
+    }
+}
+
+// The few-rows form holds a strip's whole K in registers: up to 8 K steps a wave of four (gate_up), 12 a wave (down).
+constexpr int64_t kFewMaxHidden = 4096, kFewMaxInter = 1536;
+// Up to this many activation elements an expert (rows x hidden) the weights bound the few-rows form and it is ahead; beyond,
+// every strip's workgroup reading all of its expert's rows does.  Whole calls, few against many rows: 128 experts of 2048 x
+// 768, top 8: 16 tokens 92 / 153 us, 128: 135 / 212, 512: 200 / 214, 640: 219 / 214, 1024: 283 / 227; 32 experts of 3584 x
+// 1536, top 4: 16 tokens 112 / 152, 128: 153 / 161, 256: 196 / 172; 64 experts of 1024 x 512, top 6: 64 tokens 40 / 76,
+// 640: 73 / 81, 1024: 91 / 81.
+constexpr int64_t kFewElementsPerExpert = 72 * 1024;
+
 struct ExpertsPlan {
-    int64_t rows;  // rows of the expert-grouped layout (their bound)
+    bool few;
+    int64_t rows;   // rows of the expert-grouped layout (their bound)
+    int64_t slots;  // experts that can have a row
     size_t row_tokens, row_experts, row_map, weights, m_sizes, m_offsets, route, xq, xs, h, hs, out, bytes;
 };
 
 static ExpertsPlan experts_plan(int64_t tokens, int topk, int experts, int64_t hidden, int64_t inter) {
     ExpertsPlan p{};
     const int64_t pairs = tokens * topk;
-    const int64_t touched = pairs < experts ? pairs : experts;
-    p.rows = (pairs + touched * 127) / 128 * 128;
+    p.few = pairs * hidden <= kFewElementsPerExpert * experts && hidden <= kFewMaxHidden && inter <= kFewMaxInter;
+    p.slots = pairs < experts ? pairs : experts;
+    p.rows = p.few ? pairs : (pairs + p.slots * 127) / 128 * 128;
     size_t at = 0;
     auto take = [&](size_t bytes) {
         const size_t here = at;
@@ -29,16 +236,17 @@ static ExpertsPlan experts_plan(int64_t tokens, int topk, int experts, int64_t h
         return here;
     };
     p.row_tokens = take((size_t)p.rows * 4);
-    p.row_experts = take((size_t)p.rows * 4);
+    p.row_experts = take(p.few ? 0 : (size_t)p.rows * 4);
     p.row_map = take((size_t)pairs * 4);
     p.weights = take((size_t)pairs * 2);
     p.m_sizes = take((size_t)experts * 4);
     p.m_offsets = take((size_t)experts * 4);
     p.route = take(cfp8_route_tokens_workspace_bytes(tokens, topk, experts));
-    p.xq = take((size_t)p.rows * (size_t)hidden);
-    p.xs = take((size_t)p.rows * (size_t)(hidden / 128) * 4);
-    p.h = take((size_t)p.rows * (size_t)inter);
-    p.hs = take((size_t)p.rows * (size_t)(inter / 128) * 4);
+    const size_t xrows = (size_t)(p.few ? tokens : p.rows);
+    p.xq = take(xrows * (size_t)hidden);
+    p.xs = take(xrows * (size_t)(hidden / 128) * 4);
+    p.h = take((size_t)p.rows * (size_t)inter * (p.few ? 2 : 1));
+    p.hs = take(p.few ? 0 : (size_t)p.rows * (size_t)(inter / 128) * 4);
     p.out = take((size_t)p.rows * (size_t)hidden * 2);
     p.bytes = at;
     return p;
@@ -73,18 +281,41 @@ extern "C" int cfp8_moe_experts(const void* x, int64_t ld_x, int64_t tokens, int
     auto i32 = [&](size_t at) { return reinterpret_cast<int32_t*>(ws + at); };
     auto f32 = [&](size_t at) { return reinterpret_cast<float*>(ws + at); };
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (int rc = cfp8_route_tokens(indices, index_bytes, token_mask, tokens, topk, experts, 128, CFP8_ROUTE_END_NOT_PADDING, p.rows,
-                                   i32(p.row_tokens), i32(p.row_experts), i32(p.row_map), nullptr, weights, weights_dtype, ws + p.weights,
-                                   i32(p.m_sizes), i32(p.m_offsets), ws + p.route, cfp8_route_tokens_workspace_bytes(tokens, topk, experts), stream))
+    if (int rc = cfp8_route_tokens(indices, index_bytes, token_mask, tokens, topk, experts, p.few ? 1 : 128, CFP8_ROUTE_END_NOT_PADDING, p.rows,
+                                   i32(p.row_tokens), p.few ? nullptr : i32(p.row_experts), i32(p.row_map), nullptr, weights, weights_dtype,
+                                   ws + p.weights, i32(p.m_sizes), i32(p.m_offsets), ws + p.route,
+                                   cfp8_route_tokens_workspace_bytes(tokens, topk, experts), stream))
         return rc;
-    if (int rc = cfp8_scatter_quant_group128(x, ld_x, tokens, hidden, i32(p.row_map), topk, i32(p.row_tokens), p.rows, ws + p.xq, hidden, f32(p.xs), stream))
-        return rc;
-    if (int rc = cfp8_gemm_grouped_swiglu_quant(ws + p.xq, hidden, f32(p.xs), gate_up, gate_up_scales, i32(p.row_experts), ws + p.h, inter,
-                                                f32(p.hs), p.rows, inter, hidden, experts, stream))
-        return rc;
-    if (int rc = cfp8_gemm_grouped_block128(ws + p.h, inter, f32(p.hs), down, down_scales, i32(p.row_experts), ws + p.out, hidden, CFP8_OUT_BF16,
-                                            p.rows, hidden, inter, experts, stream))
-        return rc;
+    if (p.few) {
+        if (int rc = cfp8_quant_group128(x, tokens, hidden, ld_x, ws + p.xq, hidden, f32(p.xs), CFP8_GROUP_MODE_DIV, stream)) return rc;
+        FewArgs f{};
+        f.xq = ws + p.xq;
+        f.xs = f32(p.xs);
+        f.w = static_cast<const uint8_t*>(gate_up);
+        f.ws = gate_up_scales;
+        f.row_tokens = i32(p.row_tokens);
+        f.sizes = i32(p.m_sizes);
+        f.ends = i32(p.m_offsets);
+        f.h = reinterpret_cast<uint16_t*>(ws + p.h);
+        f.out = reinterpret_cast<uint16_t*>(ws + p.out);
+        f.experts = experts;
+        f.hidden = (int)hidden;
+        f.inter = (int)inter;
+        launch_few_gate_up<(int)(kFewMaxHidden / 512)>((int)((hidden / 128 + 3) / 4), dim3((unsigned)(inter / 16), (unsigned)p.slots), st, f);
+        f.w = static_cast<const uint8_t*>(down);
+        f.ws = down_scales;
+        launch_few_down<(int)(kFewMaxInter / 128)>((int)(inter / 128), dim3((unsigned)(hidden / 128), (unsigned)p.slots), st, f);
+        if (int rc = check_launch("moe_experts")) return rc;
+    } else {
+        if (int rc = cfp8_scatter_quant_group128(x, ld_x, tokens, hidden, i32(p.row_map), topk, i32(p.row_tokens), p.rows, ws + p.xq, hidden, f32(p.xs), stream))
+            return rc;
+        if (int rc = cfp8_gemm_grouped_swiglu_quant(ws + p.xq, hidden, f32(p.xs), gate_up, gate_up_scales, i32(p.row_experts), ws + p.h, inter,
+                                                    f32(p.hs), p.rows, inter, hidden, experts, stream))
+            return rc;
+        if (int rc = cfp8_gemm_grouped_block128(ws + p.h, inter, f32(p.hs), down, down_scales, i32(p.row_experts), ws + p.out, hidden, CFP8_OUT_BF16,
+                                                p.rows, hidden, inter, experts, stream))
+            return rc;
+    }
     return cfp8_combine_rows(ws + p.out, hidden, p.rows, i32(p.row_map), ws + p.weights, CFP8_IN_BF16, tokens, topk, hidden,
                              CFP8_COMBINE_BF16_STEPS, y, ld_y, stream);
 }

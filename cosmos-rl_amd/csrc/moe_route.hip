@@ -19,9 +19,9 @@ namespace cfp8 {
 
 constexpr int kRouteThreads = 1024, kRouteWaves = kRouteThreads / 64;
 constexpr int kRouteMaxExperts = 1024;
-// Pairs up to which one workgroup does it all (its histogram included): at 4096 pairs four rounds of the placing loop
-// cost about what a second launch costs.
-constexpr int kRouteOneLaunchPairs = 4096;
+// Pairs up to which one workgroup does it all (its histogram included): one round of the placing loop, 8 us.  2048 pairs
+// take 14 us that way and 12 us in two launches.
+constexpr int kRouteOneLaunchPairs = 1024;
 constexpr int kRouteMaxBlocks = 128;
 
 struct RouteArgs {
