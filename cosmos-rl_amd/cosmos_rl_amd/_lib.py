@@ -69,6 +69,9 @@ SIGNATURES = {
     "cfp8_quant_mxfp4": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_void_p]),
     "cfp8_gemm_mxfp4": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64,
                                 c_int, c_int64, c_int64, c_int64, c_void_p]),
+    "cfp8_gemm_partial_bytes": (c_size_t, [c_int, c_int64, c_int64, c_int64]),
+    "cfp8_gemm_mxfp4_split": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_int, c_int64, c_int64,
+                                      c_int64, c_void_p, c_size_t, c_void_p]),
     "cfp8_linear_mxfp4": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_int, c_int64, c_int64, c_int64,
                                   c_void_p, c_size_t, c_void_p]),
     "cfp8_gather_quant_group128": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_void_p, c_void_p]),
@@ -110,7 +113,7 @@ def load() -> ctypes.CDLL:
     return lib
 
 
-DISPATCH_ROWWISE, DISPATCH_LINEAR, DISPATCH_BLOCK, DISPATCH_GROUPED, DISPATCH_GROUPED_SWIGLU = range(5)
+DISPATCH_ROWWISE, DISPATCH_LINEAR, DISPATCH_BLOCK, DISPATCH_GROUPED, DISPATCH_GROUPED_SWIGLU, DISPATCH_MXFP4 = range(6)
 
 
 def gemm_dispatch_info(kind: int, M: int, N: int, K: int, out_dtype: int = OUT_BF16, cus: int = 256,

@@ -371,6 +371,13 @@ def gemm_mxfp4(lhs: Tuple[torch.Tensor, torch.Tensor], rhs: Tuple[torch.Tensor, 
         out = torch.empty((M, N), dtype=out_dtype, device=a.device)
     elif tuple(out.shape) != (M, N) or not out.is_contiguous():
         raise ValueError("out must be a contiguous [M, N] tensor")
+    lib = _lib.load()
+    if not grouped:
+        need = lib.cfp8_gemm_partial_bytes(_lib.DISPATCH_MXFP4, M, N, K)
+        part = torch.empty(need, dtype=torch.uint8, device=a.device) if need else None
+        _lib.check(lib.cfp8_gemm_mxfp4_split(a.data_ptr(), K, sa.data_ptr(), w.data_ptr(), K // 2, ws.data_ptr(), K // 32, out.data_ptr(), N,
+                                             _out_code(out.dtype), M, N, K, _ptr(part), need, _stream()))
+        return out
     mi = 0
     if grouped:
         _need_gpu(m_indices)
@@ -378,8 +385,8 @@ def gemm_mxfp4(lhs: Tuple[torch.Tensor, torch.Tensor], rhs: Tuple[torch.Tensor, 
             raise ValueError("m_indices must have one entry per row")
         m_indices = m_indices.to(torch.int32).contiguous()
         mi = m_indices.data_ptr()
-    _lib.check(_lib.load().cfp8_gemm_mxfp4(a.data_ptr(), K, sa.data_ptr(), w.data_ptr(), K // 2, ws.data_ptr(), K // 32,
-                                          mi, E if grouped else 0, out.data_ptr(), N, _out_code(out.dtype), M, N, K, _stream()))
+    _lib.check(lib.cfp8_gemm_mxfp4(a.data_ptr(), K, sa.data_ptr(), w.data_ptr(), K // 2, ws.data_ptr(), K // 32,
+                                   mi, E, out.data_ptr(), N, _out_code(out.dtype), M, N, K, _stream()))
     return out
 
 
@@ -402,7 +409,7 @@ def linear_mxfp4(x: torch.Tensor, weight: Tuple[torch.Tensor, torch.Tensor],
     w, ws = w.contiguous(), ws.contiguous()
     out = torch.empty((M, N), dtype=out_dtype or x.dtype, device=x.device)
     lib = _lib.load()
-    wsb = lib.cfp8_linear_workspace_bytes(M, K)
+    wsb = lib.cfp8_linear_workspace_bytes(M, K) + lib.cfp8_gemm_partial_bytes(_lib.DISPATCH_MXFP4, M, N, K)
     work = torch.empty(max(wsb, 1), dtype=torch.uint8, device=x.device)
     ld_x = x2.stride(0) if M > 1 else K
     _lib.check(lib.cfp8_linear_mxfp4(x2.data_ptr(), ld_x, w.data_ptr(), K // 2, ws.data_ptr(), K // 32, out.data_ptr(), N,

@@ -27,6 +27,7 @@
 #include <atomic>
 
 #include "cfp8_common.h"
+#include "gemm_ring.h"
 
 namespace cfp8 {
 
@@ -1771,9 +1772,45 @@ static int launch_mx4(Mx4Args p, int out_dtype, hipStream_t st) {
 
 }  // namespace cfp8
 
-extern "C" int cfp8_gemm_mxfp4(const void* a, int64_t ld_a, const float* sa, const void* w, int64_t ld_w, const void* ws,
-                               int64_t ld_ws, const int32_t* m_indices, int64_t num_groups, void* out, int64_t ld_out,
-                               int out_dtype, int64_t M, int64_t N, int64_t K, void* stream) {
+namespace cfp8 {
+// What the tile kernels below the dispatch would take for M > 128 rows, in microseconds: rounds of tiles on the CUs (a
+// partial round of one-tile workgroups costs less than a whole one) times K steps, fitted to 35 timed shapes.  Infinite
+// where only the register-staged tiles would be left, which the ring kernel beats everywhere.
+static double mx4_tiles_cost(int64_t M, int64_t N, int64_t K, bool aligned256, int cus) {
+    const double kt = (double)((K + 127) / 128);
+    auto rounds = [&](int64_t tiles) {
+        const int64_t full = tiles / cus, rem = tiles % cus;
+        return full == 0 ? 1.0 : (double)full + (rem ? 0.5 + 0.5 * (double)rem / cus : 0.0);
+    };
+    const int64_t t256 = (M + 127) / 128 * ((N + 255) / 256), t512 = (M + 127) / 128 * ((N + 511) / 512);
+    if (aligned256 && (M / 256) * (N / 256) >= 128) return 4.0 + rounds((M / 256) * (N / 256)) * (kt * 1.3 + 3.0);
+    if (t512 >= 256 && (N + 511) / 512 * 512 - N <= N / 8) return 4.0 + rounds(t512) * (kt * 1.85 + 1.5);
+    if (t256 >= 64) return 4.0 + rounds(t256) * (kt * (0.6 + 0.3 * (t256 < cus ? (double)t256 / cus : 1.0)) + 1.0);
+    return 1e30;
+}
+
+// One product, ungrouped, with partial sums' memory or none: the ring kernel or the tile kernels.
+static int gemm_mx4_dense(Mx4Args& p, float* partial, size_t partial_bytes, int out_dtype, hipStream_t st, bool& taken) {
+    taken = false;
+    RingArgs r{};
+    r.a = p.a; r.w = p.w; r.ws = p.ws; r.sa = p.sa; r.out = p.out; r.partial = partial;
+    r.ld_a = p.ld_a; r.ld_w = p.ld_w; r.ld_ws = p.ld_ws; r.ld_out = p.ld_out;
+    r.M = p.M; r.N = p.N; r.K = p.K;
+    // (up to 4 tokens of K <= 4096 cfp8_linear_mxfp4 is one launch, whose bits the kernel for 16 tokens gives)
+    if ((p.M <= 4 && p.K <= 4096) || !ring_takes(kRingMx, r, out_dtype)) return CFP8_OK;
+    const RingPlan plan = ring_plan(kRingMx, p.M, p.N, p.K, partial_bytes, mx4_cu_count());
+    if (p.M > 128) {
+        const bool aligned256 = p.M % 256 == 0 && p.N % 256 == 0 && p.K % 128 == 0 && p.ld_ws % 4 == 0 && (reinterpret_cast<uintptr_t>(p.ws) & 3u) == 0;
+        if (mx4_tiles_cost(p.M, p.N, p.K, aligned256, mx4_cu_count()) <= plan.cost) return CFP8_OK;
+    }
+    taken = true;
+    return launch_ring(kRingMx, r, plan, out_dtype, st);
+}
+}  // namespace cfp8
+
+static int gemm_mxfp4_in(const void* a, int64_t ld_a, const float* sa, const void* w, int64_t ld_w, const void* ws,
+                         int64_t ld_ws, const int32_t* m_indices, int64_t num_groups, void* out, int64_t ld_out,
+                         int out_dtype, int64_t M, int64_t N, int64_t K, float* partial, size_t partial_bytes, void* stream) {
     using namespace cfp8;
     if (M < 0 || N < 0 || K < 0 || num_groups < 0) return set_error(CFP8_EINVAL, "gemm_mxfp4: negative shape");
     if (out_dtype != CFP8_OUT_BF16 && out_dtype != CFP8_OUT_F32) return set_error(CFP8_EINVAL, "gemm_mxfp4: out_dtype must be CFP8_OUT_BF16 or CFP8_OUT_F32");
@@ -1803,6 +1840,11 @@ extern "C" int cfp8_gemm_mxfp4(const void* a, int64_t ld_a, const float* sa, con
     p.ld_a = ld_a; p.ld_w = ld_w; p.ld_ws = ld_ws; p.ld_out = ld_out;
     p.M = (int)M; p.N = (int)N; p.K = (int)K;
     hipStream_t st = static_cast<hipStream_t>(stream);
+    if (!m_indices) {
+        bool taken = false;
+        const int rc = gemm_mx4_dense(p, partial, partial_bytes, out_dtype, st, taken);
+        if (rc || taken) return rc;
+    }
     if (M <= 16 && !m_indices) return launch_mx4_gemv(p, out_dtype, st);
     if (M <= 16) return launch_mx4<16, 64, 1, 4, 2>(p, out_dtype, st);
     // 17..128 tokens on a wide weight: the strip kernel (a narrow weight leaves most CUs without a strip)
@@ -1846,6 +1888,20 @@ extern "C" int cfp8_gemm_mxfp4(const void* a, int64_t ld_a, const float* sa, con
     return launch_mx4<128, 128, 2, 2, 1>(p, out_dtype, st);
 }
 
+extern "C" int cfp8_gemm_mxfp4(const void* a, int64_t ld_a, const float* sa, const void* w, int64_t ld_w, const void* ws,
+                               int64_t ld_ws, const int32_t* m_indices, int64_t num_groups, void* out, int64_t ld_out,
+                               int out_dtype, int64_t M, int64_t N, int64_t K, void* stream) {
+    return gemm_mxfp4_in(a, ld_a, sa, w, ld_w, ws, ld_ws, m_indices, num_groups, out, ld_out, out_dtype, M, N, K, nullptr, 0, stream);
+}
+
+extern "C" int cfp8_gemm_mxfp4_split(const void* a, int64_t ld_a, const float* sa, const void* w, int64_t ld_w, const void* ws,
+                                     int64_t ld_ws, void* out, int64_t ld_out, int out_dtype, int64_t M, int64_t N, int64_t K,
+                                     void* workspace, size_t workspace_bytes, void* stream) {
+    if (workspace_bytes && (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 255u)))
+        return cfp8::set_error(CFP8_EINVAL, "gemm_mxfp4_split: workspace must be 256-byte aligned");
+    return gemm_mxfp4_in(a, ld_a, sa, w, ld_w, ws, ld_ws, nullptr, 0, out, ld_out, out_dtype, M, N, K, static_cast<float*>(workspace), workspace_bytes,
+                         stream);
+}
 
 namespace cfp8 {
 // quant_rowwise.hip
@@ -1889,5 +1945,8 @@ extern "C" int cfp8_linear_mxfp4(const void* x, int64_t ld_x, const void* w, int
     float* sx = reinterpret_cast<float*>(qx + (((size_t)M * (size_t)K + 255) & ~(size_t)255));
     if (int rc = check_device()) return rc;
     if (int rc = launch_quant_rowwise(x, M, K, ld_x, qx, K, sx, false, st)) return rc;
-    return cfp8_gemm_mxfp4(qx, K, sx, w, ld_w, ws, ld_ws, nullptr, 0, out, ld_out, out_dtype, M, N, K, stream);
+    // what the workspace holds beyond the quantised activation is room for partial sums
+    const size_t base = cfp8_linear_workspace_bytes(M, K);
+    return gemm_mxfp4_in(qx, K, sx, w, ld_w, ws, ld_ws, nullptr, 0, out, ld_out, out_dtype, M, N, K,
+                         reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + base), workspace_bytes - base, stream);
 }

@@ -1,0 +1,32 @@
+// Interface of the ring GEMM (gemm_ring.hip) to the entry points.
+#pragma once
+
+#include "cfp8_common.h"
+
+namespace cfp8 {
+
+enum : int { kRingRow = 0, kRingBlock = 1, kRingMx = 2 };
+
+struct RingArgs {
+    const uint8_t* a;      // activations e4m3 [M, K]
+    const uint8_t* w;      // weights e4m3 [N, K], kRingMx: packed e2m1 [N, K / 2]
+    const uint8_t* ws;     // kRingMx: e8m0 [N, K / 32]
+    const float* sa;       // [M]; kRingBlock: [M, K / 128]
+    const float* sb;       // kRingRow: [N]; kRingBlock: see the strides
+    const uint16_t* bias;  // bf16 [N] or null
+    void* out;
+    float* partial;        // [slices, M, N] when slices > 1
+    int64_t ld_a, ld_w, ld_ws, ld_out, sb_stride_n, sb_stride_k;
+    int M, N, K;
+    int tiles_m, tiles_n, slices, slice_steps;
+};
+
+struct RingPlan {
+    int bm, bn, slices;
+    double cost;           // microseconds, estimated
+};
+RingPlan ring_plan(int mode, int64_t M, int64_t N, int64_t K, size_t partial_bytes, int cus);
+bool ring_takes(int mode, const RingArgs& p, int out_dtype);  // whether the operands fit what the kernel assumes
+int launch_ring(int mode, RingArgs& p, const RingPlan& plan, int out_dtype, hipStream_t st);
+
+}  // namespace cfp8

@@ -1,0 +1,507 @@
+// Ring GEMM: the middle of the range of token counts, where 256 x 256 tiles leave CUs idle or hold rows that do not
+// exist, and where a narrow weight with a long K has fewer tiles than the GPU has CUs.
+//
+//   out[m, n] = sum_k x[m, k] * w[n, k], scaled rowwise, by 1x128 / 128x128 blocks, or with MXFP4 weights
+//
+// A workgroup of four waves (2 x 2) owns a tile of BM x BN over one slice of K.  Both operand tiles of a K step go from
+// global memory straight into LDS through a ring of S stages, as deep as the LDS allows; a step's fragments are read a
+// step ahead, under the MFMAs of the step before, so that no MFMA waits for LDS and the workgroup's one barrier per step
+// finds every wave's reads done:
+//
+//   step kt:  wait for the loads of tile kt + 1 (those of the S - 2 tiles behind it stay in flight), barrier
+//             request tile kt + S into the stage of tile kt, whose fragments are in registers
+//             per MFMA one fragment read of tile kt + 1
+//
+// Every edge is a bound of a buffer descriptor: rows beyond M and N, chunks beyond K in the last step (K need only be a
+// multiple of 16, of 32 for MXFP4) and steps beyond the slice are per-lane offsets past the end, which a direct-to-LDS
+// load turns into zeros without a fetch.  So any M, N % 16 and K run at full speed, and the count of loads per step, which
+// the hand-written waits rely on, is the same everywhere.
+//
+// LDS layout of a stage: row-major, 16-byte chunk c of row r at position c ^ f(r).  A lane (row = lane & 15, q = lane >> 4)
+// of an e4m3 fragment reads chunks q and q + 4 - the K positions that go with an e2m1 lane's 32 codes, and as good as any
+// other two where both operands are e4m3.  The LDS serves a 16-byte read sixteen lanes at a time, lanes 0-3, 12-15, 20-23,
+// 24-27 first; f(r) = (bit 1 of r) << 1 | (bit 3 of r) << 2 puts those sixteen on sixteen different bank groups (128-byte
+// rows), and (bit 3 of r) << 1 does so for the 64-byte rows of e2m1.
+//
+// What bounds it (1111 x 3584 x 18944 rowwise, 252 tiles of 128 x 128, 87 us where tiles of 256 x 128 took 156 us; compiled
+// out one at a time): the multiplications and fragment reads alone 48 us, the loads alone 85 us - 32 KiB a CU and step at 57 B/ns,
+// 72 % of them from the XCD's L2, the rest from the memory-side cache or HBM (with both operands in that cache 68 us).  Other
+// row pitches and K steps rotated between workgroups or XCDs move it by at most 10 % either way.
+// MXFP4, 200 tokens: 2176 x 14848 20 against 142 us on the register-staged tiles, 3456 x 11264 27 against 108 us.
+//
+// Slices of K: fp32 partial sums into caller memory, summed in slice order with scales, bias and conversion by
+// ring_reduce_kernel.
+#include <atomic>
+#include <stdio.h>
+#include <stdlib.h>
+#include <type_traits>
+
+#include "gemm_internal.h"
+#include "gemm_ring.h"
+
+namespace cfp8 {
+
+constexpr uint32_t kOutside = 0xF0000000u;  // a per-lane offset that no descriptor here covers (they end at or below 0xEFFFFFFF)
+
+template <int MODE, int BM, int BN>
+struct RingShape {
+    static constexpr int LX = BM / 32, LW = MODE == kRingMx ? BN / 64 : BN / 32, LS = MODE == kRingMx ? 1 : 0;  // loads per wave and step
+    static constexpr int XS = BM * 128, WS = MODE == kRingMx ? BN * 64 : BN * 128, SS = MODE == kRingMx ? 1024 : 0;
+    static constexpr int STAGE = XS + WS + SS;
+    // block scaling keeps room for the slice's scales
+    static constexpr int S0 = (MODE == kRingBlock ? 128 : 160) * 1024 / STAGE;
+    static constexpr int S = S0 > 8 ? 8 : S0;
+};
+
+template <int MODE, int BM, int BN, bool SPLIT, bool OUT_F32>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_ring_kernel(const RingArgs p) {
+    using Sh = RingShape<MODE, BM, BN>;
+    constexpr int LX = Sh::LX, LW = Sh::LW, LS = Sh::LS, L = LX + LW + LS, S = Sh::S;
+    constexpr int TM = BM / 32, TN = BN / 32;  // 16 x 16 tiles per wave
+    constexpr int WB = S * Sh::XS, SB = WB + S * Sh::WS;
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    typedef __attribute__((address_space(3))) void lds_void;
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wm = wave & 1, wn = wave >> 1;
+    const int lrow = lane & 15, quarter = lane >> 4;
+    int tm, tn, slice;
+    {
+        const int tiles = p.tiles_m * p.tiles_n;
+        slice = SPLIT ? (int)blockIdx.x / tiles : 0;
+        const int pid = (int)blockIdx.x - slice * tiles;
+        // Every XCD (workgroups are dealt to the eight round robin) takes a contiguous range of tiles in bands of equal
+        // height, about four tile rows: what its workgroups load in common comes through its L2 once.  (Bands of up to 3, 4,
+        // 6, 8, 12 and 16 rows: 1111 x 37888 x 3584 184, 184, 197, 197, 195 and 194 us, 1024 x 3584 x 18944 86, 84, 84, 88,
+        // 88 and 88 us, level within 3 % elsewhere.)
+        const int xcd = pid & 7, local = pid >> 3, base = tiles >> 3, rem = tiles & 7;
+        const int lin = xcd * base + (xcd < rem ? xcd : rem) + local;
+        const int bands = (p.tiles_m + 3) >> 2, low = p.tiles_m / bands, high = p.tiles_m - low * bands;  // `high` bands of low + 1 rows first
+        const int split = high * (low + 1) * p.tiles_n;
+        const int rows = lin < split ? low + 1 : low;
+        const int at = lin < split ? lin : lin - split;
+        const int g = at / (rows * p.tiles_n), in = at - g * rows * p.tiles_n;
+        tm = (lin < split ? 0 : high * (low + 1)) + g * rows + in % rows;
+        tn = in / rows;
+    }
+    const int m0 = tm * BM, n0 = tn * BN;
+    const int KT = (p.K + 127) >> 7, tail = p.K & 127;
+    const int kbeg = SPLIT ? slice * p.slice_steps : 0;
+    const int kend = SPLIT ? (kbeg + p.slice_steps < KT ? kbeg + p.slice_steps : KT) : KT;
+
+    const int steps = kend - kbeg;
+
+    // descriptors: this wave's first row of the tile, ending with the matrix
+    constexpr uint32_t kMost = 0xEFFFFFFFu;
+    auto bytes_left = [&](int64_t rows, int64_t ld) -> uint32_t {
+        const int64_t b = rows > 0 ? rows * ld : 0;
+        return b < (int64_t)kMost ? (uint32_t)b : kMost;
+    };
+    constexpr int WROWS = MODE == kRingMx ? 16 : 8;  // weight rows of one load
+    uint64_t a_at = reinterpret_cast<uint64_t>(p.a) + (uint64_t)(m0 + wave * 8) * (uint64_t)p.ld_a;
+    uint64_t w_at = reinterpret_cast<uint64_t>(p.w) + (uint64_t)(n0 + wave * WROWS) * (uint64_t)p.ld_w;
+    uint32_t a_end = bytes_left((int64_t)p.M - m0 - wave * 8, p.ld_a), w_end = bytes_left((int64_t)p.N - n0 - wave * WROWS, p.ld_w);
+    uint32_t a_step = 32u * (uint32_t)p.ld_a, w_step = (uint32_t)(4 * WROWS) * (uint32_t)p.ld_w;
+    uint64_t s_at = 0;
+    uint32_t s_end = 0;
+    if (MODE == kRingMx) {
+        s_at = reinterpret_cast<uint64_t>(p.ws) + (uint64_t)(n0 + wave * (BN / 4)) * (uint64_t)p.ld_ws;
+        s_end = bytes_left((int64_t)p.N - n0 - wave * (BN / 4), p.ld_ws);
+    }
+    asm volatile("" : "+s"(a_at), "+s"(w_at), "+s"(a_end), "+s"(w_end), "+s"(a_step), "+s"(w_step), "+s"(s_at), "+s"(s_end));
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(a_at), 0, (int)a_end, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(w_at), 0, (int)w_end, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(s_at), 0, (int)s_end, 0x00020000);
+    // a load of 8 rows x 128 bytes: row lane >> 3, whose chunk position lane & 7 holds chunk position ^ f(row)
+    const uint32_t c8 = (uint32_t)((lane & 7) ^ ((((lane >> 4) & 1) << 1) | ((wave & 1) << 2)));
+    const uint32_t va = (uint32_t)(lane >> 3) * (uint32_t)p.ld_a + c8 * 16;
+    const uint32_t va_tail = tail && c8 * 16 >= (uint32_t)tail ? kOutside : va;  // the last step of a K that is no multiple of 128
+    uint32_t vw, vw_tail, vs = kOutside;
+    if (MODE == kRingMx) {  // 16 rows x 64 bytes
+        const uint32_t c4 = (uint32_t)((lane & 3) ^ (((lane >> 5) & 1) << 1));
+        vw = (uint32_t)(lane >> 2) * (uint32_t)p.ld_w + c4 * 16;
+        vw_tail = tail && c4 * 32 >= (uint32_t)tail ? kOutside : vw;
+        if (lane < BN / 4) vs = (uint32_t)lane * (uint32_t)p.ld_ws;
+    } else {
+        vw = (uint32_t)(lane >> 3) * (uint32_t)p.ld_w + c8 * 16;
+        vw_tail = tail && c8 * 16 >= (uint32_t)tail ? kOutside : vw;
+    }
+    auto dma = [&](int kt, int st, int l) {  // load l of the step's LX + LW + LS
+        const bool in = kt < kend, at_tail = kt == KT - 1;
+        if (l < LX)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_void*)(smem + st * Sh::XS + (wave + 4 * l) * 1024), 16,
+                                                     in ? (at_tail ? va_tail : va) : kOutside, (uint32_t)l * a_step + ((uint32_t)kt << 7), 0, 0);
+        else if (l < LX + LW)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_void*)(smem + WB + st * Sh::WS + (wave + 4 * (l - LX)) * 1024), 16,
+                                                     in ? (at_tail ? vw_tail : vw) : kOutside,
+                                                     (uint32_t)(l - LX) * w_step + ((uint32_t)kt << (MODE == kRingMx ? 6 : 7)), 0, 0);
+        else  // the step's four scale bytes of a row; in a last step that is shorter the four that end with the row
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)(smem + SB + st * 1024 + wave * 256), 4, in ? vs : kOutside,
+                                                     at_tail && tail ? (uint32_t)(p.K >> 5) - 4u : (uint32_t)kt << 2, 0, 0);
+    };
+
+    // fragments of 16 rows
+    const int xo = (wm * (BM / 2) + lrow) * 128 + ((quarter ^ ((((lrow >> 1) & 1) << 1) | (((lrow >> 3) & 1) << 2))) << 4);
+    const int wo = MODE == kRingMx ? WB + (wn * (BN / 2) + lrow) * 64 + ((quarter ^ (((lrow >> 3) & 1) << 1)) << 4)
+                                   : WB + (wn * (BN / 2) + lrow) * 128 + ((quarter ^ ((((lrow >> 1) & 1) << 1) | (((lrow >> 3) & 1) << 2))) << 4);
+    const int xo2 = xo ^ 64, wo2 = wo ^ 64;  // the row's chunk q + 4 (a stage and a tile of rows begin on multiples of 128)
+    auto frag8 = [&](int at, int at2) {
+        const i32x4 lo = *reinterpret_cast<const i32x4*>(smem + at);
+        const i32x4 hi = *reinterpret_cast<const i32x4*>(smem + at2);
+        return i32x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    };
+    auto wfrag = [&](int stage, int i) {
+        if (MODE == kRingMx) {
+            const i32x4 v = *reinterpret_cast<const i32x4*>(smem + stage * Sh::WS + wo + i * 1024);
+            return i32x8{v[0], v[1], v[2], v[3], 0, 0, 0, 0};
+        }
+        return frag8(stage * Sh::WS + wo + i * 2048, stage * Sh::WS + wo2 + i * 2048);
+    };
+    auto xfrag = [&](int stage, int j) { return frag8(stage * Sh::XS + xo + j * 2048, stage * Sh::XS + xo2 + j * 2048); };
+    auto scale_word = [&](int st, int i) -> u32 {  // e8m0 bytes of this lane's row, one per quarter
+        const int n = wn * (BN / 2) + i * 16 + lrow;
+        return *reinterpret_cast<const u32*>(smem + SB + st * 1024 + (n / (BN / 4)) * 256 + (n % (BN / 4)) * 4);
+    };
+
+    // block scaling: the slice's activation scales, [row][step] with an odd pitch, and the weight scales of the tile's one or
+    // two 128-blocks of N
+    const int spitch = p.slice_steps | 1;
+    float* const sa_lds = reinterpret_cast<float*>(smem + SB);
+    float* const sb_lds = sa_lds + BM * spitch;
+    if (MODE == kRingBlock) {
+        for (int i = t; i < BM * steps; i += 256) {
+            const int r = i / steps, c = i - r * steps;
+            sa_lds[r * spitch + c] = m0 + r < p.M ? p.sa[(int64_t)(m0 + r) * KT + kbeg + c] : 0.f;
+        }
+        for (int i = t; i < steps; i += 256) sb_lds[i] = p.sb[(int64_t)(n0 >> 7) * p.sb_stride_n + (int64_t)(kbeg + i) * p.sb_stride_k];
+    }
+    static_assert(MODE != kRingBlock || BN <= 128, "a tile lies in one 128-block of N");
+
+    f32x4 acc[TN][TM];
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // Fragments: the weight tiles' and the last token tile's twice (a step's and the next one's), the other token tiles' once,
+    // replaced in place behind their last MFMA.
+    i32x8 W[2][TN], XL[2], X[TM - 1];
+    u32 wword[2][TN];         // kRingMx: the scale word of the weight tile's row
+    float xs[2][TM], ss[2];   // kRingBlock: activation scales and weight scale of a step
+    auto read_w = [&](int b, int st, int i) {
+        W[b][i] = wfrag(st, i);
+        if (MODE == kRingMx) wword[b][i] = scale_word(st, i);
+    };
+    auto read_s = [&](int b, int kt) {
+        if (MODE == kRingBlock) {
+            const int c = kt < kend ? kt - kbeg : 0;
+            ss[b] = sb_lds[c];
+#pragma unroll
+            for (int j = 0; j < TM; ++j) xs[b][j] = sa_lds[(wm * (BM / 2) + j * 16 + lrow) * spitch + c];
+        }
+    };
+    f32x4 pr[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};  // kRingBlock: products not yet added
+    float pr_f = 0.f;
+
+#pragma unroll
+    for (int d = 0; d < S; ++d)
+#pragma unroll
+        for (int l = 0; l < L; ++l) dma(kbeg + d, d, l);
+    // tile 0 has landed when at most the loads of the S - 1 tiles behind it are outstanding
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 1) * L) : "memory");
+    int stage = 0;
+    auto step = [&](auto B, int kt) {
+        constexpr int b = decltype(B)::value;
+        constexpr int SLOTS = TM * TN;
+        // all waves hold tile kt's fragments; tile kt + 1 has landed when at most S - 2 tiles' loads are outstanding
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * L) : "memory");
+        const int freed = stage;
+        stage = stage == S - 1 ? 0 : stage + 1;
+        int wsc[TN];
+        if (MODE == kRingMx) {
+#pragma unroll
+            for (int i = 0; i < TN; ++i) {
+                u32 v = wword[b][i];
+                if (tail && kt == KT - 1) v >>= (u32)(4 - (tail >> 5)) * 8;
+                wsc[i] = (int)(v >> (quarter * 8));
+            }
+        }
+        float f[TM];
+#pragma unroll
+        for (int j = 0; j < TM; ++j) f[j] = MODE == kRingBlock ? xs[b][j] * ss[b] : 0.f;
+#pragma unroll
+        for (int g = 0; g < SLOTS; ++g) {
+            const int j = g / TN, i = g % TN;
+            const i32x8 xf = j == TM - 1 ? XL[b] : X[j];
+            if (MODE == kRingBlock) {
+                const f32x4 old = pr[g & 1];
+                pr[g & 1] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(W[b][i], xf, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
+                const int og = g >= 2 ? g - 2 : SLOTS + g - 2, oj = og / TN, oi = og % TN;
+                const float of = g >= 2 ? f[oj] : pr_f;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[oi][oj][e] = __builtin_fmaf(old[e], of, acc[oi][oj][e]);
+            } else if (MODE == kRingMx) {
+                acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(W[b][i], xf, acc[i][j], 4, 0, 0, wsc[i], 0, 0x7F7F7F7F);
+            } else {
+                acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(W[b][i], xf, acc[i][j], 0, 0, 0, 0, 0, 0);
+            }
+            // (an MFMA is a pure function of registers: pinned, or the compiler moves it past the fences below)
+            if (MODE == kRingBlock) asm volatile("" : "+v"(pr[g & 1]));
+            else asm volatile("" : "+v"(acc[i][j]));
+            // behind the MFMA: a fragment of the next step where one is due, and the loads spread over the step
+            if (g == 0) XL[b ^ 1] = xfrag(stage, TM - 1);
+            if (g == 0) read_s(b ^ 1, kt + 1);
+            if (g >= 1 && g <= TN) read_w(b ^ 1, stage, g - 1);
+            if (g > TN && g % TN == 1) X[g / TN - 1] = xfrag(stage, g / TN - 1);
+#pragma unroll
+            for (int l = 0; l < L; ++l)
+                if (l * SLOTS / L == g) dma(kt + S, freed, l);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        pr_f = f[TM - 1];
+    };
+    auto first = [&](auto B) {
+        constexpr int b = decltype(B)::value;
+#pragma unroll
+        for (int i = 0; i < TN; ++i) read_w(b, 0, i);
+#pragma unroll
+        for (int j = 0; j < TM - 1; ++j) X[j] = xfrag(0, j);
+        XL[b] = xfrag(0, TM - 1);
+        read_s(b, kbeg);
+    };
+    // Two steps a round, so that the register sets alternate; an odd step goes first.  (With an exit in the middle of the
+    // round the compiler gives the accumulators two sets of registers as well.)
+    int kt = kbeg;
+    if (steps & 1) {
+        first(std::integral_constant<int, 1>{});
+        step(std::integral_constant<int, 1>{}, kt++);
+    } else {
+        first(std::integral_constant<int, 0>{});
+    }
+    for (; kt < kend; kt += 2) {
+        step(std::integral_constant<int, 0>{}, kt);
+        step(std::integral_constant<int, 1>{}, kt + 1);
+    }
+    if (MODE == kRingBlock) {
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[TN - 2 + g][TM - 1][e] = __builtin_fmaf(pr[g][e], pr_f, acc[TN - 2 + g][TM - 1][e]);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may land in LDS once the workgroup has gone
+
+    if (SPLIT) {
+        float* const part = p.partial + (int64_t)slice * p.M * p.N;
+#pragma unroll
+        for (int j = 0; j < TM; ++j) {
+            const int m = m0 + wm * (BM / 2) + j * 16 + lrow;
+            if (m >= p.M) continue;
+#pragma unroll
+            for (int i = 0; i < TN; ++i) {
+                const int n = n0 + wn * (BN / 2) + i * 16 + quarter * 4;
+                if (n < p.N) *reinterpret_cast<f32x4*>(part + (int64_t)m * p.N + n) = acc[i][j];
+            }
+        }
+        return;
+    }
+    float sam[TM];
+    f32x4 sbn[TN], bia[TN];
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+        const int m = m0 + wm * (BM / 2) + j * 16 + lrow;
+        sam[j] = MODE != kRingBlock ? p.sa[m < p.M ? m : p.M - 1] : 1.f;
+    }
+#pragma unroll
+    for (int i = 0; i < TN; ++i) {
+        const int n = n0 + wn * (BN / 2) + i * 16 + quarter * 4, nn = n < p.N ? n : 0;
+        sbn[i] = MODE == kRingRow ? *reinterpret_cast<const f32x4*>(p.sb + nn) : f32x4{1.f, 1.f, 1.f, 1.f};
+        bia[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (p.bias) {
+            const uint2 b = *reinterpret_cast<const uint2*>(p.bias + nn);
+            bia[i] = f32x4{bf16_lo(b.x), bf16_hi(b.x), bf16_lo(b.y), bf16_hi(b.y)};
+        }
+    }
+    auto value = [&](int i, int j) {
+        f32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = acc[i][j][e] * sam[j] * sbn[i][e] + bia[i][e];
+        return v;
+    };
+    if constexpr (OUT_F32) {
+#pragma unroll
+        for (int j = 0; j < TM; ++j) {
+            const int m = m0 + wm * (BM / 2) + j * 16 + lrow;
+            if (m >= p.M) continue;
+#pragma unroll
+            for (int i = 0; i < TN; ++i) {
+                const int n = n0 + wn * (BN / 2) + i * 16 + quarter * 4;
+                if (n < p.N) *reinterpret_cast<f32x4*>(static_cast<float*>(p.out) + (int64_t)m * p.ld_out + n) = value(i, j);
+            }
+        }
+    } else {
+        // turned through LDS (the ring is free behind a barrier): 16 bytes per lane, BN bytes of a row at a time
+        constexpr int PITCH = BN + 16, LPR = BN / 16, RPI = 64 / LPR;  // a wave's row is BN / 2 values
+        __syncthreads();
+        uint8_t* const buf = smem + wave * (BM / 2) * PITCH;
+#pragma unroll
+        for (int j = 0; j < TM; ++j)
+#pragma unroll
+            for (int i = 0; i < TN; ++i) {
+                const f32x4 v = value(i, j);
+                *reinterpret_cast<uint2*>(buf + (j * 16 + lrow) * PITCH + (i * 16 + quarter * 4) * 2) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+            }
+        const int rr = lane / LPR, rc = lane % LPR;
+#pragma unroll
+        for (int r = 0; r < BM / 2; r += RPI) {
+            const int m = m0 + wm * (BM / 2) + r + rr, n = n0 + wn * (BN / 2) + rc * 8;
+            const i32x4 d = *reinterpret_cast<const i32x4*>(buf + (r + rr) * PITCH + rc * 16);
+            if (m < p.M && n < p.N) *reinterpret_cast<i32x4*>(static_cast<uint16_t*>(p.out) + (int64_t)m * p.ld_out + n) = d;
+        }
+    }
+}
+
+// Sum of the slices in order, scales, bias, conversion; one thread per four columns.
+template <int MODE, bool OUT_F32>
+__global__ __launch_bounds__(256) void ring_reduce_kernel(const RingArgs p) {
+    const int nq = p.N >> 2;
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (int64_t)p.M * nq) return;
+    const int m = (int)(i / nq), n = (int)(i - (int64_t)m * nq) * 4;
+    const float* const at = p.partial + (int64_t)m * p.N + n;
+    f32x4 v = *reinterpret_cast<const f32x4*>(at);
+#pragma unroll 4
+    for (int s = 1; s < p.slices; ++s) {
+        const f32x4 o = *reinterpret_cast<const f32x4*>(at + (int64_t)s * p.M * p.N);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] += o[e];
+    }
+    const float sam = MODE != kRingBlock ? p.sa[m] : 1.f;
+    const f32x4 sbn = MODE == kRingRow ? *reinterpret_cast<const f32x4*>(p.sb + n) : f32x4{1.f, 1.f, 1.f, 1.f};
+    f32x4 bia = {0.f, 0.f, 0.f, 0.f};
+    if (p.bias) {
+        const uint2 b = *reinterpret_cast<const uint2*>(p.bias + n);
+        bia = f32x4{bf16_lo(b.x), bf16_hi(b.x), bf16_lo(b.y), bf16_hi(b.y)};
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = v[e] * sam * sbn[e] + bia[e];
+    if (OUT_F32) *reinterpret_cast<f32x4*>(static_cast<float*>(p.out) + (int64_t)m * p.ld_out + n) = v;
+    else *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.out) + (int64_t)m * p.ld_out + n) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+}
+
+template <int MODE, int BM, int BN, bool SPLIT>
+static int launch_ring_cfg(RingArgs& p, int out_dtype, hipStream_t st) {
+    using Sh = RingShape<MODE, BM, BN>;
+    p.tiles_m = (p.M + BM - 1) / BM;
+    p.tiles_n = (p.N + BN - 1) / BN;
+    const int64_t blocks = (int64_t)p.tiles_m * p.tiles_n * p.slices;
+    if (blocks > 0x7FFFFFFFll) return set_error(CFP8_EINVAL, "gemm: too many tiles for one launch");
+    size_t lds = (size_t)Sh::S * Sh::STAGE;
+    if (MODE == kRingBlock) lds += ((size_t)BM * (p.slice_steps | 1) + p.slice_steps) * sizeof(float);
+    static_assert(Sh::S >= 3 && (size_t)4 * (BM / 2) * (BN + 16) <= (size_t)Sh::S * Sh::STAGE, "ring LDS");
+    const int f32 = out_dtype == CFP8_OUT_F32;
+    using Kern = void (*)(const RingArgs);
+    const Kern kern = SPLIT || !f32 ? static_cast<Kern>(gemm_ring_kernel<MODE, BM, BN, SPLIT, false>) : static_cast<Kern>(gemm_ring_kernel<MODE, BM, BN, false, true>);
+    static std::atomic<bool> raised[65][2];
+    const int slot = device_slot();
+    if (slot == 64) raised[64][f32].store(false, std::memory_order_relaxed);
+    if (int rc = raise_lds_limit(reinterpret_cast<const void*>(kern), 160 * 1024, raised[slot][f32])) return rc;
+    {
+        char name[80];
+        snprintf(name, sizeof(name), "gemm_ring<%s,%d,%d>%s slices=%d", MODE == kRingRow ? "rowwise" : MODE == kRingBlock ? "block" : "mxfp4", BM, BN,
+                 p.K & 127 ? " ktail" : "", p.slices);
+        if (!note_launch(name, (unsigned)blocks, 256, lds)) return CFP8_OK;
+    }
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), lds, st, p);
+    if (SPLIT) {
+        const unsigned rb = (unsigned)(((int64_t)p.M * (p.N >> 2) + 255) / 256);
+        if (f32) hipLaunchKernelGGL((ring_reduce_kernel<MODE, true>), dim3(rb), dim3(256), 0, st, p);
+        else hipLaunchKernelGGL((ring_reduce_kernel<MODE, false>), dim3(rb), dim3(256), 0, st, p);
+    }
+    return check_launch("gemm");
+}
+
+template <int MODE>
+static int launch_ring_mode(RingArgs& p, const RingPlan& plan, int out_dtype, hipStream_t st) {
+    const int KT = (p.K + 127) >> 7;
+    p.slice_steps = (KT + plan.slices - 1) / plan.slices;
+    p.slices = (KT + p.slice_steps - 1) / p.slice_steps;
+#define CFP8_RING(BM, BN) \
+    if (plan.bm == BM && plan.bn == BN) return p.slices > 1 ? launch_ring_cfg<MODE, BM, BN, true>(p, out_dtype, st) : launch_ring_cfg<MODE, BM, BN, false>(p, out_dtype, st)
+    CFP8_RING(128, 128);
+    CFP8_RING(64, 128);
+    CFP8_RING(128, 64);
+    CFP8_RING(64, 64);
+#undef CFP8_RING
+    return set_error(CFP8_EINVAL, "gemm: no such ring tile");
+}
+
+// The tile and the number of slices with the least estimated time.  The estimate is a fixed time per launch plus, per
+// round of workgroups on the CUs, K steps times the tile's step time (longer the more CUs load at once) plus the tile's
+// ends, not below the operands' bytes at the rate they come in; slices add the reduction's launch and their partial sums'
+// way out and back.  The constants are fitted to 1150 (rowwise), 1500 (block) and 1400 (MXFP4) timed combinations of 90
+// shapes each (1 .. 8192 tokens, weights of 896 .. 37888 rows, K 896 .. 18944): the choice is within 1 % of the best
+// combination on average, 13 % at worst.
+struct RingRates {
+    double step[4], load[4];  // 128 x 128, 64 x 128, 128 x 64, 64 x 64: microseconds a step, and what a full GPU adds
+    double launch, ends, partial, bytes, reduce;
+};
+static const RingRates kRates[3] = {
+    {{0.359, 0.207, 0.240, 0.131}, {0.336, 0.589, 0.233, 0.522}, 3.0, 2.0, 4.2, 4.7, 2.1},
+    {{0.579, 0.302, 0.460, 0.223}, {0.182, 0.443, 0.014, 0.320}, 3.5, 2.1, 5.0, 5.4, 2.3},
+    {{0.432, 0.328, 0.308, 0.182}, {0.177, 0.196, 0.028, 0.158}, 3.6, 2.1, 4.3, 4.4, 2.3},
+};
+static const int kTiles[4][2] = {{128, 128}, {64, 128}, {128, 64}, {64, 64}};
+constexpr int kRingMaxSlices = 16;
+
+// block scaling: the scales of a slice in LDS beside the ring
+static bool ring_scales_fit(int bm, int64_t steps) { return ((int64_t)bm * (steps | 1) + steps) * 4 <= 32 * 1024; }
+
+RingPlan ring_plan(int mode, int64_t M, int64_t N, int64_t K, size_t partial_bytes, int cus) {
+    const RingRates& r = kRates[mode];
+    const int64_t KT = (K + 127) / 128;
+    RingPlan best{0, 0, 0, 1e30};
+    const double bytes = (double)N * K * (mode == kRingMx ? 0.53 : 1.0) + (double)M * K;
+    for (int c = 0; c < 4; ++c) {
+        const int bm = kTiles[c][0], bn = kTiles[c][1];
+        if (bm == 128 && M <= 64) continue;
+        const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+        for (int s = 1; s <= kRingMaxSlices; ++s) {
+            const int64_t steps = (KT + s - 1) / s;
+            if (s > 1 && (steps < 3 || (KT + steps - 1) / steps != s || tiles * s > 2 * cus || (size_t)s * (size_t)M * (size_t)N * 4 > partial_bytes)) continue;
+            if (mode == kRingBlock && !ring_scales_fit(bm, steps)) continue;
+            const int64_t full = tiles * s / cus, rem = tiles * s % cus;
+            const double part = (double)rem / cus;
+            double us = r.launch + full * (steps * r.step[c] * (1 + r.load[c]) + r.ends);
+            if (rem) us += steps * r.step[c] * (1 + r.load[c] * (full ? 1.0 : part) * part) + r.ends;
+            const double stream = r.launch + bytes / (r.bytes * 1e6);
+            if (us < stream) us = stream;
+            if (s > 1) us += r.reduce + 8.0 * s * M * N / (r.partial * 1e6);
+            if (us < best.cost) best = {bm, bn, s, us};
+        }
+    }
+    return best;
+}
+
+bool ring_takes(int mode, const RingArgs& p, int out_dtype) {
+    // a tile's byte offsets plus the outside offset stay below 2^32
+    if (p.ld_a >= (1 << 21) || p.ld_w >= (1 << 21) || p.ld_ws >= (1 << 21)) return false;
+    if (mode == kRingMx && p.K < 128) return false;                   // the last step's scale word ends with its row
+    if (mode == kRingBlock && p.K % 128) return false;
+    if (out_dtype == CFP8_OUT_BF16 && (p.ld_out % 8 || !aligned16(p.out))) return false;
+    return (reinterpret_cast<uintptr_t>(p.bias) & 7u) == 0 && aligned16(p.out);
+}
+
+int launch_ring(int mode, RingArgs& p, const RingPlan& plan, int out_dtype, hipStream_t st) {
+    if (mode == kRingRow) return launch_ring_mode<kRingRow>(p, plan, out_dtype, st);
+    if (mode == kRingBlock) return launch_ring_mode<kRingBlock>(p, plan, out_dtype, st);
+    return launch_ring_mode<kRingMx>(p, plan, out_dtype, st);
+}
+
+}  // namespace cfp8
+
+extern "C" size_t cfp8_gemm_partial_bytes(int kind, int64_t M, int64_t N, int64_t K) {
+    using namespace cfp8;
+    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    const int mode = kind == CFP8_DISPATCH_BLOCK ? kRingBlock : kind == CFP8_DISPATCH_MXFP4 ? kRingMx : kRingRow;
+    const RingPlan plan = ring_plan(mode, M, N, K, ~(size_t)0, cu_count());
+    return plan.slices > 1 ? (size_t)plan.slices * (size_t)M * (size_t)N * 4 : 0;
+}

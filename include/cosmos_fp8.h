@@ -338,6 +338,18 @@ int cfp8_gemm_mxfp4(const void* a, int64_t ld_a, const float* sa, const void* w,
                     int64_t ld_ws, const int32_t* m_indices, int64_t num_groups, void* out, int64_t ld_out,
                     int out_dtype, int64_t M, int64_t N, int64_t K, void* stream);
 
+/* fp32 partial sums: how much memory a product needs to be cut into slices of K where that is the fastest way (a weight
+ * with few rows and a long K; 0: it is not).  kind: CFP8_DISPATCH_ROWWISE, _BLOCK or _MXFP4.  The entry points named
+ * *_split, and cfp8_linear_mxfp4 beyond its quantised activations, take that memory as a workspace (256-byte aligned);
+ * with less of it they choose among what fits.  The slices are summed in order, so results do not vary from run to run. */
+#define CFP8_DISPATCH_MXFP4 5
+size_t cfp8_gemm_partial_bytes(int kind, int64_t M, int64_t N, int64_t K);
+
+/* cfp8_gemm_mxfp4 on one weight matrix with memory for partial sums. */
+int cfp8_gemm_mxfp4_split(const void* a, int64_t ld_a, const float* sa, const void* w, int64_t ld_w, const void* ws,
+                          int64_t ld_ws, void* out, int64_t ld_out, int out_dtype, int64_t M, int64_t N, int64_t K,
+                          void* workspace, size_t workspace_bytes, void* stream);
+
 /* The linear layer on MXFP4 weights from bf16 activations: per-token dynamic FP8 quantisation of x (bf16 [M, K], ld_x in
  * elements, multiple of 8, x 16-byte aligned; the arithmetic of cfp8_quant_rowwise) followed by cfp8_gemm_mxfp4 on one
  * weight matrix.  Up to 4 tokens with K <= 4096 run as one launch (the quantisation inside the weight-streaming
