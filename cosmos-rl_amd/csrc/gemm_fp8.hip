@@ -1991,11 +1991,17 @@ __global__ __launch_bounds__(NTL * 128) void gemm_rowwise_skinny_kernel(const Ge
 // ---------------------------------------------------------------------------
 // Rowwise GEMM for M <= 16 (single-token decode): no LDS staging and no barrier
 // in the loop.  A workgroup owns 16 weight rows; its four waves split K (wave w
-// takes K steps w, w + 4, ...), each issuing the loads of eight K steps (16 KiB
-// of weights per wave) before the first MFMA.  The few activation rows come
-// straight from global memory (they stay in L2), rows >= M are zero.
+// takes K steps w, w + 4, ...), each issuing the loads of a chunk of NI K steps
+// before the first MFMA: all of its steps if they are at most eight, else equal
+// chunks of at most eight (16 KiB of weights per wave).  Loads for steps that do
+// not exist cost as much as others: with eight for every K, 9728 x 896 took 11.1 us
+// against 4.6, 23552 x 1152 21.3 against 8.0.  The loads are cacheable: streaming
+// ones were slower wherever a launch has more workgroups than fit at once (37888 x
+// 3584 33.3 against 25.4 us, 5.4 TB/s, M = 1; 45 against 37 us at M = 16, where L2
+// also returns 16 activation rows for 16 weight rows, which bounds it).  The few
+// activation rows come straight from global memory (they stay in L2), rows >= M repeat row 0.
 // ---------------------------------------------------------------------------
-template <bool OUT_F32>
+template <int NI, bool OUT_F32>
 __global__ __launch_bounds__(256) void gemm_rowwise_gemv_kernel(const GemmArgs p) {
     __shared__ __attribute__((aligned(16))) float red[3 * 64 * 4];
     const int t = threadIdx.x, lane = t & 63;
@@ -2003,33 +2009,32 @@ __global__ __launch_bounds__(256) void gemm_rowwise_gemv_kernel(const GemmArgs p
     const int lrow = lane & 15, quarter = lane >> 4;
     const int n0 = blockIdx.x * 16;
     const int KT = p.K >> 7;
-    const int wrow = n0 + lrow;
-    const bool wok = wrow < p.N, xok = lrow < p.M;
-    const uint8_t* wptr = p.b + (int64_t)(wok ? wrow : 0) * p.ld_b + quarter * 32;
+    const bool xok = lrow < p.M;
+    const uint8_t* wptr = p.b + (int64_t)(n0 + lrow) * p.ld_b + quarter * 32;  // N % 16 == 0: the 16 rows are there
     const uint8_t* xptr = p.a + (int64_t)(xok ? lrow : 0) * p.ld_a + quarter * 32;
     f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int base = wave; base < KT; base += 32) {
-        u32x4 wl[8], wh[8], xl[8], xh[8];
+    for (int base = wave; base < KT; base += 4 * NI) {
+        u32x4 wl[NI], wh[NI], xl[NI], xh[NI];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
+        for (int i = 0; i < NI; ++i) {
             const int kt = base + 4 * i;
-            const bool in = kt < KT;
-            const int64_t off = (int64_t)(in ? kt : 0) << 7;
-            wl[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wptr + off));
-            wh[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wptr + off + 16));
+            if (kt >= KT) continue;
+            const int64_t off = (int64_t)kt << 7;
+            wl[i] = *reinterpret_cast<const u32x4*>(wptr + off);
+            wh[i] = *reinterpret_cast<const u32x4*>(wptr + off + 16);
             xl[i] = *reinterpret_cast<const u32x4*>(xptr + off);
             xh[i] = *reinterpret_cast<const u32x4*>(xptr + off + 16);
         }
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const bool in = base + 4 * i < KT;
+        for (int i = 0; i < NI; ++i) {
+            if (base + 4 * i >= KT) continue;
             i32x8 fw, fx;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                fw[e] = (in && wok) ? (int)wl[i][e] : 0;
-                fw[4 + e] = (in && wok) ? (int)wh[i][e] : 0;
-                fx[e] = (in && xok) ? (int)xl[i][e] : 0;
-                fx[4 + e] = (in && xok) ? (int)xh[i][e] : 0;
+                fw[e] = (int)wl[i][e];
+                fw[4 + e] = (int)wh[i][e];
+                fx[e] = (int)xl[i][e];
+                fx[4 + e] = (int)xh[i][e];
             }
             acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fw, fx, acc, 0, 0, 0, 0, 0, 0);
         }
@@ -2038,7 +2043,7 @@ __global__ __launch_bounds__(256) void gemm_rowwise_gemv_kernel(const GemmArgs p
     __syncthreads();
     if (wave == 0) {
         const int n = n0 + quarter * 4, m = lrow;
-        if (n < p.N && m < p.M) {
+        if (m < p.M) {
 #pragma unroll
             for (int w = 0; w < 3; ++w) {
                 const f32x4 o = *reinterpret_cast<const f32x4*>(red + (w * 64 + lane) * 4);
@@ -2058,15 +2063,17 @@ __global__ __launch_bounds__(256) void gemm_rowwise_gemv_kernel(const GemmArgs p
 }
 
 // ---------------------------------------------------------------------------
-// FP8 linear for at most 4 tokens and K <= 4096 in ONE launch: the gemv kernel above with the per-token
+// FP8 linear for at most 4 tokens and K <= 4096 (8192 for one) in ONE launch: the gemv kernel above with the per-token
 // quantisation folded in.  Every workgroup first requests its weights (all of a wave's K steps are in
 // flight before anything else happens), then its 256 threads quantise the tokens together - each
-// thread holds at most two 16-byte vectors of a token between the amax and the cast, exactly the
+// thread holds at most two (four) 16-byte vectors of a token between the amax and the cast, exactly the
 // arithmetic of the rowwise quantiser - into LDS, from where the MFMA fragments are read.  The
-// quantisation hides behind the weight loads, and the separate launch (5 us plus the gap between two
-// launches, a quarter of a single-token call) is gone.  Results are bit-identical to the two-launch path.
+// quantisation hides behind the weight loads, and the separate launch (3 us plus the gap between two
+// launches) is gone: 896 x 4864 10.2 -> 6.1 us, 18944 x 3584 20.1 -> 15.5 us with the loads as above.  At four
+// tokens the quantisation in every workgroup costs what the launch would (18944 x 2560 15.9 us either way), beyond
+// that more; and 8192 is what a wave's registers hold.  Results are bit-identical to the two-launch path.
 // ---------------------------------------------------------------------------
-template <int MR, bool OUT_F32>
+template <int MR, int NI, bool OUT_F32>
 __global__ __launch_bounds__(256) void linear_gemv_fused_kernel(const uint4* __restrict__ x, int64_t ldx, const GemmArgs p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t xq[];  // [M][K] fp8
     __shared__ __attribute__((aligned(16))) float red[3 * 64 * 4];
@@ -2075,28 +2082,29 @@ __global__ __launch_bounds__(256) void linear_gemv_fused_kernel(const uint4* __r
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int lrow = lane & 15, quarter = lane >> 4;
     const int n0 = blockIdx.x * 16;
-    const int KT = p.K >> 7;  // <= 32: one batch of 8 K steps per wave
-    const int wrow = n0 + lrow;
-    const bool wok = wrow < p.N, xok = lrow < p.M;
-    const uint8_t* wptr = p.b + (int64_t)(wok ? wrow : 0) * p.ld_b + quarter * 32;
-    u32x4 wl[8], wh[8];
+    const int KT = p.K >> 7;  // <= 4 NI: all of a wave's K steps at once
+    const bool xok = lrow < p.M;
+    const uint8_t* wptr = p.b + (int64_t)(n0 + lrow) * p.ld_b + quarter * 32;
+    u32x4 wl[NI], wh[NI];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int kt = wave + 4 * i;
-        const int64_t off = (int64_t)(kt < KT ? kt : 0) << 7;
-        wl[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wptr + off));
-        wh[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wptr + off + 16));
+    for (int i = 0; i < NI; ++i) {
+        // (a wave without this step repeats the last one: under a branch the loads were sunk behind the barriers, 17664 x
+        // 2176 17 against 11 us)
+        const int kt = wave + 4 * i < KT ? wave + 4 * i : KT - 1;
+        wl[i] = *reinterpret_cast<const u32x4*>(wptr + ((int64_t)kt << 7));
+        wh[i] = *reinterpret_cast<const u32x4*>(wptr + ((int64_t)kt << 7) + 16);
     }
     // the tokens (MR >= M of them): amax, scale, cast - rows >= M read row 0 and are never used
     const int nvec = p.K >> 3;
-    uint4 v[MR][2];
+    constexpr int NV = (NI + 3) / 4;
+    uint4 v[MR][NV];
     float scale[MR];
 #pragma unroll
     for (int r = 0; r < MR; ++r) {
         const uint4* xr = x + (int64_t)(r < p.M ? r : 0) * ldx;
         u32 m = 0;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+        for (int j = 0; j < NV; ++j) {
             const int idx = t + 256 * j;
             v[r][j] = idx < nvec ? xr[idx] : make_uint4(0, 0, 0, 0);
             m = absmax8(m, v[r][j]);
@@ -2112,7 +2120,7 @@ __global__ __launch_bounds__(256) void linear_gemv_fused_kernel(const uint4* __r
         const Divider d(scale[r]);
         if (r < p.M) {
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
+            for (int j = 0; j < NV; ++j) {
                 const int idx = t + 256 * j;
                 if (idx < nvec) *reinterpret_cast<uint2*>(xq + (int64_t)r * p.K + idx * 8) = cast8(v[r][j], d);
             }
@@ -2122,18 +2130,18 @@ __global__ __launch_bounds__(256) void linear_gemv_fused_kernel(const uint4* __r
     f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
     const uint8_t* xrow = xq + (xok ? lrow : 0) * p.K + quarter * 32;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < NI; ++i) {
         const int kt = wave + 4 * i;
-        const bool in = kt < KT;
-        const u32x4 xl = *reinterpret_cast<const u32x4*>(xrow + ((in ? kt : 0) << 7));
-        const u32x4 xh = *reinterpret_cast<const u32x4*>(xrow + ((in ? kt : 0) << 7) + 16);
+        if (kt >= KT) continue;
+        const u32x4 xl = *reinterpret_cast<const u32x4*>(xrow + (kt << 7));
+        const u32x4 xh = *reinterpret_cast<const u32x4*>(xrow + (kt << 7) + 16);
         i32x8 fw, fx;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            fw[e] = (in && wok) ? (int)wl[i][e] : 0;
-            fw[4 + e] = (in && wok) ? (int)wh[i][e] : 0;
-            fx[e] = (in && xok) ? (int)xl[e] : 0;
-            fx[4 + e] = (in && xok) ? (int)xh[e] : 0;
+            fw[e] = (int)wl[i][e];
+            fw[4 + e] = (int)wh[i][e];
+            fx[e] = (int)xl[e];
+            fx[4 + e] = (int)xh[e];
         }
         acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fw, fx, acc, 0, 0, 0, 0, 0, 0);
     }
@@ -2141,7 +2149,7 @@ __global__ __launch_bounds__(256) void linear_gemv_fused_kernel(const uint4* __r
     __syncthreads();
     if (wave == 0) {
         const int n = n0 + quarter * 4, m = lrow;
-        if (n < p.N && m < p.M) {
+        if (m < p.M) {
 #pragma unroll
             for (int w = 0; w < 3; ++w) {
                 const f32x4 o = *reinterpret_cast<const f32x4*>(red + (w * 64 + lane) * 4);
@@ -2164,30 +2172,42 @@ __global__ __launch_bounds__(256) void linear_gemv_fused_kernel(const uint4* __r
 
 // whether the one-launch kernel above takes the call
 static bool fused_gemv_applies(int64_t M, int64_t K, const void* x, int64_t ld_x) {
-    return M >= 1 && M <= 4 && K <= 4096 && K % 128 == 0 && aligned16(x) && ld_x % 8 == 0;
+    return M >= 1 && M <= 4 && K <= (M == 1 ? 8192 : 4096) && K % 128 == 0 && aligned16(x) && ld_x % 8 == 0;
 }
-template <int MR>
-static int launch_linear_gemv_fused_mr(const void* x, int64_t ld_x, GemmArgs& p, int out_dtype, hipStream_t st) {
+template <int MR, int NI>
+static void launch_fused_ni(int ni, dim3 grid, size_t lds, hipStream_t st, const void* x, int64_t ld_x, const GemmArgs& p, int out_dtype) {
+    if constexpr (NI > 0) {
+        if (ni != NI) return launch_fused_ni<MR, NI - 1>(ni, grid, lds, st, x, ld_x, p, out_dtype);
+        if (out_dtype == CFP8_OUT_F32)
+            hipLaunchKernelGGL((linear_gemv_fused_kernel<MR, NI, true>), grid, dim3(256), lds, st, static_cast<const uint4*>(x), ld_x / 8, p);
+        else
+            hipLaunchKernelGGL((linear_gemv_fused_kernel<MR, NI, false>), grid, dim3(256), lds, st, static_cast<const uint4*>(x), ld_x / 8, p);
+    }
+}
+static int launch_linear_gemv_fused(const void* x, int64_t ld_x, GemmArgs& p, int out_dtype, hipStream_t st) {
     const int64_t blocks = (p.N + 15) / 16;
     const size_t lds = (size_t)p.M * (size_t)p.K;  // <= 16 KiB
     if (!note_launch("linear_gemv_fused", (unsigned)blocks, 256, lds)) return CFP8_OK;
-    if (out_dtype == CFP8_OUT_F32)
-        hipLaunchKernelGGL((linear_gemv_fused_kernel<MR, true>), dim3((unsigned)blocks), dim3(256), lds, st, static_cast<const uint4*>(x), ld_x / 8, p);
-    else
-        hipLaunchKernelGGL((linear_gemv_fused_kernel<MR, false>), dim3((unsigned)blocks), dim3(256), lds, st, static_cast<const uint4*>(x), ld_x / 8, p);
+    const int ni = ((p.K >> 7) + 3) / 4;
+    if (p.M == 1) launch_fused_ni<1, 16>(ni, dim3((unsigned)blocks), lds, st, x, ld_x, p, out_dtype);
+    else if (p.M == 2) launch_fused_ni<2, 8>(ni, dim3((unsigned)blocks), lds, st, x, ld_x, p, out_dtype);
+    else launch_fused_ni<4, 8>(ni, dim3((unsigned)blocks), lds, st, x, ld_x, p, out_dtype);
     return check_launch("linear");
 }
-static int launch_linear_gemv_fused(const void* x, int64_t ld_x, GemmArgs& p, int out_dtype, hipStream_t st) {
-    if (p.M == 1) return launch_linear_gemv_fused_mr<1>(x, ld_x, p, out_dtype, st);
-    if (p.M == 2) return launch_linear_gemv_fused_mr<2>(x, ld_x, p, out_dtype, st);
-    return launch_linear_gemv_fused_mr<4>(x, ld_x, p, out_dtype, st);
-}
 
+template <int NI>
+static void launch_gemv_ni(int ni, dim3 grid, hipStream_t st, const GemmArgs& p, int out_dtype) {
+    if constexpr (NI > 0) {
+        if (ni != NI) return launch_gemv_ni<NI - 1>(ni, grid, st, p, out_dtype);
+        if (out_dtype == CFP8_OUT_F32) hipLaunchKernelGGL((gemm_rowwise_gemv_kernel<NI, true>), grid, dim3(256), 0, st, p);
+        else hipLaunchKernelGGL((gemm_rowwise_gemv_kernel<NI, false>), grid, dim3(256), 0, st, p);
+    }
+}
 static int launch_rowwise_gemv(GemmArgs& p, int out_dtype, hipStream_t st) {
     const int64_t blocks = (p.N + 15) / 16;
     if (!note_launch("gemm_rowwise_gemv", (unsigned)blocks, 256, 0)) return CFP8_OK;
-    if (out_dtype == CFP8_OUT_F32) hipLaunchKernelGGL(gemm_rowwise_gemv_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, st, p);
-    else hipLaunchKernelGGL(gemm_rowwise_gemv_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, st, p);
+    const int steps = ((p.K >> 7) + 3) / 4, chunks = (steps + 7) / 8;
+    launch_gemv_ni<8>((steps + chunks - 1) / chunks, dim3((unsigned)blocks), st, p, out_dtype);
     return check_launch("gemm");
 }
 
