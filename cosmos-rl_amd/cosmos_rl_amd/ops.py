@@ -500,12 +500,23 @@ def scaled_mm(a: torch.Tensor, b: torch.Tensor, scale_a: torch.Tensor, scale_b: 
     out = torch.empty((M, N), dtype=out_dtype, device=a.device)
     ld_a = a.stride(0) if M > 1 else K
     ld_b = b.stride(1) if N > 1 else K
-    _lib.check(_lib.load().cfp8_scaled_mm_rowwise(a.data_ptr(), ld_a, sa.data_ptr(), b.data_ptr(), ld_b,
-                                                 sb.data_ptr(), out.data_ptr(), N, _out_code(out_dtype),
-                                                 M, N, K, _stream()))
-    if bias is not None:
+    lib = _lib.load()
+    need = lib.cfp8_gemm_partial_bytes(_lib.DISPATCH_ROWWISE, M, N, K)
+    part = torch.empty(need, dtype=torch.uint8, device=a.device) if need else None
+    fused = _fused_bias(bias, N)
+    _lib.check(lib.cfp8_scaled_mm_rowwise_split(a.data_ptr(), ld_a, sa.data_ptr(), b.data_ptr(), ld_b, sb.data_ptr(), _ptr(fused), out.data_ptr(), N,
+                                                _out_code(out_dtype), M, N, K, _ptr(part), need, _stream()))
+    if bias is not None and fused is None:
         out = out + bias
     return out
+
+
+def _fused_bias(bias: Optional[torch.Tensor], n: int) -> Optional[torch.Tensor]:
+    """The bias as the GEMM epilogues take it - one bf16 value per column - or None."""
+    if bias is None or bias.dtype != torch.bfloat16 or bias.dim() != 1 or bias.shape[0] != n or not bias.is_cuda:
+        return None
+    bias = bias.contiguous()
+    return bias if bias.data_ptr() % 8 == 0 else None
 
 
 def fp8_linear(x: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor,
@@ -529,19 +540,21 @@ def fp8_linear(x: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor
     lib = _lib.load()
     need = lib.cfp8_linear_workspace_bytes(M, K)
     if workspace is None or workspace.numel() * workspace.element_size() < need:
-        # the larger size lets the library split K where that pays (few weight rows, long K, 17..64 tokens)
-        workspace = torch.empty(max(lib.cfp8_linear_workspace_bytes_split(M, N, K), 256), dtype=torch.uint8, device=x.device)
+        # the larger size lets the library cut K into slices where that pays (few weight rows, long K)
+        need += lib.cfp8_gemm_partial_bytes(_lib.DISPATCH_ROWWISE, M, N, K)
+        workspace = torch.empty(max(need, 256), dtype=torch.uint8, device=x.device)
     sw = weight_scale.reshape(-1)
     if sw.dtype != torch.float32 or not sw.is_contiguous():
         sw = sw.contiguous().float()
     out = torch.empty((M, N), dtype=out_dtype, device=x.device)
     ld_x = x2.stride(0) if M > 1 else K
     ld_w = weight.stride(1) if N > 1 else K
-    _lib.check(lib.cfp8_linear_rowwise(x2.data_ptr(), ld_x, weight.data_ptr(), ld_w, sw.data_ptr(),
-                                      out.data_ptr(), N, _out_code(out_dtype), M, N, K,
-                                      workspace.data_ptr(), workspace.numel() * workspace.element_size(),
-                                      _stream()))
-    if bias is not None:
+    fused = _fused_bias(bias, N)
+    _lib.check(lib.cfp8_linear_rowwise_split(x2.data_ptr(), ld_x, weight.data_ptr(), ld_w, sw.data_ptr(), _ptr(fused),
+                                             out.data_ptr(), N, _out_code(out_dtype), M, N, K,
+                                             workspace.data_ptr(), workspace.numel() * workspace.element_size(),
+                                             _stream()))
+    if bias is not None and fused is None:
         out = out + bias
     return out.reshape(*x.shape[:-1], N)
 

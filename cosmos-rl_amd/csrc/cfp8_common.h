@@ -268,6 +268,19 @@ __device__ __forceinline__ u32 pack_bf16x2(float a, float b) {
     return __builtin_bit_cast(u32, __builtin_convertvector(v, bf16x2_t));
 }
 
+// four scaled sums plus a bias of four packed bf16, as an output of the GEMMs: with bf16 output the product is rounded
+// first and the sum again, what adding the bias to a bf16 product gives; kNoBias (-0.0) leaves every value as it is
+constexpr u32 kNoBias = 0x80008000u;
+template <bool OUT_F32>
+__device__ __forceinline__ f32x4 plus_bias(f32x4 v, u32 b0, u32 b1) {
+    if (!OUT_F32) {
+        const u32 p0 = pack_bf16x2(v[0], v[1]), p1 = pack_bf16x2(v[2], v[3]);
+        v = f32x4{bf16_lo(p0), bf16_hi(p0), bf16_lo(p1), bf16_hi(p1)};
+    }
+    v[0] += bf16_lo(b0); v[1] += bf16_hi(b0); v[2] += bf16_lo(b1); v[3] += bf16_hi(b1);
+    return v;
+}
+
 // exp(t) as a fixed sequence of IEEE fp32 operations (range reduction by ln2 in two parts, Taylor
 // polynomial of degree 7 in Horner form with fused multiply-adds, exact scaling): every step is
 // correctly rounded, so a CPU that runs the same sequence gets the same bits.  |error| < 2 ulp.

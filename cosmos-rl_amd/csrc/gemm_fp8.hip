@@ -29,6 +29,7 @@
 
 #include "cfp8_common.h"
 #include "gemm_internal.h"
+#include "gemm_ring.h"
 
 namespace cfp8 {
 
@@ -638,11 +639,16 @@ __global__ __launch_bounds__(256) void gemm_rowwise_256_kernel(const GemmArgs p)
 // workgroup's wait for the few that have a tile in it.  Those tiles are cut into quarters of 128 x 128 instead, dealt
 // to all workgroups behind their last full tile and computed by the strip kernel's ring pipeline (same products in
 // the same order of K, same epilogue arithmetic: the same bits).
-template <int BM, int TN, bool OUT_F32>
+//
+// EDGE: the same for any M and N (N % 16 == 0), with a bias.  Descriptors end with their matrix: rows and columns beyond it
+// arrive as zeros, and the stores of the epilogue are issued in buffer form with an offset beyond the descriptor where
+// there is nothing to store, so that their number stays what the waits count on.  A remainder of at most 128 rows or
+// columns is not a row or column of tiles but of quarter tiles (p.edge_rows, p.edge_cols), dealt out behind those of the last round.
+template <int BM, int TN, bool OUT_F32, bool BIAS = false>
 __device__ __forceinline__ void rowwise_strip_block(const GemmArgs& p, uint8_t* const smem, const int m0, const int n0, const int t);
 
-template <bool OUT_F32>
-__global__ __launch_bounds__(256) void gemm_rowwise_256p_kernel(const GemmArgs p) {
+template <bool OUT_F32, bool EDGE>
+__device__ __forceinline__ void rowwise_256p(const GemmArgs& p) {
     constexpr int BM = 256, BN = 256;
     constexpr int XS = BM * 128, WS = BN * 128;
     constexpr int WBASE = 2 * XS;
@@ -669,8 +675,9 @@ __global__ __launch_bounds__(256) void gemm_rowwise_256p_kernel(const GemmArgs p
         n0 = tn * BN;
         const uint64_t aw = reinterpret_cast<uint64_t>(p.a) + ((uint64_t)m0 + (uint64_t)wave * 8) * (uint64_t)p.ld_a;
         const uint64_t bw = reinterpret_cast<uint64_t>(p.b) + ((uint64_t)n0 + (uint64_t)wave * 8) * (uint64_t)p.ld_b;
-        ra = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(aw), 0, 0xFFFFFFFF, 0x00020000);
-        rb = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(bw), 0, 0xFFFFFFFF, 0x00020000);
+        auto left = [](int64_t rows, int64_t ld) -> int { return rows <= 0 ? 0 : rows * ld < 0xEFFFFFFFll ? (int)(uint32_t)(rows * ld) : (int)0xEFFFFFFFu; };
+        ra = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(aw), 0, EDGE ? left((int64_t)p.M - m0 - wave * 8, p.ld_a) : (int)0xFFFFFFFF, 0x00020000);
+        rb = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(bw), 0, EDGE ? left((int64_t)p.N - n0 - wave * 8, p.ld_b) : (int)0xFFFFFFFF, 0x00020000);
     };
     auto dma_x = [&](__amdgpu_buffer_rsrc_t r, int kt, int stage, int i) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)(smem + stage * XS + (wave + 4 * i) * 1024), 16, va_lane,
@@ -764,12 +771,18 @@ __global__ __launch_bounds__(256) void gemm_rowwise_256p_kernel(const GemmArgs p
             if (kt == last) {
                 // the weight stage of this step stays free for the epilogue; it takes the tile's scales now
                 uint8_t* dst = smem + WBASE + ws * WS + 24576 + wave * 256;
+                const int rows = p.M - m0 - wave * 64, cols = p.N - n0 - wave * 64;
                 const __amdgpu_buffer_rsrc_t rsa = __builtin_amdgcn_make_buffer_rsrc(
-                    const_cast<float*>(p.sa) + m0 + wave * 64, 0, 0xFFFFFFFF, 0x00020000);
+                    const_cast<float*>(p.sa) + m0 + wave * 64, 0, EDGE ? (rows > 0 ? rows * 4 : 0) : (int)0xFFFFFFFF, 0x00020000);
                 const __amdgpu_buffer_rsrc_t rsb = __builtin_amdgcn_make_buffer_rsrc(
-                    const_cast<float*>(p.sb) + n0 + wave * 64, 0, 0xFFFFFFFF, 0x00020000);
+                    const_cast<float*>(p.sb) + n0 + wave * 64, 0, EDGE ? (cols > 0 ? cols * 4 : 0) : (int)0xFFFFFFFF, 0x00020000);
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, (lds_void*)dst, 4, (uint32_t)lane * 4u, 0, 0, 0);
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rsb, (lds_void*)(dst + 1024), 4, (uint32_t)lane * 4u, 0, 0, 0);
+                if constexpr (EDGE) {  // the bias of the wave's 64 columns, two a lane
+                    const __amdgpu_buffer_rsrc_t rsc = __builtin_amdgcn_make_buffer_rsrc(
+                        const_cast<uint16_t*>(p.bias) + n0 + wave * 64, 0, p.bias && cols > 0 ? (cols < 64 ? cols * 2 : 128) : 0, 0x00020000);
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsc, (lds_void*)(dst + 2048), 4, (uint32_t)lane * 4u, 0, 0, 0);
+                }
                 ws_free = ws;
             }
 #pragma unroll
@@ -804,6 +817,26 @@ __global__ __launch_bounds__(256) void gemm_rowwise_256p_kernel(const GemmArgs p
         f32x4 sbn[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) sbn[i] = *reinterpret_cast<const f32x4*>(scale_lds + 256 + wn * 128 + i * 16 + quarter * 4);
+        // EDGE: the tile's part of the output, ending with the matrix; the bias as packed bf16
+        __amdgpu_buffer_rsrc_t ro;
+        uint2 bia[8];
+        if constexpr (EDGE) {
+            constexpr int ES = OUT_F32 ? 4 : 2;
+            const int64_t rows = p.M - m0 < BM ? p.M - m0 : BM;
+            ro = __builtin_amdgcn_make_buffer_rsrc(static_cast<uint8_t*>(p.out) + ((int64_t)m0 * p.ld_out + n0) * ES, 0,
+                                                   (int)(uint32_t)(((rows - 1) * p.ld_out + (p.N - n0)) * ES), 0x00020000);
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                bia[i] = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint8_t*>(scale_lds) + 2048 + (wn * 2 + (i >> 2)) * 256 +
+                                                         (i & 3) * 32 + quarter * 8);
+        }
+        auto value = [&](int i, int j) {
+            f32x4 v = acc[i][j];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = v[e] * sam[j] * sbn[i][e];
+            if constexpr (EDGE) v = plus_bias<OUT_F32>(v, bia[i].x, bia[i].y);
+            return v;
+        };
         if (OUT_F32) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
@@ -811,9 +844,11 @@ __global__ __launch_bounds__(256) void gemm_rowwise_256p_kernel(const GemmArgs p
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
                     const int m = m0 + wm * 128 + j * 16 + lrow;
-                    f32x4 v = acc[i][j];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = v[e] * sam[j] * sbn[i][e];
+                    const f32x4 v = value(i, j);
+                    if constexpr (EDGE)
+                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), ro,
+                                                               n < p.N ? ((uint32_t)(m - m0) * (uint32_t)p.ld_out + (uint32_t)(n - n0)) * 4u : 0xF0000000u, 0, 2);
+                    else
                     __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(static_cast<float*>(p.out) + (int64_t)m * p.ld_out + n));
                 }
             }
@@ -827,9 +862,7 @@ __global__ __launch_bounds__(256) void gemm_rowwise_256p_kernel(const GemmArgs p
             for (int j = 0; j < 8; ++j) {
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
-                    f32x4 v = acc[i][j];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = v[e] * sam[j] * sbn[i][e];
+                    const f32x4 v = value(i, j);
                     // written as an instruction: in front of an LDS store it knows of, the compiler waits for the loads
                     // of the next tile that are still on their way into other parts of LDS
                     const uint64_t two = (uint64_t)pack_bf16x2(v[0], v[1]) | ((uint64_t)pack_bf16x2(v[2], v[3]) << 32);
@@ -841,6 +874,11 @@ __global__ __launch_bounds__(256) void gemm_rowwise_256p_kernel(const GemmArgs p
                     const int row = r * 4 + rd_row;
                     const i32x4 d = *reinterpret_cast<const i32x4*>(ebuf + row * EST + rd_chunk * 16);
                     const int m = m0 + wm * 128 + j * 16 + row;
+                    if constexpr (EDGE) {
+                        const int n = wn * 128 + rd_chunk * 8;
+                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, d), ro,
+                                                               n < p.N - n0 ? ((uint32_t)(m - m0) * (uint32_t)p.ld_out + (uint32_t)n) * 2u : 0xF0000000u, 0, 2);
+                    } else
                     __builtin_nontemporal_store(
                         d, reinterpret_cast<i32x4*>(static_cast<uint16_t*>(p.out) + (int64_t)m * p.ld_out + n0 + wn * 128 + rd_chunk * 8));
                 }
@@ -877,13 +915,29 @@ __global__ __launch_bounds__(256) void gemm_rowwise_256p_kernel(const GemmArgs p
     for (unsigned i = 0; i < sizeof(GemmArgs) / 4; ++i) copy[i] = words[i];
     GemmArgs late;
     __builtin_memcpy(&late, copy, sizeof(late));
-    for (int u = (int)blockIdx.x; u < 4 * late.tail_tiles; u += (int)gridDim.x) {
+    const int units = 4 * late.tail_tiles + (EDGE ? late.edge_rows + late.edge_cols : 0);
+    for (int u = (int)blockIdx.x; u < units; u += (int)gridDim.x) {
         __syncthreads();  // every wave is done with the stages (the last tile's epilogue buffer, the quarter before)
+        if constexpr (EDGE) {
+            // the remainders: edge_rows quarter tiles below the last row of tiles, edge_cols beside their last column
+            const int e = u - 4 * late.tail_tiles;
+            if (e >= 0) {
+                const int me = e < late.edge_rows ? late.tiles_m * BM : (e - late.edge_rows) * 128;
+                const int ne = e < late.edge_rows ? e * 128 : late.tiles_n * BN;
+                rowwise_strip_block<128, 8, OUT_F32, true>(late, smem, me, ne, t_late);
+                continue;
+            }
+        }
         int tm, tn;
         tile_of_block(late.tiles_m * late.tiles_n - late.tail_tiles + (u >> 2), late.tiles_m, late.tiles_n, tm, tn);
-        rowwise_strip_block<128, 8, OUT_F32>(late, smem, tm * BM + (u & 1) * 128, tn * BN + ((u >> 1) & 1) * 128, t_late);
+        rowwise_strip_block<128, 8, OUT_F32, EDGE>(late, smem, tm * BM + (u & 1) * 128, tn * BN + ((u >> 1) & 1) * 128, t_late);
     }
 }
+
+template <bool OUT_F32>
+__global__ __launch_bounds__(256) void gemm_rowwise_256p_kernel(const GemmArgs p) { rowwise_256p<OUT_F32, false>(p); }
+template <bool OUT_F32>
+__global__ __launch_bounds__(256) void gemm_rowwise_edge_kernel(const GemmArgs p) { rowwise_256p<OUT_F32, true>(p); }
 
 // ---------------------------------------------------------------------------
 // The same pipeline on 256 x 128 tiles (256 activation rows, 128 weight rows), for problems whose 256 x 256
@@ -1806,6 +1860,60 @@ static int launch_rowwise_256p(GemmArgs& p, int out_dtype, hipStream_t st) {
     return check_launch("gemm");
 }
 
+// The edge form's division of a problem: a remainder of rows (and of columns) is either a last row of whole tiles or quarter
+// tiles.  The estimated times, in microseconds a K step: a whole tile on every CU 1.35, a quarter tile 0.5, or 1.0 for
+// quarters of a row remainder, which read all of the weight again (8192 x 18944 x 3584, nine rounds and one of quarters, 405
+// us; 1111 x 37888 x 3584 180 us with 87 rows as quarters, 2.3 rounds of tiles and 2.4 of quarters).
+struct EdgePlan {
+    int tiles_m, tiles_n, tail, edge_rows, edge_cols;
+    double cost;
+};
+static EdgePlan edge_plan(int64_t M, int64_t N, int64_t K, int cus) {
+    EdgePlan best{};
+    best.cost = 1e30;
+    const double whole = (double)(K / 128) * 1.35 + 6.0;
+    for (int up = 0; up < 4; ++up) {
+        const int64_t tm = M / 256 + (up & 1), tn = N / 256 + (up >> 1);
+        if (up & 1 ? M % 256 == 0 : M % 256 > 128) continue;  // (quarter tiles: one row of them at most)
+        if (up & 2 ? N % 256 == 0 : N % 256 > 128) continue;
+        const int64_t tiles = tm * tn, rem = tiles % cus;
+        if (tiles < cus || tiles > 0x7FFFFFFFll) continue;
+        const int64_t rows = M > tm * 256 ? (N + 127) / 128 : 0;
+        const int64_t cols = N > tn * 256 ? ((M < tm * 256 ? M : tm * 256) + 127) / 128 : 0;
+        const double quarter = (double)(K / 128) * (rows ? 1.0 : 0.5) + 4.0;
+        for (int64_t tail = 0; tail <= rem; tail += rem ? rem : 1) {
+            const int64_t units = 4 * tail + rows + cols;
+            const double cost = 4.0 + (double)((tiles - tail + cus - 1) / cus) * whole + (double)((units + cus - 1) / cus) * quarter;
+            if (cost < best.cost) best = EdgePlan{(int)tm, (int)tn, (int)tail, (int)rows, (int)cols, cost};
+        }
+    }
+    return best;
+}
+static bool edge_takes(const GemmArgs& p, int out_dtype) {
+    return p.K % 128 == 0 && p.K >= 384 && p.ld_a < (1 << 21) && p.ld_b < (1 << 21) && p.ld_out < (1 << 20) && aligned16(p.out) &&
+           (p.ld_out * (out_dtype == CFP8_OUT_F32 ? 4 : 2)) % 16 == 0 && (reinterpret_cast<uintptr_t>(p.bias) & 7u) == 0;
+}
+static int launch_rowwise_edge(GemmArgs& p, const EdgePlan& e, int out_dtype, hipStream_t st) {
+    p.tiles_m = e.tiles_m; p.tiles_n = e.tiles_n;
+    p.tail_tiles = e.tail; p.edge_rows = e.edge_rows; p.edge_cols = e.edge_cols;
+    constexpr size_t lds = (size_t)(2 + 3) * 256 * 128;
+    static std::atomic<bool> raised[65][2];  // zero-initialised
+    const int v = out_dtype == CFP8_OUT_F32 ? 1 : 0;
+    const void* fn = v ? reinterpret_cast<const void*>(gemm_rowwise_edge_kernel<true>) : reinterpret_cast<const void*>(gemm_rowwise_edge_kernel<false>);
+    const int slot = device_slot();
+    if (slot == 64) raised[64][v].store(false, std::memory_order_relaxed);
+    if (int rc = raise_lds_limit(fn, lds, raised[slot][v])) return rc;
+    const unsigned blocks = (unsigned)cu_count();
+    {
+        char name[80];
+        snprintf(name, sizeof(name), "gemm_rowwise_edge tail=%d edges=%d", e.tail, e.edge_rows + e.edge_cols);
+        if (!note_launch(name, blocks, 256, lds)) return CFP8_OK;
+    }
+    if (v) hipLaunchKernelGGL(gemm_rowwise_edge_kernel<true>, dim3(blocks), dim3(256), lds, st, p);
+    else hipLaunchKernelGGL(gemm_rowwise_edge_kernel<false>, dim3(blocks), dim3(256), lds, st, p);
+    return check_launch("gemm");
+}
+
 static int launch_rowwise_256x128(GemmArgs& p, int out_dtype, hipStream_t st) {
     p.tiles_m = p.M / 256;
     p.tiles_n = p.N / 128;
@@ -2055,6 +2163,10 @@ __global__ __launch_bounds__(256) void gemm_rowwise_gemv_kernel(const GemmArgs p
             f32x4 v;
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] = acc[e] * sam * sbn[e];
+            if (p.bias) {
+                const uint2 b = *reinterpret_cast<const uint2*>(p.bias + n);
+                v = plus_bias<OUT_F32>(v, b.x, b.y);
+            }
             if (OUT_F32) *reinterpret_cast<f32x4*>(static_cast<float*>(p.out) + (int64_t)m * p.ld_out + n) = v;
             else *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.out) + (int64_t)m * p.ld_out + n) =
                     make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
@@ -2163,6 +2275,10 @@ __global__ __launch_bounds__(256) void linear_gemv_fused_kernel(const uint4* __r
             f32x4 o;
 #pragma unroll
             for (int e = 0; e < 4; ++e) o[e] = acc[e] * sam * sbn[e];
+            if (p.bias) {
+                const uint2 b = *reinterpret_cast<const uint2*>(p.bias + n);
+                o = plus_bias<OUT_F32>(o, b.x, b.y);
+            }
             if (OUT_F32) *reinterpret_cast<f32x4*>(static_cast<float*>(p.out) + (int64_t)m * p.ld_out + n) = o;
             else *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.out) + (int64_t)m * p.ld_out + n) =
                     make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
@@ -2223,7 +2339,7 @@ static int launch_rowwise_gemv(GemmArgs& p, int out_dtype, hipStream_t st) {
 // Rows beyond M and N are not fetched: the descriptors end with the matrix and a direct-to-LDS load writes zero for a
 // lane beyond its descriptor.  Wave w computes token rows w BM / 4 ... against all TN weight tiles.
 // ---------------------------------------------------------------------------
-template <int BM, int TN, bool OUT_F32>
+template <int BM, int TN, bool OUT_F32, bool BIAS>
 __device__ __forceinline__ void rowwise_strip_block(const GemmArgs& p, uint8_t* const smem, const int m0, const int n0, const int t) {
     constexpr int BN = TN * 16;
     constexpr int WROWS = (BN + 31) / 32 * 32;          // weight rows requested per step: 8 per wave and load
@@ -2284,6 +2400,16 @@ __device__ __forceinline__ void rowwise_strip_block(const GemmArgs& p, uint8_t* 
         const int n = n0 + i * 16 + quarter * 4;
         sbn[i] = *(const gbl_f32x4*)(sb_g + (n < p.N ? n : 0));
     }
+    typedef __attribute__((address_space(1))) const u32x2 gbl_u32x2;
+    typedef __attribute__((address_space(1))) const uint16_t gbl_u16;
+    u32x2 bia[BIAS ? TN : 1];
+    if (BIAS) {
+#pragma unroll
+        for (int i = 0; i < TN; ++i) {
+            const int n = n0 + i * 16 + quarter * 4;
+            bia[i] = p.bias ? *(const gbl_u32x2*)((const gbl_u16*)p.bias + (n < p.N ? n : 0)) : u32x2{kNoBias, kNoBias};
+        }
+    }
 
     f32x4 acc[TN][XT];
 #pragma unroll
@@ -2343,6 +2469,7 @@ __device__ __forceinline__ void rowwise_strip_block(const GemmArgs& p, uint8_t* 
             f32x4 v;
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] = acc[i][j][e] * sam[j] * sbn[i][e];
+            if (BIAS) v = plus_bias<OUT_F32>(v, bia[i][0], bia[i][1]);
             typedef __attribute__((address_space(1))) f32x4 gbl_out4;
             typedef __attribute__((address_space(1))) u32x2 gbl_out2;
             typedef __attribute__((address_space(1))) float gbl_outf;
@@ -3201,6 +3328,77 @@ static int launch_gemm(GemmArgs& p, int out_dtype, hipStream_t st) {
     return launch_cfg<256, 256, 2, 4, kRowwise>(p, out_dtype, st);
 }
 
+// out += bias in place, for the kernels that do not take a bias themselves
+template <bool OUT_F32>
+__global__ __launch_bounds__(256) void bias_rows_kernel(void* out, int64_t ld_out, const uint16_t* __restrict__ bias, int M, int nq) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;  // one thread per 4 consecutive columns
+    if (i >= (int64_t)M * nq) return;
+    const int64_t m = i / nq, n = (i - m * nq) * 4;
+    const uint2 b = *reinterpret_cast<const uint2*>(bias + n);
+    if (OUT_F32) {
+        f32x4* const o = reinterpret_cast<f32x4*>(static_cast<float*>(out) + m * ld_out + n);
+        f32x4 v = *o;
+        v[0] += bf16_lo(b.x); v[1] += bf16_hi(b.x); v[2] += bf16_lo(b.y); v[3] += bf16_hi(b.y);
+        *o = v;
+    } else {
+        uint2* const o = reinterpret_cast<uint2*>(static_cast<uint16_t*>(out) + m * ld_out + n);
+        const uint2 v = *o;
+        *o = make_uint2(pack_bf16x2(bf16_lo(v.x) + bf16_lo(b.x), bf16_hi(v.x) + bf16_hi(b.x)),
+                        pack_bf16x2(bf16_lo(v.y) + bf16_lo(b.y), bf16_hi(v.y) + bf16_hi(b.y)));
+    }
+}
+
+// Rowwise product with a bias and memory for partial sums: the form with the least estimated time among the ring kernel
+// (gemm_ring.hip), the walking 256 x 256 tiles with edges, and, up to 128 tokens, the weight streamers of launch_gemm.
+// The streamers' estimates, in microseconds: up to 16 tokens the larger of the weights' way in (token rows come from L2 beside
+// them) and the chunks of K one after the other, beyond that rounds of strips times K steps.  Timed with weights that no cache
+// holds, ring / launch_gemm: 739 x 1024 x 1024 5.8 / 21.7 us, 152 x 1792 x 12672 17 / 88, 1061 x 2560 x 7936 40 / 75, 637 x
+// 18944 x 3584 63 / 64, 21 x 896 x 17152 11 / 33, 42 x 32768 x 2560 20 / 28; 33 x 37888 x 3584, two full rounds of strips,
+// 37 / 30.
+static int launch_rowwise_best(GemmArgs& p, int out_dtype, hipStream_t st) {
+    const int cus = cu_count();
+    RingArgs r{};
+    r.a = p.a; r.w = p.b; r.sa = p.sa; r.sb = p.sb; r.bias = p.bias; r.out = p.out;
+    r.partial = p.partial;
+    r.ld_a = p.ld_a; r.ld_w = p.ld_b; r.ld_out = p.ld_out;
+    r.M = p.M; r.N = p.N; r.K = p.K;
+    RingPlan ring{0, 0, 0, 1e30};
+    if (ring_takes(kRingRow, r, out_dtype)) ring = ring_plan(kRingRow, p.M, p.N, p.K, p.partial_bytes, cus);
+    EdgePlan edge{};
+    edge.cost = 1e30;
+    if (p.M > 128 && edge_takes(p, out_dtype)) edge = edge_plan(p.M, p.N, p.K, cus);
+    double stream = 1e30;
+    if (p.M <= 128 && p.K % 128 == 0) {
+        const double kt = p.K / 128, bytes = (double)p.N * p.K;
+        auto rounds = [&](int rows) { return (double)(((int64_t)(p.N + rows - 1) / rows + cus - 1) / cus); };
+        const bool narrow = (p.N + 79) / 80 < 128;
+        if (p.M <= 16) {
+            const double chunks = (p.K / 128 + 31) / 32, latency = chunks * (2.4 + 0.1 * p.M), stream_in = bytes * (1 + p.M / 32.0) / 5.4e6;
+            stream = 2.0 + (latency > stream_in ? latency : stream_in);
+        } else {
+            const double step = p.M <= 64 ? (narrow ? 0.22 : 0.50) : (narrow ? 0.32 : 0.85), in = bytes / 4.7e6;
+            const double run = rounds(narrow ? 32 : 80) * kt * step;
+            stream = 3.5 + (run > in ? run : in);
+            if (p.bias) stream += 4.0;
+        }
+    }
+    if (ring.cost < 1e30 && ring.cost <= edge.cost && ring.cost <= stream) return launch_ring(kRingRow, r, ring, out_dtype, st);
+    // (without a bias and without remainders launch_gemm's form of the same tiles is 2 % faster)
+    const bool even = p.M % 256 == 0 && p.N % 256 == 0 && !p.bias;
+    if (edge.cost < 1e30 && edge.cost <= stream && !even) return launch_rowwise_edge(p, edge, out_dtype, st);
+    float* const partial = p.partial;
+    p.partial = nullptr;  // (launch_gemm's own slices are those of cfp8_linear_rowwise)
+    if (int rc = launch_gemm<kRowwise>(p, out_dtype, st)) return rc;
+    p.partial = partial;
+    if (!p.bias || (p.M <= 16 && p.K % 128 == 0)) return CFP8_OK;  // (the kernel for 16 tokens takes the bias itself)
+    const int64_t blocks = ((int64_t)p.M * (p.N / 4) + 255) / 256;
+    if (blocks > 0x7FFFFFFFll) return set_error(CFP8_EINVAL, "gemm: too large for one launch");
+    if (!note_launch("bias_rows", (unsigned)blocks, 256, 0)) return CFP8_OK;
+    if (out_dtype == CFP8_OUT_F32) hipLaunchKernelGGL(bias_rows_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, st, p.out, p.ld_out, p.bias, p.M, p.N / 4);
+    else hipLaunchKernelGGL(bias_rows_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, st, p.out, p.ld_out, p.bias, p.M, p.N / 4);
+    return check_launch("gemm");
+}
+
 static int check_common(const char* who, const void* a, const void* b, const float* sa, const float* sb,
                         const void* out, int64_t ld_a, int64_t ld_b, int64_t ld_out, int out_dtype, int64_t M,
                         int64_t N, int64_t K, int k_unit = 128) {
@@ -3313,6 +3511,30 @@ extern "C" int cfp8_scaled_mm_rowwise(const void* a, int64_t ld_a, const float* 
     return launch_gemm<kRowwise>(p, out_dtype, static_cast<hipStream_t>(stream));
 }
 
+extern "C" int cfp8_scaled_mm_rowwise_split(const void* a, int64_t ld_a, const float* sa, const void* b, int64_t ld_b,
+                                            const float* sb, const void* bias, void* out, int64_t ld_out, int out_dtype, int64_t M,
+                                            int64_t N, int64_t K, void* workspace, size_t workspace_bytes, void* stream) {
+    using namespace cfp8;
+    if (int rc = check_common("scaled_mm_rowwise_split", a, b, sa, sb, out, ld_a, ld_b, ld_out, out_dtype, M, N, K, 16)) return rc;
+    if (M == 0 || N == 0) return CFP8_OK;
+    if (reinterpret_cast<uintptr_t>(bias) & 7u) return set_error(CFP8_EINVAL, "scaled_mm_rowwise_split: bias must be 8-byte aligned");
+    if (workspace_bytes && (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 255u)))
+        return set_error(CFP8_EINVAL, "scaled_mm_rowwise_split: workspace must be 256-byte aligned");
+    if (int rc = check_device()) return rc;
+    GemmArgs p{};
+    p.a = static_cast<const uint8_t*>(a);
+    p.b = static_cast<const uint8_t*>(b);
+    p.sa = sa;
+    p.sb = sb;
+    p.bias = static_cast<const uint16_t*>(bias);
+    p.out = out;
+    p.ld_a = ld_a; p.ld_b = ld_b; p.ld_out = ld_out;
+    p.M = (int)M; p.N = (int)N; p.K = (int)K;
+    p.partial = static_cast<float*>(workspace);
+    p.partial_bytes = workspace_bytes;
+    return launch_rowwise_best(p, out_dtype, static_cast<hipStream_t>(stream));
+}
+
 extern "C" size_t cfp8_linear_workspace_bytes(int64_t M, int64_t K) {
     if (M <= 0 || K <= 0) return 0;
     const size_t q = ((size_t)M * (size_t)K + 255) & ~(size_t)255;
@@ -3363,6 +3585,39 @@ extern "C" int cfp8_linear_rowwise(const void* x, int64_t ld_x, const void* w, i
     p.partial = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + base);
     p.partial_bytes = workspace_bytes - base;
     return launch_gemm<kRowwise>(p, out_dtype, st);
+}
+
+extern "C" int cfp8_linear_rowwise_split(const void* x, int64_t ld_x, const void* w, int64_t ld_w, const float* w_scale, const void* bias,
+                                         void* out, int64_t ld_out, int out_dtype, int64_t M, int64_t N, int64_t K,
+                                         void* workspace, size_t workspace_bytes, void* stream) {
+    using namespace cfp8;
+    if (M < 0 || N < 0 || K <= 0) return set_error(CFP8_EINVAL, "linear_rowwise_split: bad shape");
+    if (M == 0 || N == 0) return CFP8_OK;
+    const size_t base = cfp8_linear_workspace_bytes(M, K);
+    if (!workspace || workspace_bytes < base)
+        return set_error(CFP8_EWORKSPACE, "linear_rowwise_split: workspace of %zu bytes needed, %zu given", base, workspace_bytes);
+    if (reinterpret_cast<uintptr_t>(workspace) & 255u) return set_error(CFP8_EINVAL, "linear_rowwise_split: workspace must be 256-byte aligned");
+    if (!x || !aligned16(x) || ld_x % 8 || ld_x < K) return set_error(CFP8_EINVAL, "linear_rowwise_split: bad activation pointer or leading dimension");
+    if (reinterpret_cast<uintptr_t>(bias) & 7u) return set_error(CFP8_EINVAL, "linear_rowwise_split: bias must be 8-byte aligned");
+    uint8_t* qx = static_cast<uint8_t*>(workspace);
+    float* sx = reinterpret_cast<float*>(qx + (((size_t)M * (size_t)K + 255) & ~(size_t)255));
+    if (int rc = check_common("linear_rowwise_split", qx, w, sx, w_scale, out, K, ld_w, ld_out, out_dtype, M, N, K, 16)) return rc;
+    if (int rc = check_device()) return rc;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    GemmArgs p{};
+    p.a = qx;
+    p.b = static_cast<const uint8_t*>(w);
+    p.sa = sx;
+    p.sb = w_scale;
+    p.bias = static_cast<const uint16_t*>(bias);
+    p.out = out;
+    p.ld_a = K; p.ld_b = ld_w; p.ld_out = ld_out;
+    p.M = (int)M; p.N = (int)N; p.K = (int)K;
+    p.partial = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + base);
+    p.partial_bytes = workspace_bytes - base;
+    if (fused_gemv_applies(M, K, x, ld_x)) return launch_linear_gemv_fused(x, ld_x, p, out_dtype, st);
+    if (int rc = launch_quant_rowwise(x, M, K, ld_x, qx, K, sx, false, st)) return rc;
+    return launch_rowwise_best(p, out_dtype, st);
 }
 
 extern "C" int cfp8_gemm_block128(const void* a, int64_t ld_a, const float* sa, const void* b, int64_t ld_b,

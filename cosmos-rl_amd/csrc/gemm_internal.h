@@ -32,6 +32,9 @@ struct GemmArgs {
     int unit_parts;
     // gemm_rowwise_256p_kernel: tiles of the last, at most half-full round, computed as quarter tiles by all workgroups
     int tail_tiles;
+    // gemm_rowwise_edge_kernel: bf16 [N] or null; quarter tiles below the last row of tiles and beside their last column
+    const uint16_t* bias;
+    int edge_rows, edge_cols;
 };
 
 // ---- host side (gemm_fp8.hip) ---------------------------------------------

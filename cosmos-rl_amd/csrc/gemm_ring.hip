@@ -18,10 +18,11 @@
 // the hand-written waits rely on, is the same everywhere.
 //
 // LDS layout of a stage: row-major, 16-byte chunk c of row r at position c ^ f(r).  A lane (row = lane & 15, q = lane >> 4)
-// of an e4m3 fragment reads chunks q and q + 4 - the K positions that go with an e2m1 lane's 32 codes, and as good as any
-// other two where both operands are e4m3.  The LDS serves a 16-byte read sixteen lanes at a time, lanes 0-3, 12-15, 20-23,
-// 24-27 first; f(r) = (bit 1 of r) << 1 | (bit 3 of r) << 2 puts those sixteen on sixteen different bank groups (128-byte
-// rows), and (bit 3 of r) << 1 does so for the 64-byte rows of e2m1.
+// of an e4m3 fragment reads chunks 2 q and 2 q + 1, as in the other FP8 kernels (so that an unsliced product has their
+// bits), against e2m1 weights chunks q and q + 4: the K positions that go with an e2m1 lane's 32 codes.  The LDS serves a
+// 16-byte read sixteen lanes at a time, lanes 0-3, 12-15, 20-23, 24-27 first; f(r) = bit 1 of r | (bit 3 of r) << 2 puts
+// those sixteen on sixteen different bank groups for the first pair of chunks, (bit 1 of r) << 1 | (bit 3 of r) << 2 for the
+// second, and (bit 3 of r) << 1 for the 64-byte rows of e2m1.
 //
 // What bounds it (1111 x 3584 x 18944 rowwise, 252 tiles of 128 x 128, 87 us where tiles of 256 x 128 took 156 us; compiled
 // out one at a time): the multiplications and fragment reads alone 48 us, the loads alone 85 us - 32 KiB a CU and step at 57 B/ns,
@@ -113,7 +114,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(w_at), 0, (int)w_end, 0x00020000);
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(s_at), 0, (int)s_end, 0x00020000);
     // a load of 8 rows x 128 bytes: row lane >> 3, whose chunk position lane & 7 holds chunk position ^ f(row)
-    const uint32_t c8 = (uint32_t)((lane & 7) ^ ((((lane >> 4) & 1) << 1) | ((wave & 1) << 2)));
+    constexpr int F1 = MODE == kRingMx ? 1 : 0;  // where bit 1 of the row goes
+    const uint32_t c8 = (uint32_t)((lane & 7) ^ ((((lane >> 4) & 1) << F1) | ((wave & 1) << 2)));
     const uint32_t va = (uint32_t)(lane >> 3) * (uint32_t)p.ld_a + c8 * 16;
     const uint32_t va_tail = tail && c8 * 16 >= (uint32_t)tail ? kOutside : va;  // the last step of a K that is no multiple of 128
     uint32_t vw, vw_tail, vs = kOutside;
@@ -141,10 +143,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
     };
 
     // fragments of 16 rows
-    const int xo = (wm * (BM / 2) + lrow) * 128 + ((quarter ^ ((((lrow >> 1) & 1) << 1) | (((lrow >> 3) & 1) << 2))) << 4);
+    const int fr = (((lrow >> 1) & 1) << F1) | (((lrow >> 3) & 1) << 2), c0 = MODE == kRingMx ? quarter : 2 * quarter;
+    const int xo = (wm * (BM / 2) + lrow) * 128 + ((c0 ^ fr) << 4);
     const int wo = MODE == kRingMx ? WB + (wn * (BN / 2) + lrow) * 64 + ((quarter ^ (((lrow >> 3) & 1) << 1)) << 4)
-                                   : WB + (wn * (BN / 2) + lrow) * 128 + ((quarter ^ ((((lrow >> 1) & 1) << 1) | (((lrow >> 3) & 1) << 2))) << 4);
-    const int xo2 = xo ^ 64, wo2 = wo ^ 64;  // the row's chunk q + 4 (a stage and a tile of rows begin on multiples of 128)
+                                   : WB + (wn * (BN / 2) + lrow) * 128 + ((c0 ^ fr) << 4);
+    constexpr int kOther = MODE == kRingMx ? 64 : 16;  // the lane's second chunk (a stage and a tile of rows begin on multiples of 128)
+    const int xo2 = xo ^ kOther, wo2 = wo ^ kOther;
     auto frag8 = [&](int at, int at2) {
         const i32x4 lo = *reinterpret_cast<const i32x4*>(smem + at);
         const i32x4 hi = *reinterpret_cast<const i32x4*>(smem + at2);
@@ -304,7 +308,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
         return;
     }
     float sam[TM];
-    f32x4 sbn[TN], bia[TN];
+    f32x4 sbn[TN];
+    uint2 bia[TN];
 #pragma unroll
     for (int j = 0; j < TM; ++j) {
         const int m = m0 + wm * (BM / 2) + j * 16 + lrow;
@@ -314,17 +319,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
     for (int i = 0; i < TN; ++i) {
         const int n = n0 + wn * (BN / 2) + i * 16 + quarter * 4, nn = n < p.N ? n : 0;
         sbn[i] = MODE == kRingRow ? *reinterpret_cast<const f32x4*>(p.sb + nn) : f32x4{1.f, 1.f, 1.f, 1.f};
-        bia[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (p.bias) {
-            const uint2 b = *reinterpret_cast<const uint2*>(p.bias + nn);
-            bia[i] = f32x4{bf16_lo(b.x), bf16_hi(b.x), bf16_lo(b.y), bf16_hi(b.y)};
-        }
+        bia[i] = p.bias ? *reinterpret_cast<const uint2*>(p.bias + nn) : make_uint2(kNoBias, kNoBias);
     }
     auto value = [&](int i, int j) {
         f32x4 v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = acc[i][j][e] * sam[j] * sbn[i][e] + bia[i][e];
-        return v;
+        for (int e = 0; e < 4; ++e) v[e] = acc[i][j][e] * sam[j] * sbn[i][e];
+        return plus_bias<OUT_F32>(v, bia[i].x, bia[i].y);
     };
     if constexpr (OUT_F32) {
 #pragma unroll
@@ -376,13 +377,10 @@ __global__ __launch_bounds__(256) void ring_reduce_kernel(const RingArgs p) {
     }
     const float sam = MODE != kRingBlock ? p.sa[m] : 1.f;
     const f32x4 sbn = MODE == kRingRow ? *reinterpret_cast<const f32x4*>(p.sb + n) : f32x4{1.f, 1.f, 1.f, 1.f};
-    f32x4 bia = {0.f, 0.f, 0.f, 0.f};
-    if (p.bias) {
-        const uint2 b = *reinterpret_cast<const uint2*>(p.bias + n);
-        bia = f32x4{bf16_lo(b.x), bf16_hi(b.x), bf16_lo(b.y), bf16_hi(b.y)};
-    }
+    const uint2 b = p.bias ? *reinterpret_cast<const uint2*>(p.bias + n) : make_uint2(kNoBias, kNoBias);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = v[e] * sam * sbn[e] + bia[e];
+    for (int e = 0; e < 4; ++e) v[e] = v[e] * sam * sbn[e];
+    v = plus_bias<OUT_F32>(v, b.x, b.y);
     if (OUT_F32) *reinterpret_cast<f32x4*>(static_cast<float*>(p.out) + (int64_t)m * p.ld_out + n) = v;
     else *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.out) + (int64_t)m * p.ld_out + n) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
 }
@@ -437,17 +435,17 @@ static int launch_ring_mode(RingArgs& p, const RingPlan& plan, int out_dtype, hi
 // The tile and the number of slices with the least estimated time.  The estimate is a fixed time per launch plus, per
 // round of workgroups on the CUs, K steps times the tile's step time (longer the more CUs load at once) plus the tile's
 // ends, not below the operands' bytes at the rate they come in; slices add the reduction's launch and their partial sums'
-// way out and back.  The constants are fitted to 1150 (rowwise), 1500 (block) and 1400 (MXFP4) timed combinations of 90
-// shapes each (1 .. 8192 tokens, weights of 896 .. 37888 rows, K 896 .. 18944): the choice is within 1 % of the best
-// combination on average, 13 % at worst.
+// way out and back.  The constants are fitted to all combinations of 120 shapes each (1 .. 8192 tokens, weights of 896 ..
+// 37888 rows, K 896 .. 18944), timed with operands that no cache holds: the choice is within 2 % of the best combination on
+// average, 20 % at worst.
 struct RingRates {
     double step[4], load[4];  // 128 x 128, 64 x 128, 128 x 64, 64 x 64: microseconds a step, and what a full GPU adds
     double launch, ends, partial, bytes, reduce;
 };
 static const RingRates kRates[3] = {
-    {{0.359, 0.207, 0.240, 0.131}, {0.336, 0.589, 0.233, 0.522}, 3.0, 2.0, 4.2, 4.7, 2.1},
-    {{0.579, 0.302, 0.460, 0.223}, {0.182, 0.443, 0.014, 0.320}, 3.5, 2.1, 5.0, 5.4, 2.3},
-    {{0.432, 0.328, 0.308, 0.182}, {0.177, 0.196, 0.028, 0.158}, 3.6, 2.1, 4.3, 4.4, 2.3},
+    {{0.560, 0.371, 0.388, 0.208}, {0.003, 0.108, 0.000, 0.293}, 2.3, 1.7, 3.8, 3.7, 2.8},
+    {{0.708, 0.388, 0.509, 0.230}, {0.000, 0.197, 0.000, 0.415}, 3.8, 2.3, 4.2, 4.4, 1.9},
+    {{0.631, 0.493, 0.399, 0.201}, {0.000, 0.150, 0.079, 0.323}, 3.4, 1.7, 3.6, 3.2, 2.3},
 };
 static const int kTiles[4][2] = {{128, 128}, {64, 128}, {128, 64}, {64, 64}};
 constexpr int kRingMaxSlices = 16;

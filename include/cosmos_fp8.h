@@ -345,6 +345,17 @@ int cfp8_gemm_mxfp4(const void* a, int64_t ld_a, const float* sa, const void* w,
 #define CFP8_DISPATCH_MXFP4 5
 size_t cfp8_gemm_partial_bytes(int kind, int64_t M, int64_t N, int64_t K);
 
+/* cfp8_scaled_mm_rowwise and cfp8_linear_rowwise with a bias (bf16 [N] or null, 8-byte aligned; added to the
+ * product as it would have been written, i.e. with bf16 output to the rounded product) and memory for partial sums; the second takes it behind the quantised activations, in a
+ * workspace of cfp8_linear_workspace_bytes(M, K) + cfp8_gemm_partial_bytes(CFP8_DISPATCH_ROWWISE, M, N, K) bytes or, with
+ * fewer slices, at least the first of the two. */
+int cfp8_scaled_mm_rowwise_split(const void* a, int64_t ld_a, const float* sa, const void* b, int64_t ld_b, const float* sb,
+                                 const void* bias, void* out, int64_t ld_out, int out_dtype, int64_t M, int64_t N, int64_t K,
+                                 void* workspace, size_t workspace_bytes, void* stream);
+int cfp8_linear_rowwise_split(const void* x, int64_t ld_x, const void* w, int64_t ld_w, const float* w_scale, const void* bias,
+                              void* out, int64_t ld_out, int out_dtype, int64_t M, int64_t N, int64_t K, void* workspace,
+                              size_t workspace_bytes, void* stream);
+
 /* cfp8_gemm_mxfp4 on one weight matrix with memory for partial sums. */
 int cfp8_gemm_mxfp4_split(const void* a, int64_t ld_a, const float* sa, const void* w, int64_t ld_w, const void* ws,
                           int64_t ld_ws, void* out, int64_t ld_out, int out_dtype, int64_t M, int64_t N, int64_t K,

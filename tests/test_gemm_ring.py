@@ -51,3 +51,42 @@ def test_mxfp4(dev, M, N, K):
             _lib.check(_lib.load().cfp8_gemm_mxfp4_split(q.data_ptr(), K, s.data_ptr(), w.data_ptr(), K // 2, ws.data_ptr(), K // 32, out.data_ptr(),
                                                          N + 8, ops._out_code(dtype), M, N, K, part.data_ptr(), have, _stream()))
             _check(out, want, M, N, dtype, 0.0)
+
+
+def _rowwise_want(q, s, w, sw, bias):
+    want = (q.double() * s.double().reshape(-1, 1)) @ (w.double() * sw.double().reshape(-1, 1)).t()
+    return (want if bias is None else want + bias.double()).cpu()
+
+
+# the shapes above, the walking tiles with remainders of rows and columns below, at and above half a tile, and a partial round
+@pytest.mark.parametrize("M,N,K", SHAPES + TAILS + [(1, 400, 1152), (3, 272, 4864), (16, 144, 4224), (90, 10256, 128), (4000, 4112, 384), (4096 + 120, 4096 + 112, 512),
+                                                    (4096 + 130, 4096 + 144, 384), (2100, 9216, 640), (8000, 4352, 512)])
+@pytest.mark.parametrize("biased", [False, True])
+def test_rowwise(dev, M, N, K, biased):
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g, device=dev).to(torch.bfloat16)
+    q, s = ops.quant_rowwise(x)
+    w, sw = ops.quant_rowwise((torch.randn(N, K, generator=g, device=dev) * 0.05).to(torch.bfloat16))
+    bias = torch.randn(N, generator=g, device=dev).to(torch.bfloat16) if biased else None
+    want = _rowwise_want(q, s, w, sw, bias)
+    part, need = _partial(_lib.DISPATCH_ROWWISE, M, N, K, dev)
+    for dtype in (torch.float32, torch.bfloat16):
+        for have in {0, need // 2, need}:
+            out = _out(M, N, dev, dtype)
+            _lib.check(_lib.load().cfp8_scaled_mm_rowwise_split(q.data_ptr(), K, s.data_ptr(), w.data_ptr(), K, sw.data_ptr(), ops._ptr(bias),
+                                                                out.data_ptr(), N + 8, ops._out_code(dtype), M, N, K, part.data_ptr(), have, _stream()))
+            # (a bf16 product is rounded before the bias is added and the sum again: 2^-9 of it more at most)
+            _check(out, want, M, N, dtype, 2.0 ** -9 if biased and dtype == torch.bfloat16 else 0.0)
+            y = ops.fp8_linear(x, w.t(), sw, bias=bias, out_dtype=dtype)
+            if have == need:
+                assert torch.equal(y, out[:M, :N])
+                if biased:
+                    assert torch.equal(y, ops.fp8_linear(x, w.t(), sw, out_dtype=dtype) + bias)
+
+
+def test_rowwise_bias_of_another_kind(dev):
+    """A bias that no epilogue takes (fp32) is added as torch adds it."""
+    x = torch.randn(5, 256, device=dev).to(torch.bfloat16)
+    w, sw = ops.quant_rowwise(torch.randn(48, 256, device=dev).to(torch.bfloat16))
+    b = torch.randn(48, device=dev)
+    assert torch.equal(ops.fp8_linear(x, w.t(), sw, bias=b), ops.fp8_linear(x, w.t(), sw) + b)
