@@ -91,6 +91,8 @@ SIGNATURES = {
                                           c_int64, c_void_p, c_size_t, c_void_p]),
     "cfp8_gemm_block128": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_int64,
                                    c_void_p, c_int64, c_int, c_int64, c_int64, c_int64, c_void_p]),
+    "cfp8_gemm_block128_split": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_int64,
+                                         c_void_p, c_int64, c_int, c_int64, c_int64, c_int64, c_void_p, c_size_t, c_void_p]),
     "cfp8_gemm_dispatch_info": (c_int, [c_int, c_int64, c_int64, c_int64, c_int, c_int, c_int, c_char_p, c_size_t]),
     "cfp8_gemm_grouped_block128": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                            c_int64, c_int, c_int64, c_int64, c_int64, c_int64, c_void_p]),

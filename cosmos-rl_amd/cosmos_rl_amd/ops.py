@@ -585,9 +585,12 @@ def gemm_fp8_fp8_bf16_nt(lhs: Tuple[torch.Tensor, torch.Tensor], rhs: Tuple[torc
         raise ValueError(f"lhs scales must be [{M}, {kb}], got {tuple(sa.shape)}")
     if not out.is_contiguous():
         raise ValueError("out must be contiguous")
-    _lib.check(_lib.load().cfp8_gemm_block128(a.data_ptr(), K, sa.data_ptr(), b.data_ptr(), K, sb.data_ptr(),
-                                             stride_n, stride_k, out.data_ptr(), N, _out_code(out.dtype),
-                                             M, N, K, _stream()))
+    lib = _lib.load()
+    partial = lib.cfp8_gemm_partial_bytes(_lib.DISPATCH_BLOCK, M, N, K)
+    work = torch.empty(partial, dtype=torch.uint8, device=a.device) if partial else None
+    _lib.check(lib.cfp8_gemm_block128_split(a.data_ptr(), K, sa.data_ptr(), b.data_ptr(), K, sb.data_ptr(),
+                                            stride_n, stride_k, out.data_ptr(), N, _out_code(out.dtype),
+                                            M, N, K, _ptr(work), partial, _stream()))
     return out
 
 

@@ -3399,6 +3399,72 @@ static int launch_rowwise_best(GemmArgs& p, int out_dtype, hipStream_t st) {
     return check_launch("gemm");
 }
 
+// Block-scaled product with memory for partial sums, the least of three estimates (microseconds):
+//   ring    the ring kernel (gemm_ring.hip) on all rows
+//   middle  the register-staged 128 x 128 tiles of launch_gemm, two workgroups a CU: 1.55 a K step with two of them, 0.7 to 1.0
+//           with one
+//   full    launch_gemm's full tiles on the first M / 256 * 256 rows, 2.05 a K step for 256 x 256 and 1.16 for 256 x 128, and one
+//           of the others on the rows that are left
+// Few tokens and narrow weights go to the ring kernel, whose loads are many steps ahead and whose slices fill the GPU; in the
+// middle its four waves are behind the others' eight, which do the scaling of one half of the waves under the other's products.
+// Timed with weights that no cache holds, launch_gemm / ring: 24 x 18432 x 7168 61.9 / 58.6 us, 22 x 9600 x 4608 35 / 24, 8 x
+// 2176 x 4352 26.5 / 13.5, 123 x 1792 x 5120 43 / 16, 171 x 16000 x 2560 28.8 / 29.4, 600 x 9472 x 5248 67 / 78, 1000 x 9728 x
+// 5248 98 / 114; full tiles with a ring kernel behind them 3000 x 4480 x 3200 86 / 76.
+struct BlockPlan {
+    int64_t body;   // rows of the full tiles
+    RingPlan ring;  // the others (bm == 0: launch_gemm)
+};
+static RingPlan block_rows_plan(int64_t M, int64_t N, int64_t K, size_t partial_bytes, int cus) {
+    RingPlan ring = ring_plan(kRingBlock, M, N, K, partial_bytes, cus);
+    if (M <= 64) return ring;
+    const int64_t KT = K / 128, tiles = ((M + 127) / 128) * ((N + 127) / 128), full = tiles / (2 * cus), rem = tiles % (2 * cus);
+    const double part = (double)rem / cus, step = part <= 1.0 ? 0.7 + 0.3 * part : 1.15 + 0.2 * part;
+    const double middle = 5.0 + (double)full * ((double)KT * 1.55 + 3.0) + (rem ? (double)KT * step : 0.0);
+    // (several rounds of 128 x 128 ring tiles take about 15 % longer than estimated)
+    if (middle < ring.cost * (M > 256 ? 1.15 : 1.0)) ring = {0, 0, 0, middle};
+    return ring;
+}
+static BlockPlan block_plan(int64_t M, int64_t N, int64_t K, size_t partial_bytes, int cus) {
+    BlockPlan best{0, block_rows_plan(M, N, K, partial_bytes, cus)};
+    const int64_t KT = K / 128, body = M / 256 * 256, tm = body / 256;
+    if (body <= 512 || N % 128 || tm * (N / 128) < 384 || KT > kMaxTileWeightScales) return best;
+    double full = 6.0 + (double)((tm * (N / 128) + cus - 1) / cus) * ((double)KT * 1.16 + (KT <= kPersistentBlockSteps ? 1.0 : 4.0));
+    if (N % 256 == 0 && KT >= 16 && KT <= 1024) {  // as launch_gemm has it
+        const int64_t tn = N / 256, tiles = tm * tn, rem = tiles % cus;
+        const int64_t cut = rem > 0 && rem * 2 <= cus ? (rem + tm - 1) / tm : 0;
+        const int64_t head = tm * (tn - cut), rounds = (head + cus - 1) / cus;
+        if (head >= cus && head * 5 >= rounds * cus * 4) full = 6.0 + (double)(rounds * KT) * 2.05 + (cut ? 6.0 + (double)KT * 1.16 : 0.0);
+    }
+    if (full >= best.ring.cost) return best;
+    RingPlan rest{0, 0, 0, 0.0};
+    if (M > body) rest = block_rows_plan(M - body, N, K, partial_bytes, cus);
+    if (full + rest.cost < best.ring.cost) best = {body, rest};
+    return best;
+}
+size_t block_partial_bytes(int64_t M, int64_t N, int64_t K) {
+    const BlockPlan b = block_plan(M, N, K, ~(size_t)0, cu_count());
+    return b.ring.slices > 1 ? (size_t)b.ring.slices * (size_t)(M - b.body) * (size_t)N * 4 : 0;
+}
+static int launch_block_best(GemmArgs& p, int out_dtype, hipStream_t st) {
+    const int64_t elem = out_dtype == CFP8_OUT_F32 ? 4 : 2;
+    const BlockPlan plan = block_plan(p.M, p.N, p.K, p.partial_bytes, cu_count());
+    RingArgs r{};
+    r.a = p.a + plan.body * p.ld_a; r.w = p.b; r.sa = p.sa + plan.body * (p.K >> 7); r.sb = p.sb;
+    r.out = static_cast<uint8_t*>(p.out) + plan.body * p.ld_out * elem;
+    r.partial = p.partial;
+    r.ld_a = p.ld_a; r.ld_w = p.ld_b; r.ld_out = p.ld_out;
+    r.sb_stride_n = p.sb_stride_n; r.sb_stride_k = p.sb_stride_k;
+    r.M = p.M - (int)plan.body; r.N = p.N; r.K = p.K;
+    // (rows of the rest that launch_gemm takes: it splits them off itself)
+    if (r.M == 0 || !plan.ring.bm || !ring_takes(kRingBlock, r, out_dtype)) return launch_gemm<kBlock>(p, out_dtype, st);
+    if (plan.body) {
+        GemmArgs body = p;
+        body.M = (int)plan.body;
+        if (int rc = launch_gemm<kBlock>(body, out_dtype, st)) return rc;
+    }
+    return launch_ring(kRingBlock, r, plan.ring, out_dtype, st);
+}
+
 static int check_common(const char* who, const void* a, const void* b, const float* sa, const float* sb,
                         const void* out, int64_t ld_a, int64_t ld_b, int64_t ld_out, int out_dtype, int64_t M,
                         int64_t N, int64_t K, int k_unit = 128) {
@@ -3638,6 +3704,29 @@ extern "C" int cfp8_gemm_block128(const void* a, int64_t ld_a, const float* sa, 
     p.sb_stride_n = sb_stride_n; p.sb_stride_k = sb_stride_k;
     p.M = (int)M; p.N = (int)N; p.K = (int)K;
     return launch_gemm<kBlock>(p, out_dtype, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int cfp8_gemm_block128_split(const void* a, int64_t ld_a, const float* sa, const void* b, int64_t ld_b, const float* sb,
+                                        int64_t sb_stride_n, int64_t sb_stride_k, void* out, int64_t ld_out, int out_dtype, int64_t M,
+                                        int64_t N, int64_t K, void* workspace, size_t workspace_bytes, void* stream) {
+    using namespace cfp8;
+    if (int rc = check_common("gemm_block128_split", a, b, sa, sb, out, ld_a, ld_b, ld_out, out_dtype, M, N, K)) return rc;
+    if (M == 0 || N == 0) return CFP8_OK;
+    if (workspace_bytes && (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 255u)))
+        return set_error(CFP8_EINVAL, "gemm_block128_split: workspace must be 256-byte aligned");
+    if (int rc = check_device()) return rc;
+    GemmArgs p{};
+    p.a = static_cast<const uint8_t*>(a);
+    p.b = static_cast<const uint8_t*>(b);
+    p.sa = sa;
+    p.sb = sb;
+    p.out = out;
+    p.ld_a = ld_a; p.ld_b = ld_b; p.ld_out = ld_out;
+    p.sb_stride_n = sb_stride_n; p.sb_stride_k = sb_stride_k;
+    p.M = (int)M; p.N = (int)N; p.K = (int)K;
+    p.partial = static_cast<float*>(workspace);
+    p.partial_bytes = workspace_bytes;
+    return launch_block_best(p, out_dtype, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int cfp8_gemm_grouped_block128(const void* a, int64_t ld_a, const float* sa, const void* b,

@@ -43,6 +43,7 @@ bool note_launch(const char* kernel, unsigned grid, unsigned block, size_t lds);
 int raise_lds_limit(const void* fn, size_t lds, std::atomic<bool>& flag);         // once per (device, function)
 int device_slot();                                                                // 0..63, 64 = not cached
 int cu_count();                                                                   // compute units of the current device
+size_t block_partial_bytes(int64_t M, int64_t N, int64_t K);                      // of the block-scaled product's slices of K
 
 // ---- units of the kernels in which a workgroup walks rows of tiles ----------
 // The schedule for tiles_m tile rows of tiles_n tiles on `cus` workgroups: one workgroup per CU.  Tile rows beyond the

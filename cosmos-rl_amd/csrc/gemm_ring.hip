@@ -499,7 +499,8 @@ int launch_ring(int mode, RingArgs& p, const RingPlan& plan, int out_dtype, hipS
 extern "C" size_t cfp8_gemm_partial_bytes(int kind, int64_t M, int64_t N, int64_t K) {
     using namespace cfp8;
     if (M <= 0 || N <= 0 || K <= 0) return 0;
-    const int mode = kind == CFP8_DISPATCH_BLOCK ? kRingBlock : kind == CFP8_DISPATCH_MXFP4 ? kRingMx : kRingRow;
+    if (kind == CFP8_DISPATCH_BLOCK) return block_partial_bytes(M, N, K);
+    const int mode = kind == CFP8_DISPATCH_MXFP4 ? kRingMx : kRingRow;
     const RingPlan plan = ring_plan(mode, M, N, K, ~(size_t)0, cu_count());
     return plan.slices > 1 ? (size_t)plan.slices * (size_t)M * (size_t)N * 4 : 0;
 }

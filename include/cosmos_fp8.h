@@ -452,6 +452,11 @@ int cfp8_gemm_block128(const void* a, int64_t ld_a, const float* sa,
                        void* out, int64_t ld_out, int out_dtype,
                        int64_t M, int64_t N, int64_t K, void* stream);
 
+/* cfp8_gemm_block128 with memory for partial sums (cfp8_gemm_partial_bytes(CFP8_DISPATCH_BLOCK, M, N, K), or less). */
+int cfp8_gemm_block128_split(const void* a, int64_t ld_a, const float* sa, const void* b, int64_t ld_b, const float* sb,
+                             int64_t sb_stride_n, int64_t sb_stride_k, void* out, int64_t ld_out, int out_dtype,
+                             int64_t M, int64_t N, int64_t K, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Grouped contiguous block-scaled GEMM.  Row r of a belongs to expert
  * m_indices[r] (int32, device); groups are contiguous and start on multiples of
  * 128 rows; rows with a negative index are padding and are not written.

@@ -90,3 +90,23 @@ def test_rowwise_bias_of_another_kind(dev):
     w, sw = ops.quant_rowwise(torch.randn(48, 256, device=dev).to(torch.bfloat16))
     b = torch.randn(48, device=dev)
     assert torch.equal(ops.fp8_linear(x, w.t(), sw, bias=b), ops.fp8_linear(x, w.t(), sw) + b)
+
+
+# the shapes above, scales of a slice that do not fit beside the ring's stages on 128 rows (63 steps and more), full tiles with
+# and without rows behind them
+@pytest.mark.parametrize("M,N,K", SHAPES + [(1, 2048, 7168), (24, 18432, 1152), (70, 4112, 8192), (1000, 1536, 1664), (1024 + 5, 24576, 384), (2048 + 130, 12288, 2048)])
+@pytest.mark.parametrize("kn", [False, True])
+def test_block(dev, M, N, K, kn):
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    q, s = ops.groupwise_activation_quant(torch.randn(M, K, generator=g, device=dev).to(torch.bfloat16))
+    w = (torch.randn(N, K, generator=g, device=dev) * 0.05).to(torch.float8_e4m3fn)
+    sw = torch.rand(-(-N // 128), K // 128, generator=g, device=dev) + 0.5
+    want = ((q.double() * s.double().repeat_interleave(128, 1)) @ (w.double() * sw.double().repeat_interleave(128, 0)[:N].repeat_interleave(128, 1)).t()).cpu()
+    sb, strides = (sw.t().contiguous(), (1, sw.shape[0])) if kn else (sw, (K // 128, 1))
+    part, need = _partial(_lib.DISPATCH_BLOCK, M, N, K, dev)
+    for dtype in (torch.float32, torch.bfloat16):
+        for have in {0, need // 2, need}:
+            out = _out(M, N, dev, dtype)
+            _lib.check(_lib.load().cfp8_gemm_block128_split(q.data_ptr(), K, s.data_ptr(), w.data_ptr(), K, sb.data_ptr(), *strides, out.data_ptr(), N + 8,
+                                                            ops._out_code(dtype), M, N, K, part.data_ptr(), have, _stream()))
+            _check(out, want, M, N, dtype, 0.0)
