@@ -33,6 +33,7 @@
 // Slices of K: fp32 partial sums into caller memory, summed in slice order with scales, bias and conversion by
 // ring_reduce_kernel.
 #include <atomic>
+#include <math.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <type_traits>
@@ -44,19 +45,20 @@ namespace cfp8 {
 
 constexpr uint32_t kOutside = 0xF0000000u;  // a per-lane offset that no descriptor here covers (they end at or below 0xEFFFFFFF)
 
-template <int MODE, int BM, int BN>
+// PER: the LDS is shared by PER workgroups a CU
+template <int MODE, int BM, int BN, int PER>
 struct RingShape {
     static constexpr int LX = BM / 32, LW = MODE == kRingMx ? BN / 64 : BN / 32, LS = MODE == kRingMx ? 1 : 0;  // loads per wave and step
     static constexpr int XS = BM * 128, WS = MODE == kRingMx ? BN * 64 : BN * 128, SS = MODE == kRingMx ? 1024 : 0;
     static constexpr int STAGE = XS + WS + SS;
     // block scaling keeps room for the slice's scales
-    static constexpr int S0 = (MODE == kRingBlock ? 128 : 160) * 1024 / STAGE;
+    static constexpr int S0 = (MODE == kRingBlock ? 128 : 160) * 1024 / PER / STAGE;
     static constexpr int S = S0 > 8 ? 8 : S0;
 };
 
-template <int MODE, int BM, int BN, bool SPLIT, bool OUT_F32>
+template <int MODE, int BM, int BN, int PER, bool SPLIT, bool OUT_F32>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_ring_kernel(const RingArgs p) {
-    using Sh = RingShape<MODE, BM, BN>;
+    using Sh = RingShape<MODE, BM, BN, PER>;
     constexpr int LX = Sh::LX, LW = Sh::LW, LS = Sh::LS, L = LX + LW + LS, S = Sh::S;
     constexpr int TM = BM / 32, TN = BN / 32;  // 16 x 16 tiles per wave
     constexpr int WB = S * Sh::XS, SB = WB + S * Sh::WS;
@@ -385,9 +387,9 @@ __global__ __launch_bounds__(256) void ring_reduce_kernel(const RingArgs p) {
     else *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.out) + (int64_t)m * p.ld_out + n) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
 }
 
-template <int MODE, int BM, int BN, bool SPLIT>
+template <int MODE, int BM, int BN, int PER, bool SPLIT>
 static int launch_ring_cfg(RingArgs& p, int out_dtype, hipStream_t st) {
-    using Sh = RingShape<MODE, BM, BN>;
+    using Sh = RingShape<MODE, BM, BN, PER>;
     p.tiles_m = (p.M + BM - 1) / BM;
     p.tiles_n = (p.N + BN - 1) / BN;
     const int64_t blocks = (int64_t)p.tiles_m * p.tiles_n * p.slices;
@@ -397,7 +399,7 @@ static int launch_ring_cfg(RingArgs& p, int out_dtype, hipStream_t st) {
     static_assert(Sh::S >= 3 && (size_t)4 * (BM / 2) * (BN + 16) <= (size_t)Sh::S * Sh::STAGE, "ring LDS");
     const int f32 = out_dtype == CFP8_OUT_F32;
     using Kern = void (*)(const RingArgs);
-    const Kern kern = SPLIT || !f32 ? static_cast<Kern>(gemm_ring_kernel<MODE, BM, BN, SPLIT, false>) : static_cast<Kern>(gemm_ring_kernel<MODE, BM, BN, false, true>);
+    const Kern kern = SPLIT || !f32 ? static_cast<Kern>(gemm_ring_kernel<MODE, BM, BN, PER, SPLIT, false>) : static_cast<Kern>(gemm_ring_kernel<MODE, BM, BN, PER, false, true>);
     static std::atomic<bool> raised[65][2];
     const int slot = device_slot();
     if (slot == 64) raised[64][f32].store(false, std::memory_order_relaxed);
@@ -417,61 +419,71 @@ static int launch_ring_cfg(RingArgs& p, int out_dtype, hipStream_t st) {
     return check_launch("gemm");
 }
 
+// Workgroups a CU that a tile's ring leaves room for.  Two of 64 x 64 rowwise, with rings of 5 instead of 8 stages, take
+// each other's prologues, epilogues and uneven rounds: 33 x 37888 x 3584 33.8 -> 30.1 us, 621 x 20480 x 2304
+// MXFP4 50.9 -> 37.9 us; a ring of two 128 x 128 e4m3 stages, or of two block-scaled 64 x 128 ones, would be none.
+constexpr int ring_per_cu(int mode, int bm, int bn) { return mode == kRingMx || bm * bn == 64 * 64 || (mode == kRingRow && bm * bn == 64 * 128) ? 2 : 1; }
+
 template <int MODE>
 static int launch_ring_mode(RingArgs& p, const RingPlan& plan, int out_dtype, hipStream_t st) {
     const int KT = (p.K + 127) >> 7;
     p.slice_steps = (KT + plan.slices - 1) / plan.slices;
     p.slices = (KT + p.slice_steps - 1) / p.slice_steps;
 #define CFP8_RING(BM, BN) \
-    if (plan.bm == BM && plan.bn == BN) return p.slices > 1 ? launch_ring_cfg<MODE, BM, BN, true>(p, out_dtype, st) : launch_ring_cfg<MODE, BM, BN, false>(p, out_dtype, st)
+    if (plan.bm == BM && plan.bn == BN) \
+        return p.slices > 1 ? launch_ring_cfg<MODE, BM, BN, ring_per_cu(MODE, BM, BN), true>(p, out_dtype, st) \
+                            : launch_ring_cfg<MODE, BM, BN, ring_per_cu(MODE, BM, BN), false>(p, out_dtype, st)
     CFP8_RING(128, 128);
     CFP8_RING(64, 128);
-    CFP8_RING(128, 64);
+    if constexpr (MODE != kRingBlock) CFP8_RING(128, 64);
     CFP8_RING(64, 64);
 #undef CFP8_RING
     return set_error(CFP8_EINVAL, "gemm: no such ring tile");
 }
 
-// The tile and the number of slices with the least estimated time.  The estimate is a fixed time per launch plus, per
-// round of workgroups on the CUs, K steps times the tile's step time (longer the more CUs load at once) plus the tile's
-// ends, not below the operands' bytes at the rate they come in; slices add the reduction's launch and their partial sums'
-// way out and back.  The constants are fitted to all combinations of 120 shapes each (1 .. 8192 tokens, weights of 896 ..
-// 37888 rows, K 896 .. 18944), timed with operands that no cache holds: the choice is within 2 % of the best combination on
-// average, 20 % at worst.
+// The tile and the number of slices with the least estimated time.  The estimate adds up rounds of workgroups on the CUs, each
+// K steps times the tile's step time (longer the more CUs load at once, and as long as for two everywhere as soon as one CU
+// holds two) plus the tile's ends; joins it with the operands' bytes at the rate they come in, (a^4 + b^4)^(1/4), since neither
+// hides the other near where they meet; and adds a fixed time per launch and, for slices, the reduction's launch and their
+// partial sums' way out and back.  The constants are fitted to all combinations of 112 to 144 shapes each (3 .. 3000 tokens,
+// weights of 896 .. 37888 rows, K 896 .. 18944), timed with weights that no cache holds: the choice is within 2 % of the best
+// combination on average, 20 % at worst.
 struct RingRates {
-    double step[4], load[4];  // 128 x 128, 64 x 128, 128 x 64, 64 x 64: microseconds a step, and what a full GPU adds
+    double step[4], load[4], two[4];  // 128 x 128, 64 x 128, 128 x 64, 64 x 64: microseconds a step; what a full GPU adds; what two a CU add
     double launch, ends, partial, bytes, reduce;
 };
 static const RingRates kRates[3] = {
-    {{0.560, 0.371, 0.388, 0.208}, {0.003, 0.108, 0.000, 0.293}, 2.3, 1.7, 3.8, 3.7, 2.8},
-    {{0.708, 0.388, 0.509, 0.230}, {0.000, 0.197, 0.000, 0.415}, 3.8, 2.3, 4.2, 4.4, 1.9},
-    {{0.631, 0.493, 0.399, 0.201}, {0.000, 0.150, 0.079, 0.323}, 3.4, 1.7, 3.6, 3.2, 2.3},
+    {{0.464, 0.312, 0.308, 0.169}, {0.249, 0.427, 0.168, 0.371}, {0.0, 0.637, 0.854, 1.062}, 2.4, 0.8, 4.8, 5.0, 2.5},
+    {{0.658, 0.393, 0.0, 0.263}, {0.100, 0.335, 0.0, 0.283}, {0.0, 0.0, 0.0, 0.362}, 2.3, 1.2, 4.3, 4.9, 2.3},
+    {{0.491, 0.343, 0.294, 0.210}, {0.097, 0.287, 0.213, 0.115}, {0.789, 0.793, 0.894, 1.104}, 3.1, 0.4, 4.7, 3.4, 2.7},
 };
 static const int kTiles[4][2] = {{128, 128}, {64, 128}, {128, 64}, {64, 64}};
 constexpr int kRingMaxSlices = 16;
 
 // block scaling: the scales of a slice in LDS beside the ring
-static bool ring_scales_fit(int bm, int64_t steps) { return ((int64_t)bm * (steps | 1) + steps) * 4 <= 32 * 1024; }
+static bool ring_scales_fit(int bm, int bn, int64_t steps) {
+    return ((int64_t)bm * (steps | 1) + steps) * 4 <= 32 * 1024 / ring_per_cu(kRingBlock, bm, bn);
+}
 
 RingPlan ring_plan(int mode, int64_t M, int64_t N, int64_t K, size_t partial_bytes, int cus) {
     const RingRates& r = kRates[mode];
     const int64_t KT = (K + 127) / 128;
     RingPlan best{0, 0, 0, 1e30};
-    const double bytes = (double)N * K * (mode == kRingMx ? 0.53 : 1.0) + (double)M * K;
+    const double in = ((double)N * K * (mode == kRingMx ? 0.53 : 1.0) + (double)M * K) / (r.bytes * 1e6);
     for (int c = 0; c < 4; ++c) {
-        const int bm = kTiles[c][0], bn = kTiles[c][1];
-        if (bm == 128 && M <= 64) continue;
+        const int bm = kTiles[c][0], bn = kTiles[c][1], per = ring_per_cu(mode, bm, bn);
+        if ((bm == 128 && M <= 64) || (mode == kRingBlock && c == 2)) continue;
         const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
         for (int s = 1; s <= kRingMaxSlices; ++s) {
             const int64_t steps = (KT + s - 1) / s;
-            if (s > 1 && (steps < 3 || (KT + steps - 1) / steps != s || tiles * s > 2 * cus || (size_t)s * (size_t)M * (size_t)N * 4 > partial_bytes)) continue;
-            if (mode == kRingBlock && !ring_scales_fit(bm, steps)) continue;
-            const int64_t full = tiles * s / cus, rem = tiles * s % cus;
-            const double part = (double)rem / cus;
-            double us = r.launch + full * (steps * r.step[c] * (1 + r.load[c]) + r.ends);
-            if (rem) us += steps * r.step[c] * (1 + r.load[c] * (full ? 1.0 : part) * part) + r.ends;
-            const double stream = r.launch + bytes / (r.bytes * 1e6);
-            if (us < stream) us = stream;
+            if (s > 1 && (steps < 3 || (KT + steps - 1) / steps != s || tiles * s > 4 * cus || (size_t)s * (size_t)M * (size_t)N * 4 > partial_bytes)) continue;
+            if (mode == kRingBlock && !ring_scales_fit(bm, bn, steps)) continue;
+            const int64_t full = tiles * s / (per * cus), rem = tiles * s % (per * cus);
+            const double part = (double)rem / cus, step = (double)steps * r.step[c];
+            double us = (double)full * (step * (1 + r.load[c] + r.two[c]) + per * r.ends);
+            if (part > 1) us += step * (1 + r.load[c] + r.two[c]) + 2 * r.ends;
+            else if (rem) us += step * (1 + r.load[c] * (full ? part : part * part)) + r.ends;
+            us = r.launch + sqrt(sqrt(us * us * us * us + in * in * in * in));
             if (s > 1) us += r.reduce + 8.0 * s * M * N / (r.partial * 1e6);
             if (us < best.cost) best = {bm, bn, s, us};
         }
