@@ -5,7 +5,10 @@
 
 namespace cfp8 {
 
-enum : int { kRingRow = 0, kRingBlock = 1, kRingMx = 2 };
+// kRingGateUp, kRingDown: block-scaled products of MoE experts on rows that lie expert behind expert; the first one gathers its
+// rows from the tokens and ends in SwiGLU
+enum : int { kRingRow = 0, kRingBlock = 1, kRingMx = 2, kRingGateUp = 3, kRingDown = 4 };
+constexpr int kRingGroupRows = 64;
 
 struct RingArgs {
     const uint8_t* a;      // activations e4m3 [M, K]
@@ -17,6 +20,10 @@ struct RingArgs {
     void* out;
     float* partial;        // [slices, M, N] when slices > 1
     int64_t ld_a, ld_w, ld_ws, ld_out, sb_stride_n, sb_stride_k;
+    const int32_t* row_tokens;  // kRingGateUp: the token of every row; M is then the number of tokens
+    const int32_t* sizes;       // kRingGateUp, kRingDown: rows of every expert, and their inclusive cumulative sum
+    const int32_t* ends;
+    int experts;
     int M, N, K;
     int tiles_m, tiles_n, slices, slice_steps;
 };
@@ -27,6 +34,8 @@ struct RingPlan {
 };
 RingPlan ring_plan(int mode, int64_t M, int64_t N, int64_t K, size_t partial_bytes, int cus);
 bool ring_takes(int mode, const RingArgs& p, int out_dtype);  // whether the operands fit what the kernel assumes
+bool ring_grouped_takes(int64_t K);
+int launch_ring_grouped(int mode, RingArgs& p, int64_t row_tiles, hipStream_t st);
 int launch_ring(int mode, RingArgs& p, const RingPlan& plan, int out_dtype, hipStream_t st);
 
 }  // namespace cfp8

@@ -30,6 +30,10 @@
 // row pitches and K steps rotated between workgroups or XCDs move it by at most 10 % either way.
 // MXFP4, 200 tokens: 2176 x 14848 20 against 142 us on the register-staged tiles, 3456 x 11264 27 against 108 us.
 //
+// kRingGateUp, kRingDown: 64 x 128 tiles of a MoE layer's experts, rows gathered from the tokens, SwiGLU at the end of the first
+// (128 experts of 2048 x 768, 777 tokens top 8: the whole call 231 -> 179 us against padded tiles of 128 rows).  Bound by the
+// weights' way in, hence two workgroups a CU: one loads while the other looks its tile up or leaves.
+//
 // Slices of K: fp32 partial sums into caller memory, summed in slice order with scales, bias and conversion by
 // ring_reduce_kernel.
 #include <atomic>
@@ -45,6 +49,10 @@ namespace cfp8 {
 
 constexpr uint32_t kOutside = 0xF0000000u;  // a per-lane offset that no descriptor here covers (they end at or below 0xEFFFFFFF)
 
+constexpr bool ring_grouped(int mode) { return mode == kRingGateUp || mode == kRingDown; }
+constexpr bool ring_blocks(int mode) { return mode == kRingBlock || ring_grouped(mode); }  // 1x128 and 128x128 scales
+constexpr int ring_scale_room(int mode) { return mode == kRingBlock ? 32 * 1024 : ring_grouped(mode) ? 16 * 1024 : 0; }
+
 // PER: the LDS is shared by PER workgroups a CU
 template <int MODE, int BM, int BN, int PER>
 struct RingShape {
@@ -52,9 +60,43 @@ struct RingShape {
     static constexpr int XS = BM * 128, WS = MODE == kRingMx ? BN * 64 : BN * 128, SS = MODE == kRingMx ? 1024 : 0;
     static constexpr int STAGE = XS + WS + SS;
     // block scaling keeps room for the slice's scales
-    static constexpr int S0 = (MODE == kRingBlock ? 128 : 160) * 1024 / PER / STAGE;
+    static constexpr int S0 = (160 * 1024 - ring_scale_room(MODE)) / PER / STAGE;
     static constexpr int S = S0 > 8 ? 8 : S0;
 };
+
+// kRingGateUp, kRingDown: the workgroup's tile.  Row tiles are numbered expert by expert; every XCD takes a contiguous eighth of
+// them, tile by tile all of its columns, so that an expert's rows and weights come through one L2.
+struct RowTile {
+    int expert, row, end, tn;  // expert < 0: there is none
+};
+template <int BM>
+__device__ __forceinline__ RowTile ring_row_tile(const RingArgs& p, int lane) {
+    auto tiles_of = [&](int e) { return e < p.experts ? (p.sizes[e] + BM - 1) / BM : 0; };
+    int total = 0;
+    for (int e0 = 0; e0 < p.experts; e0 += 64) total += tiles_of(e0 + lane);
+    for (int d = 1; d < 64; d <<= 1) total += __shfl_xor(total, d);
+    total = __builtin_amdgcn_readfirstlane(total);
+    const int local = (int)blockIdx.x >> 3, per = (total + 7) >> 3, k = local / p.tiles_n;
+    int at = ((int)blockIdx.x & 7) * per + k;
+    if (k >= per || at >= total) return {-1, 0, 0, 0};
+    for (int e0 = 0; e0 < p.experts; e0 += 64) {
+        const int n = tiles_of(e0 + lane);
+        int sum = n;  // inclusive
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(sum, d);
+            if (lane >= d) sum += o;
+        }
+        const uint64_t mine = __ballot(at >= sum - n && at < sum);
+        if (mine) {
+            const int bit = __ffsll((unsigned long long)mine) - 1, e = e0 + bit;
+            const int end = __builtin_amdgcn_readfirstlane(p.ends[e]);
+            const int start = end - __builtin_amdgcn_readfirstlane(p.sizes[e]);
+            return {e, start + (at - (__builtin_amdgcn_readlane(sum, bit) - __builtin_amdgcn_readlane(n, bit))) * BM, end, local - k * p.tiles_n};
+        }
+        at -= __builtin_amdgcn_readlane(sum, 63);
+    }
+    return {-1, 0, 0, 0};
+}
 
 template <int MODE, int BM, int BN, int PER, bool SPLIT, bool OUT_F32>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_ring_kernel(const RingArgs p) {
@@ -68,8 +110,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wm = wave & 1, wn = wave >> 1;
     const int lrow = lane & 15, quarter = lane >> 4;
-    int tm, tn, slice;
-    {
+    int tm = 0, tn, slice = 0, expert = 0, m0, mend;  // rows m0 .. mend - 1 at most
+    if (ring_grouped(MODE)) {
+        const RowTile rt = ring_row_tile<BM>(p, lane);
+        if (rt.expert < 0) return;
+        tn = rt.tn;
+        expert = rt.expert;
+        m0 = rt.row;
+        mend = rt.end;
+    } else {
         const int tiles = p.tiles_m * p.tiles_n;
         slice = SPLIT ? (int)blockIdx.x / tiles : 0;
         const int pid = (int)blockIdx.x - slice * tiles;
@@ -86,8 +135,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
         const int g = at / (rows * p.tiles_n), in = at - g * rows * p.tiles_n;
         tm = (lin < split ? 0 : high * (low + 1)) + g * rows + in % rows;
         tn = in / rows;
+        m0 = tm * BM;
+        mend = p.M;
     }
-    const int m0 = tm * BM, n0 = tn * BN;
+    const int n0 = tn * BN;
     const int KT = (p.K + 127) >> 7, tail = p.K & 127;
     const int kbeg = SPLIT ? slice * p.slice_steps : 0;
     const int kend = SPLIT ? (kbeg + p.slice_steps < KT ? kbeg + p.slice_steps : KT) : KT;
@@ -101,9 +152,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
         return b < (int64_t)kMost ? (uint32_t)b : kMost;
     };
     constexpr int WROWS = MODE == kRingMx ? 16 : 8;  // weight rows of one load
-    uint64_t a_at = reinterpret_cast<uint64_t>(p.a) + (uint64_t)(m0 + wave * 8) * (uint64_t)p.ld_a;
-    uint64_t w_at = reinterpret_cast<uint64_t>(p.w) + (uint64_t)(n0 + wave * WROWS) * (uint64_t)p.ld_w;
-    uint32_t a_end = bytes_left((int64_t)p.M - m0 - wave * 8, p.ld_a), w_end = bytes_left((int64_t)p.N - n0 - wave * WROWS, p.ld_w);
+    // (kRingGateUp: rows of the tokens wherever they lie)
+    uint64_t a_at = reinterpret_cast<uint64_t>(p.a) + (MODE == kRingGateUp ? 0 : (uint64_t)(m0 + wave * 8) * (uint64_t)p.ld_a);
+    uint64_t w_at = reinterpret_cast<uint64_t>(p.w) + ((uint64_t)expert * (uint64_t)p.N + (uint64_t)(n0 + wave * WROWS)) * (uint64_t)p.ld_w;
+    uint32_t a_end = bytes_left(MODE == kRingGateUp ? (int64_t)p.M : (int64_t)mend - m0 - wave * 8, p.ld_a), w_end = bytes_left((int64_t)p.N - n0 - wave * WROWS, p.ld_w);
     uint32_t a_step = 32u * (uint32_t)p.ld_a, w_step = (uint32_t)(4 * WROWS) * (uint32_t)p.ld_w;
     uint64_t s_at = 0;
     uint32_t s_end = 0;
@@ -130,11 +182,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
         vw = (uint32_t)(lane >> 3) * (uint32_t)p.ld_w + c8 * 16;
         vw_tail = tail && c8 * 16 >= (uint32_t)tail ? kOutside : vw;
     }
+    uint32_t va_row[LX];  // kRingGateUp
     auto dma = [&](int kt, int st, int l) {  // load l of the step's LX + LW + LS
         const bool in = kt < kend, at_tail = kt == KT - 1;
+        const uint32_t xa = MODE == kRingGateUp ? va_row[l < LX ? l : 0] : at_tail ? va_tail : va;
         if (l < LX)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_void*)(smem + st * Sh::XS + (wave + 4 * l) * 1024), 16,
-                                                     in ? (at_tail ? va_tail : va) : kOutside, (uint32_t)l * a_step + ((uint32_t)kt << 7), 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_void*)(smem + st * Sh::XS + (wave + 4 * l) * 1024), 16, in ? xa : kOutside,
+                                                     (MODE == kRingGateUp ? 0u : (uint32_t)l * a_step) + ((uint32_t)kt << 7), 0, 0);
         else if (l < LX + LW)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_void*)(smem + WB + st * Sh::WS + (wave + 4 * (l - LX)) * 1024), 16,
                                                      in ? (at_tail ? vw_tail : vw) : kOutside,
@@ -169,8 +223,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
         return *reinterpret_cast<const u32*>(smem + SB + st * 1024 + (n / (BN / 4)) * 256 + (n % (BN / 4)) * 4);
     };
 
-    // block scaling: the slice's activation scales, [row][step] with an odd pitch, and the weight scales of the tile's one or
-    // two 128-blocks of N
+    // block scaling: the slice's activation scales, [row][step] with an odd pitch, and the weight scales of the tile's block of N
+    // (kRingGateUp: of its 64 gate and 64 up features, which lie in two)
+    constexpr int NB = MODE == kRingGateUp ? 2 : 1;
     const int spitch = p.slice_steps | 1;
     float* const sa_lds = reinterpret_cast<float*>(smem + SB);
     float* const sb_lds = sa_lds + BM * spitch;
@@ -181,7 +236,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
         }
         for (int i = t; i < steps; i += 256) sb_lds[i] = p.sb[(int64_t)(n0 >> 7) * p.sb_stride_n + (int64_t)(kbeg + i) * p.sb_stride_k];
     }
-    static_assert(MODE != kRingBlock || BN <= 128, "a tile lies in one 128-block of N");
+    static_assert(!ring_blocks(MODE) || BN <= 128, "a tile lies in one 128-block of N");
 
     f32x4 acc[TN][TM];
 #pragma unroll
@@ -192,28 +247,61 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
     // replaced in place behind their last MFMA.
     i32x8 W[2][TN], XL[2], X[TM - 1];
     u32 wword[2][TN];         // kRingMx: the scale word of the weight tile's row
-    float xs[2][TM], ss[2];   // kRingBlock: activation scales and weight scale of a step
+    float xs[2][TM], ss[2][NB];  // block scaling: activation scales and weight scales of a step
     auto read_w = [&](int b, int st, int i) {
         W[b][i] = wfrag(st, i);
         if (MODE == kRingMx) wword[b][i] = scale_word(st, i);
     };
     auto read_s = [&](int b, int kt) {
-        if (MODE == kRingBlock) {
+        if (ring_blocks(MODE)) {
             const int c = kt < kend ? kt - kbeg : 0;
-            ss[b] = sb_lds[c];
+#pragma unroll
+            for (int u = 0; u < NB; ++u) ss[b][u] = sb_lds[u * steps + c];
 #pragma unroll
             for (int j = 0; j < TM; ++j) xs[b][j] = sa_lds[(wm * (BM / 2) + j * 16 + lrow) * spitch + c];
         }
     };
-    f32x4 pr[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};  // kRingBlock: products not yet added
-    float pr_f = 0.f;
+    f32x4 pr[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};  // block scaling: products not yet added
+    float pr_f[NB];
+#pragma unroll
+    for (int u = 0; u < NB; ++u) pr_f[u] = 0.f;
 
+    if (ring_grouped(MODE)) {
+        // weights first: they do not wait for the row's token to be known; then tokens and scales, four threads a row
+        static_assert(!ring_grouped(MODE) || BM == 64, "256 threads, four a row");
 #pragma unroll
-    for (int d = 0; d < S; ++d)
+        for (int d = 0; d < S; ++d)
 #pragma unroll
-        for (int l = 0; l < L; ++l) dma(kbeg + d, d, l);
-    // tile 0 has landed when at most the loads of the S - 1 tiles behind it are outstanding
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 1) * L) : "memory");
+            for (int l = LX; l < L; ++l) dma(d, d, l);
+        const int srow = m0 + (t >> 2) < mend ? m0 + (t >> 2) : mend - 1;
+        int64_t stoken = srow;
+        if (MODE == kRingGateUp) {
+            stoken = p.row_tokens[srow];
+#pragma unroll
+            for (int l = 0; l < LX; ++l) {
+                const int row = m0 + wave * 8 + 32 * l + (lane >> 3);
+                const uint32_t token = (uint32_t)p.row_tokens[row < mend ? row : mend - 1];
+                va_row[l] = row < mend ? token * (uint32_t)p.ld_a + c8 * 16 : kOutside;
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < S; ++d)
+#pragma unroll
+            for (int l = 0; l < LX; ++l) dma(d, d, l);
+        const float* const sp = p.sa + stoken * KT;
+        float* const sl = sa_lds + (t >> 2) * spitch;
+        for (int c = t & 3; c < KT; c += 4) sl[c] = sp[c];
+        const float* const wp = p.sb + ((int64_t)expert * (p.N >> 7) + (MODE == kRingGateUp ? 2 * (n0 >> 8) : n0 >> 7)) * KT;  // (two rows that follow each other)
+        if (t < NB * KT) sb_lds[t] = wp[t];
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    } else {
+#pragma unroll
+        for (int d = 0; d < S; ++d)
+#pragma unroll
+            for (int l = 0; l < L; ++l) dma(kbeg + d, d, l);
+        // tile 0 has landed when at most the loads of the S - 1 tiles behind it are outstanding
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 1) * L) : "memory");
+    }
     int stage = 0;
     auto step = [&](auto B, int kt) {
         constexpr int b = decltype(B)::value;
@@ -231,18 +319,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
                 wsc[i] = (int)(v >> (quarter * 8));
             }
         }
-        float f[TM];
+        float f[TM][NB];
 #pragma unroll
-        for (int j = 0; j < TM; ++j) f[j] = MODE == kRingBlock ? xs[b][j] * ss[b] : 0.f;
+        for (int j = 0; j < TM; ++j)
+#pragma unroll
+            for (int u = 0; u < NB; ++u) f[j][u] = ring_blocks(MODE) ? xs[b][j] * ss[b][u] : 0.f;
 #pragma unroll
         for (int g = 0; g < SLOTS; ++g) {
             const int j = g / TN, i = g % TN;
             const i32x8 xf = j == TM - 1 ? XL[b] : X[j];
-            if (MODE == kRingBlock) {
+            if (ring_blocks(MODE)) {
                 const f32x4 old = pr[g & 1];
                 pr[g & 1] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(W[b][i], xf, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
                 const int og = g >= 2 ? g - 2 : SLOTS + g - 2, oj = og / TN, oi = og % TN;
-                const float of = g >= 2 ? f[oj] : pr_f;
+                const float of = g >= 2 ? f[oj][oi % NB] : pr_f[g % NB];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) acc[oi][oj][e] = __builtin_fmaf(old[e], of, acc[oi][oj][e]);
             } else if (MODE == kRingMx) {
@@ -251,7 +341,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
                 acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(W[b][i], xf, acc[i][j], 0, 0, 0, 0, 0, 0);
             }
             // (an MFMA is a pure function of registers: pinned, or the compiler moves it past the fences below)
-            if (MODE == kRingBlock) asm volatile("" : "+v"(pr[g & 1]));
+            if (ring_blocks(MODE)) asm volatile("" : "+v"(pr[g & 1]));
             else asm volatile("" : "+v"(acc[i][j]));
             // behind the MFMA: a fragment of the next step where one is due, and the loads spread over the step
             if (g == 0) XL[b ^ 1] = xfrag(stage, TM - 1);
@@ -263,7 +353,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
                 if (l * SLOTS / L == g) dma(kt + S, freed, l);
             __builtin_amdgcn_sched_barrier(0);
         }
-        pr_f = f[TM - 1];
+#pragma unroll
+        for (int u = 0; u < NB; ++u) pr_f[u] = f[TM - 1][u];
     };
     auto first = [&](auto B) {
         constexpr int b = decltype(B)::value;
@@ -287,14 +378,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
         step(std::integral_constant<int, 0>{}, kt);
         step(std::integral_constant<int, 1>{}, kt + 1);
     }
-    if (MODE == kRingBlock) {
+    if (ring_blocks(MODE)) {
 #pragma unroll
         for (int g = 0; g < 2; ++g)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[TN - 2 + g][TM - 1][e] = __builtin_fmaf(pr[g][e], pr_f, acc[TN - 2 + g][TM - 1][e]);
+            for (int e = 0; e < 4; ++e) acc[TN - 2 + g][TM - 1][e] = __builtin_fmaf(pr[g][e], pr_f[g % NB], acc[TN - 2 + g][TM - 1][e]);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may land in LDS once the workgroup has gone
 
+    if constexpr (MODE == kRingGateUp) {
+        // 16 gate rows, then the 16 up rows of the same features
+#pragma unroll
+        for (int j = 0; j < TM; ++j) {
+            const int m = m0 + wm * (BM / 2) + j * 16 + lrow;
+            if (m >= mend) continue;
+#pragma unroll
+            for (int i = 0; i < TN; i += 2) {
+                const f32x4 g = acc[i][j], u = acc[i + 1][j];
+                u32 h0, h1;
+                swiglu_quad(pack_bf16x2(g[0], g[1]), pack_bf16x2(g[2], g[3]), pack_bf16x2(u[0], u[1]), pack_bf16x2(u[2], u[3]), h0, h1);
+                const int n = ((n0 + wn * (BN / 2) + i * 16) >> 1) + quarter * 4;
+                *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.out) + (int64_t)m * p.ld_out + n) = make_uint2(h0, h1);
+            }
+        }
+        return;
+    }
     if (SPLIT) {
         float* const part = p.partial + (int64_t)slice * p.M * p.N;
 #pragma unroll
@@ -315,7 +423,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
 #pragma unroll
     for (int j = 0; j < TM; ++j) {
         const int m = m0 + wm * (BM / 2) + j * 16 + lrow;
-        sam[j] = MODE != kRingBlock ? p.sa[m < p.M ? m : p.M - 1] : 1.f;
+        sam[j] = !ring_blocks(MODE) ? p.sa[m < p.M ? m : p.M - 1] : 1.f;
     }
 #pragma unroll
     for (int i = 0; i < TN; ++i) {
@@ -333,7 +441,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
 #pragma unroll
         for (int j = 0; j < TM; ++j) {
             const int m = m0 + wm * (BM / 2) + j * 16 + lrow;
-            if (m >= p.M) continue;
+            if (m >= mend) continue;
 #pragma unroll
             for (int i = 0; i < TN; ++i) {
                 const int n = n0 + wn * (BN / 2) + i * 16 + quarter * 4;
@@ -357,7 +465,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
         for (int r = 0; r < BM / 2; r += RPI) {
             const int m = m0 + wm * (BM / 2) + r + rr, n = n0 + wn * (BN / 2) + rc * 8;
             const i32x4 d = *reinterpret_cast<const i32x4*>(buf + (r + rr) * PITCH + rc * 16);
-            if (m < p.M && n < p.N) *reinterpret_cast<i32x4*>(static_cast<uint16_t*>(p.out) + (int64_t)m * p.ld_out + n) = d;
+            if (m < mend && n < p.N) *reinterpret_cast<i32x4*>(static_cast<uint16_t*>(p.out) + (int64_t)m * p.ld_out + n) = d;
         }
     }
 }
@@ -399,7 +507,10 @@ static int launch_ring_cfg(RingArgs& p, int out_dtype, hipStream_t st) {
     static_assert(Sh::S >= 3 && (size_t)4 * (BM / 2) * (BN + 16) <= (size_t)Sh::S * Sh::STAGE, "ring LDS");
     const int f32 = out_dtype == CFP8_OUT_F32;
     using Kern = void (*)(const RingArgs);
-    const Kern kern = SPLIT || !f32 ? static_cast<Kern>(gemm_ring_kernel<MODE, BM, BN, PER, SPLIT, false>) : static_cast<Kern>(gemm_ring_kernel<MODE, BM, BN, PER, false, true>);
+    Kern kern = gemm_ring_kernel<MODE, BM, BN, PER, SPLIT, false>;
+    if constexpr (!SPLIT) {
+        if (f32) kern = gemm_ring_kernel<MODE, BM, BN, PER, false, true>;
+    }
     static std::atomic<bool> raised[65][2];
     const int slot = device_slot();
     if (slot == 64) raised[64][f32].store(false, std::memory_order_relaxed);
@@ -498,6 +609,32 @@ bool ring_takes(int mode, const RingArgs& p, int out_dtype) {
     if (mode == kRingBlock && p.K % 128) return false;
     if (out_dtype == CFP8_OUT_BF16 && (p.ld_out % 8 || !aligned16(p.out))) return false;
     return (reinterpret_cast<uintptr_t>(p.bias) & 7u) == 0 && aligned16(p.out);
+}
+
+// The two products of a MoE layer's experts: `row_tiles` bounds the number of tiles of kRingGroupRows rows.
+bool ring_grouped_takes(int64_t K) { return K % 128 == 0 && (K / 128 | 1) * kRingGroupRows * 4 + 2 * (K / 128) * 4 <= ring_scale_room(kRingDown) / 2; }
+
+template <int MODE>
+static int launch_ring_grouped_mode(RingArgs& p, int64_t row_tiles, hipStream_t st) {
+    constexpr int BM = kRingGroupRows, BN = 128;
+    using Sh = RingShape<MODE, BM, BN, 2>;
+    p.tiles_n = p.N / BN;
+    p.slice_steps = p.K >> 7;
+    p.slices = 1;
+    const int64_t blocks = (row_tiles + 7) / 8 * 8 * p.tiles_n;
+    if (blocks > 0x7FFFFFFFll) return set_error(CFP8_EINVAL, "gemm: too many tiles for one launch");
+    const size_t lds = (size_t)Sh::S * Sh::STAGE + ((size_t)BM * (p.slice_steps | 1) + 2 * p.slice_steps) * sizeof(float);
+    static_assert(Sh::S >= 3 && (size_t)4 * (BM / 2) * (BN + 16) <= (size_t)Sh::S * Sh::STAGE, "ring LDS");
+    static std::atomic<bool> raised[65];
+    const int slot = device_slot();
+    if (slot == 64) raised[64].store(false, std::memory_order_relaxed);
+    if (int rc = raise_lds_limit(reinterpret_cast<const void*>(gemm_ring_kernel<MODE, BM, BN, 2, false, false>), 160 * 1024, raised[slot])) return rc;
+    if (!note_launch(MODE == kRingGateUp ? "gemm_ring<gate_up,64,128>" : "gemm_ring<down,64,128>", (unsigned)blocks, 256, lds)) return CFP8_OK;
+    hipLaunchKernelGGL((gemm_ring_kernel<MODE, BM, BN, 2, false, false>), dim3((unsigned)blocks), dim3(256), lds, st, p);
+    return check_launch("gemm");
+}
+int launch_ring_grouped(int mode, RingArgs& p, int64_t row_tiles, hipStream_t st) {
+    return mode == kRingGateUp ? launch_ring_grouped_mode<kRingGateUp>(p, row_tiles, st) : launch_ring_grouped_mode<kRingDown>(p, row_tiles, st);
 }
 
 int launch_ring(int mode, RingArgs& p, const RingPlan& plan, int out_dtype, hipStream_t st) {

@@ -1,18 +1,22 @@
 // The experts of one MoE layer on routed tokens as one call: routing, 1x128 quantisation of the tokens, the gate_up product
 // with SwiGLU, the down product and the weighted sum over each token's experts - launches only, on caller memory.
 //
-// Two forms, by the mean number of rows an expert gets:
+// Three forms, by the mean number of rows an expert gets:
 //
 //   many rows   Every expert's rows are padded to tiles of 128 (experts without a row get none), the tokens quantised into
 //               that layout (cfp8_scatter_quant_group128) and multiplied by the grouped GEMMs of the training path.  A
 //               group's rows of padding are zeros all the way: a walking GEMM carries a row's last products into the first
 //               step of its next tile with a scale of zero, so what multiplies there must be finite.  Rows past the last
 //               group are not touched.
+//   middle      A chunk of prefill: all experts' weights are read, for less than a tile of 128 rows each.  Rows lie one
+//               behind the other without padding; the ring kernel takes tiles of 64 of one expert's rows (gemm_ring.hip:
+//               kRingGateUp reads them from the quantised tokens and ends in SwiGLU, kRingDown), two workgroups a CU.  The
+//               hidden activation is quantised in between, since a 1x128 group of it is spread over two workgroups.
 //   few rows    A decode batch: reading the weights of the experts that have a row is all the time there is, and tiles of
-//               128 rows would hold one or two.  Rows lie one behind the other without padding; a workgroup takes a strip
-//               of ONE expert's weight rows, requests all of its K into registers before anything else, and then walks
-//               the expert's rows in tiles of 16 (few_gate_up_kernel, few_down_kernel).
-#include "cfp8_common.h"
+//               64 rows would hold one or two.  A workgroup takes a strip of ONE expert's weight rows, requests all of its
+//               K into registers before anything else, and then walks the expert's rows in tiles of 16
+//               (few_gate_up_kernel, few_down_kernel).
+#include "gemm_ring.h"
 
 namespace cfp8 {
 
@@ -209,26 +213,33 @@ static void launch_few_down(int ni, dim3 grid, hipStream_t st, const FewArgs& p)
 
 // The few-rows form holds a strip's whole K in registers: up to 8 K steps a wave of four (gate_up), 12 a wave (down).
 constexpr int64_t kFewMaxHidden = 4096, kFewMaxInter = 1536;
-// Up to this many activation elements an expert (rows x hidden) the weights bound the few-rows form and it is ahead; beyond,
-// every strip's workgroup reading all of its expert's rows does.  Whole calls, few against many rows: 128 experts of 2048 x
-// 768, top 8: 16 tokens 92 / 153 us, 128: 135 / 212, 512: 200 / 214, 640: 219 / 214, 1024: 283 / 227; 32 experts of 3584 x
-// 1536, top 4: 16 tokens 112 / 152, 128: 153 / 161, 256: 196 / 172; 64 experts of 1024 x 512, top 6: 64 tokens 40 / 76,
-// 640: 73 / 81, 1024: 91 / 81.
-constexpr int64_t kFewElementsPerExpert = 72 * 1024;
+// Mean rows an expert up to which a form is taken.  The few-rows form reads an expert's rows once for every strip of 16
+// features, the middle one once for every 128 columns but holds 64 rows in a tile; from about two of those tiles on the grouped
+// GEMMs' larger tiles need fewer loads a product.  Whole calls, few / middle / many rows, us: 128 experts of 2048 x 768, top 8:
+// 8 rows an expert 136 / 146 / 214, 16: 160 / 151 / 212, 49: 241 / 179 / 231, 96: 370 / 233 / 246, 128: 455 / 266 / 256; 32 of
+// 3584 x 1536, top 4: 8: 128 / 130 / 162, 16: 152 / 133 / 161, 97: 363 / 190 / 212, 128: 438 / 225 / 209; 64 of 1024 x 512, top 6:
+// 12: 42 / 44 / 71, 24: 50 / 47 / 74, 96: 88 / 62 / 77, 144: 112 / 76 / 92.
+constexpr int64_t kFewRowsPerExpert = 10, kMiddleRowsPerExpert = 112;
+
+enum class Form { kFew, kMiddle, kMany };
+constexpr int64_t kMiddleRowsPerExpert = 128;
 
 struct ExpertsPlan {
-    bool few;
+    Form form;
     int64_t rows;   // rows of the expert-grouped layout (their bound)
     int64_t slots;  // experts that can have a row
-    size_t row_tokens, row_experts, row_map, weights, m_sizes, m_offsets, route, xq, xs, h, hs, out, bytes;
+    size_t row_tokens, row_experts, row_map, weights, m_sizes, m_offsets, route, xq, xs, h, hq, hs, out, bytes;
 };
 
 static ExpertsPlan experts_plan(int64_t tokens, int topk, int experts, int64_t hidden, int64_t inter) {
     ExpertsPlan p{};
     const int64_t pairs = tokens * topk;
-    p.few = pairs * hidden <= kFewElementsPerExpert * experts && hidden <= kFewMaxHidden && inter <= kFewMaxInter;
+    if (pairs <= kFewRowsPerExpert * experts && hidden <= kFewMaxHidden && inter <= kFewMaxInter) p.form = Form::kFew;
+    else if (pairs <= kMiddleRowsPerExpert * experts && ring_grouped_takes(hidden) && ring_grouped_takes(inter) && tokens * hidden < (int64_t)1 << 31) p.form = Form::kMiddle;
+    else p.form = Form::kMany;
+    const bool many = p.form == Form::kMany;
     p.slots = pairs < experts ? pairs : experts;
-    p.rows = p.few ? pairs : (pairs + p.slots * 127) / 128 * 128;
+    p.rows = many ? (pairs + p.slots * 127) / 128 * 128 : pairs;
     size_t at = 0;
     auto take = [&](size_t bytes) {
         const size_t here = at;
@@ -236,17 +247,18 @@ static ExpertsPlan experts_plan(int64_t tokens, int topk, int experts, int64_t h
         return here;
     };
     p.row_tokens = take((size_t)p.rows * 4);
-    p.row_experts = take(p.few ? 0 : (size_t)p.rows * 4);
+    p.row_experts = take(many ? (size_t)p.rows * 4 : 0);
     p.row_map = take((size_t)pairs * 4);
     p.weights = take((size_t)pairs * 2);
     p.m_sizes = take((size_t)experts * 4);
     p.m_offsets = take((size_t)experts * 4);
     p.route = take(cfp8_route_tokens_workspace_bytes(tokens, topk, experts));
-    const size_t xrows = (size_t)(p.few ? tokens : p.rows);
+    const size_t xrows = (size_t)(many ? p.rows : tokens);
     p.xq = take(xrows * (size_t)hidden);
     p.xs = take(xrows * (size_t)(hidden / 128) * 4);
-    p.h = take((size_t)p.rows * (size_t)inter * (p.few ? 2 : 1));
-    p.hs = take(p.few ? 0 : (size_t)p.rows * (size_t)(inter / 128) * 4);
+    p.h = take(many ? 0 : (size_t)p.rows * (size_t)inter * 2);
+    p.hq = take(p.form == Form::kFew ? 0 : (size_t)p.rows * (size_t)inter);
+    p.hs = take(p.form == Form::kFew ? 0 : (size_t)p.rows * (size_t)(inter / 128) * 4);
     p.out = take((size_t)p.rows * (size_t)hidden * 2);
     p.bytes = at;
     return p;
@@ -281,12 +293,27 @@ extern "C" int cfp8_moe_experts(const void* x, int64_t ld_x, int64_t tokens, int
     auto i32 = [&](size_t at) { return reinterpret_cast<int32_t*>(ws + at); };
     auto f32 = [&](size_t at) { return reinterpret_cast<float*>(ws + at); };
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (int rc = cfp8_route_tokens(indices, index_bytes, token_mask, tokens, topk, experts, p.few ? 1 : 128, CFP8_ROUTE_END_NOT_PADDING, p.rows,
-                                   i32(p.row_tokens), p.few ? nullptr : i32(p.row_experts), i32(p.row_map), nullptr, weights, weights_dtype,
+    if (int rc = cfp8_route_tokens(indices, index_bytes, token_mask, tokens, topk, experts, p.form == Form::kMany ? 128 : 1, CFP8_ROUTE_END_NOT_PADDING, p.rows,
+                                   i32(p.row_tokens), p.form == Form::kMany ? i32(p.row_experts) : nullptr, i32(p.row_map), nullptr, weights, weights_dtype,
                                    ws + p.weights, i32(p.m_sizes), i32(p.m_offsets), ws + p.route,
                                    cfp8_route_tokens_workspace_bytes(tokens, topk, experts), stream))
         return rc;
-    if (p.few) {
+    if (p.form == Form::kMiddle) {
+        if (int rc = cfp8_quant_group128(x, tokens, hidden, ld_x, ws + p.xq, hidden, f32(p.xs), CFP8_GROUP_MODE_DIV, stream)) return rc;
+        const int64_t row_tiles = p.slots + p.rows / kRingGroupRows;
+        RingArgs r{};
+        r.a = ws + p.xq; r.w = static_cast<const uint8_t*>(gate_up); r.sa = f32(p.xs); r.sb = gate_up_scales; r.out = ws + p.h;
+        r.ld_a = r.ld_w = hidden; r.ld_out = inter;
+        r.row_tokens = i32(p.row_tokens); r.sizes = i32(p.m_sizes); r.ends = i32(p.m_offsets);
+        r.experts = experts;
+        r.M = (int)tokens; r.N = (int)(2 * inter); r.K = (int)hidden;
+        if (int rc = launch_ring_grouped(kRingGateUp, r, row_tiles, st)) return rc;
+        if (int rc = cfp8_quant_group128(ws + p.h, p.rows, inter, inter, ws + p.hq, inter, f32(p.hs), CFP8_GROUP_MODE_DIV, stream)) return rc;
+        r.a = ws + p.hq; r.w = static_cast<const uint8_t*>(down); r.sa = f32(p.hs); r.sb = down_scales; r.out = ws + p.out;
+        r.ld_a = r.ld_w = inter; r.ld_out = hidden;
+        r.M = (int)p.rows; r.N = (int)hidden; r.K = (int)inter;
+        if (int rc = launch_ring_grouped(kRingDown, r, row_tiles, st)) return rc;
+    } else if (p.form == Form::kFew) {
         if (int rc = cfp8_quant_group128(x, tokens, hidden, ld_x, ws + p.xq, hidden, f32(p.xs), CFP8_GROUP_MODE_DIV, stream)) return rc;
         FewArgs f{};
         f.xq = ws + p.xq;
@@ -309,10 +336,10 @@ extern "C" int cfp8_moe_experts(const void* x, int64_t ld_x, int64_t tokens, int
     } else {
         if (int rc = cfp8_scatter_quant_group128(x, ld_x, tokens, hidden, i32(p.row_map), topk, i32(p.row_tokens), p.rows, ws + p.xq, hidden, f32(p.xs), stream))
             return rc;
-        if (int rc = cfp8_gemm_grouped_swiglu_quant(ws + p.xq, hidden, f32(p.xs), gate_up, gate_up_scales, i32(p.row_experts), ws + p.h, inter,
+        if (int rc = cfp8_gemm_grouped_swiglu_quant(ws + p.xq, hidden, f32(p.xs), gate_up, gate_up_scales, i32(p.row_experts), ws + p.hq, inter,
                                                     f32(p.hs), p.rows, inter, hidden, experts, stream))
             return rc;
-        if (int rc = cfp8_gemm_grouped_block128(ws + p.h, inter, f32(p.hs), down, down_scales, i32(p.row_experts), ws + p.out, hidden, CFP8_OUT_BF16,
+        if (int rc = cfp8_gemm_grouped_block128(ws + p.hq, inter, f32(p.hs), down, down_scales, i32(p.row_experts), ws + p.out, hidden, CFP8_OUT_BF16,
                                                 p.rows, hidden, inter, experts, stream))
             return rc;
     }
