@@ -222,8 +222,6 @@ constexpr int64_t kFewMaxHidden = 4096, kFewMaxInter = 1536;
 constexpr int64_t kFewRowsPerExpert = 10, kMiddleRowsPerExpert = 112;
 
 enum class Form { kFew, kMiddle, kMany };
-constexpr int64_t kMiddleRowsPerExpert = 128;
-
 struct ExpertsPlan {
     Form form;
     int64_t rows;   // rows of the expert-grouped layout (their bound)
