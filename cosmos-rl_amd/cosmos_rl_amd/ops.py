@@ -409,7 +409,9 @@ def linear_mxfp4(x: torch.Tensor, weight: Tuple[torch.Tensor, torch.Tensor],
     w, ws = w.contiguous(), ws.contiguous()
     out = torch.empty((M, N), dtype=out_dtype or x.dtype, device=x.device)
     lib = _lib.load()
-    wsb = lib.cfp8_linear_workspace_bytes(M, K) + lib.cfp8_gemm_partial_bytes(_lib.DISPATCH_MXFP4, M, N, K)
+    wsb = lib.cfp8_linear_workspace_bytes(M, K)
+    if M > 4 or K > 4096:  # (below, one launch that takes no partial sums)
+        wsb += lib.cfp8_gemm_partial_bytes(_lib.DISPATCH_MXFP4, M, N, K)
     work = torch.empty(max(wsb, 1), dtype=torch.uint8, device=x.device)
     ld_x = x2.stride(0) if M > 1 else K
     _lib.check(lib.cfp8_linear_mxfp4(x2.data_ptr(), ld_x, w.data_ptr(), K // 2, ws.data_ptr(), K // 32, out.data_ptr(), N,

@@ -578,25 +578,28 @@ static bool ring_scales_fit(int bm, int bn, int64_t steps) {
 
 RingPlan ring_plan(int mode, int64_t M, int64_t N, int64_t K, size_t partial_bytes, int cus) {
     const RingRates& r = kRates[mode];
-    const int64_t KT = (K + 127) / 128;
+    const uint32_t KT = (uint32_t)((K + 127) / 128);
     RingPlan best{0, 0, 0, 1e30};
     const double in = ((double)N * K * (mode == kRingMx ? 0.53 : 1.0) + (double)M * K) / (r.bytes * 1e6);
     for (int c = 0; c < 4; ++c) {
         const int bm = kTiles[c][0], bn = kTiles[c][1], per = ring_per_cu(mode, bm, bn);
         if ((bm == 128 && M <= 64) || (mode == kRingBlock && c == 2)) continue;
-        const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-        for (int s = 1; s <= kRingMaxSlices; ++s) {
-            const int64_t steps = (KT + s - 1) / s;
-            if (s > 1 && (steps < 3 || (KT + steps - 1) / steps != s || tiles * s > 4 * cus || (size_t)s * (size_t)M * (size_t)N * 4 > partial_bytes)) continue;
+        const int64_t tiles64 = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+        // (32-bit divisions: a small product waits for this on the host)
+        const uint32_t tiles = (uint32_t)(tiles64 < (1 << 26) ? tiles64 : 1 << 26), slots = (uint32_t)(per * cus);
+        for (uint32_t s = 1; s <= kRingMaxSlices; ++s) {
+            const uint32_t steps = (KT + s - 1) / s;
+            if (s > 1 && (steps < 3 || tiles * s > 4 * (uint32_t)cus || (size_t)s * (size_t)M * (size_t)N * 4 > partial_bytes)) break;
+            if (s > 1 && (KT + steps - 1) / steps != s) continue;
             if (mode == kRingBlock && !ring_scales_fit(bm, bn, steps)) continue;
-            const int64_t full = tiles * s / (per * cus), rem = tiles * s % (per * cus);
+            const uint32_t full = tiles * s / slots, rem = tiles * s - full * slots;
             const double part = (double)rem / cus, step = (double)steps * r.step[c];
             double us = (double)full * (step * (1 + r.load[c] + r.two[c]) + per * r.ends);
             if (part > 1) us += step * (1 + r.load[c] + r.two[c]) + 2 * r.ends;
             else if (rem) us += step * (1 + r.load[c] * (full ? part : part * part)) + r.ends;
             us = r.launch + sqrt(sqrt(us * us * us * us + in * in * in * in));
-            if (s > 1) us += r.reduce + 8.0 * s * M * N / (r.partial * 1e6);
-            if (us < best.cost) best = {bm, bn, s, us};
+            if (s > 1) us += r.reduce + 8.0 * s * (double)M * (double)N / (r.partial * 1e6);
+            if (us < best.cost) best = {bm, bn, (int)s, us};
         }
     }
     return best;
