@@ -505,7 +505,7 @@ def scaled_mm(a: torch.Tensor, b: torch.Tensor, scale_a: torch.Tensor, scale_b: 
     lib = _lib.load()
     need = lib.cfp8_gemm_partial_bytes(_lib.DISPATCH_ROWWISE, M, N, K)
     part = torch.empty(need, dtype=torch.uint8, device=a.device) if need else None
-    fused = _fused_bias(bias, N)
+    fused = _fused_bias(bias, N, out.device)
     _lib.check(lib.cfp8_scaled_mm_rowwise_split(a.data_ptr(), ld_a, sa.data_ptr(), b.data_ptr(), ld_b, sb.data_ptr(), _ptr(fused), out.data_ptr(), N,
                                                 _out_code(out_dtype), M, N, K, _ptr(part), need, _stream()))
     if bias is not None and fused is None:
@@ -513,12 +513,20 @@ def scaled_mm(a: torch.Tensor, b: torch.Tensor, scale_a: torch.Tensor, scale_b: 
     return out
 
 
-def _fused_bias(bias: Optional[torch.Tensor], n: int) -> Optional[torch.Tensor]:
-    """The bias as the GEMM epilogues take it - one bf16 value per column - or None."""
-    if bias is None or bias.dtype != torch.bfloat16 or bias.dim() != 1 or bias.shape[0] != n or not bias.is_cuda:
+def _fused_bias(bias: Optional[torch.Tensor], n: int, device: torch.device) -> Optional[torch.Tensor]:
+    """The bias as the GEMM epilogues take it - one bf16 value per column - or None where torch adds it: other types and
+    shapes, and a bias that torch follows (a gradient, a tangent, a batched or otherwise wrapped tensor)."""
+    if bias is None or type(bias) not in (torch.Tensor, torch.nn.Parameter) or bias.dtype != torch.bfloat16:
+        return None
+    if bias.dim() != 1 or bias.shape[0] != n or bias.device != device or (bias.requires_grad and torch.is_grad_enabled()):
+        return None
+    if torch.autograd.forward_ad.unpack_dual(bias).tangent is not None:
         return None
     bias = bias.contiguous()
-    return bias if bias.data_ptr() % 8 == 0 else None
+    try:
+        return bias if bias.data_ptr() % 8 == 0 else None
+    except RuntimeError:  # (a tensor of torch.func has no storage)
+        return None
 
 
 def fp8_linear(x: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor,
@@ -551,7 +559,7 @@ def fp8_linear(x: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor
     out = torch.empty((M, N), dtype=out_dtype, device=x.device)
     ld_x = x2.stride(0) if M > 1 else K
     ld_w = weight.stride(1) if N > 1 else K
-    fused = _fused_bias(bias, N)
+    fused = _fused_bias(bias, N, out.device)
     _lib.check(lib.cfp8_linear_rowwise_split(x2.data_ptr(), ld_x, weight.data_ptr(), ld_w, sw.data_ptr(), _ptr(fused),
                                              out.data_ptr(), N, _out_code(out_dtype), M, N, K,
                                              workspace.data_ptr(), workspace.numel() * workspace.element_size(),

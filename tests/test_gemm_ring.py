@@ -110,3 +110,23 @@ def test_block(dev, M, N, K, kn):
             _lib.check(_lib.load().cfp8_gemm_block128_split(q.data_ptr(), K, s.data_ptr(), w.data_ptr(), K, sb.data_ptr(), *strides, out.data_ptr(), N + 8,
                                                             ops._out_code(dtype), M, N, K, part.data_ptr(), have, _stream()))
             _check(out, want, M, N, dtype, 0.0)
+
+
+def test_a_bias_that_torch_follows(dev):
+    """the epilogue adds a bias only where nothing else would see the addition"""
+    x = torch.randn(33, 256, device=dev).to(torch.bfloat16)
+    q, s = ops.scaled_fp8_quant((torch.randn(384, 256, device=dev) * 0.05).to(torch.bfloat16), use_per_token_if_dynamic=True)
+    bias = torch.randn(384, device=dev).to(torch.bfloat16)
+    want = ops.fp8_linear(x, q.t(), s, bias=bias)
+    learnt = torch.nn.Parameter(bias.clone())
+    got = ops.fp8_linear(x, q.t(), s, bias=learnt)
+    got.sum().backward()
+    assert torch.equal(got.detach(), want) and bool((learnt.grad == 33).all())
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(bias, torch.ones_like(bias))
+        tangent = torch.autograd.forward_ad.unpack_dual(ops.fp8_linear(x, q.t(), s, bias=dual)).tangent
+    assert tangent is not None and bool((tangent == 1).all())
+    many = torch.func.vmap(lambda b: ops.fp8_linear(x, q.t(), s, bias=b))(torch.stack([bias, bias + 1]))
+    assert torch.equal(many[0], want)
+    with pytest.raises(RuntimeError):
+        ops.fp8_linear(x, q.t(), s, bias=bias.cpu())
