@@ -670,6 +670,15 @@ def grouped_gemm_swiglu_quant(lhs: Tuple[torch.Tensor, torch.Tensor], rhs_interl
     return q, s
 
 
+def token_mask_of(token_mask: Optional[torch.Tensor], indices: torch.Tensor) -> Optional[torch.Tensor]:
+    """The mask as the routing kernel reads it: one byte per token of ``indices`` [T, topk], on its GPU."""
+    if token_mask is None:
+        return None
+    if token_mask.device != indices.device or token_mask.dim() > 1:
+        raise ValueError("token_mask must be a [tokens] tensor on the GPU of indices")
+    return token_mask.to(torch.bool).expand(indices.shape[0]).contiguous()
+
+
 def moe_experts(x: torch.Tensor, token_mask: Optional[torch.Tensor], weights: torch.Tensor, indices: torch.Tensor,
                 gate_up_interleaved: Tuple[torch.Tensor, torch.Tensor], down: Tuple[torch.Tensor, torch.Tensor]) -> torch.Tensor:
     """The experts of one MoE layer on routed tokens in one library call (``GroupedExperts.forward`` on one rank,
@@ -690,15 +699,13 @@ def moe_experts(x: torch.Tensor, token_mask: Optional[torch.Tensor], weights: to
         indices = indices.to(torch.int64)
     if weights.dtype not in (torch.bfloat16, torch.float32):
         weights = weights.to(torch.bfloat16)
-    if token_mask is not None and token_mask.dtype != torch.bool:
-        token_mask = token_mask.to(torch.bool)
+    token_mask = token_mask_of(token_mask, indices)
     indices, weights, gu, gus, dn, dns = (t.contiguous() for t in (indices, weights, gu, gus, dn, dns))
-    mask = token_mask.contiguous() if token_mask is not None else None
     y = torch.empty((T, H), dtype=torch.bfloat16, device=x.device)
     lib = _lib.load()
     need = lib.cfp8_moe_experts_workspace_bytes(T, topk, E, H, I)
     work = torch.empty(max(need, 1), dtype=torch.uint8, device=x.device)
-    _lib.check(lib.cfp8_moe_experts(x.data_ptr(), x.stride(0) if T > 1 else H, T, H, indices.data_ptr(), indices.element_size(), _ptr(mask),
+    _lib.check(lib.cfp8_moe_experts(x.data_ptr(), x.stride(0) if T > 1 else H, T, H, indices.data_ptr(), indices.element_size(), _ptr(token_mask),
                                     weights.data_ptr(), _lib.IN_F32 if weights.dtype == torch.float32 else _lib.IN_BF16, topk, E,
                                     gu.data_ptr(), gus.data_ptr(), dn.data_ptr(), dns.data_ptr(), I, y.data_ptr(), H, work.data_ptr(), need,
                                     _stream()))

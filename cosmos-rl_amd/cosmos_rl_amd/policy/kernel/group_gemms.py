@@ -158,7 +158,7 @@ class DSGroupGEMM(GroupGEMMStrategy):
         down_fp8, down_s = module.get_parameter("down_proj_fp8"), module.get_parameter("down_proj_scales")
         if inter % ops.BLOCK or hidden % ops.BLOCK or hidden != x.shape[1] or indices.shape[1] > 64 or n_experts > _lib.ROUTE_MAX_EXPERTS:
             return None
-        if x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16 or down_fp8.shape[0] != n_experts or hidden > _lib.SWIGLU_GEMM_MAX_K:
+        if x.stride(1) != 1 or x.stride(0) % 8 or x.stride(0) < hidden or x.data_ptr() % 16 or down_fp8.shape[0] != n_experts or hidden > _lib.SWIGLU_GEMM_MAX_K:
             return None
         return ops.moe_experts(x, token_mask, weights, indices, self._interleaved(module), (down_fp8, down_s))
 

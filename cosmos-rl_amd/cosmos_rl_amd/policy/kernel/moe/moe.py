@@ -15,7 +15,7 @@ from typing import Optional
 
 import torch
 
-from cosmos_rl_amd import _lib
+from cosmos_rl_amd import _lib, ops
 from cosmos_rl_amd.policy.kernel.moe.indices import generate_permute_indices, permute_tokens
 
 __all__ = ["TokenRouting", "route_tokens", "combine_expert_outputs", "grouped_experts_forward"]
@@ -67,8 +67,7 @@ def route_tokens(indices: torch.Tensor, token_mask: Optional[torch.Tensor], n_ex
     if indices.dtype not in (torch.int32, torch.int64):
         indices = indices.to(torch.int64)
     indices = indices.contiguous()
-    if token_mask is not None:
-        token_mask = token_mask.to(torch.bool).contiguous()
+    token_mask = ops.token_mask_of(token_mask, indices)
     lib = _lib.load()
     row_tokens = torch.empty(capacity, dtype=torch.int32, device=dev)
     row_map = torch.empty((T, K), dtype=torch.int32, device=dev)

@@ -76,3 +76,22 @@ def test_one_call_experts_refuses_a_small_workspace(dev):
     args = lambda n: _lib.load().cfp8_moe_experts(t.data_ptr(), 256, 4, 256, t.data_ptr(), 8, None, t.data_ptr(), 0, 2, 2, t.data_ptr(), t.data_ptr(),
                                                   t.data_ptr(), t.data_ptr(), 128, t.data_ptr(), 256, t.data_ptr(), n, None)
     assert need > 0 and args(need - 1) == _lib.EWORKSPACE
+
+
+def test_token_masks_of_other_forms(dev):
+    from cosmos_rl_amd.policy.kernel.moe.moe import grouped_experts_forward, route_tokens
+    E, T, H, I = 4, 6, 256, 128
+    strategy, module = _module(dev, E, H, I, 3)
+    g = torch.Generator(device=dev).manual_seed(4)
+    x = torch.randn(T, H, generator=g, device=dev).to(torch.bfloat16)
+    idx = torch.rand(T, E, generator=g, device=dev).topk(2, dim=1).indices
+    w = torch.rand(T, 2, generator=g, device=dev).to(torch.bfloat16)
+    want = grouped_experts_forward(x, None, w, idx, strategy, module, E)
+    one = torch.ones(1, dtype=torch.bool, device=dev)
+    for mask in (one, one[0], torch.ones(T, dtype=torch.int64, device=dev)):   # one value for all tokens, whole numbers
+        assert torch.equal(grouped_experts_forward(x, mask, w, idx, strategy, module, E), want)
+    for mask in (torch.ones(T, dtype=torch.bool), one.expand(T - 1)):          # on the host, too short: refused before a launch
+        with pytest.raises((ValueError, RuntimeError)):
+            grouped_experts_forward(x, mask, w, idx, strategy, module, E)
+        with pytest.raises((ValueError, RuntimeError)):
+            route_tokens(idx, mask, E)
