@@ -2103,11 +2103,13 @@ __global__ __launch_bounds__(NTL * 128) void gemm_rowwise_skinny_kernel(const Ge
 // before the first MFMA: all of its steps if they are at most eight, else equal
 // chunks of at most eight (16 KiB of weights per wave).  Loads for steps that do
 // not exist cost as much as others: with eight for every K, 9728 x 896 took 11.1 us
-// against 4.6, 23552 x 1152 21.3 against 8.0.  The loads are cacheable: streaming
-// ones were slower wherever a launch has more workgroups than fit at once (37888 x
-// 3584 33.3 against 25.4 us, 5.4 TB/s, M = 1; 45 against 37 us at M = 16, where L2
-// also returns 16 activation rows for 16 weight rows, which bounds it).  The few
-// activation rows come straight from global memory (they stay in L2), rows >= M repeat row 0.
+// against 4.6, 23552 x 1152 21.3 against 8.0.  The weights' loads are streaming ones:
+// cacheable ones push the lines that the kernels before have written out of L2, and
+// wait for them.  37888 x 3584 at 16 tokens, streaming and cacheable: 30.1 / 33.1 us
+// (5.4 TB/s at one token) behind kernels that wrote little, 34.0 / 59.8 us behind one that left
+// L2 full of its output; only one token with nothing to write back is faster cacheable,
+// 28.3 / 24.6 us, against 31.8 / 49.4 us otherwise.  The few activation rows come
+// straight from global memory (they stay in L2), rows >= M repeat row 0.
 // ---------------------------------------------------------------------------
 template <int NI, bool OUT_F32>
 __global__ __launch_bounds__(256) void gemm_rowwise_gemv_kernel(const GemmArgs p) {
@@ -2128,8 +2130,8 @@ __global__ __launch_bounds__(256) void gemm_rowwise_gemv_kernel(const GemmArgs p
             const int kt = base + 4 * i;
             if (kt >= KT) continue;
             const int64_t off = (int64_t)kt << 7;
-            wl[i] = *reinterpret_cast<const u32x4*>(wptr + off);
-            wh[i] = *reinterpret_cast<const u32x4*>(wptr + off + 16);
+            wl[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wptr + off));
+            wh[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wptr + off + 16));
             xl[i] = *reinterpret_cast<const u32x4*>(xptr + off);
             xh[i] = *reinterpret_cast<const u32x4*>(xptr + off + 16);
         }
@@ -2181,7 +2183,7 @@ __global__ __launch_bounds__(256) void gemm_rowwise_gemv_kernel(const GemmArgs p
 // thread holds at most two (four) 16-byte vectors of a token between the amax and the cast, exactly the
 // arithmetic of the rowwise quantiser - into LDS, from where the MFMA fragments are read.  The
 // quantisation hides behind the weight loads, and the separate launch (3 us plus the gap between two
-// launches) is gone: 896 x 4864 10.2 -> 6.1 us, 18944 x 3584 20.1 -> 15.5 us with the loads as above.  At four
+// launches) is gone: 896 x 4864 10.2 -> 6.1 us; 18944 x 3584 takes 16.2 us.  At four
 // tokens the quantisation in every workgroup costs what the launch would (18944 x 2560 15.9 us either way), beyond
 // that more; and 8192 is what a wave's registers hold.  Results are bit-identical to the two-launch path.
 // ---------------------------------------------------------------------------
@@ -2203,8 +2205,8 @@ __global__ __launch_bounds__(256) void linear_gemv_fused_kernel(const uint4* __r
         // (a wave without this step repeats the last one: under a branch the loads were sunk behind the barriers, 17664 x
         // 2176 17 against 11 us)
         const int kt = wave + 4 * i < KT ? wave + 4 * i : KT - 1;
-        wl[i] = *reinterpret_cast<const u32x4*>(wptr + ((int64_t)kt << 7));
-        wh[i] = *reinterpret_cast<const u32x4*>(wptr + ((int64_t)kt << 7) + 16);
+        wl[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wptr + ((int64_t)kt << 7)));
+        wh[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wptr + ((int64_t)kt << 7) + 16));
     }
     // the tokens (MR >= M of them): amax, scale, cast - rows >= M read row 0 and are never used
     const int nvec = p.K >> 3;
