@@ -35,7 +35,7 @@ struct RingPlan {
 RingPlan ring_plan(int mode, int64_t M, int64_t N, int64_t K, size_t partial_bytes, int cus);
 bool ring_takes(int mode, const RingArgs& p, int out_dtype);  // whether the operands fit what the kernel assumes
 bool ring_grouped_takes(int64_t K);
-int launch_ring_grouped(int mode, RingArgs& p, int64_t row_tiles, hipStream_t st);
+int launch_ring_grouped(int mode, RingArgs& p, int64_t row_tiles, bool once, hipStream_t st);
 int launch_ring(int mode, RingArgs& p, const RingPlan& plan, int out_dtype, hipStream_t st);
 
 }  // namespace cfp8

@@ -98,7 +98,8 @@ __device__ __forceinline__ RowTile ring_row_tile(const RingArgs& p, int lane) {
     return {-1, 0, 0, 0};
 }
 
-template <int MODE, int BM, int BN, int PER, bool SPLIT, bool OUT_F32>
+// ONCE: one row of tiles, so that no line of the weights is read twice; it is loaded as a stream (see ring_streams)
+template <int MODE, int BM, int BN, int PER, bool SPLIT, bool OUT_F32, bool ONCE = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_ring_kernel(const RingArgs p) {
     using Sh = RingShape<MODE, BM, BN, PER>;
     constexpr int LX = Sh::LX, LW = Sh::LW, LS = Sh::LS, L = LX + LW + LS, S = Sh::S;
@@ -192,7 +193,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
         else if (l < LX + LW)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_void*)(smem + WB + st * Sh::WS + (wave + 4 * (l - LX)) * 1024), 16,
                                                      in ? (at_tail ? vw_tail : vw) : kOutside,
-                                                     (uint32_t)(l - LX) * w_step + ((uint32_t)kt << (MODE == kRingMx ? 6 : 7)), 0, 0);
+                                                     (uint32_t)(l - LX) * w_step + ((uint32_t)kt << (MODE == kRingMx ? 6 : 7)), 0, ONCE ? 2 : 0);
         else  // the step's four scale bytes of a row; in a last step that is shorter the four that end with the row
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)(smem + SB + st * 1024 + wave * 256), 4, in ? vs : kOutside,
                                                      at_tail && tail ? (uint32_t)(p.K >> 5) - 4u : (uint32_t)kt << 2, 0, 0);
@@ -495,6 +496,15 @@ __global__ __launch_bounds__(256) void ring_reduce_kernel(const RingArgs p) {
     else *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.out) + (int64_t)m * p.ld_out + n) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
 }
 
+// Tiles whose weights are loaded as a stream where there is one row of them.  Cacheable loads push the lines that the kernels
+// before have written out of L2 and wait for them.  33 tokens, cacheable and streaming: 37888 x
+// 3584 34.6 and 32.0 us, 3584 x 18944 23.1 and 22.6, behind a kernel that left L2 full of its output 60.9 and 35.8, 37.5
+// and 26.3; block-scaled 24 x 18432 x 7168 with its quantiser 36.2 and 34.0.  With more rows of tiles, whose workgroups
+// share the weights through L2, it is the other way round (four linears at 1111 tokens 299 and 321 us).
+// Not for MXFP4: half a line a step, and the other half is gone before its step (64 x 18944 x 3584 17.1 us cacheable, 20.2
+// as a stream; behind a kernel that filled L2 with its output 29.1 and 23.4).
+constexpr bool ring_streams(int mode, int bm) { return mode != kRingMx && bm == 64; }
+
 template <int MODE, int BM, int BN, int PER, bool SPLIT>
 static int launch_ring_cfg(RingArgs& p, int out_dtype, hipStream_t st) {
     using Sh = RingShape<MODE, BM, BN, PER>;
@@ -511,10 +521,20 @@ static int launch_ring_cfg(RingArgs& p, int out_dtype, hipStream_t st) {
     if constexpr (!SPLIT) {
         if (f32) kern = gemm_ring_kernel<MODE, BM, BN, PER, false, true>;
     }
-    static std::atomic<bool> raised[65][2];
+    int form = f32;
+    if constexpr (ring_streams(MODE, BM)) {
+        if (p.tiles_m == 1) {
+            form += 2;
+            kern = gemm_ring_kernel<MODE, BM, BN, PER, SPLIT, false, true>;
+            if constexpr (!SPLIT) {
+                if (f32) kern = gemm_ring_kernel<MODE, BM, BN, PER, false, true, true>;
+            }
+        }
+    }
+    static std::atomic<bool> raised[65][4];
     const int slot = device_slot();
-    if (slot == 64) raised[64][f32].store(false, std::memory_order_relaxed);
-    if (int rc = raise_lds_limit(reinterpret_cast<const void*>(kern), 160 * 1024, raised[slot][f32])) return rc;
+    if (slot == 64) raised[64][form].store(false, std::memory_order_relaxed);
+    if (int rc = raise_lds_limit(reinterpret_cast<const void*>(kern), 160 * 1024, raised[slot][form])) return rc;
     {
         char name[80];
         snprintf(name, sizeof(name), "gemm_ring<%s,%d,%d>%s slices=%d", MODE == kRingRow ? "rowwise" : MODE == kRingBlock ? "block" : "mxfp4", BM, BN,
@@ -617,7 +637,7 @@ bool ring_takes(int mode, const RingArgs& p, int out_dtype) {
 // The two products of a MoE layer's experts: `row_tiles` bounds the number of tiles of kRingGroupRows rows.
 bool ring_grouped_takes(int64_t K) { return K % 128 == 0 && (K / 128 | 1) * kRingGroupRows * 4 + 2 * (K / 128) * 4 <= ring_scale_room(kRingDown) / 2; }
 
-template <int MODE>
+template <int MODE, bool ONCE>
 static int launch_ring_grouped_mode(RingArgs& p, int64_t row_tiles, hipStream_t st) {
     constexpr int BM = kRingGroupRows, BN = 128;
     using Sh = RingShape<MODE, BM, BN, 2>;
@@ -631,13 +651,15 @@ static int launch_ring_grouped_mode(RingArgs& p, int64_t row_tiles, hipStream_t 
     static std::atomic<bool> raised[65];
     const int slot = device_slot();
     if (slot == 64) raised[64].store(false, std::memory_order_relaxed);
-    if (int rc = raise_lds_limit(reinterpret_cast<const void*>(gemm_ring_kernel<MODE, BM, BN, 2, false, false>), 160 * 1024, raised[slot])) return rc;
+    if (int rc = raise_lds_limit(reinterpret_cast<const void*>(gemm_ring_kernel<MODE, BM, BN, 2, false, false, ONCE>), 160 * 1024, raised[slot])) return rc;
     if (!note_launch(MODE == kRingGateUp ? "gemm_ring<gate_up,64,128>" : "gemm_ring<down,64,128>", (unsigned)blocks, 256, lds)) return CFP8_OK;
-    hipLaunchKernelGGL((gemm_ring_kernel<MODE, BM, BN, 2, false, false>), dim3((unsigned)blocks), dim3(256), lds, st, p);
+    hipLaunchKernelGGL((gemm_ring_kernel<MODE, BM, BN, 2, false, false, ONCE>), dim3((unsigned)blocks), dim3(256), lds, st, p);
     return check_launch("gemm");
 }
-int launch_ring_grouped(int mode, RingArgs& p, int64_t row_tiles, hipStream_t st) {
-    return mode == kRingGateUp ? launch_ring_grouped_mode<kRingGateUp>(p, row_tiles, st) : launch_ring_grouped_mode<kRingDown>(p, row_tiles, st);
+// `once`: hardly an expert has a second tile of rows.
+int launch_ring_grouped(int mode, RingArgs& p, int64_t row_tiles, bool once, hipStream_t st) {
+    if (once) return mode == kRingGateUp ? launch_ring_grouped_mode<kRingGateUp, true>(p, row_tiles, st) : launch_ring_grouped_mode<kRingDown, true>(p, row_tiles, st);
+    return mode == kRingGateUp ? launch_ring_grouped_mode<kRingGateUp, false>(p, row_tiles, st) : launch_ring_grouped_mode<kRingDown, false>(p, row_tiles, st);
 }
 
 int launch_ring(int mode, RingArgs& p, const RingPlan& plan, int out_dtype, hipStream_t st) {

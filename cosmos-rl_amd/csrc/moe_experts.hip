@@ -220,6 +220,11 @@ constexpr int64_t kFewMaxHidden = 4096, kFewMaxInter = 1536;
 // 3584 x 1536, top 4: 8: 128 / 130 / 162, 16: 152 / 133 / 161, 97: 363 / 190 / 212, 128: 438 / 225 / 209; 64 of 1024 x 512, top 6:
 // 12: 42 / 44 / 71, 24: 50 / 47 / 74, 96: 88 / 62 / 77, 144: 112 / 76 / 92.
 constexpr int64_t kFewRowsPerExpert = 10, kMiddleRowsPerExpert = 112;
+// Up to here the weights of the middle form are loaded as a stream: an expert seldom has a second tile of 64 rows, which reads
+// them again.  128 experts of 2048 x 768, rows an expert, the whole call cacheable and streaming, us: 12.5 148.8 / 137.9, 25
+// 155.6 / 146.5, 49 168.4 / 163.0, 62 194.9 / 203.8, 88 232.6 / 274.3; 32 experts of 3584 x 1536: 32 134.4 / 123.4, 75
+// 190.2 / 214.2.
+constexpr int64_t kOnceRowsPerExpert = 52;
 
 enum class Form { kFew, kMiddle, kMany };
 struct ExpertsPlan {
@@ -299,18 +304,19 @@ extern "C" int cfp8_moe_experts(const void* x, int64_t ld_x, int64_t tokens, int
     if (p.form == Form::kMiddle) {
         if (int rc = cfp8_quant_group128(x, tokens, hidden, ld_x, ws + p.xq, hidden, f32(p.xs), CFP8_GROUP_MODE_DIV, stream)) return rc;
         const int64_t row_tiles = p.slots + p.rows / kRingGroupRows;
+        const bool once = p.rows <= kOnceRowsPerExpert * experts;
         RingArgs r{};
         r.a = ws + p.xq; r.w = static_cast<const uint8_t*>(gate_up); r.sa = f32(p.xs); r.sb = gate_up_scales; r.out = ws + p.h;
         r.ld_a = r.ld_w = hidden; r.ld_out = inter;
         r.row_tokens = i32(p.row_tokens); r.sizes = i32(p.m_sizes); r.ends = i32(p.m_offsets);
         r.experts = experts;
         r.M = (int)tokens; r.N = (int)(2 * inter); r.K = (int)hidden;
-        if (int rc = launch_ring_grouped(kRingGateUp, r, row_tiles, st)) return rc;
+        if (int rc = launch_ring_grouped(kRingGateUp, r, row_tiles, once, st)) return rc;
         if (int rc = cfp8_quant_group128(ws + p.h, p.rows, inter, inter, ws + p.hq, inter, f32(p.hs), CFP8_GROUP_MODE_DIV, stream)) return rc;
         r.a = ws + p.hq; r.w = static_cast<const uint8_t*>(down); r.sa = f32(p.hs); r.sb = down_scales; r.out = ws + p.out;
         r.ld_a = r.ld_w = inter; r.ld_out = hidden;
         r.M = (int)p.rows; r.N = (int)hidden; r.K = (int)inter;
-        if (int rc = launch_ring_grouped(kRingDown, r, row_tiles, st)) return rc;
+        if (int rc = launch_ring_grouped(kRingDown, r, row_tiles, once, st)) return rc;
     } else if (p.form == Form::kFew) {
         if (int rc = cfp8_quant_group128(x, tokens, hidden, ld_x, ws + p.xq, hidden, f32(p.xs), CFP8_GROUP_MODE_DIV, stream)) return rc;
         FewArgs f{};
