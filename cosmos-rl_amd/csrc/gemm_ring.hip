@@ -31,7 +31,7 @@
 // MXFP4, 200 tokens: 2176 x 14848 20 against 142 us on the register-staged tiles, 3456 x 11264 27 against 108 us.
 //
 // kRingGateUp, kRingDown: 64 x 128 tiles of a MoE layer's experts, rows gathered from the tokens, SwiGLU at the end of the first
-// (128 experts of 2048 x 768, 777 tokens top 8: the whole call 231 -> 179 us against padded tiles of 128 rows).  Bound by the
+// (128 experts of 2048 x 768, 777 tokens top 8: the whole call 231 -> 166 us against padded tiles of 128 rows).  Bound by the
 // weights' way in, hence two workgroups a CU: one loads while the other looks its tile up or leaves.
 //
 // Slices of K: fp32 partial sums into caller memory, summed in slice order with scales, bias and conversion by

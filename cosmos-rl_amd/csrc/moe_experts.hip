@@ -216,7 +216,7 @@ constexpr int64_t kFewMaxHidden = 4096, kFewMaxInter = 1536;
 // Mean rows an expert up to which a form is taken.  The few-rows form reads an expert's rows once for every strip of 16
 // features, the middle one once for every 128 columns but holds 64 rows in a tile; from about two of those tiles on the grouped
 // GEMMs' larger tiles need fewer loads a product.  Whole calls, few / middle / many rows, us: 128 experts of 2048 x 768, top 8:
-// 8 rows an expert 136 / 146 / 214, 16: 160 / 151 / 212, 49: 241 / 179 / 231, 96: 370 / 233 / 246, 128: 455 / 266 / 256; 32 of
+// 8 rows an expert 136 / 146 / 214, 16: 160 / 151 / 212, 49: 241 / 166 / 231, 96: 370 / 233 / 246, 128: 455 / 266 / 256; 32 of
 // 3584 x 1536, top 4: 8: 128 / 130 / 162, 16: 152 / 133 / 161, 97: 363 / 190 / 212, 128: 438 / 225 / 209; 64 of 1024 x 512, top 6:
 // 12: 42 / 44 / 71, 24: 50 / 47 / 74, 96: 88 / 62 / 77, 144: 112 / 76 / 92.
 constexpr int64_t kFewRowsPerExpert = 10, kMiddleRowsPerExpert = 112;
