@@ -501,9 +501,10 @@ __global__ __launch_bounds__(256) void ring_reduce_kernel(const RingArgs p) {
 // 3584 34.6 and 32.0 us, 3584 x 18944 23.1 and 22.6, behind a kernel that left L2 full of its output 60.9 and 35.8, 37.5
 // and 26.3; block-scaled 24 x 18432 x 7168 with its quantiser 36.2 and 34.0.  With more rows of tiles, whose workgroups
 // share the weights through L2, it is the other way round (four linears at 1111 tokens 299 and 321 us).
-// Not for MXFP4: half a line a step, and the other half is gone before its step (64 x 18944 x 3584 17.1 us cacheable, 20.2
-// as a stream; behind a kernel that filled L2 with its output 29.1 and 23.4).
-constexpr bool ring_streams(int mode, int bm) { return mode != kRingMx && bm == 64; }
+// MXFP4 takes half a line a step, and some of the other halves are gone before theirs, so that up to 128 rows streaming loads
+// are the slower ones behind small writes and the faster ones behind large ones (64 x 18944 x 3584 17.1 cacheable and 20.2,
+// 29.1 and 23.4; 16 x 37888 x 3584 25.6 and 27.7, 37.4 and 31.4); taken for what they bound.
+constexpr bool ring_streams(int mode, int bm) { return mode == kRingMx || bm == 64; }
 
 template <int MODE, int BM, int BN, int PER, bool SPLIT>
 static int launch_ring_cfg(RingArgs& p, int out_dtype, hipStream_t st) {
@@ -523,7 +524,7 @@ static int launch_ring_cfg(RingArgs& p, int out_dtype, hipStream_t st) {
     }
     int form = f32;
     if constexpr (ring_streams(MODE, BM)) {
-        if (p.tiles_m == 1) {
+        if (MODE == kRingMx ? p.M <= 128 : p.tiles_m == 1) {
             form += 2;
             kern = gemm_ring_kernel<MODE, BM, BN, PER, SPLIT, false, true>;
             if constexpr (!SPLIT) {
