@@ -57,16 +57,21 @@ __device__ __forceinline__ i32x8 few_frag(const u32x4& lo, const u32x4& hi) {
 
 // ---------------------------------------------------------------------------
 // gate_up and SwiGLU.  A workgroup of four waves: 16 gate rows and the 16 up rows of the same features (neighbours in the
-// interleaved weight); wave w takes K steps w, w + 4, ... (NI of them), all of whose weights it requests at once.  A lane
-// reads bytes 16 q .. 16 q + 15 and 64 + 16 q .. of a K step (q = lane >> 4) of both operands: which K positions a lane
-// holds is free as long as both operands agree, and this way a load takes 64 contiguous bytes of each of 16 rows.
-// (Cacheable loads: 55 -> 49 us for the 258 MB of 16 tokens' experts against streaming ones, 2048 x 768; with four waves
-// a SIMD 47 us = 5.5 TB/s, 69 us = 5.8 TB/s once every expert has a row.)  The four waves' sums meet in LDS; h = bf16(bf16(silu(gate)) * up) leaves as bf16, since a 1x128 group of it is spread
-// over eight workgroups.
+// interleaved weight); wave w takes K steps w, w + 4, ... (NI of them), all of whose weights it requests at once.  Results
+// have the bits of the grouped GEMMs: a lane reads bytes 32 q .. 32 q + 31 of a K step (q = lane >> 4) of both operands, as
+// their fragments have them, and the steps' products meet in LDS unscaled, 16 steps a phase, from where one wave scales and
+// adds them in the order of K.  h = bf16(bf16(silu(gate)) * up) leaves as bf16, since a 1x128 group of it is spread over
+// eight workgroups.
+// Bound by the weights' way in.  Whole calls, 128 experts of 2048 x 768, top 8, us: 16 tokens 95.5, 64 130.3 (91.5 and 126.6
+// with loads of 64 contiguous bytes and every wave's own sum, which moves roundings: 2 of the 4 us are the loads).
+// Cacheable against streaming loads, in both kernels: 16 tokens 96.2 / 102.0 behind kernels that write little, 143 / 106 behind
+// one that left L2 full of its output; 64 tokens 131.6 / 141.7 and 180 / 147; 16 tokens on 4096 x 1536 282 / 310 and 326 / 316.
+// Cacheable, since what runs in front of a decode batch's experts writes a few hundred kilobytes.
 // ---------------------------------------------------------------------------
 template <int NI>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NI <= 4 ? 4 : 2))) void few_gate_up_kernel(const FewArgs p) {
-    __shared__ __attribute__((aligned(16))) f32x4 red[2][4][2][64];
+    __shared__ __attribute__((aligned(16))) f32x4 prod[16][2][64];
+    __shared__ float factor[16][2][16];
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int lrow = lane & 15, quarter = lane >> 4;
@@ -74,16 +79,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NI <= 4 ? 4
     int start, end;
     const int e = few_expert(p, (int)blockIdx.y, lane, start, end);
     if (e < 0) return;
-    const uint8_t* const wg = p.w + ((int64_t)e * 2 * p.inter + strip * 32 + lrow) * p.hidden + quarter * 16;
+    const uint8_t* const wg = p.w + ((int64_t)e * 2 * p.inter + strip * 32 + lrow) * p.hidden + quarter * 32;
     const uint8_t* const wu = wg + (int64_t)16 * p.hidden;
     u32x4 w[NI][4];
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
         const int kt = wave + 4 * i < KT ? wave + 4 * i : KT - 1;
         w[i][0] = *reinterpret_cast<const u32x4*>(wg + (kt << 7));
-        w[i][1] = *reinterpret_cast<const u32x4*>(wg + (kt << 7) + 64);
+        w[i][1] = *reinterpret_cast<const u32x4*>(wg + (kt << 7) + 16);
         w[i][2] = *reinterpret_cast<const u32x4*>(wu + (kt << 7));
-        w[i][3] = *reinterpret_cast<const u32x4*>(wu + (kt << 7) + 64);
+        w[i][3] = *reinterpret_cast<const u32x4*>(wu + (kt << 7) + 16);
     }
     float sg[NI], su[NI];
     const float* const sp = p.ws + ((int64_t)e * (p.inter >> 6) + 2 * (strip >> 3)) * KT;
@@ -93,11 +98,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NI <= 4 ? 4
         sg[i] = sp[kt];
         su[i] = sp[KT + kt];
     }
-    int turn = 0;
-    for (int r0 = start; r0 < end; r0 += 16, turn ^= 1) {
+    for (int r0 = start; r0 < end; r0 += 16) {
         const int row = r0 + lrow;
         const int64_t token = p.row_tokens[row < end ? row : end - 1];
-        const uint8_t* const xp = p.xq + token * p.hidden + quarter * 16;
+        const uint8_t* const xp = p.xq + token * p.hidden + quarter * 32;
         const float* const xsp = p.xs + token * KT;
         u32x4 x[NI][2];
         float xs[NI];
@@ -105,34 +109,46 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NI <= 4 ? 4
         for (int i = 0; i < NI; ++i) {
             const int kt = wave + 4 * i < KT ? wave + 4 * i : KT - 1;
             x[i][0] = *reinterpret_cast<const u32x4*>(xp + (kt << 7));
-            x[i][1] = *reinterpret_cast<const u32x4*>(xp + (kt << 7) + 64);
+            x[i][1] = *reinterpret_cast<const u32x4*>(xp + (kt << 7) + 16);
             xs[i] = xsp[kt];
         }
+        const bool adds = wave == ((r0 - start) >> 4 & 3) && row < end;  // the tiles' sums are taken in turn
         f32x4 g = {0.f, 0.f, 0.f, 0.f}, u = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            if (i == NI - 1 && wave + 4 * i >= KT) continue;
-            const i32x8 xf = few_frag(x[i][0], x[i][1]);
-            const f32x4 pg = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(few_frag(w[i][0], w[i][1]), xf, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
-            const f32x4 pu = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(few_frag(w[i][2], w[i][3]), xf, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
-            const float fg = xs[i] * sg[i], fu = xs[i] * su[i];
+        for (int ph = 0; ph < (NI + 3) / 4; ++ph) {
+            if (ph || r0 != start) __syncthreads();  // the sums of the phase before have been taken
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                g[k] = __builtin_fmaf(pg[k], fg, g[k]);
-                u[k] = __builtin_fmaf(pu[k], fu, u[k]);
+            for (int i = 4 * ph; i < NI && i < 4 * ph + 4; ++i) {
+                if (i == NI - 1 && wave + 4 * i >= KT) continue;
+                const i32x8 xf = few_frag(x[i][0], x[i][1]);
+                const f32x4 pg = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(few_frag(w[i][0], w[i][1]), xf, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
+                const f32x4 pu = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(few_frag(w[i][2], w[i][3]), xf, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
+                const int at = wave + 4 * (i - 4 * ph);
+                if (row < end) {
+                    prod[at][0][lane] = pg;
+                    prod[at][1][lane] = pu;
+                    if (quarter == 0) {
+                        factor[at][0][lrow] = xs[i] * sg[i];
+                        factor[at][1][lrow] = xs[i] * su[i];
+                    }
+                }
+            }
+            __syncthreads();
+            if (adds) {
+                const int steps = KT - 16 * ph < 16 ? KT - 16 * ph : 16;
+#pragma unroll 4
+                for (int s = 0; s < steps; ++s) {
+                    const f32x4 pg = prod[s][0][lane], pu = prod[s][1][lane];
+                    const float fg = factor[s][0][lrow], fu = factor[s][1][lrow];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        g[k] = __builtin_fmaf(pg[k], fg, g[k]);
+                        u[k] = __builtin_fmaf(pu[k], fu, u[k]);
+                    }
+                }
             }
         }
-        red[turn][wave][0][lane] = g;
-        red[turn][wave][1][lane] = u;
-        // one barrier a tile: the buffer written two tiles on has been read before its writers pass the next barrier
-        __syncthreads();
-        if (wave == ((r0 - start) >> 4 & 3) && row < end) {
-#pragma unroll
-            for (int v = 1; v < 4; ++v) {
-                const f32x4 og = red[turn][(wave + v) & 3][0][lane], ou = red[turn][(wave + v) & 3][1][lane];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) g[k] += og[k], u[k] += ou[k];
-            }
+        if (adds) {
             u32 h0, h1;
             swiglu_quad(pack_bf16x2(g[0], g[1]), pack_bf16x2(g[2], g[3]), pack_bf16x2(u[0], u[1]), pack_bf16x2(u[2], u[3]), h0, h1);
             *reinterpret_cast<uint2*>(p.h + (int64_t)row * p.inter + strip * 16 + quarter * 4) = make_uint2(h0, h1);
@@ -142,8 +158,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NI <= 4 ? 4
 
 // ---------------------------------------------------------------------------
 // down.  A workgroup of eight waves: 128 weight rows, 16 a wave over the whole of K (NI = inter / 128 steps), all requested
-// at once; under those loads the workgroup quantises 16 rows of h (1x128, as the quantiser does) into LDS.  27 us for the
-// 129 MB of 16 tokens' experts (2048 x 768), 39 us for all 201 MB; the grouped GEMM on tiles of 128 rows took 68 us.
+// at once; under those loads the workgroup quantises 16 rows of h (1x128, as the quantiser does) into LDS.  About 27 us
+// for the 129 MB of 16 tokens' experts (2048 x 768); the grouped GEMM on tiles of 128 rows took 68 us.
 // ---------------------------------------------------------------------------
 template <int NI>
 __global__ __launch_bounds__(512) void few_down_kernel(const FewArgs p) {
@@ -157,12 +173,12 @@ __global__ __launch_bounds__(512) void few_down_kernel(const FewArgs p) {
     const int e = few_expert(p, (int)blockIdx.y, lane, start, end);
     if (e < 0) return;
     const int n0 = (int)blockIdx.x * 128 + wave * 16;
-    const uint8_t* const wp = p.w + ((int64_t)e * p.hidden + n0 + lrow) * p.inter + quarter * 16;
+    const uint8_t* const wp = p.w + ((int64_t)e * p.hidden + n0 + lrow) * p.inter + quarter * 32;
     u32x4 w[NI][2];
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
         w[i][0] = *reinterpret_cast<const u32x4*>(wp + (i << 7));
-        w[i][1] = *reinterpret_cast<const u32x4*>(wp + (i << 7) + 64);
+        w[i][1] = *reinterpret_cast<const u32x4*>(wp + (i << 7) + 16);
     }
     float sw[NI];
     const float* const sp = p.ws + ((int64_t)e * (p.hidden >> 7) + blockIdx.x) * NI;
@@ -183,8 +199,8 @@ __global__ __launch_bounds__(512) void few_down_kernel(const FewArgs p) {
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
-            const u32x4 lo = *reinterpret_cast<const u32x4*>(&q[turn][rr * PITCH + i * 128 + quarter * 16]);
-            const u32x4 hi = *reinterpret_cast<const u32x4*>(&q[turn][rr * PITCH + i * 128 + 64 + quarter * 16]);
+            const u32x4 lo = *reinterpret_cast<const u32x4*>(&q[turn][rr * PITCH + i * 128 + quarter * 32]);
+            const u32x4 hi = *reinterpret_cast<const u32x4*>(&q[turn][rr * PITCH + i * 128 + quarter * 32 + 16]);
             const f32x4 pr = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(few_frag(w[i][0], w[i][1]), few_frag(lo, hi), f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
             const float f = qs[turn][rr][i] * sw[i];
 #pragma unroll
