@@ -120,13 +120,15 @@ def load() -> ctypes.CDLL:
 
 
 DISPATCH_ROWWISE, DISPATCH_LINEAR, DISPATCH_BLOCK, DISPATCH_GROUPED, DISPATCH_GROUPED_SWIGLU, DISPATCH_MXFP4 = range(6)
+DISPATCH_LARGE_WORKSPACE, DISPATCH_SPLIT, DISPATCH_NO_MEMORY, DISPATCH_BIAS = 1, 2, 4, 8  # flags of gemm_dispatch_info
 
 
 def gemm_dispatch_info(kind: int, M: int, N: int, K: int, out_dtype: int = OUT_BF16, cus: int = 256,
-                       with_split_workspace: bool = False) -> str:
-    """The kernels a GEMM entry point would launch for a problem ("name grid=.. block=.. lds=..; ..."); needs no GPU."""
+                       with_split_workspace: bool = False, flags: int = 0) -> str:
+    """The kernels a GEMM entry point would launch for a problem ("name grid=.. block=.. lds=..; ..."); needs no GPU.
+    DISPATCH_SPLIT in ``flags``: the entry point that the operators in ``ops`` call."""
     buf = ctypes.create_string_buffer(1024)
-    check(load().cfp8_gemm_dispatch_info(kind, M, N, K, out_dtype, cus, int(with_split_workspace), buf, len(buf)))
+    check(load().cfp8_gemm_dispatch_info(kind, M, N, K, out_dtype, cus, flags | (DISPATCH_LARGE_WORKSPACE if with_split_workspace else 0), buf, len(buf)))
     return buf.value.decode()
 
 

@@ -3493,13 +3493,13 @@ int launch_quant_rowwise(const void* x, int64_t rows, int64_t cols, int64_t ld_x
 
 }  // namespace cfp8
 
-extern "C" int cfp8_gemm_dispatch_info(int kind, int64_t M, int64_t N, int64_t K, int out_dtype, int cus, int with_split_workspace,
+extern "C" int cfp8_gemm_dispatch_info(int kind, int64_t M, int64_t N, int64_t K, int out_dtype, int cus, int flags,
                                        char* buf, size_t buf_bytes) {
     using namespace cfp8;
     if (!buf || buf_bytes == 0) return set_error(CFP8_EINVAL, "gemm_dispatch_info: no buffer");
     buf[0] = 0;
     const bool rowwise_kind = kind == CFP8_DISPATCH_ROWWISE || kind == CFP8_DISPATCH_LINEAR;
-    if (M <= 0 || N <= 0 || K <= 0 || K % (rowwise_kind ? 16 : 128) || N % 16 || M > 0x7FFFFFFFll || N > 0x7FFFFFFFll || K > 0x7FFFFFFFll || cus <= 0)
+    if (M <= 0 || N <= 0 || K <= 0 || K % (rowwise_kind ? 16 : kind == CFP8_DISPATCH_MXFP4 ? 32 : 128) || N % 16 || M > 0x7FFFFFFFll || N > 0x7FFFFFFFll || K > 0x7FFFFFFFll || cus <= 0)
         return set_error(CFP8_EINVAL, "gemm_dispatch_info: bad shape or compute-unit count");
     if (out_dtype != CFP8_OUT_BF16 && out_dtype != CFP8_OUT_F32) return set_error(CFP8_EINVAL, "gemm_dispatch_info: unknown out_dtype %d", out_dtype);
     // operands that pass every alignment test; nothing dereferences them
@@ -3514,31 +3514,43 @@ extern "C" int cfp8_gemm_dispatch_info(int kind, int64_t M, int64_t N, int64_t K
     p.h_scales = reinterpret_cast<float*>(fake);
     p.ld_a = K; p.ld_b = K; p.ld_out = N;
     p.M = (int)M; p.N = (int)N; p.K = (int)K;
+    const bool split = flags & CFP8_DISPATCH_SPLIT;
+    if (split && (kind == CFP8_DISPATCH_GROUPED || kind == CFP8_DISPATCH_GROUPED_SWIGLU))
+        return set_error(CFP8_EINVAL, "gemm_dispatch_info: the grouped products have no form with partial sums");
     g_rec.dry = true;
     g_rec.cus = cus;
     g_rec.len = 0;
     g_rec.text[0] = 0;
     int rc = CFP8_OK;
+    if (split) {
+        const int bytes_of = kind == CFP8_DISPATCH_LINEAR ? CFP8_DISPATCH_ROWWISE : kind;
+        p.partial = reinterpret_cast<float*>(fake);
+        p.partial_bytes = flags & CFP8_DISPATCH_NO_MEMORY ? 0 : cfp8_gemm_partial_bytes(bytes_of, M, N, K);
+        p.bias = reinterpret_cast<const uint16_t*>(flags & CFP8_DISPATCH_BIAS ? fake : 0);
+    }
     const int64_t kb = K / 128, nb = (N + 127) / 128;
     switch (kind) {
         case CFP8_DISPATCH_ROWWISE:
-            rc = launch_gemm<kRowwise>(p, out_dtype, nullptr);
+            rc = split ? launch_rowwise_best(p, out_dtype, nullptr) : launch_gemm<kRowwise>(p, out_dtype, nullptr);
             break;
         case CFP8_DISPATCH_LINEAR:
             if (fused_gemv_applies(M, K, reinterpret_cast<const void*>(fake), K)) {
                 rc = launch_linear_gemv_fused(reinterpret_cast<const void*>(fake), K, p, out_dtype, nullptr);
             } else {
                 note_launch("quant_rowwise", 0, 256, 0);
-                if (with_split_workspace) {
+                if (flags & CFP8_DISPATCH_LARGE_WORKSPACE) {
                     p.partial = reinterpret_cast<float*>(fake);
                     p.partial_bytes = cfp8_linear_workspace_bytes_split(M, N, K) - cfp8_linear_workspace_bytes(M, K);
                 }
-                rc = launch_gemm<kRowwise>(p, out_dtype, nullptr);
+                rc = split ? launch_rowwise_best(p, out_dtype, nullptr) : launch_gemm<kRowwise>(p, out_dtype, nullptr);
             }
             break;
         case CFP8_DISPATCH_BLOCK:
             p.sb_stride_n = kb; p.sb_stride_k = 1;
-            rc = launch_gemm<kBlock>(p, out_dtype, nullptr);
+            rc = split ? launch_block_best(p, out_dtype, nullptr) : launch_gemm<kBlock>(p, out_dtype, nullptr);
+            break;
+        case CFP8_DISPATCH_MXFP4:
+            rc = mx4_dispatch(reinterpret_cast<const void*>(fake), M, N, K, out_dtype, split, p.partial_bytes);
             break;
         case CFP8_DISPATCH_GROUPED:
             p.sb_stride_n = kb; p.sb_stride_k = 1; p.sb_stride_e = nb * kb;

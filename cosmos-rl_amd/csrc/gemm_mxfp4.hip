@@ -27,6 +27,7 @@
 #include <atomic>
 
 #include "cfp8_common.h"
+#include "gemm_internal.h"
 #include "gemm_ring.h"
 
 namespace cfp8 {
@@ -1510,7 +1511,7 @@ __global__ __launch_bounds__(256) void gemm_mxfp4_strip_kernel(const Mx4Args p) 
 
 // more dynamic LDS than the default 64 KiB: the limit is raised once per device and kernel
 static int ensure_lds(const void* fn, size_t lds, std::atomic<bool> (&raised)[64]) {
-    if (lds <= 64 * 1024) return CFP8_OK;
+    if (lds <= 64 * 1024 || dry_run()) return CFP8_OK;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return set_error(CFP8_ELAUNCH, "gemm_mxfp4: no current device");
     const bool cached = dev >= 0 && dev < 64;
@@ -1523,25 +1524,11 @@ static int ensure_lds(const void* fn, size_t lds, std::atomic<bool> (&raised)[64
     return CFP8_OK;
 }
 
-// compute units of the current device (256 if the query fails), cached per device ordinal
-static int mx4_cu_count() {
-    static std::atomic<int> cached[64];  // zero-initialised
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) {
-        (void)hipGetLastError();
-        return 256;
-    }
-    if (dev >= 0 && dev < 64) {
-        const int c = cached[dev].load(std::memory_order_relaxed);
-        if (c > 0) return c;
-    }
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) {
-        (void)hipGetLastError();
-        return 256;
-    }
-    if (dev >= 0 && dev < 64) cached[dev].store(cus, std::memory_order_relaxed);
-    return cus;
+// for the launch record (gemm_internal.h); false: nothing is to be launched
+static bool mx4_launches(const char* kernel, int bm, int bn, unsigned grid, unsigned block, size_t lds) {
+    char name[64];
+    snprintf(name, sizeof(name), bn ? "gemm_mxfp4_%s<%d,%d>" : bm ? "gemm_mxfp4_%s<%d>" : "gemm_mxfp4_%s", kernel, bm, bn);
+    return note_launch(name, grid, block, lds);
 }
 
 static int launch_mx4_256(Mx4Args p, int out_dtype, hipStream_t st) {
@@ -1553,6 +1540,7 @@ static int launch_mx4_256(Mx4Args p, int out_dtype, hipStream_t st) {
     const void* fn = f32 ? reinterpret_cast<const void*>(gemm_mxfp4_256_kernel<true>) : reinterpret_cast<const void*>(gemm_mxfp4_256_kernel<false>);
     if (int rc = ensure_lds(fn, lds, raised[f32])) return rc;
     const unsigned blocks = (unsigned)(p.tiles_m * p.tiles_n);
+    if (!mx4_launches("tile", 256, 256, blocks, 256, lds)) return CFP8_OK;
     if (f32) hipLaunchKernelGGL(gemm_mxfp4_256_kernel<true>, dim3(blocks), dim3(256), lds, st, p);
     else hipLaunchKernelGGL(gemm_mxfp4_256_kernel<false>, dim3(blocks), dim3(256), lds, st, p);
     return check_launch("gemm_mxfp4");
@@ -1568,6 +1556,7 @@ static int launch_mx4_128(Mx4Args p, int out_dtype, hipStream_t st) {
     static std::atomic<bool> raised[2][64];
     const void* fn = f32 ? reinterpret_cast<const void*>(gemm_mxfp4_128_kernel<true>) : reinterpret_cast<const void*>(gemm_mxfp4_128_kernel<false>);
     if (int rc = ensure_lds(fn, lds, raised[f32])) return rc;
+    if (!mx4_launches("tile", 128, 256, (unsigned)tiles, 256, lds)) return CFP8_OK;
     if (f32) hipLaunchKernelGGL(gemm_mxfp4_128_kernel<true>, dim3((unsigned)tiles), dim3(256), lds, st, p);
     else hipLaunchKernelGGL(gemm_mxfp4_128_kernel<false>, dim3((unsigned)tiles), dim3(256), lds, st, p);
     return check_launch("gemm_mxfp4");
@@ -1583,6 +1572,7 @@ static int launch_mx4_128x512(Mx4Args p, int out_dtype, hipStream_t st) {
     static std::atomic<bool> raised[2][64];
     const void* fn = f32 ? reinterpret_cast<const void*>(gemm_mxfp4_128x512_kernel<true>) : reinterpret_cast<const void*>(gemm_mxfp4_128x512_kernel<false>);
     if (int rc = ensure_lds(fn, lds, raised[f32])) return rc;
+    if (!mx4_launches("tile", 128, 512, (unsigned)tiles, 256, lds)) return CFP8_OK;
     if (f32) hipLaunchKernelGGL(gemm_mxfp4_128x512_kernel<true>, dim3((unsigned)tiles), dim3(256), lds, st, p);
     else hipLaunchKernelGGL(gemm_mxfp4_128x512_kernel<false>, dim3((unsigned)tiles), dim3(256), lds, st, p);
     return check_launch("gemm_mxfp4");
@@ -1599,6 +1589,7 @@ static int launch_mx4_strip(Mx4Args p, int out_dtype, hipStream_t st) {
     static std::atomic<bool> raised[2][64];
     const void* fn = f32 ? reinterpret_cast<const void*>(gemm_mxfp4_strip_kernel<BM, true>) : reinterpret_cast<const void*>(gemm_mxfp4_strip_kernel<BM, false>);
     if (int rc = ensure_lds(fn, lds, raised[f32])) return rc;
+    if (!mx4_launches("strip", BM, 0, (unsigned)blocks, 256, lds)) return CFP8_OK;
     if (f32) hipLaunchKernelGGL((gemm_mxfp4_strip_kernel<BM, true>), dim3((unsigned)blocks), dim3(256), lds, st, p);
     else hipLaunchKernelGGL((gemm_mxfp4_strip_kernel<BM, false>), dim3((unsigned)blocks), dim3(256), lds, st, p);
     return check_launch("gemm_mxfp4");
@@ -1616,6 +1607,7 @@ static int launch_mx4_skinny(const Mx4Args& p, int out_dtype, hipStream_t st) {
                          : reinterpret_cast<const void*>(gemm_mxfp4_skinny_kernel<TM, NTL, KS, PC, false>);
     static std::atomic<bool> raised[2][64];
     if (int rc = ensure_lds(fn, lds, raised[f32])) return rc;
+    if (!mx4_launches("skinny", TM, NTL, blocks, NTL * 128, lds)) return CFP8_OK;
     if (f32) hipLaunchKernelGGL((gemm_mxfp4_skinny_kernel<TM, NTL, KS, PC, true>), dim3(blocks), dim3(NTL * 128), lds, st, p);
     else hipLaunchKernelGGL((gemm_mxfp4_skinny_kernel<TM, NTL, KS, PC, false>), dim3(blocks), dim3(NTL * 128), lds, st, p);
     return check_launch("gemm_mxfp4");
@@ -1741,10 +1733,12 @@ static int launch_mx4_gemv(const Mx4Args& p, int out_dtype, hipStream_t st) {
     const unsigned blocks = (unsigned)((p.N + 15) / 16);
     const size_t x_lds = (size_t)p.M * ((size_t)((p.K + 127) / 128) * 128 + 16);
     if (p.M <= kGemvLdsRows && x_lds <= 32 * 1024) {
+        if (!mx4_launches("gemv_lds", 0, 0, blocks, 256, x_lds)) return CFP8_OK;
         if (out_dtype == CFP8_OUT_F32) hipLaunchKernelGGL(gemm_mxfp4_gemv_lds_kernel<true>, dim3(blocks), dim3(256), x_lds, st, p);
         else hipLaunchKernelGGL(gemm_mxfp4_gemv_lds_kernel<false>, dim3(blocks), dim3(256), x_lds, st, p);
         return check_launch("gemm_mxfp4");
     }
+    if (!mx4_launches("gemv", 0, 0, blocks, 256, 0)) return CFP8_OK;
     if (out_dtype == CFP8_OUT_F32) hipLaunchKernelGGL(gemm_mxfp4_gemv_kernel<true>, dim3(blocks), dim3(256), 0, st, p);
     else hipLaunchKernelGGL(gemm_mxfp4_gemv_kernel<false>, dim3(blocks), dim3(256), 0, st, p);
     return check_launch("gemm_mxfp4");
@@ -1763,6 +1757,7 @@ static int launch_mx4(Mx4Args p, int out_dtype, hipStream_t st) {
     const void* fn = f32 ? reinterpret_cast<const void*>(gemm_mxfp4_kernel<BM, BN, WM, WN, KB, true>)
                          : reinterpret_cast<const void*>(gemm_mxfp4_kernel<BM, BN, WM, WN, KB, false>);
     if (int rc = ensure_lds(fn, lds, raised[f32])) return rc;
+    if (!mx4_launches("staged", BM, BN, (unsigned)tiles, WM * WN * 64, lds)) return CFP8_OK;
     if (out_dtype == CFP8_OUT_F32)
         hipLaunchKernelGGL((gemm_mxfp4_kernel<BM, BN, WM, WN, KB, true>), dim3((unsigned)tiles), dim3(WM * WN * 64), lds, st, p);
     else
@@ -1799,14 +1794,79 @@ static int gemm_mx4_dense(Mx4Args& p, float* partial, size_t partial_bytes, int 
     r.M = p.M; r.N = p.N; r.K = p.K;
     // (up to 4 tokens of K <= 4096 cfp8_linear_mxfp4 is one launch, whose bits the kernel for 16 tokens gives)
     if ((p.M <= 4 && p.K <= 4096) || !ring_takes(kRingMx, r, out_dtype)) return CFP8_OK;
-    const RingPlan plan = ring_plan(kRingMx, p.M, p.N, p.K, partial_bytes, mx4_cu_count());
+    const RingPlan plan = ring_plan(kRingMx, p.M, p.N, p.K, partial_bytes, cu_count());
     if (p.M > 128) {
         const bool aligned256 = p.M % 256 == 0 && p.N % 256 == 0 && p.K % 128 == 0 && p.ld_ws % 4 == 0 && (reinterpret_cast<uintptr_t>(p.ws) & 3u) == 0;
         // (many rounds of ring tiles take about 5 % longer than estimated)
-        if (mx4_tiles_cost(p.M, p.N, p.K, aligned256, mx4_cu_count()) <= plan.cost * (p.M > 1000 ? 1.05 : 1.0)) return CFP8_OK;
+        if (mx4_tiles_cost(p.M, p.N, p.K, aligned256, cu_count()) <= plan.cost * (p.M > 1000 ? 1.05 : 1.0)) return CFP8_OK;
     }
     taken = true;
     return launch_ring(kRingMx, r, plan, out_dtype, st);
+}
+}  // namespace cfp8
+
+namespace cfp8 {
+static int launch_mx4_best(Mx4Args& p, float* partial, size_t partial_bytes, int out_dtype, hipStream_t st) {
+    const int64_t M = p.M, N = p.N, K = p.K, ld_w = p.ld_w, ld_ws = p.ld_ws, ld_out = p.ld_out;
+    const void* const ws = p.ws;
+    void* const out = p.out;
+    const int32_t* const m_indices = p.m_indices;
+    if (!m_indices) {
+        bool taken = false;
+        const int rc = gemm_mx4_dense(p, partial, partial_bytes, out_dtype, st, taken);
+        if (rc || taken) return rc;
+    }
+    if (M <= 16 && !m_indices) return launch_mx4_gemv(p, out_dtype, st);
+    if (M <= 16) return launch_mx4<16, 64, 1, 4, 2>(p, out_dtype, st);
+    // 17..128 tokens on a wide weight: the strip kernel (a narrow weight leaves most CUs without a strip)
+    if (M <= 128 && !m_indices && K >= 128 && (N + 79) / 80 >= 128) return M <= 64 ? launch_mx4_strip<64>(p, out_dtype, st) : launch_mx4_strip<128>(p, out_dtype, st);
+    if (M <= 64 && !m_indices) {
+        // few weight rows: narrow workgroups, so that there are enough of them
+        const bool narrow = (N + 15) / 16 <= 512;
+        if (M <= 32) return narrow ? launch_mx4_skinny<2, 3>(p, out_dtype, st) : launch_mx4_skinny<2, 5>(p, out_dtype, st);
+        return narrow ? launch_mx4_skinny<4, 3>(p, out_dtype, st) : launch_mx4_skinny<4, 5>(p, out_dtype, st);
+    }
+    if (M <= 32) return launch_mx4<32, 64, 1, 4, 2>(p, out_dtype, st);
+    if (M <= 64) return launch_mx4<64, 64, 1, 4, 2>(p, out_dtype, st);
+    // 256 x 256 tiles of the direct-to-LDS pipeline once they fill at least half of the GPU
+    const bool out16 = (reinterpret_cast<uintptr_t>(out) & 15u) == 0 && (ld_out * (out_dtype == CFP8_OUT_F32 ? 4 : 2)) % 16 == 0;
+    if (!m_indices && M % 256 == 0 && N % 256 == 0 && K % 128 == 0 && ld_ws % 4 == 0 && (reinterpret_cast<uintptr_t>(ws) & 3u) == 0 &&
+        out16 && (M / 256) * (N / 256) >= 128 && (M / 256) * (N / 256) <= 0x7FFFFFFFll) {
+        // One workgroup per CU and equal tiles: the launch runs in rounds of as many tiles as there are CUs, and a last
+        // round that is at most half full costs a whole round.  Then the last tile-columns go to a second launch on
+        // smaller tiles and the first launch ends on a full round.
+        const int64_t tm = M / 256, tn = N / 256, cus = cu_count(), rem = (tm * tn) % cus;
+        const int64_t cut = (rem + tm - 1) / tm;  // tile-columns that hold the partial round
+        if (tm * tn > cus && rem > 0 && rem * 2 <= cus && cut < tn) {
+            Mx4Args head = p;
+            head.N = (int)((tn - cut) * 256);
+            if (int rc = launch_mx4_256(head, out_dtype, st)) return rc;
+            Mx4Args tail = p;
+            tail.N = (int)(cut * 256);
+            tail.w = p.w + (int64_t)head.N * ld_w;
+            tail.ws = p.ws + (int64_t)head.N * ld_ws;
+            tail.out = static_cast<uint8_t*>(out) + (int64_t)head.N * (out_dtype == CFP8_OUT_F32 ? 4 : 2);
+            return launch_mx4_128(tail, out_dtype, st);
+        }
+        return launch_mx4_256(p, out_dtype, st);
+    }
+    // every other shape with enough 128 x 256 tiles, and the grouped layout: the same pipeline with edges
+    // (128 x 512 tiles when that still gives every CU a tile and wastes under an eighth of the last tile-column)
+    // (its byte offsets inside a tile reach 463 weight rows: the pitch must stay below 2^23 for 32 bits)
+    if (out16 && K >= 128 && ld_w < (1ll << 23) && (M + 127) / 128 * ((N + 511) / 512) >= 256 && (N + 511) / 512 * 512 - N <= N / 8)
+        return launch_mx4_128x512(p, out_dtype, st);
+    if (out16 && K >= 128 && (M + 127) / 128 * ((N + 255) / 256) >= 64) return launch_mx4_128(p, out_dtype, st);
+    return launch_mx4<128, 128, 2, 2, 1>(p, out_dtype, st);
+}
+
+int mx4_dispatch(const void* any, int64_t M, int64_t N, int64_t K, int out_dtype, bool split, size_t partial_bytes) {
+    Mx4Args p{};
+    p.a = p.w = p.ws = static_cast<const uint8_t*>(any);
+    p.sa = static_cast<const float*>(any);
+    p.out = const_cast<void*>(any);
+    p.ld_a = K; p.ld_w = K / 2; p.ld_ws = K / 32; p.ld_out = N;
+    p.M = (int)M; p.N = (int)N; p.K = (int)K;
+    return launch_mx4_best(p, split ? static_cast<float*>(p.out) : nullptr, split ? partial_bytes : 0, out_dtype, nullptr);
 }
 }  // namespace cfp8
 
@@ -1841,53 +1901,7 @@ static int gemm_mxfp4_in(const void* a, int64_t ld_a, const float* sa, const voi
     p.out = out;
     p.ld_a = ld_a; p.ld_w = ld_w; p.ld_ws = ld_ws; p.ld_out = ld_out;
     p.M = (int)M; p.N = (int)N; p.K = (int)K;
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    if (!m_indices) {
-        bool taken = false;
-        const int rc = gemm_mx4_dense(p, partial, partial_bytes, out_dtype, st, taken);
-        if (rc || taken) return rc;
-    }
-    if (M <= 16 && !m_indices) return launch_mx4_gemv(p, out_dtype, st);
-    if (M <= 16) return launch_mx4<16, 64, 1, 4, 2>(p, out_dtype, st);
-    // 17..128 tokens on a wide weight: the strip kernel (a narrow weight leaves most CUs without a strip)
-    if (M <= 128 && !m_indices && K >= 128 && (N + 79) / 80 >= 128) return M <= 64 ? launch_mx4_strip<64>(p, out_dtype, st) : launch_mx4_strip<128>(p, out_dtype, st);
-    if (M <= 64 && !m_indices) {
-        // few weight rows: narrow workgroups, so that there are enough of them
-        const bool narrow = (N + 15) / 16 <= 512;
-        if (M <= 32) return narrow ? launch_mx4_skinny<2, 3>(p, out_dtype, st) : launch_mx4_skinny<2, 5>(p, out_dtype, st);
-        return narrow ? launch_mx4_skinny<4, 3>(p, out_dtype, st) : launch_mx4_skinny<4, 5>(p, out_dtype, st);
-    }
-    if (M <= 32) return launch_mx4<32, 64, 1, 4, 2>(p, out_dtype, st);
-    if (M <= 64) return launch_mx4<64, 64, 1, 4, 2>(p, out_dtype, st);
-    // 256 x 256 tiles of the direct-to-LDS pipeline once they fill at least half of the GPU
-    const bool out16 = (reinterpret_cast<uintptr_t>(out) & 15u) == 0 && (ld_out * (out_dtype == CFP8_OUT_F32 ? 4 : 2)) % 16 == 0;
-    if (!m_indices && M % 256 == 0 && N % 256 == 0 && K % 128 == 0 && ld_ws % 4 == 0 && (reinterpret_cast<uintptr_t>(ws) & 3u) == 0 &&
-        out16 && (M / 256) * (N / 256) >= 128 && (M / 256) * (N / 256) <= 0x7FFFFFFFll) {
-        // One workgroup per CU and equal tiles: the launch runs in rounds of as many tiles as there are CUs, and a last
-        // round that is at most half full costs a whole round.  Then the last tile-columns go to a second launch on
-        // smaller tiles and the first launch ends on a full round.
-        const int64_t tm = M / 256, tn = N / 256, cus = mx4_cu_count(), rem = (tm * tn) % cus;
-        const int64_t cut = (rem + tm - 1) / tm;  // tile-columns that hold the partial round
-        if (tm * tn > cus && rem > 0 && rem * 2 <= cus && cut < tn) {
-            Mx4Args head = p;
-            head.N = (int)((tn - cut) * 256);
-            if (int rc = launch_mx4_256(head, out_dtype, st)) return rc;
-            Mx4Args tail = p;
-            tail.N = (int)(cut * 256);
-            tail.w = p.w + (int64_t)head.N * ld_w;
-            tail.ws = p.ws + (int64_t)head.N * ld_ws;
-            tail.out = static_cast<uint8_t*>(out) + (int64_t)head.N * (out_dtype == CFP8_OUT_F32 ? 4 : 2);
-            return launch_mx4_128(tail, out_dtype, st);
-        }
-        return launch_mx4_256(p, out_dtype, st);
-    }
-    // every other shape with enough 128 x 256 tiles, and the grouped layout: the same pipeline with edges
-    // (128 x 512 tiles when that still gives every CU a tile and wastes under an eighth of the last tile-column)
-    // (its byte offsets inside a tile reach 463 weight rows: the pitch must stay below 2^23 for 32 bits)
-    if (out16 && K >= 128 && ld_w < (1ll << 23) && (M + 127) / 128 * ((N + 511) / 512) >= 256 && (N + 511) / 512 * 512 - N <= N / 8)
-        return launch_mx4_128x512(p, out_dtype, st);
-    if (out16 && K >= 128 && (M + 127) / 128 * ((N + 255) / 256) >= 64) return launch_mx4_128(p, out_dtype, st);
-    return launch_mx4<128, 128, 2, 2, 1>(p, out_dtype, st);
+    return launch_mx4_best(p, partial, partial_bytes, out_dtype, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int cfp8_gemm_mxfp4(const void* a, int64_t ld_a, const float* sa, const void* w, int64_t ld_w, const void* ws,

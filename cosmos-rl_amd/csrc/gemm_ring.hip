@@ -536,15 +536,17 @@ static int launch_ring_cfg(RingArgs& p, int out_dtype, hipStream_t st) {
     const int slot = device_slot();
     if (slot == 64) raised[64][form].store(false, std::memory_order_relaxed);
     if (int rc = raise_lds_limit(reinterpret_cast<const void*>(kern), 160 * 1024, raised[slot][form])) return rc;
+    const unsigned rb = (unsigned)(((int64_t)p.M * (p.N >> 2) + 255) / 256);
     {
         char name[80];
         snprintf(name, sizeof(name), "gemm_ring<%s,%d,%d>%s slices=%d", MODE == kRingRow ? "rowwise" : MODE == kRingBlock ? "block" : "mxfp4", BM, BN,
                  p.K & 127 ? " ktail" : "", p.slices);
-        if (!note_launch(name, (unsigned)blocks, 256, lds)) return CFP8_OK;
+        const bool real = note_launch(name, (unsigned)blocks, 256, lds);
+        if (SPLIT) note_launch("ring_reduce", rb, 256, 0);
+        if (!real) return CFP8_OK;
     }
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), lds, st, p);
     if (SPLIT) {
-        const unsigned rb = (unsigned)(((int64_t)p.M * (p.N >> 2) + 255) / 256);
         if (f32) hipLaunchKernelGGL((ring_reduce_kernel<MODE, true>), dim3(rb), dim3(256), 0, st, p);
         else hipLaunchKernelGGL((ring_reduce_kernel<MODE, false>), dim3(rb), dim3(256), 0, st, p);
     }

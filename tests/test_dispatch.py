@@ -103,6 +103,36 @@ def test_dispatch_limits_of_the_walking_forms():
         assert "ktail" in info(ROW, M, N, K) and "ktail" in info(LIN, M, N, K)
 
 
+# What the operators in ops.py launch: the entry points with memory for partial sums, which choose by estimated time.
+S, NONE, BIAS, MX = L.DISPATCH_SPLIT, L.DISPATCH_NO_MEMORY, L.DISPATCH_BIAS, L.DISPATCH_MXFP4
+OPERATORS = [
+    ("linear, one token: one launch", (LIN, 1, 3584, 3584), S, ["linear_gemv_fused"]),
+    ("linear, 1111 tokens, gate_up: the edge form, the last rows as whole tiles", (LIN, 1111, 37888, 3584), S,
+     ["quant_rowwise", "gemm_rowwise_edge tail=0 edges=0 grid=256"]),
+    ("1111 tokens, one round and 114 tiles: those as quarter tiles", (ROW, 1111, 18944, 3584), S, ["gemm_rowwise_edge tail=114 edges=0"]),
+    ("1111 tokens, down: a round of ring tiles", (ROW, 1111, 3584, 18944), S, ["gemm_ring<rowwise,128,128> slices=1 grid=252"]),
+    ("full tiles without a bias: the walking form", (ROW, 8192, 4608, 3584), S, ["gemm_rowwise_256p tail=64"]),
+    ("full tiles with a bias: the edge form, which adds it", (ROW, 8192, 4608, 3584), S | BIAS, ["gemm_rowwise_edge tail=64 edges=0"]),
+    ("a narrow weight and a long K: slices", (ROW, 200, 896, 18944), S, ["gemm_ring<rowwise,", "ring_reduce"]),
+    ("... none without memory", (ROW, 200, 896, 18944), S | NONE, ["gemm_ring<rowwise,"]),
+    ("K of 16 k: the ring kernel masks its last step", (ROW, 200, 2880, 2896), S | BIAS, ["gemm_ring<rowwise,64,64> ktail"]),
+    ("block, a decode batch", (BLK, 24, 18432, 7168), S, ["gemm_ring<block,64,128> slices=1 grid=144"]),
+    ("block, full tiles", (BLK, 4096, 18432, 7168), S, ["gemm_block_256 grid=1024", "gemm_block_w8<256,128,block>"]),
+    ("block, full tiles and a ring kernel behind them", (BLK, 3000, 4480, 3200), S, ["gemm_block_w8p<256,128,block>", "gemm_ring<block,64,64>"]),
+    ("block, some hundred rows on a wide weight: staged tiles", (BLK, 600, 9472, 5248), S, ["gemm_kernel<128,128,2,2,block>"]),
+    ("mxfp4, up to four tokens of a short K: as the one-launch linear", (MX, 4, 896, 896), S, ["gemm_mxfp4_gemv_lds"]),
+    ("mxfp4, 200 tokens", (MX, 200, 37888, 3584), S, ["gemm_ring<mxfp4,128,128> slices=1 grid=592"]),
+    ("mxfp4, full tiles", (MX, 8192, 18944, 3584), S, ["gemm_mxfp4_tile<256,256>", "gemm_mxfp4_tile<128,256>"]),
+    ("mxfp4, K below a step", (MX, 100, 96, 96), S, ["gemm_mxfp4_staged<128,128>"]),
+]
+
+
+@pytest.mark.parametrize("name,args,flags,want", OPERATORS, ids=[c[0] for c in OPERATORS])
+def test_dispatch_of_the_operators(name, args, flags, want):
+    got = L.gemm_dispatch_info(*args, flags=flags).split("; ")
+    assert len(got) == len(want) and all(w in g for w, g in zip(want, got)), got
+
+
 def test_dispatch_info_rejects_bad_arguments():
     lib = L.load()
     import ctypes
@@ -112,5 +142,7 @@ def test_dispatch_info_rejects_bad_arguments():
     assert lib.cfp8_gemm_dispatch_info(9, 128, 128, 128, 0, 256, 0, buf, 64) == L.EINVAL        # kind
     assert lib.cfp8_gemm_dispatch_info(GRP, 100, 256, 128, 0, 256, 0, buf, 64) == L.EINVAL      # grouped M % 128
     assert lib.cfp8_gemm_dispatch_info(ROW, 128, 128, 128, 0, 256, 0, None, 0) == L.EINVAL
+    assert lib.cfp8_gemm_dispatch_info(MX, 128, 128, 112, 0, 256, 0, buf, 64) == L.EINVAL       # MXFP4: K % 32
+    assert lib.cfp8_gemm_dispatch_info(GRP, 128, 256, 128, 0, 256, S, buf, 64) == L.EINVAL      # no partial sums there
     # a short buffer truncates, it does not overflow
     assert lib.cfp8_gemm_dispatch_info(ROW, 8192, 18944, 3584, 0, 256, 0, buf, 16) == 0 and len(buf.value) == 15
