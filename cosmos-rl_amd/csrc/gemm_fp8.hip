@@ -3352,11 +3352,15 @@ __global__ __launch_bounds__(256) void bias_rows_kernel(void* out, int64_t ld_ou
 
 // Rowwise product with a bias and memory for partial sums: the form with the least estimated time among the ring kernel
 // (gemm_ring.hip), the walking 256 x 256 tiles with edges, and, up to 128 tokens, the weight streamers of launch_gemm.
-// The streamers' estimates, in microseconds: up to 16 tokens the larger of the weights' way in (token rows come from L2 beside
-// them) and the chunks of K one after the other, beyond that rounds of strips times K steps.  Timed with weights that no cache
-// holds, ring / launch_gemm: 739 x 1024 x 1024 5.8 / 21.7 us, 152 x 1792 x 12672 17 / 88, 1061 x 2560 x 7936 40 / 75, 637 x
-// 18944 x 3584 63 / 64, 21 x 896 x 17152 11 / 33, 42 x 32768 x 2560 20 / 28; 33 x 37888 x 3584, two full rounds of strips,
-// 37 / 30.
+// The streamers' estimates, in microseconds: up to 16 tokens the weights' way in (token rows come from L2 beside
+// them) joined with the chunks of K one after the other, beyond that rounds of strips times K steps; fitted to 468 shapes of 5 to
+// 128 tokens, timed behind small writes and behind one that left L2 full, to the mean of the two, 5 and 4 % off on average.
+// Within 8 % of each other the streamers are taken, which lose less behind large writes (33 x 18944 x 3584 with the token quantiser
+// 19.9 / 23.7 us, ring 21.1 / 25.6), and within 25 % beyond 96 tokens, where the ring kernel's second row of tiles of 64 fills up
+// (121 x 3328 x 3328 15.7 / 18.5, ring 16.1 / 21.4).
+// Timed with weights that no cache holds, ring / launch_gemm: 739 x 1024 x 1024 5.8 / 21.7 us, 152 x 1792 x 12672 17 / 88, 1061
+// x 2560 x 7936 40 / 75, 637 x 18944 x 3584 63 / 64, 21 x 896 x 17152 11 / 33, 33 x 25344 x 2560 15.0 / 23.6; 33 x 18944 x 3584, one
+// round of strips, 17.3 / 16.4, 64 x 2048 x 1536 7.0 / 6.2, 16 x 1792 x 1792 6.8 / 4.3.
 static int launch_rowwise_best(GemmArgs& p, int out_dtype, hipStream_t st) {
     const int cus = cu_count();
     RingArgs r{};
@@ -3372,17 +3376,18 @@ static int launch_rowwise_best(GemmArgs& p, int out_dtype, hipStream_t st) {
     double stream = 1e30;
     if (p.M <= 128 && p.K % 128 == 0) {
         const double kt = p.K / 128, bytes = (double)p.N * p.K;
-        auto rounds = [&](int rows) { return (double)(((int64_t)(p.N + rows - 1) / rows + cus - 1) / cus); };
-        const bool narrow = (p.N + 79) / 80 < 128;
         if (p.M <= 16) {
-            const double chunks = (p.K / 128 + 31) / 32, latency = chunks * (2.4 + 0.1 * p.M), stream_in = bytes * (1 + p.M / 32.0) / 5.4e6;
-            stream = 2.0 + (latency > stream_in ? latency : stream_in);
+            const int steps = ((p.K >> 7) + 3) / 4, chunks = (steps + 7) / 8;  // as launch_rowwise_gemv has them
+            const double latency = chunks * (1.25 + 0.137 * ((steps + chunks - 1) / chunks) * (1 + 0.045 * p.M));
+            const double in = bytes * (1 + 0.03 * p.M) / 5.35e6 + 0.097 * chunks * p.N / 4096;
+            stream = 1.9 + sqrt(latency * latency + in * in);
         } else {
-            const double step = p.M <= 64 ? (narrow ? 0.22 : 0.50) : (narrow ? 0.32 : 0.85), in = bytes / 4.7e6;
-            const double run = rounds(narrow ? 32 : 80) * kt * step;
-            stream = 3.5 + (run > in ? run : in);
-            if (p.bias) stream += 4.0;
+            const bool narrow = (p.N + 79) / 80 < 128;  // as launch_rowwise_strip has it
+            const int strips = (p.N + (narrow ? 31 : 79)) / (narrow ? 32 : 80);
+            stream = 1.5 + ((strips + cus - 1) / cus) * (1.5 + kt * (p.M <= 64 ? (narrow ? 0.215 : 0.451) : (narrow ? 0.32 : 0.626))) + bytes / 30e6;
+            if (p.bias) stream += 4.0;  // (bias_rows_kernel)
         }
+        stream /= p.M <= 96 ? 1.08 : 1.25;
     }
     if (ring.cost < 1e30 && ring.cost <= edge.cost && ring.cost <= stream) return launch_ring(kRingRow, r, ring, out_dtype, st);
     // (without a bias and without remainders launch_gemm's form of the same tiles is 2 % faster)

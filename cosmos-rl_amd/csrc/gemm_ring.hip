@@ -98,7 +98,7 @@ __device__ __forceinline__ RowTile ring_row_tile(const RingArgs& p, int lane) {
     return {-1, 0, 0, 0};
 }
 
-// ONCE: one row of tiles, so that no line of the weights is read twice; it is loaded as a stream (see ring_streams)
+// ONCE: the weights are loaded as a stream (see ring_once)
 template <int MODE, int BM, int BN, int PER, bool SPLIT, bool OUT_F32, bool ONCE = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_ring_kernel(const RingArgs p) {
     using Sh = RingShape<MODE, BM, BN, PER>;
@@ -496,15 +496,25 @@ __global__ __launch_bounds__(256) void ring_reduce_kernel(const RingArgs p) {
     else *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.out) + (int64_t)m * p.ld_out + n) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
 }
 
-// Tiles whose weights are loaded as a stream where there is one row of them.  Cacheable loads push the lines that the kernels
-// before have written out of L2 and wait for them.  33 tokens, cacheable and streaming: 37888 x
-// 3584 34.6 and 32.0 us, 3584 x 18944 23.1 and 22.6, behind a kernel that left L2 full of its output 60.9 and 35.8, 37.5
-// and 26.3; block-scaled 24 x 18432 x 7168 with its quantiser 36.2 and 34.0.  With more rows of tiles, whose workgroups
-// share the weights through L2, it is the other way round (four linears at 1111 tokens 299 and 321 us).
-// MXFP4 takes half a line a step, and some of the other halves are gone before theirs, so that up to 128 rows streaming loads
-// are the slower ones behind small writes and the faster ones behind large ones (64 x 18944 x 3584 17.1 cacheable and 20.2,
-// 29.1 and 23.4; 16 x 37888 x 3584 25.6 and 27.7, 37.4 and 31.4); taken for what they bound.
-constexpr bool ring_streams(int mode, int bm) { return mode == kRingMx || bm == 64; }
+// Whether the weights are loaded as a stream: where there is one row of tiles, so that no line of them is read twice; for two rows of
+// tiles of 64, MXFP4 always and rowwise when the weights are more than 14 MiB, close to half of the eight L2s.  Cacheable loads push
+// the lines that the kernels before have written out of L2 and wait for them.  Cacheable and streaming, us, and the
+// same behind a kernel that left L2 full of its output:
+//   one row of tiles   33 x 37888 x 3584 34.6 32.0, 60.9 35.8; 33 x 3584 x 18944 23.1 22.6, 37.5 26.3; 128 x 37888 x 3584 44.3 43.2,
+//                      68.0 48.2; 80 x 25344 x 2560 18.9 17.9, 32.2 22.4; block-scaled 24 x 18432 x 7168 with its quantiser 36.2 34.0
+//   two of 64 rows     80 x 2944 x 2432 7.0 8.6, 12.6 11.8; 80 x 4608 x 3584 9.6 10.4, 16.0 14.8; 128 x 6144 x 3072 11.2 10.9, 17.0 14.2
+// With more rows of tiles, whose workgroups share the weights through L2, it is the other way round (four linears at 1111
+// tokens 299 and 321 us).
+// MXFP4 takes half a line a step, and some of the other halves are gone before theirs, so that streaming loads are as a rule the
+// slower ones behind small writes and the faster ones behind large ones, on one row of tiles (64 x 18944 x 3584 17.1 cacheable and
+// 20.0, 29.1 and 23.3; 128 x 20480 x 2304 14.2 and 15.6, 23.6 and 19.6) as on two of 64 (128 x 6144 x 3072 11.2 and 11.3, 15.7 and
+// 14.3; 105 x 4608 x 3328 12.4 and 11.6, 15.2 and 14.2); taken for what they bound.
+static bool ring_once(int mode, const RingArgs& p) {
+    if (mode == kRingMx) return p.M <= 128;
+    if (p.tiles_m == 1) return mode != kRingBlock || p.M <= 64;  // (block-scaled 65 .. 128 rows: within 5 % either way)
+    return mode == kRingRow && p.M <= 128 && (int64_t)p.N * p.K > 14 << 20;
+}
+constexpr bool ring_streams(int mode, int bm) { return mode != kRingBlock || bm == 64; }  // tiles that can have that form
 
 template <int MODE, int BM, int BN, int PER, bool SPLIT>
 static int launch_ring_cfg(RingArgs& p, int out_dtype, hipStream_t st) {
@@ -524,7 +534,7 @@ static int launch_ring_cfg(RingArgs& p, int out_dtype, hipStream_t st) {
     }
     int form = f32;
     if constexpr (ring_streams(MODE, BM)) {
-        if (MODE == kRingMx ? p.M <= 128 : p.tiles_m == 1) {
+        if (ring_once(MODE, p)) {
             form += 2;
             kern = gemm_ring_kernel<MODE, BM, BN, PER, SPLIT, false, true>;
             if constexpr (!SPLIT) {
@@ -581,7 +591,9 @@ static int launch_ring_mode(RingArgs& p, const RingPlan& plan, int out_dtype, hi
 // hides the other near where they meet; and adds a fixed time per launch and, for slices, the reduction's launch and their
 // partial sums' way out and back.  The constants are fitted to all combinations of 112 to 144 shapes each (3 .. 3000 tokens,
 // weights of 896 .. 37888 rows, K 896 .. 18944), timed with weights that no cache holds: the choice is within 2 % of the best
-// combination on average, 20 % at worst.
+// combination on average, 20 % at worst.  Those for up to 128 rows, rowwise and MXFP4, are fitted to 468 shapes of 5 to
+// 128 rows, each timed behind small writes and behind one that left L2 full, to the mean of the two: 4 and 5 % off on
+// average, the choice within 1 % of the best combination, 15 % at worst.
 struct RingRates {
     double step[4], load[4], two[4];  // 128 x 128, 64 x 128, 128 x 64, 64 x 64: microseconds a step; what a full GPU adds; what two a CU add
     double launch, ends, partial, bytes, reduce;
@@ -590,6 +602,11 @@ static const RingRates kRates[3] = {
     {{0.464, 0.312, 0.308, 0.169}, {0.249, 0.427, 0.168, 0.371}, {0.0, 0.637, 0.854, 1.062}, 2.4, 0.8, 4.8, 5.0, 2.5},
     {{0.658, 0.393, 0.0, 0.263}, {0.100, 0.335, 0.0, 0.283}, {0.0, 0.0, 0.0, 0.362}, 2.3, 1.2, 4.3, 4.9, 2.3},
     {{0.491, 0.343, 0.294, 0.210}, {0.097, 0.287, 0.213, 0.115}, {0.789, 0.793, 0.894, 1.104}, 3.1, 0.4, 4.7, 3.4, 2.7},
+};
+static const RingRates kFewRates[3] = {
+    {{0.587, 0.418, 0.387, 0.223}, {0.296, 0.465, 0.130, 0.331}, {0.0, 0.845, 0.886, 1.338}, 2.88, 0.34, 4.17, 7.97, 2.26},
+    {},
+    {{0.630, 0.523, 0.447, 0.290}, {0.170, 0.317, 0.0, 0.121}, {0.942, 0.883, 0.965, 1.274}, 2.51, 0.0, 4.22, 5.52, 2.86},
 };
 static const int kTiles[4][2] = {{128, 128}, {64, 128}, {128, 64}, {64, 64}};
 constexpr int kRingMaxSlices = 16;
@@ -600,7 +617,8 @@ static bool ring_scales_fit(int bm, int bn, int64_t steps) {
 }
 
 RingPlan ring_plan(int mode, int64_t M, int64_t N, int64_t K, size_t partial_bytes, int cus) {
-    const RingRates& r = kRates[mode];
+    const bool few = mode != kRingBlock && M <= 128;
+    const RingRates& r = few ? kFewRates[mode] : kRates[mode];
     const uint32_t KT = (uint32_t)((K + 127) / 128);
     RingPlan best{0, 0, 0, 1e30};
     const double in = ((double)N * K * (mode == kRingMx ? 0.53 : 1.0) + (double)M * K) / (r.bytes * 1e6);
@@ -620,6 +638,7 @@ RingPlan ring_plan(int mode, int64_t M, int64_t N, int64_t K, size_t partial_byt
             double us = (double)full * (step * (1 + r.load[c] + r.two[c]) + per * r.ends);
             if (part > 1) us += step * (1 + r.load[c] + r.two[c]) + 2 * r.ends;
             else if (rem) us += step * (1 + r.load[c] * (full ? part : part * part)) + r.ends;
+            if (few) us *= 0.9 + 0.2 * (double)M / (double)((M + bm - 1) / bm * bm);  // rows that do not exist are not loaded
             us = r.launch + sqrt(sqrt(us * us * us * us + in * in * in * in));
             if (s > 1) us += r.reduce + 8.0 * s * (double)M * (double)N / (r.partial * 1e6);
             if (us < best.cost) best = {bm, bn, (int)s, us};

@@ -116,6 +116,17 @@ OPERATORS = [
     ("a narrow weight and a long K: slices", (ROW, 200, 896, 18944), S, ["gemm_ring<rowwise,", "ring_reduce"]),
     ("... none without memory", (ROW, 200, 896, 18944), S | NONE, ["gemm_ring<rowwise,"]),
     ("K of 16 k: the ring kernel masks its last step", (ROW, 200, 2880, 2896), S | BIAS, ["gemm_ring<rowwise,64,64> ktail"]),
+    ("17 to 128 tokens, a round of strips", (ROW, 33, 18944, 3584), S, ["gemm_rowwise_strip<64,5> grid=237"]),
+    ("... which has no bias of its own", (ROW, 33, 18944, 3584), S | BIAS, ["gemm_ring<rowwise,64,128> slices=1 grid=148"]),
+    ("... 64 tokens", (ROW, 64, 18944, 3584), S, ["gemm_rowwise_strip<64,5> grid=237"]),
+    ("... a narrow weight", (ROW, 33, 4608, 3584), S, ["gemm_rowwise_strip<64,2> grid=144"]),
+    ("two rounds of strips and a little: ring tiles", (ROW, 33, 25344, 2560), S, ["gemm_ring<rowwise,64,128> slices=1"]),
+    ("65 to 96 tokens: tiles of 64 rows or of 128", (ROW, 80, 2944, 2432), S, ["gemm_ring<rowwise,64,64> slices=1"]),
+    ("... a wide weight", (ROW, 80, 32768, 2560), S, ["gemm_ring<rowwise,128,128> slices=1"]),
+    ("128 tokens on the widest weight: two rounds of strips", (ROW, 128, 37888, 3584), S, ["gemm_rowwise_strip<128,5>"]),
+    ("33 tokens, down: slices", (ROW, 33, 3584, 18944), S, ["gemm_ring<rowwise,64,64> slices=4", "ring_reduce"]),
+    ("16 tokens on a small weight", (ROW, 16, 1792, 1792), S, ["gemm_rowwise_gemv"]),
+    ("16 tokens on a wide weight", (ROW, 16, 37888, 3584), S, ["gemm_ring<rowwise,64,64> slices=1"]),
     ("block, a decode batch", (BLK, 24, 18432, 7168), S, ["gemm_ring<block,64,128> slices=1 grid=144"]),
     ("block, full tiles", (BLK, 4096, 18432, 7168), S, ["gemm_block_256 grid=1024", "gemm_block_w8<256,128,block>"]),
     ("block, full tiles and a ring kernel behind them", (BLK, 3000, 4480, 3200), S, ["gemm_block_w8p<256,128,block>", "gemm_ring<block,64,64>"]),
