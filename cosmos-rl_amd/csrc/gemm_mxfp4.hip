@@ -1729,10 +1729,13 @@ static int launch_linear_mx4_fused_mr(const void* x, int64_t ld_x, const Mx4Args
     return check_launch("linear_mxfp4");
 }
 
+static size_t mx4_gemv_lds(int64_t M, int64_t K) { return (size_t)M * ((size_t)((K + 127) / 128) * 128 + 16); }
+static bool mx4_gemv_in_lds(int64_t M, int64_t K) { return M <= kGemvLdsRows && mx4_gemv_lds(M, K) <= 32 * 1024; }
+
 static int launch_mx4_gemv(const Mx4Args& p, int out_dtype, hipStream_t st) {
     const unsigned blocks = (unsigned)((p.N + 15) / 16);
-    const size_t x_lds = (size_t)p.M * ((size_t)((p.K + 127) / 128) * 128 + 16);
-    if (p.M <= kGemvLdsRows && x_lds <= 32 * 1024) {
+    const size_t x_lds = mx4_gemv_lds(p.M, p.K);
+    if (mx4_gemv_in_lds(p.M, p.K)) {
         if (!mx4_launches("gemv_lds", 0, 0, blocks, 256, x_lds)) return CFP8_OK;
         if (out_dtype == CFP8_OUT_F32) hipLaunchKernelGGL(gemm_mxfp4_gemv_lds_kernel<true>, dim3(blocks), dim3(256), x_lds, st, p);
         else hipLaunchKernelGGL(gemm_mxfp4_gemv_lds_kernel<false>, dim3(blocks), dim3(256), x_lds, st, p);
@@ -1785,7 +1788,25 @@ static double mx4_tiles_cost(int64_t M, int64_t N, int64_t K, bool aligned256, i
     return 1e30;
 }
 
-// One product, ungrouped, with partial sums' memory or none: the ring kernel or the tile kernels.
+// The same for up to 128 rows: the kernels that stream the weights - a round of workgroups each 16 rows wide and the chunks of K
+// one after the other up to 16 tokens, rounds of strips times K steps beyond - fitted to 258 shapes of 5 to 128 rows, each timed behind
+// small writes and behind one that left L2 full, to the mean of the two (2 to 4 % off on average).  Infinite for narrow weights of 17 rows
+// and more: the ring kernel is the faster one there without slices too (17 x 1664 x 1664 6.5 us both, 64 x 1536 x 8960 30 against 33).
+static double mx4_streams_cost(int64_t M, int64_t N, int64_t K, int cus) {
+    const double codes = (double)N * (double)K;
+    const int64_t kt = (K + 127) / 128;
+    if (M <= 16) {
+        const double chunks = (double)((kt + 4 * kGemvDepth - 1) / (4 * kGemvDepth)), steps = (double)((kt + 3) / 4);
+        const double more = (double)(((N + 15) / 16 + cus - 1) / cus - 1);
+        if (mx4_gemv_in_lds(M, K)) return 1.8 + chunks * (1.93 + 0.035 * M + 1.24 * more) + steps * (0.026 + 0.024 * M) + codes * (1 + 0.047 * M) / 13.8e6;
+        return 2.1 + chunks * (2.2 + 2.7 * more) + steps * 0.009 * M + codes * (1 + 0.014 * M) / 19.4e6;
+    }
+    const int64_t strips = (N + 79) / 80;
+    if (strips < 128) return 1e30;
+    return 1.82 + (double)((strips + cus - 1) / cus) * (2.9 + (double)kt * (M <= 64 ? 0.378 : 0.595)) + codes / 23.7e6;
+}
+
+// One product, ungrouped, with partial sums' memory or none: the ring kernel or the others.
 static int gemm_mx4_dense(Mx4Args& p, float* partial, size_t partial_bytes, int out_dtype, hipStream_t st, bool& taken) {
     taken = false;
     RingArgs r{};
@@ -1795,7 +1816,11 @@ static int gemm_mx4_dense(Mx4Args& p, float* partial, size_t partial_bytes, int 
     // (up to 4 tokens of K <= 4096 cfp8_linear_mxfp4 is one launch, whose bits the kernel for 16 tokens gives)
     if ((p.M <= 4 && p.K <= 4096) || !ring_takes(kRingMx, r, out_dtype)) return CFP8_OK;
     const RingPlan plan = ring_plan(kRingMx, p.M, p.N, p.K, partial_bytes, cu_count());
-    if (p.M > 128) {
+    if (p.M <= 128) {
+        // (the ring kernel where it is ahead by more than the estimates are off: 18944 x 3584 at 33 tokens 19.5 against 17.4 us,
+        // 16 x 3584 x 3584 8.2 against 6.2, but 33 x 25344 x 2560 15.3 against 25.3)
+        if (mx4_streams_cost(p.M, p.N, p.K, cu_count()) <= plan.cost * 1.05) return CFP8_OK;
+    } else {
         const bool aligned256 = p.M % 256 == 0 && p.N % 256 == 0 && p.K % 128 == 0 && p.ld_ws % 4 == 0 && (reinterpret_cast<uintptr_t>(p.ws) & 3u) == 0;
         // (many rounds of ring tiles take about 5 % longer than estimated)
         if (mx4_tiles_cost(p.M, p.N, p.K, aligned256, cu_count()) <= plan.cost * (p.M > 1000 ? 1.05 : 1.0)) return CFP8_OK;

@@ -132,6 +132,13 @@ OPERATORS = [
     ("block, full tiles and a ring kernel behind them", (BLK, 3000, 4480, 3200), S, ["gemm_block_w8p<256,128,block>", "gemm_ring<block,64,64>"]),
     ("block, some hundred rows on a wide weight: staged tiles", (BLK, 600, 9472, 5248), S, ["gemm_kernel<128,128,2,2,block>"]),
     ("mxfp4, up to four tokens of a short K: as the one-launch linear", (MX, 4, 896, 896), S, ["gemm_mxfp4_gemv_lds"]),
+    ("mxfp4, 17 to 128 tokens, a round of strips", (MX, 64, 18944, 3584), S, ["gemm_mxfp4_strip<64> grid=237"]),
+    ("... without memory", (MX, 64, 18944, 3584), 0, ["gemm_mxfp4_strip<64> grid=237"]),
+    ("mxfp4, two rounds of strips and a little: ring tiles", (MX, 33, 25344, 2560), S, ["gemm_ring<mxfp4,64,128> slices=1"]),
+    ("mxfp4, 16 tokens on a small weight", (MX, 16, 3584, 3584), S, ["gemm_mxfp4_gemv"]),
+    ("mxfp4, 8 tokens on a small weight", (MX, 8, 896, 896), S, ["gemm_mxfp4_gemv_lds"]),
+    ("mxfp4, a narrow weight and a long K: slices", (MX, 33, 896, 18944), S, ["gemm_ring<mxfp4,64,64>", "ring_reduce"]),
+    ("... without memory", (MX, 33, 896, 18944), 0, ["gemm_ring<mxfp4,64,64> slices=1 grid=14"]),
     ("mxfp4, 200 tokens", (MX, 200, 37888, 3584), S, ["gemm_ring<mxfp4,128,128> slices=1 grid=592"]),
     ("mxfp4, full tiles", (MX, 8192, 18944, 3584), S, ["gemm_mxfp4_tile<256,256>", "gemm_mxfp4_tile<128,256>"]),
     ("mxfp4, K below a step", (MX, 100, 96, 96), S, ["gemm_mxfp4_staged<128,128>"]),
