@@ -7,7 +7,7 @@ from cosmos_rl_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
 
-# rows around a tile's 64 and 128, columns that end inside a wave's share, one K step and a few (the ring is 5 to 10 deep), odd
+# rows around a tile's 64 and 128, columns that end inside a wave's share, one K step and a few (the ring is 3 to 8 deep), odd
 # and even numbers of steps, a last step of 32 .. 112; long K with few columns: slices
 SHAPES = [(5, 16, 128), (17, 48, 384), (63, 144, 640), (64, 128, 1152), (65, 272, 896), (127, 80, 256), (128, 1040, 2304), (129, 256, 1280),
           (200, 400, 12800), (33, 208, 18944), (300, 4624, 512), (7, 4096, 4224)]
@@ -58,7 +58,7 @@ def _rowwise_want(q, s, w, sw, bias):
     return (want if bias is None else want + bias.double()).cpu()
 
 
-# the shapes above, the walking tiles with remainders of rows and columns below, at and above half a tile, and a partial round
+# the shapes above, the streamers of few tokens, and thousands of rows with remainders of tiles of 128
 @pytest.mark.parametrize("M,N,K", SHAPES + TAILS + [(1, 400, 1152), (3, 272, 4864), (16, 144, 4224), (90, 10256, 128), (4000, 4112, 384), (4096 + 120, 4096 + 112, 512),
                                                     (4096 + 130, 4096 + 144, 384), (2100, 9216, 640), (8000, 4352, 512)])
 @pytest.mark.parametrize("biased", [False, True])
@@ -82,6 +82,48 @@ def test_rowwise(dev, M, N, K, biased):
                 assert torch.equal(y, out[:M, :N])
                 if biased:
                     assert torch.equal(y, ops.fp8_linear(x, w.t(), sw, out_dtype=dtype) + bias)
+
+
+# the walking 256 x 256 tiles with edges.  Remainders of rows (1, 6, 64, 129) and of columns (16, 144) as quarter tiles and as a last
+# row or column of whole ones, each alone and both, with a partial last round dealt out as quarter tiles and without: (M, N, K), whether
+# there is one, whether a remainder is quarter tiles
+EDGES = [((2310, 12288, 512), False, False), ((2304, 18960, 640), False, False), ((2310, 12304, 512), False, False), ((2310, 12432, 512), False, False),
+         ((2177, 18960, 640), False, False), ((2048, 8208, 1152), False, True), ((2048, 8336, 1152), True, False), ((2177, 8192, 1152), True, False),
+         ((2049, 8208, 1152), True, True), ((2177, 8208, 1152), True, True), ((1536, 12304, 1152), True, True), ((1600, 12432, 1792), True, True),
+         ((2049, 9216, 2560), True, True), ((2048, 8192, 640), False, False), ((2304, 8192, 1152), True, False)]
+
+
+# (full tiles without a bias take the walking form without edges)
+@pytest.mark.parametrize("shape,tail,quarters,biased", [(*e, b) for b in (False, True) for e in EDGES if b or e[0][0] % 256 or e[0][1] % 256])
+def test_rowwise_edges(dev, shape, tail, quarters, biased):
+    M, N, K = shape
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    took = _lib.gemm_dispatch_info(_lib.DISPATCH_ROWWISE, M, N, K, cus=cus, flags=_lib.DISPATCH_SPLIT | (_lib.DISPATCH_BIAS if biased else 0))
+    assert took.startswith("gemm_rowwise_edge") and ("tail=0" not in took) == tail and ("edges=0" not in took) == quarters, took
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    q, s = ops.quant_rowwise(torch.randn(M, K, generator=g, device=dev).to(torch.bfloat16))
+    w, sw = ops.quant_rowwise((torch.randn(N, K, generator=g, device=dev) * 0.05).to(torch.bfloat16))
+    bias = torch.randn(N, generator=g, device=dev).to(torch.bfloat16) if biased else None
+    want = _rowwise_want(q, s, w, sw, bias)
+    for dtype in (torch.float32, torch.bfloat16):
+        runs = []
+        for _ in range(3):  # (a missing wait between a tile's stores and the next one's loads would show as a difference)
+            out = _out(M, N, dev, dtype)
+            _lib.check(_lib.load().cfp8_scaled_mm_rowwise_split(q.data_ptr(), K, s.data_ptr(), w.data_ptr(), K, sw.data_ptr(), ops._ptr(bias),
+                                                                out.data_ptr(), N + 8, ops._out_code(dtype), M, N, K, None, 0, _stream()))
+            runs.append(out)
+        assert torch.equal(runs[0], runs[1]) and torch.equal(runs[0], runs[2])
+        _check(runs[0], want, M, N, dtype, 2.0 ** -9 if biased and dtype == torch.bfloat16 else 0.0)
+        # the bits of the other kernels, cut along N into calls that the entry point without partial sums takes, the bias added as torch does
+        cut = (N // 256 + 1) // 2 * 256
+        parts = []
+        for n0, n1 in ((0, cut), (cut, N)):
+            o = torch.empty(M, n1 - n0, dtype=dtype, device=dev)
+            _lib.check(_lib.load().cfp8_scaled_mm_rowwise(q.data_ptr(), K, s.data_ptr(), w[n0:].data_ptr(), K, sw[n0:].data_ptr(), o.data_ptr(), n1 - n0,
+                                                          ops._out_code(dtype), M, n1 - n0, K, _stream()))
+            parts.append(o if bias is None else o + bias[n0:n1])
+        same = M if M % 256 == 0 or M % 256 > 16 else M // 256 * 256  # (the kernel for up to 16 rows adds the sums of four waves)
+        assert torch.equal(runs[0][:same, :N], torch.cat(parts, 1)[:same])
 
 
 def test_rowwise_bias_of_another_kind(dev):

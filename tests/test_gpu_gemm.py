@@ -561,14 +561,11 @@ def test_walking_kernels_repeatable(dev):
                     if not runs:
                         sx = torch.rand(M, 1, generator=g, device=dev) + 0.5
                         sw = torch.rand(N, 1, generator=g, device=dev) + 0.5
-                    runs.append(ops.scaled_mm(a, b.t(), sx, sw.t(), out_dtype=dt))
                 else:
                     if not runs:
                         sx = torch.rand(M, K // 128, generator=g, device=dev) + 0.5
                         sw = torch.rand(N // 128, K // 128, generator=g, device=dev) + 0.5
-                    o = torch.empty(M, N, dtype=dt, device=dev)
-                    ops.gemm_fp8_fp8_bf16_nt((a, sx), (b, sw), o)
-                    runs.append(o)
+                runs.append(_walking(dev, mode, a, sx, b, sw, dt))
             assert all(torch.equal(runs[0], r) for r in runs[1:]), f"{mode} {M}x{N}x{K} {dt}: runs differ"
 
 
@@ -660,9 +657,28 @@ def test_grouped_short_k_kernel_equal_to_sliced_calls(dev):
         assert torch.equal(wide[:, :N], ref) and bool((wide[:, N:] == 3.0).all())
 
 
+def _walking(dev, mode, a, sx, b, sw, dt):
+    """The product from the entry point that has no memory for partial sums: the walking kernels, where the operators may
+    take others."""
+    from cosmos_rl_amd import _lib
+    (M, K), N = a.shape, b.shape[0]
+    kind = _lib.DISPATCH_ROWWISE if mode == "row" else _lib.DISPATCH_BLOCK
+    took = _lib.gemm_dispatch_info(kind, M, N, K, out_dtype=ops._out_code(dt), cus=torch.cuda.get_device_properties(dev).multi_processor_count)
+    assert ("gemm_rowwise_256p" if mode == "row" else "gemm_block_w8p") in took, took
+    out, stream = torch.empty(M, N, dtype=dt, device=dev), torch.cuda.current_stream().cuda_stream
+    if mode == "row":
+        _lib.check(_lib.load().cfp8_scaled_mm_rowwise(a.data_ptr(), K, sx.data_ptr(), b.data_ptr(), K, sw.data_ptr(), out.data_ptr(), N, ops._out_code(dt),
+                                                      M, N, K, stream))
+    else:
+        _lib.check(_lib.load().cfp8_gemm_block128(a.data_ptr(), K, sx.data_ptr(), b.data_ptr(), K, sw.data_ptr(), K // 128, 1, out.data_ptr(), N,
+                                                  ops._out_code(dt), M, N, K, stream))
+    return out
+
+
 def test_walking_kernels_equal_to_sliced_calls(dev):
     """Rowwise and block-scaled: a problem with more tiles than CUs (the walking kernels) against the same problem cut
-    along N into calls that fit one round of workgroups (one tile per workgroup, or the generic kernel): same bits."""
+    along N into calls that fit one round of workgroups (one tile per workgroup, or the generic kernel), and against
+    what the operators take for it: same bits."""
     g = torch.Generator(device=dev).manual_seed(9)
     # (the third to fifth: a last round of 16, 96 and 40 tiles, which the walking kernel's workgroups take as quarter tiles)
     for mode, (M, N, K), cuts in (("row", (2304, 11520, 512), 3), ("row", (8192, 7680, 896), 6), ("row", (2048, 8704, 512), 2),
@@ -691,7 +707,8 @@ def test_walking_kernels_equal_to_sliced_calls(dev):
                     o = torch.empty(M, n1 - n0, dtype=dt, device=dev)
                     ops.gemm_fp8_fp8_bf16_nt((a, sx), (b[n0:n1], sw[n0 // 128:n1 // 128].clone()), o)
                     parts.append(o)
-            assert torch.equal(torch.cat(parts, 1), whole), f"{mode} {M}x{N}x{K} {dt}: walking form differs from the sliced calls"
+            assert torch.equal(torch.cat(parts, 1), whole), f"{mode} {M}x{N}x{K} {dt}: the whole differs from the sliced calls"
+            assert torch.equal(_walking(dev, mode, a, sx, b, sw, dt), whole), f"{mode} {M}x{N}x{K} {dt}: walking form differs"
 
 
 def test_random_shapes_all_dispatch_paths(dev):
