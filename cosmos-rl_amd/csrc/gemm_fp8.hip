@@ -647,6 +647,11 @@ __global__ __launch_bounds__(256) void gemm_rowwise_256_kernel(const GemmArgs p)
 template <int BM, int TN, bool OUT_F32, bool BIAS = false>
 __device__ __forceinline__ void rowwise_strip_block(const GemmArgs& p, uint8_t* const smem, const int m0, const int n0, const int t);
 
+// what the edge form reads where there is no bias: 64 columns of kNoBias
+__device__ const u32 kNoBiasRow[32] = {kNoBias, kNoBias, kNoBias, kNoBias, kNoBias, kNoBias, kNoBias, kNoBias, kNoBias, kNoBias, kNoBias,
+                                       kNoBias, kNoBias, kNoBias, kNoBias, kNoBias, kNoBias, kNoBias, kNoBias, kNoBias, kNoBias, kNoBias,
+                                       kNoBias, kNoBias, kNoBias, kNoBias, kNoBias, kNoBias, kNoBias, kNoBias, kNoBias, kNoBias};
+
 template <bool OUT_F32, bool EDGE>
 __device__ __forceinline__ void rowwise_256p(const GemmArgs& p) {
     constexpr int BM = 256, BN = 256;
@@ -779,8 +784,9 @@ __device__ __forceinline__ void rowwise_256p(const GemmArgs& p) {
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, (lds_void*)dst, 4, (uint32_t)lane * 4u, 0, 0, 0);
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rsb, (lds_void*)(dst + 1024), 4, (uint32_t)lane * 4u, 0, 0, 0);
                 if constexpr (EDGE) {  // the bias of the wave's 64 columns, two a lane
-                    const __amdgpu_buffer_rsrc_t rsc = __builtin_amdgcn_make_buffer_rsrc(
-                        const_cast<uint16_t*>(p.bias) + n0 + wave * 64, 0, p.bias && cols > 0 ? (cols < 64 ? cols * 2 : 128) : 0, 0x00020000);
+                    const uint16_t* const bias = p.bias ? p.bias + n0 + wave * 64 : reinterpret_cast<const uint16_t*>(kNoBiasRow);
+                    const __amdgpu_buffer_rsrc_t rsc =
+                        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(bias), 0, cols > 0 ? (cols < 64 ? cols * 2 : 128) : 0, 0x00020000);
                     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsc, (lds_void*)(dst + 2048), 4, (uint32_t)lane * 4u, 0, 0, 0);
                 }
                 ws_free = ws;
@@ -849,7 +855,7 @@ __device__ __forceinline__ void rowwise_256p(const GemmArgs& p) {
                         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), ro,
                                                                n < p.N ? ((uint32_t)(m - m0) * (uint32_t)p.ld_out + (uint32_t)(n - n0)) * 4u : 0xF0000000u, 0, 2);
                     else
-                    __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(static_cast<float*>(p.out) + (int64_t)m * p.ld_out + n));
+                        __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(static_cast<float*>(p.out) + (int64_t)m * p.ld_out + n));
                 }
             }
         } else {
@@ -878,9 +884,10 @@ __device__ __forceinline__ void rowwise_256p(const GemmArgs& p) {
                         const int n = wn * 128 + rd_chunk * 8;
                         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, d), ro,
                                                                n < p.N - n0 ? ((uint32_t)(m - m0) * (uint32_t)p.ld_out + (uint32_t)n) * 2u : 0xF0000000u, 0, 2);
-                    } else
-                    __builtin_nontemporal_store(
-                        d, reinterpret_cast<i32x4*>(static_cast<uint16_t*>(p.out) + (int64_t)m * p.ld_out + n0 + wn * 128 + rd_chunk * 8));
+                    } else {
+                        __builtin_nontemporal_store(
+                            d, reinterpret_cast<i32x4*>(static_cast<uint16_t*>(p.out) + (int64_t)m * p.ld_out + n0 + wn * 128 + rd_chunk * 8));
+                    }
                 }
             }
         }

@@ -126,6 +126,17 @@ def test_rowwise_edges(dev, shape, tail, quarters, biased):
         assert torch.equal(runs[0][:same, :N], torch.cat(parts, 1)[:same])
 
 
+@pytest.mark.parametrize("M,N,K", [(2310, 12304, 512), (33, 272, 256), (5, 48, 128)])
+def test_rowwise_without_a_bias_keeps_the_sign_of_zero(dev, M, N, K):
+    """Products that the scales take below the smallest fp32 number keep their sign: no bias is not a bias of +0."""
+    g = torch.Generator(device=dev).manual_seed(M)
+    sign = torch.where(torch.rand(M, 1, generator=g, device=dev) < 0.5, -1.0, 1.0)
+    a = (sign * torch.ones(M, K, device=dev)).to(torch.float8_e4m3fn)
+    b = torch.ones(N, K, device=dev).to(torch.float8_e4m3fn)
+    out = ops.scaled_mm(a, b.t(), torch.full((M, 1), 1e-30, device=dev), torch.full((1, N), 1e-30, device=dev), out_dtype=torch.float32)
+    assert not bool(out.any()) and torch.equal(torch.signbit(out), (sign < 0).expand(M, N))
+
+
 def test_rowwise_bias_of_another_kind(dev):
     """A bias that no epilogue takes (fp32) is added as torch adds it."""
     x = torch.randn(5, 256, device=dev).to(torch.bfloat16)
