@@ -691,6 +691,12 @@ def moe_experts(x: torch.Tensor, token_mask: Optional[torch.Tensor], weights: to
     gu, gus = gate_up_interleaved
     dn, dns = down
     _need_gpu(x, weights, indices, gu, gus, dn, dns)
+    if x.dim() != 2 or x.dtype != torch.bfloat16 or x.stride(1) != 1:
+        raise ValueError(f"expected bf16 tokens [T, H] with unit column stride, got {tuple(x.shape)} {x.dtype} strides {x.stride()}")
+    if gu.dtype != FP8_DTYPE or dn.dtype != FP8_DTYPE or gus.dtype != torch.float32 or dns.dtype != torch.float32:
+        raise ValueError(f"expected float8_e4m3fn weights with fp32 scales, got {gu.dtype}, {gus.dtype}, {dn.dtype}, {dns.dtype}")
+    if indices.dim() != 2 or gu.dim() != 3:
+        raise ValueError("expected indices [T, topk] and gate_up weights [E, 2 I, H]")
     T, H = x.shape
     E, N2, Kb = gu.shape
     I = N2 // 2

@@ -74,6 +74,23 @@ def test_one_call_experts_refuses_a_small_workspace(dev):
     assert need > 0 and args(need - 1) == _lib.EWORKSPACE
 
 
+def test_one_call_experts_refuses_other_types(dev):
+    """What the kernels would read as something else is refused before a launch."""
+    E, T, H, I = 4, 6, 256, 128
+    strategy, module = _module(dev, E, H, I, 5)
+    x = torch.randn(T, H, device=dev).to(torch.bfloat16)
+    idx = torch.rand(T, E, device=dev).topk(2, dim=1).indices
+    w = torch.rand(T, 2, device=dev).to(torch.bfloat16)
+    (gu, gus), dn, dns = strategy._interleaved(module), module.get_parameter("down_proj_fp8"), module.get_parameter("down_proj_scales")
+    assert ops.moe_experts(x, None, w, idx, (gu, gus), (dn, dns)).shape == (T, H)
+    wide = torch.randn(T, 2 * H, device=dev).to(torch.bfloat16)
+    for bad in ((x.half(), (gu, gus), (dn, dns)), (x.float(), (gu, gus), (dn, dns)), (wide[:, ::2], (gu, gus), (dn, dns)), (x[None], (gu, gus), (dn, dns)),
+                (x, (gu, gus.to(torch.bfloat16)), (dn, dns)), (x, (gu, gus), (dn, dns.double())), (x, (gu.view(torch.uint8), gus), (dn, dns)),
+                (x, (gu, gus), (dn.to(torch.bfloat16), dns))):
+        with pytest.raises(ValueError):
+            ops.moe_experts(bad[0], None, w, idx, bad[1], bad[2])
+
+
 def test_token_masks_of_other_forms(dev):
     from cosmos_rl_amd.policy.kernel.moe.moe import grouped_experts_forward, route_tokens
     E, T, H, I = 4, 6, 256, 128
