@@ -149,7 +149,10 @@ class DSGroupGEMM(GroupGEMMStrategy):
 
     def forward_experts(self, x, token_mask, weights, indices, module, n_experts):
         """``grouped_experts_forward`` as one library call, or None where the configuration or the shapes need the
-        general chain: the fused gate_up form, bf16 tokens, sizes in multiples of 128."""
+        general chain: the fused gate_up form, bf16 tokens, sizes in multiples of 128, and a strategy whose steps are
+        those of this class."""
+        if type(self).execute_from_tokens is not DSGroupGEMM.execute_from_tokens or type(self)._run is not DSGroupGEMM._run:
+            return None
         if not (self.fuse_gate_up and self.fuse_swiglu and self.fuse_epilogue) or x.dtype != torch.bfloat16 or not x.is_cuda:
             return None
         if x.dim() != 2 or indices.dim() != 2 or weights.shape != indices.shape or indices.shape[0] != x.shape[0]:

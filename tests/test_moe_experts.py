@@ -91,6 +91,32 @@ def test_one_call_experts_refuses_other_types(dev):
             ops.moe_experts(bad[0], None, w, idx, bad[1], bad[2])
 
 
+def test_strategies_with_steps_of_their_own(dev):
+    """A strategy derived from DSGroupGEMM that replaces one of its steps has that step called; one that adds to it keeps the
+    one-call form."""
+    from cosmos_rl_amd.policy.kernel.group_gemms import DSGroupGEMM
+    from cosmos_rl_amd.policy.kernel.moe.moe import grouped_experts_forward
+    calls = []
+
+    class Counted(DSGroupGEMM):
+        def _run(self, *args, **kwargs):
+            calls.append(1)
+            return super()._run(*args, **kwargs)
+
+    class Named(DSGroupGEMM):
+        name = "experts"
+
+    E, T, H, I = 4, 6, 256, 128
+    strategy, module = _module(dev, E, H, I, 6)
+    x = torch.randn(T, H, device=dev).to(torch.bfloat16)
+    idx = torch.rand(T, E, device=dev).topk(2, dim=1).indices
+    w = torch.rand(T, 2, device=dev).to(torch.bfloat16)
+    want = grouped_experts_forward(x, None, w, idx, strategy, module, E)
+    assert torch.equal(grouped_experts_forward(x, None, w, idx, Counted(torch.nn.SiLU(), fuse_gate_up=True), module, E), want) and calls == [1]
+    named = Named(torch.nn.SiLU(), fuse_gate_up=True)
+    assert torch.equal(named.forward_experts(x, None, w, idx, module, E), want)
+
+
 def test_token_masks_of_other_forms(dev):
     from cosmos_rl_amd.policy.kernel.moe.moe import grouped_experts_forward, route_tokens
     E, T, H, I = 4, 6, 256, 128
