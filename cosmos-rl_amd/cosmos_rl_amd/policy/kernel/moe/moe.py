@@ -118,7 +118,7 @@ def grouped_experts_forward(x: torch.Tensor, token_mask: Optional[torch.Tensor],
                             indices: torch.Tensor, strategy, module, n_experts: int, alignment: int = 128) -> torch.Tensor:
     """``GroupedExperts.forward(x, token_mask, weights, indices)`` (moe.py:179-285) on one rank, with the
     experts of ``module`` run by ``strategy`` (a ``GroupGEMMStrategy``) instead of the per-expert loop."""
-    if hasattr(strategy, "forward_experts"):
+    if hasattr(strategy, "forward_experts") and alignment > 0:  # (route_tokens refuses the others)
         y = strategy.forward_experts(x, token_mask, weights, indices, module, n_experts)
         if y is not None:
             return y

@@ -93,7 +93,7 @@ def test_one_call_experts_refuses_other_types(dev):
 
 def test_strategies_with_steps_of_their_own(dev):
     """A strategy derived from DSGroupGEMM that replaces one of its steps has that step called; one that adds to it keeps the
-    one-call form."""
+    one-call form.  An alignment that no layout has is refused on either way."""
     from cosmos_rl_amd.policy.kernel.group_gemms import DSGroupGEMM
     from cosmos_rl_amd.policy.kernel.moe.moe import grouped_experts_forward
     calls = []
@@ -115,6 +115,8 @@ def test_strategies_with_steps_of_their_own(dev):
     assert torch.equal(grouped_experts_forward(x, None, w, idx, Counted(torch.nn.SiLU(), fuse_gate_up=True), module, E), want) and calls == [1]
     named = Named(torch.nn.SiLU(), fuse_gate_up=True)
     assert torch.equal(named.forward_experts(x, None, w, idx, module, E), want)
+    with pytest.raises(ValueError):
+        grouped_experts_forward(x, None, w, idx, strategy, module, E, alignment=0)
 
 
 def test_token_masks_of_other_forms(dev):
