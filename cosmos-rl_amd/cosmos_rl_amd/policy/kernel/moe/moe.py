@@ -36,6 +36,7 @@ def _route_tokens_by_sorting(indices: torch.Tensor, token_mask: Optional[torch.T
     T, K = indices.shape
     dev = indices.device
     key = indices.to(torch.int64)
+    key = torch.where((key < 0) | (key > n_experts), n_experts, key)
     if token_mask is not None:
         key = torch.where(token_mask.to(torch.bool).unsqueeze(-1), key, n_experts)
     order = torch.argsort(key.reshape(-1), stable=True)
@@ -56,7 +57,8 @@ def route_tokens(indices: torch.Tensor, token_mask: Optional[torch.Tensor], n_ex
     """Expert-grouped layout of the routed (token, slot) pairs: groups in expert order, tokens ascending
     inside a group (the order ``torch.where`` gives the reference, moe.py:244-245), every group padded to
     ``alignment`` rows.  No host synchronisation: the row count is the bound ``max_rows`` (default
-    tokens * topk + n_experts * alignment); rows past the real end are padding."""
+    tokens * topk + n_experts * alignment); rows past the real end are padding.  An index that no expert has (negative,
+    ``n_experts`` and beyond) goes to no expert, like those of a masked token: nothing reads it back to refuse it."""
     if indices.dim() != 2 or not indices.is_cuda:
         raise ValueError("indices must be a [tokens, topk] GPU tensor")
     T, K = indices.shape

@@ -71,7 +71,9 @@ def test_route_tokens_more_experts_than_the_tables_hold(dev):
     """The fallback gives what the kernel gives: 1024 experts by both, the fallback asked for by name."""
     from cosmos_rl_amd.policy.kernel.moe import moe
     g = torch.Generator().manual_seed(3)
-    indices = torch.randint(0, 1024, (300, 4), generator=g).to(dev)
+    indices = torch.randint(0, 1024, (300, 4), generator=g)
+    indices[7, 1], indices[8, 3], indices[299, 0] = -3, 1024, 5000        # indices no expert has
+    indices = indices.to(dev)
     mask = (torch.rand(300, generator=g) < 0.8).to(dev)
     a = moe.route_tokens(indices, mask, 1024, 8)
     b = moe._route_tokens_by_sorting(indices, mask, 1024, 8, a.row_tokens.numel())
