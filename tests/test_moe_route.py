@@ -30,9 +30,9 @@ def _by_loops(indices, mask, E, alignment, capacity, keep_empty):
     return row_tokens, row_experts, row_map, order, sizes
 
 
-# one launch (up to 4096 pairs) and two, partial last workgroups, one expert, experts at and around powers of two and at
-# the limit of the tables, repeated experts in a token, a capacity that cuts rows off
-@pytest.mark.parametrize("T,K,E,alignment,distinct,short", [(1, 1, 1, 16, True, False), (3, 8, 128, 128, True, False), (512, 8, 128, 1, True, False),
+# one launch (up to 1024 pairs) and two on either side of the line, partial last workgroups, one expert, experts at and around
+# powers of two and at the limit of the tables, repeated experts in a token, a capacity that cuts rows off
+@pytest.mark.parametrize("T,K,E,alignment,distinct,short", [(1, 1, 1, 16, True, False), (3, 8, 128, 128, True, False), (128, 8, 64, 128, True, False), (205, 5, 64, 8, True, False), (90, 7, 40, 16, False, False), (512, 8, 128, 1, True, False),
                                                             (513, 8, 127, 128, True, False), (700, 6, 129, 16, False, False),
                                                             (2049, 3, 1024, 8, False, False), (1024, 4, 2, 64, False, True), (5000, 2, 33, 128, True, False)])
 @pytest.mark.parametrize("keep_empty", [True, False])
@@ -65,6 +65,30 @@ def test_route_tokens(dev, T, K, E, alignment, distinct, short, keep_empty):
             assert got.cpu().tolist() == ref
         assert torch.equal(mo.cpu().long(), torch.tensor(want[4]).cumsum(0))
         assert torch.equal(sw.cpu(), torch.gather(w, 1, so.cpu()).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("T,K,E,alignment,shift", [(16500, 8, 128, 128, 0.0), (33000, 8, 65, 16, 0.3), (131073, 1, 1000, 8, 0.0), (128, 8, 64, 16, 0.0)])
+def test_route_tokens_many_pairs(dev, T, K, E, alignment, shift):
+    """More pairs than 128 workgroups place in one round (131072), with partial last rounds: against a stable sort."""
+    from cosmos_rl_amd.policy.kernel.moe.moe import route_tokens
+    g = torch.Generator().manual_seed(T + E)
+    indices = (torch.rand(T, E, generator=g) + shift * torch.rand(E, generator=g)).topk(K, dim=1).indices if E * T < 20e6 else torch.randint(0, E, (T, K), generator=g)
+    mask = torch.rand(T, generator=g) < 0.9
+    r = route_tokens(indices.to(dev), mask.to(dev), E, alignment)
+    key = torch.where(mask[:, None], indices, E)
+    order = torch.sort(key.reshape(-1), stable=True).indices
+    counts = torch.bincount(key.reshape(-1), minlength=E + 1)[:E]
+    sizes = ((counts.clamp_min(alignment) + alignment - 1) // alignment * alignment)
+    ends, first = sizes.cumsum(0), counts.cumsum(0) - counts
+    row_tokens, row_of = torch.full((r.row_tokens.numel(),), -1), torch.full((T * K,), -1)
+    kept = order[:int(counts.sum())]
+    e = key.reshape(-1)[kept]
+    rows = (ends - sizes)[e] + torch.arange(kept.numel()) - first[e]
+    row_tokens[rows], row_of[kept] = kept // K, rows
+    slots = torch.sort(key, dim=1, stable=True).indices
+    assert torch.equal(r.m_sizes.cpu().long(), sizes) and torch.equal(r.m_offsets.cpu().long(), ends)
+    assert torch.equal(r.row_tokens.cpu().long(), row_tokens) and torch.equal(r.slot_order.cpu(), slots)
+    assert torch.equal(r.row_map.cpu().long(), torch.gather(row_of.view(T, K), 1, slots))
 
 
 def test_route_tokens_more_experts_than_the_tables_hold(dev):
