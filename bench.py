@@ -494,10 +494,17 @@ def run_extra(torch, lib, _lib, ops, dev, stream, gen, tensors, only=""):
         lambda: check(lib.cfp8_quant_group128(x4.data_ptr(), M4, K4, K4, qx4.data_ptr(), K4, sx4.data_ptr(), 0, stream)), copy_ceiling=True)
     o4 = torch.empty(M4, N4, dtype=torch.bfloat16, device=dev)
 
+    # (the products below go through the entry points that the operators in ops.py call, with memory for partial sums)
+    def partial(kind, m, n, k):
+        need = lib.cfp8_gemm_partial_bytes(kind, m, n, k)
+        return torch.empty(max(need, 1), dtype=torch.uint8, device=dev), need
+
+    p4, p4b = partial(_lib.DISPATCH_BLOCK, M4, N4, K4)
+
     def gemm4():
         check(lib.cfp8_quant_group128(x4.data_ptr(), M4, K4, K4, qx4.data_ptr(), K4, sx4.data_ptr(), 0, stream))
-        check(lib.cfp8_gemm_block128(qx4.data_ptr(), K4, sx4.data_ptr(), q4.data_ptr(), K4, s4.data_ptr(), 1, N4 // 128,
-                                     o4.data_ptr(), N4, 0, M4, N4, K4, stream))
+        check(lib.cfp8_gemm_block128_split(qx4.data_ptr(), K4, sx4.data_ptr(), q4.data_ptr(), K4, s4.data_ptr(), 1, N4 // 128,
+                                           o4.data_ptr(), N4, 0, M4, N4, K4, p4.data_ptr(), p4b, stream))
     mfma("gemm_block128_cfg4_4096x18432x7168_incl_act_quant", 2.0 * M4 * N4 * K4, N4 * K4 + M4 * K4 * 2 + M4 * N4 * 2, gemm4, iters=50)
     if "gemm_block128_cfg4_4096x18432x7168_incl_act_quant" in out:
         rows = torch.arange(0, M4, M4 // 16, device=dev) + 7
@@ -508,7 +515,7 @@ def run_extra(torch, lib, _lib, ops, dev, stream, gen, tensors, only=""):
             ref[:, nb:nb + 2048] = a @ wb.t()
         verify("gemm_block128_cfg4_4096x18432x7168_incl_act_quant", rel_err(o4[rows].float(), ref.to(torch.bfloat16).float()))
         del a, ref, wb
-    del x4, qx4, sx4, o4, q4, s4
+    del x4, qx4, sx4, o4, q4, s4, p4
     # a short-K block-scaled GEMM (the shape of DeepSeek-V3's q_b projection at 4096 tokens): many tiles of few K steps each
     Mq, Nq, Kq = 4096, 24576, 1536
     qxq = torch.randint(0, 120, (Mq, Kq), generator=gen, device=dev, dtype=torch.uint8)
@@ -516,10 +523,11 @@ def run_extra(torch, lib, _lib, ops, dev, stream, gen, tensors, only=""):
     sxq = torch.rand(Mq, Kq // 128, generator=gen, device=dev) + 0.5
     swq = torch.rand(Nq // 128, Kq // 128, generator=gen, device=dev) + 0.5
     oq = torch.empty(Mq, Nq, dtype=torch.bfloat16, device=dev)
+    pq, pqb = partial(_lib.DISPATCH_BLOCK, Mq, Nq, Kq)
     mfma("gemm_block128_short_k_4096x24576x1536_gemm_only", 2.0 * Mq * Nq * Kq, Nq * Kq + Mq * Kq + Mq * Nq * 2,
-         lambda: check(lib.cfp8_gemm_block128(qxq.data_ptr(), Kq, sxq.data_ptr(), qwq.data_ptr(), Kq, swq.data_ptr(), Kq // 128, 1,
-                                              oq.data_ptr(), Nq, 0, Mq, Nq, Kq, stream)), iters=50)
-    del qxq, qwq, sxq, swq, oq
+         lambda: check(lib.cfp8_gemm_block128_split(qxq.data_ptr(), Kq, sxq.data_ptr(), qwq.data_ptr(), Kq, swq.data_ptr(), Kq // 128, 1,
+                                                    oq.data_ptr(), Nq, 0, Mq, Nq, Kq, pq.data_ptr(), pqb, stream)), iters=50)
+    del qxq, qwq, sxq, swq, oq, pq
 
     # config 3: FP8 linear [M, 3584] x [18944, 3584]^T, per-token activation quant inside the call
     N3, K3 = 18944, 3584
@@ -537,11 +545,11 @@ def run_extra(torch, lib, _lib, ops, dev, stream, gen, tensors, only=""):
         chan = torch.rand(K3, generator=gen, device=dev) < 0.005
         x = torch.where(chan[None, :], x * 30, x).to(torch.bfloat16)
         o = torch.empty(M, N3, dtype=torch.bfloat16, device=dev)
-        wsb = lib.cfp8_linear_workspace_bytes(M, K3)
+        wsb = lib.cfp8_linear_workspace_bytes(M, K3) + lib.cfp8_gemm_partial_bytes(_lib.DISPATCH_ROWWISE, M, N3, K3)
         ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
         mfma(f"linear_rowwise_cfg3_M{M}", 2.0 * M * N3 * K3, N3 * K3 + 4 * N3 + M * K3 * 2 + M * N3 * 2,
-             lambda: check(lib.cfp8_linear_rowwise(x.data_ptr(), K3, qw3.data_ptr(), K3, sw3.data_ptr(), o.data_ptr(), N3, 0,
-                                                   M, N3, K3, ws.data_ptr(), wsb, stream)), iters=50)
+             lambda: check(lib.cfp8_linear_rowwise_split(x.data_ptr(), K3, qw3.data_ptr(), K3, sw3.data_ptr(), None, o.data_ptr(), N3, 0,
+                                                         M, N3, K3, ws.data_ptr(), wsb, stream)), iters=50)
         if f"linear_rowwise_cfg3_M{M}" in out:
             # (the per-token quantisation of the call is that of the rowwise quantiser, bit for bit)
             rows = torch.unique(torch.linspace(0, M - 1, 16, device=dev).long())
@@ -554,15 +562,16 @@ def run_extra(torch, lib, _lib, ops, dev, stream, gen, tensors, only=""):
             # (torch._scaled_mm) on the same bytes beside it - a comparison figure, nothing here calls it otherwise
             qx, sx = ops.quant_rowwise(x)
             fl, by = 2.0 * M * N3 * K3, N3 * K3 + 4 * N3 + M * K3 + M * N3 * 2
+            pt, ptb = partial(_lib.DISPATCH_ROWWISE, M, N3, K3)
             mfma(f"scaled_mm_rowwise_cfg3_M{M}_gemm_only", fl, by,
-                 lambda: check(lib.cfp8_scaled_mm_rowwise(qx.data_ptr(), K3, sx.data_ptr(), qw3.data_ptr(), K3, sw3.data_ptr(),
-                                                          o.data_ptr(), N3, 0, M, N3, K3, stream)), iters=50)
+                 lambda: check(lib.cfp8_scaled_mm_rowwise_split(qx.data_ptr(), K3, sx.data_ptr(), qw3.data_ptr(), K3, sw3.data_ptr(), None,
+                                                                o.data_ptr(), N3, 0, M, N3, K3, pt.data_ptr(), ptb, stream)), iters=50)
             if M == 8192:
                 # the same call back to back, without the flush: operands come from the memory-side cache, as they do
                 # for a layer's activations (not for its weights) in a running model; reported beside the cold figure
                 mfma(f"scaled_mm_rowwise_cfg3_M{M}_gemm_only_no_flush", fl, by,
-                     lambda: check(lib.cfp8_scaled_mm_rowwise(qx.data_ptr(), K3, sx.data_ptr(), qw3.data_ptr(), K3, sw3.data_ptr(),
-                                                              o.data_ptr(), N3, 0, M, N3, K3, stream)), iters=50, cold=False)
+                     lambda: check(lib.cfp8_scaled_mm_rowwise_split(qx.data_ptr(), K3, sx.data_ptr(), qw3.data_ptr(), K3, sw3.data_ptr(), None,
+                                                                    o.data_ptr(), N3, 0, M, N3, K3, pt.data_ptr(), ptb, stream)), iters=50, cold=False)
             try:
                 sb = sw3.reshape(1, N3)
                 torch._scaled_mm(qx, qw3.t(), scale_a=sx, scale_b=sb, out_dtype=torch.bfloat16)
@@ -573,7 +582,7 @@ def run_extra(torch, lib, _lib, ops, dev, stream, gen, tensors, only=""):
                          lambda: torch._scaled_mm(qx, qw3.t(), scale_a=sx, scale_b=sb, out_dtype=torch.bfloat16), iters=50, cold=False)
             except Exception as e:  # the comparison is optional: a torch build without this path must not fail the bench
                 out[f"vendor_torch_scaled_mm_rowwise_cfg3_M{M}"] = {"error": f"{type(e).__name__}: {str(e)[:120]}"}
-            del qx, sx
+            del qx, sx, pt
         del x, o, ws
     del qw3, sw3
 
@@ -590,11 +599,11 @@ def run_extra(torch, lib, _lib, ops, dev, stream, gen, tensors, only=""):
         del w
         x = torch.randn(ML, k, generator=gen, device=dev).to(torch.bfloat16)
         o = torch.empty(ML, n, dtype=torch.bfloat16, device=dev)
-        wsb = lib.cfp8_linear_workspace_bytes_split(ML, n, k)
+        wsb = lib.cfp8_linear_workspace_bytes(ML, k) + lib.cfp8_gemm_partial_bytes(_lib.DISPATCH_ROWWISE, ML, n, k)
         ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
         mfma(name, 2.0 * ML * n * k, n * k + 4 * n + ML * k * 2 + ML * n * 2,
-             lambda: check(lib.cfp8_linear_rowwise(x.data_ptr(), k, qw.data_ptr(), k, sw.data_ptr(), o.data_ptr(), n, 0,
-                                                   ML, n, k, ws.data_ptr(), wsb, stream)), iters=50)
+             lambda: check(lib.cfp8_linear_rowwise_split(x.data_ptr(), k, qw.data_ptr(), k, sw.data_ptr(), None, o.data_ptr(), n, 0,
+                                                         ML, n, k, ws.data_ptr(), wsb, stream)), iters=50)
         rows = torch.arange(0, ML, ML // 16, device=dev) + 3
         qx_v, sx_v = ops.quant_rowwise(x[rows])
         ref = (deq_e4m3(qx_v) @ deq_e4m3(qw).t()) * sx_v.double().reshape(-1, 1) * sw.double().reshape(1, -1)
@@ -623,9 +632,10 @@ def run_extra(torch, lib, _lib, ops, dev, stream, gen, tensors, only=""):
         xq = torch.randn(M, K, generator=gen, device=dev).mul_(60).to(torch.float8_e4m3fn)
         sxq = torch.rand(M, generator=gen, device=dev) + 0.5
         o = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+        pt, ptb = partial(_lib.DISPATCH_MXFP4, M, N, K)
         mfma(name, 2.0 * M * N * K, N * K // 2 + N * K // 32 + M * K + 4 * M + M * N * 2,
-             lambda: check(lib.cfp8_gemm_mxfp4(xq.data_ptr(), K, sxq.data_ptr(), w4.data_ptr(), K // 2, s4.data_ptr(), K // 32,
-                                               None, 0, o.data_ptr(), N, 0, M, N, K, stream)), iters=50)
+             lambda: check(lib.cfp8_gemm_mxfp4_split(xq.data_ptr(), K, sxq.data_ptr(), w4.data_ptr(), K // 2, s4.data_ptr(), K // 32,
+                                                     o.data_ptr(), N, 0, M, N, K, pt.data_ptr(), ptb, stream)), iters=50)
         if M == 1:
             # the same layer from bf16 activations: quantisation inside the weight-streaming kernel, one launch
             # (beside roofline_decode's M1_ms, the FP8 form of the same layer)
@@ -634,7 +644,7 @@ def run_extra(torch, lib, _lib, ops, dev, stream, gen, tensors, only=""):
                  lambda: check(lib.cfp8_linear_mxfp4(xb.data_ptr(), K, w4.data_ptr(), K // 2, s4.data_ptr(), K // 32, o.data_ptr(), N, 0,
                                                      M, N, K, None, 0, stream)), iters=50)
             del xb
-        del w4, s4, xq, sxq, o
+        del w4, s4, xq, sxq, o, pt
 
     # the grouped form on the expert shapes of GPT-OSS-20B: 32 experts, 8192 tokens routed top-4, gate_up [5760, 2880]
     # (K = 2880 is not a multiple of 128, N = 5760 not one of 512: the last K step and the last tile-column are ragged)

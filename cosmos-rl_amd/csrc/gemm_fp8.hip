@@ -23,6 +23,7 @@
 //   block:    every K step is one 128-block; its MFMA result is folded into the
 //             running sum as acc += part * (sa[m, kb] * sb[n / 128, kb]).
 #include <atomic>
+#include <math.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <type_traits>
@@ -1868,9 +1869,12 @@ static int launch_rowwise_256p(GemmArgs& p, int out_dtype, hipStream_t st) {
 }
 
 // The edge form's division of a problem: a remainder of rows (and of columns) is either a last row of whole tiles or quarter
-// tiles.  The estimated times, in microseconds a K step: a whole tile on every CU 1.35, a quarter tile 0.5, or 1.0 for
+// tiles.  Between divisions the choice weighs, in microseconds a K step, a whole tile on every CU 1.35, a quarter tile 0.5, or 1.0 for
 // quarters of a row remainder, which read all of the weight again (8192 x 18944 x 3584, nine rounds and one of quarters, 405
-// us; 1111 x 37888 x 3584 180 us with 87 rows as quarters, 2.3 rounds of tiles and 2.4 of quarters).
+// us; 1111 x 37888 x 3584 180 us with 87 rows as quarters, 2.3 rounds of tiles and 2.4 of quarters).  `cost` is the time
+// of the division taken, fitted to 198 shapes behind small and behind large writes, 2 % off on average: a last round of whole tiles
+// costs 0.6 of a full one and more the fuller it is.
+static double beside(double us, double in) { return sqrt(sqrt(us * us * us * us + in * in * in * in)); }  // neither hides the other where they meet
 struct EdgePlan {
     int tiles_m, tiles_n, tail, edge_rows, edge_cols;
     double cost;
@@ -1893,6 +1897,13 @@ static EdgePlan edge_plan(int64_t M, int64_t N, int64_t K, int cus) {
             const double cost = 4.0 + (double)((tiles - tail + cus - 1) / cus) * whole + (double)((units + cus - 1) / cus) * quarter;
             if (cost < best.cost) best = EdgePlan{(int)tm, (int)tn, (int)tail, (int)rows, (int)cols, cost};
         }
+    }
+    if (best.cost < 1e30) {
+        const int64_t tiles = (int64_t)best.tiles_m * best.tiles_n - best.tail, units = 4 * (int64_t)best.tail + best.edge_rows + best.edge_cols;
+        const double kt = (double)(K / 128), part = (double)(tiles % cus) / cus;
+        const double us = (double)(tiles / cus) * (kt * 1.39 + 4.8) + (part > 0 ? kt * 1.39 * (0.6 + 0.4 * part) + 4.8 : 0.0) +
+                          (double)((units + cus - 1) / cus) * (kt * (best.edge_rows ? 1.0 : 0.72) + 6.0);
+        best.cost = 4.3 + beside(us, ((double)N * (double)K + (double)M * (double)K) / 2.4e6);
     }
     return best;
 }
@@ -3357,17 +3368,53 @@ __global__ __launch_bounds__(256) void bias_rows_kernel(void* out, int64_t ld_ou
     }
 }
 
+// The times of launch_gemm's rowwise kernels in microseconds, for the choice below; fitted to the same shapes behind small and behind
+// large writes as the ring's, to the mean of the two, 2 to 5 % off on average.
+// Up to 128 tokens, the weight streamers: up to 16 the weights' way in (token rows come from L2 beside them) joined with the
+// chunks of K one after the other, beyond that rounds of strips times K steps.
+static double rowwise_streams_cost(int64_t M, int64_t N, int64_t K, int cus) {
+    const double kt = (double)(K / 128), bytes = (double)N * (double)K;
+    if (M <= 16) {
+        const int64_t steps = (K / 128 + 3) / 4, chunks = (steps + 7) / 8;  // as launch_rowwise_gemv has them
+        const double latency = (double)chunks * (1.25 + 0.137 * (double)((steps + chunks - 1) / chunks) * (1 + 0.045 * (double)M));
+        const double in = bytes * (1 + 0.03 * (double)M) / 5.35e6 + 0.097 * (double)chunks * (double)N / 4096;
+        return 1.9 + sqrt(latency * latency + in * in);
+    }
+    const bool narrow = (N + 79) / 80 < 128;  // as launch_rowwise_strip has it
+    const int64_t strips = (N + (narrow ? 31 : 79)) / (narrow ? 32 : 80);
+    return 1.5 + (double)((strips + cus - 1) / cus) * (1.5 + kt * (M <= 64 ? (narrow ? 0.215 : 0.451) : (narrow ? 0.32 : 0.626))) + bytes / 30e6;
+}
+// Beyond that: rounds of tiles, a last one cheaper the emptier it is, beside the operands' way in; a remainder of rows is a
+// problem of its own.
+static double rowwise_tiles_cost(int64_t M, int64_t N, int64_t K, int cus) {
+    if (M <= 128) return rowwise_streams_cost(M, N, K, cus);
+    const double kt = (double)(K / 128), in = (double)N * (double)K + (double)M * (double)K;
+    auto time = [&](int64_t tiles, double step, double load, double ends) {
+        const int64_t full = tiles / cus, rem = tiles % cus;
+        const double part = (double)rem / cus;
+        return (double)full * (kt * step * (1 + load) + ends) + (rem ? kt * step * (1 + load * (full ? part : part * part)) + ends : 0.0);
+    };
+    if (M % 256 == 0 && N % 128 == 0) {
+        const int64_t t256 = M / 256 * ((N + 255) / 256), rem = t256 % cus;
+        if (N % 256 || t256 <= 128) return 4.6 + beside(time(M / 256 * (N / 128), 0.813, 0.207, 0.0), in / 2.65e6);
+        double us = time(t256, 1.159, 0.19, 3.7);
+        if (t256 > cus && rem && rem * 2 <= cus) us = time(t256 - rem, 1.159, 0.19, 3.7) + (double)((4 * rem + cus - 1) / cus) * (kt * 0.731 + 4.7);
+        return 7.1 + beside(us, in / 2.44e6);
+    }
+    if (M <= 256) return 3.1 + time((N + 127) / 128, 0.846, 0.664, 2.1);
+    if (M > 512 && N % 256 == 0 && M % 256) return rowwise_tiles_cost(M / 256 * 256, N, K, cus) + rowwise_tiles_cost(M % 256, N, K, cus);
+    return 3.6 + beside(time((M + 255) / 256 * ((N + 255) / 256), 1.472, 0.238, 3.8), in / 2.85e6);
+}
+
 // Rowwise product with a bias and memory for partial sums: the form with the least estimated time among the ring kernel
-// (gemm_ring.hip), the walking 256 x 256 tiles with edges, and, up to 128 tokens, the weight streamers of launch_gemm.
-// The streamers' estimates, in microseconds: up to 16 tokens the weights' way in (token rows come from L2 beside
-// them) joined with the chunks of K one after the other, beyond that rounds of strips times K steps; fitted to 468 shapes of 5 to
-// 128 tokens, timed behind small writes and behind one that left L2 full, to the mean of the two, 5 and 4 % off on average.
-// Within 8 % of each other the streamers are taken, which lose less behind large writes (33 x 18944 x 3584 with the token quantiser
-// 19.9 / 23.7 us, ring 21.1 / 25.6), and within 25 % beyond 96 tokens, where the ring kernel's second row of tiles of 64 fills up
-// (121 x 3328 x 3328 15.7 / 18.5, ring 16.1 / 21.4).
-// Timed with weights that no cache holds, ring / launch_gemm: 739 x 1024 x 1024 5.8 / 21.7 us, 152 x 1792 x 12672 17 / 88, 1061
-// x 2560 x 7936 40 / 75, 637 x 18944 x 3584 63 / 64, 21 x 896 x 17152 11 / 33, 33 x 25344 x 2560 15.0 / 23.6; 33 x 18944 x 3584, one
-// round of strips, 17.3 / 16.4, 64 x 2048 x 1536 7.0 / 6.2, 16 x 1792 x 1792 6.8 / 4.3.
+// (gemm_ring.hip), the walking 256 x 256 tiles with edges, and launch_gemm.
+// Up to 128 tokens launch_gemm's streamers are taken within 8 %, which lose less behind large writes (33 x 18944 x 3584 with the
+// token quantiser 19.9 / 23.7 us behind small and large ones, ring 21.1 / 25.6), and within 25 % beyond 96 tokens, where the ring
+// kernel's second row of tiles of 64 fills up (121 x 3328 x 3328 15.7 / 18.5, ring 16.1 / 21.4).
+// Timed with weights that no cache holds, ring / launch_gemm: 21 x 896 x 17152 11 / 33, 33 x 25344 x 2560 15.0 / 23.6; 33 x 18944 x
+// 3584, one round of strips, 17.3 / 16.4, 64 x 2048 x 1536 7.0 / 6.2, 16 x 1792 x 1792 6.8 / 4.3; 739 x 1024 x 1024 5.8 / 21.7, 152 x 1792
+// x 12672 17 / 88, 1061 x 2560 x 7936 40 / 75, 1024 x 3584 x 3584 with the quantiser 24 / 31; but 2048 x 3584 x 3584, 224 of its tiles of
+// 256 x 128, 42.5 / 34.7, 4096 x 3584 x 18944 412 / 231, 1024 x 9984 x 3584 65 / 48.
 static int launch_rowwise_best(GemmArgs& p, int out_dtype, hipStream_t st) {
     const int cus = cu_count();
     RingArgs r{};
@@ -3380,26 +3427,17 @@ static int launch_rowwise_best(GemmArgs& p, int out_dtype, hipStream_t st) {
     EdgePlan edge{};
     edge.cost = 1e30;
     if (p.M > 128 && edge_takes(p, out_dtype)) edge = edge_plan(p.M, p.N, p.K, cus);
-    double stream = 1e30;
-    if (p.M <= 128 && p.K % 128 == 0) {
-        const double kt = p.K / 128, bytes = (double)p.N * p.K;
-        if (p.M <= 16) {
-            const int steps = ((p.K >> 7) + 3) / 4, chunks = (steps + 7) / 8;  // as launch_rowwise_gemv has them
-            const double latency = chunks * (1.25 + 0.137 * ((steps + chunks - 1) / chunks) * (1 + 0.045 * p.M));
-            const double in = bytes * (1 + 0.03 * p.M) / 5.35e6 + 0.097 * chunks * p.N / 4096;
-            stream = 1.9 + sqrt(latency * latency + in * in);
-        } else {
-            const bool narrow = (p.N + 79) / 80 < 128;  // as launch_rowwise_strip has it
-            const int strips = (p.N + (narrow ? 31 : 79)) / (narrow ? 32 : 80);
-            stream = 1.5 + ((strips + cus - 1) / cus) * (1.5 + kt * (p.M <= 64 ? (narrow ? 0.215 : 0.451) : (narrow ? 0.32 : 0.626))) + bytes / 30e6;
-            if (p.bias) stream += 4.0;  // (bias_rows_kernel)
-        }
-        stream /= p.M <= 96 ? 1.08 : 1.25;
+    double other = 1e30;
+    if (p.K % 128 == 0) {
+        other = rowwise_tiles_cost(p.M, p.N, p.K, cus);
+        // (bias_rows_kernel behind those that take no bias)
+        if (p.bias && p.M > 16) other += 4.0 + (p.M > 128 ? 4.0 * p.M * (double)p.N / 4e6 : 0.0);
+        if (p.M <= 128) other /= p.M <= 96 ? 1.08 : 1.25;
     }
-    if (ring.cost < 1e30 && ring.cost <= edge.cost && ring.cost <= stream) return launch_ring(kRingRow, r, ring, out_dtype, st);
+    if (ring.cost < 1e30 && ring.cost <= edge.cost && ring.cost <= other) return launch_ring(kRingRow, r, ring, out_dtype, st);
     // (without a bias and without remainders launch_gemm's form of the same tiles is 2 % faster)
     const bool even = p.M % 256 == 0 && p.N % 256 == 0 && !p.bias;
-    if (edge.cost < 1e30 && edge.cost <= stream && !even) return launch_rowwise_edge(p, edge, out_dtype, st);
+    if (edge.cost < 1e30 && edge.cost <= other && !even) return launch_rowwise_edge(p, edge, out_dtype, st);
     float* const partial = p.partial;
     p.partial = nullptr;  // (launch_gemm's own slices are those of cfp8_linear_rowwise)
     if (int rc = launch_gemm<kRowwise>(p, out_dtype, st)) return rc;

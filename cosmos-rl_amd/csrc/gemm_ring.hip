@@ -589,17 +589,15 @@ static int launch_ring_mode(RingArgs& p, const RingPlan& plan, int out_dtype, hi
 // K steps times the tile's step time (longer the more CUs load at once, and as long as for two everywhere as soon as one CU
 // holds two) plus the tile's ends; joins it with the operands' bytes at the rate they come in, (a^4 + b^4)^(1/4), since neither
 // hides the other near where they meet; and adds a fixed time per launch and, for slices, the reduction's launch and their
-// partial sums' way out and back.  The constants are fitted to all combinations of 112 to 144 shapes each (3 .. 3000 tokens,
-// weights of 896 .. 37888 rows, K 896 .. 18944), timed with weights that no cache holds: the choice is within 2 % of the best
-// combination on average, 20 % at worst.  Those for up to 128 rows, rowwise and MXFP4, are fitted to 468 shapes of 5 to
-// 128 rows, each timed behind small writes and behind one that left L2 full, to the mean of the two: 4 and 5 % off on
-// average, the choice within 1 % of the best combination, 15 % at worst.
+// partial sums' way out and back.  The constants are fitted to all combinations at some hundred shapes a mode (weights of 896 .. 37888
+// rows, K 896 .. 18944; kFewRates: 5 .. 128 rows, kRates: 129 .. 6144), each timed behind small writes and behind one that left L2
+// full, to the mean of the two: 4 to 6 % off on average, the choice within 1 % of the best combination, 15 to 20 % at worst.
 struct RingRates {
     double step[4], load[4], two[4];  // 128 x 128, 64 x 128, 128 x 64, 64 x 64: microseconds a step; what a full GPU adds; what two a CU add
     double launch, ends, partial, bytes, reduce;
 };
 static const RingRates kRates[3] = {
-    {{0.464, 0.312, 0.308, 0.169}, {0.249, 0.427, 0.168, 0.371}, {0.0, 0.637, 0.854, 1.062}, 2.4, 0.8, 4.8, 5.0, 2.5},
+    {{0.547, 0.353, 0.346, 0.228}, {0.164, 0.110, 0.131, 0.099}, {0.068, 0.771, 0.787, 0.624}, 3.66, 0.78, 5.33, 2.77, 1.86},
     {{0.658, 0.393, 0.0, 0.263}, {0.100, 0.335, 0.0, 0.283}, {0.0, 0.0, 0.0, 0.362}, 2.3, 1.2, 4.3, 4.9, 2.3},
     {{0.491, 0.343, 0.294, 0.210}, {0.097, 0.287, 0.213, 0.115}, {0.789, 0.793, 0.894, 1.104}, 3.1, 0.4, 4.7, 3.4, 2.7},
 };

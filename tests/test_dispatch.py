@@ -109,7 +109,12 @@ OPERATORS = [
     ("linear, one token: one launch", (LIN, 1, 3584, 3584), S, ["linear_gemv_fused"]),
     ("linear, 1111 tokens, gate_up: the edge form, the last rows as whole tiles", (LIN, 1111, 37888, 3584), S,
      ["quant_rowwise", "gemm_rowwise_edge tail=0 edges=0 grid=256"]),
-    ("1111 tokens, one round and 114 tiles: those as quarter tiles", (ROW, 1111, 18944, 3584), S, ["gemm_rowwise_edge tail=114 edges=0"]),
+    ("1111 tokens: four rows of tiles and strips for the rest", (ROW, 1111, 18944, 3584), S, ["gemm_rowwise_256p tail=40", "gemm_rowwise_strip<128,5>"]),
+    ("full tiles, fewer than CUs: 256 x 128", (ROW, 2048, 3584, 3584), S, ["gemm_rowwise_256x128 grid=224"]),
+    ("... a round of 256 x 256", (ROW, 4096, 3584, 18944), S, ["gemm_rowwise_256 grid=224"]),
+    ("... a short K", (ROW, 512, 9728, 896), S, ["gemm_rowwise_256x128 grid=152"]),
+    ("... too few of them: ring tiles", (ROW, 1024, 3584, 3584), S, ["gemm_ring<rowwise,128,128> slices=1 grid=224"]),
+    ("... with a bias, which they do not take", (ROW, 2048, 4608, 3584), S | BIAS, ["gemm_ring<rowwise,128,64> slices=1"]),
     ("1111 tokens, down: a round of ring tiles", (ROW, 1111, 3584, 18944), S, ["gemm_ring<rowwise,128,128> slices=1 grid=252"]),
     ("full tiles without a bias: the walking form", (ROW, 8192, 4608, 3584), S, ["gemm_rowwise_256p tail=64"]),
     ("full tiles with a bias: the edge form, which adds it", (ROW, 8192, 4608, 3584), S | BIAS, ["gemm_rowwise_edge tail=64 edges=0"]),
