@@ -3451,46 +3451,61 @@ static int launch_rowwise_best(GemmArgs& p, int out_dtype, hipStream_t st) {
     return check_launch("gemm");
 }
 
-// Block-scaled product with memory for partial sums, the least of three estimates (microseconds):
-//   ring    the ring kernel (gemm_ring.hip) on all rows
-//   middle  the register-staged 128 x 128 tiles of launch_gemm, two workgroups a CU: 1.55 a K step with two of them, 0.7 to 1.0
-//           with one
-//   full    launch_gemm's full tiles on the first M / 256 * 256 rows, 2.05 a K step for 256 x 256 and 1.16 for 256 x 128, and one
-//           of the others on the rows that are left
-// Few tokens and narrow weights go to the ring kernel, whose loads are many steps ahead and whose slices fill the GPU; in the
-// middle its four waves are behind the others' eight, which do the scaling of one half of the waves under the other's products.
-// Timed with weights that no cache holds, launch_gemm / ring: 24 x 18432 x 7168 61.9 / 58.6 us, 22 x 9600 x 4608 35 / 24, 8 x
-// 2176 x 4352 26.5 / 13.5, 123 x 1792 x 5120 43 / 16, 171 x 16000 x 2560 28.8 / 29.4, 600 x 9472 x 5248 67 / 78, 1000 x 9728 x
-// 5248 98 / 114; full tiles with a ring kernel behind them 3000 x 4480 x 3200 86 / 76.
+// The times of launch_gemm's block-scaled kernels for more than 64 rows in microseconds, kernel by kernel as it chooses them; fitted to
+// 905 shapes of 80 to 6144 rows (weights of 896 .. 37888 rows, K 896 .. 18944), each timed behind small writes and behind one
+// that left L2 full, to the mean of the two: 3 % off on average.
+static bool block_splits_rows(int64_t M, int64_t N, int64_t K) {  // into full tiles and the rest, as launch_gemm does
+    return M >= 768 && M % 256 != 0 && N % 128 == 0 && M / 256 * (N / 128) >= 384 && K / 128 <= kMaxTileWeightScales;
+}
+static double block_tiles_cost(int64_t M, int64_t N, int64_t K, int cus) {
+    const int64_t KT = K / 128;
+    const double kt = (double)KT, in = (double)N * (double)K + (double)M * (double)K;
+    auto time = [&](int64_t tiles, int per, double step, double load, double two, double ends) {
+        const int64_t full = tiles / (per * cus), rem = tiles % (per * cus);
+        const double part = (double)rem / cus;
+        double us = (double)full * (kt * step * (1 + load + two) + per * ends);
+        if (part > 1) us += kt * step * (1 + load + two) + 2 * ends;
+        else if (rem) us += kt * step * (1 + load * (full ? part : part * part)) + ends;
+        return us;
+    };
+    if (M <= 64) return 6.0 + kt * 0.3;
+    if (block_splits_rows(M, N, K)) return block_tiles_cost(M / 256 * 256, N, K, cus) + block_tiles_cost(M % 256, N, K, cus);
+    if (M % 256 == 0 && N % 256 == 0 && KT >= 16 && KT <= 1024) {
+        const int64_t tm = M / 256, tn = N / 256, tiles = tm * tn, rem = tiles % cus;
+        const int64_t cut = rem > 0 && rem * 2 <= cus ? (rem + tm - 1) / tm : 0;
+        const int64_t head = tm * (tn - cut), rounds = (head + cus - 1) / cus;
+        if (head >= cus && head * 5 >= rounds * cus * 4)
+            return 2.0 + beside(time(head, 1, 1.42, 0.196, 0.0, 7.8) + (cut ? kt * 0.755 + 8.2 : 0.0), in / 2.17e6);
+    }
+    if (M > 512 && M % 256 == 0 && N % 128 == 0 && M / 256 * (N / 128) >= 384 && KT <= kMaxTileWeightScales)
+        return 4.6 + beside(time(M / 256 * (N / 128), 1, 0.797, 0.371, 0.0, KT <= kPersistentBlockSteps ? 1.0 : 4.0), in / 1.77e6);
+    if (M > 512 && (M + 255) / 256 * ((N + 127) / 128) >= 384) return 5.0 + beside(time((M + 255) / 256 * ((N + 127) / 128), 1, 1.025, 0.098, 0.0, 2.0), in / 1.4e6);
+    return 1.9 + beside(time((M + 127) / 128 * ((N + 127) / 128), 2, 0.82, 0.088, 0.445, 1.8), in / 2.58e6);
+}
+
+// Block-scaled product with memory for partial sums, the form with the least estimated time: the ring kernel (gemm_ring.hip) on
+// all rows, launch_gemm on all of them, or launch_gemm's full tiles on the first M / 256 * 256 rows and the ring kernel on the
+// rest.  Up to 64 rows the ring kernel's loads, many steps ahead, and its slices win everywhere.  In the middle its four waves are
+// behind the others' eight, which do the scaling of one half of the waves under the other's products.
+// Timed with weights that no cache holds, launch_gemm / ring: 22 x 9600 x 4608 35 / 24 us, 8 x 2176 x 4352 26.5 / 13.5, 123 x 1792 x
+// 5120 43 / 16, 256 x 3584 x 18944 126 / 41, 171 x 16000 x 2560 28.8 / 29.4; but 256 x 23552 x 3200 41.6 / 47.1, 600 x 9472 x 5248 67 / 78, 1024 x 9728 x 896
+// 21.8 / 25.2, 2816 x 3328 x 1280 26.3 / 29.8; full tiles with a ring kernel behind them 3000 x 4480 x 3200 86 / 76.  The choice is within
+// 1 % of the best on average, 9 % at worst.
 struct BlockPlan {
     int64_t body;   // rows of the full tiles
     RingPlan ring;  // the others (bm == 0: launch_gemm)
 };
-static RingPlan block_rows_plan(int64_t M, int64_t N, int64_t K, size_t partial_bytes, int cus) {
-    RingPlan ring = ring_plan(kRingBlock, M, N, K, partial_bytes, cus);
-    if (M <= 64) return ring;
-    const int64_t KT = K / 128, tiles = ((M + 127) / 128) * ((N + 127) / 128), full = tiles / (2 * cus), rem = tiles % (2 * cus);
-    const double part = (double)rem / cus, step = part <= 1.0 ? 0.7 + 0.3 * part : 1.15 + 0.2 * part;
-    const double middle = 5.0 + (double)full * ((double)KT * 1.55 + 3.0) + (rem ? (double)KT * step : 0.0);
-    // (several rounds of 128 x 128 ring tiles take about 15 % longer than estimated)
-    if (middle < ring.cost * (M > 256 ? 1.15 : 1.0)) ring = {0, 0, 0, middle};
-    return ring;
-}
 static BlockPlan block_plan(int64_t M, int64_t N, int64_t K, size_t partial_bytes, int cus) {
-    BlockPlan best{0, block_rows_plan(M, N, K, partial_bytes, cus)};
-    const int64_t KT = K / 128, body = M / 256 * 256, tm = body / 256;
-    if (body <= 512 || N % 128 || tm * (N / 128) < 384 || KT > kMaxTileWeightScales) return best;
-    double full = 6.0 + (double)((tm * (N / 128) + cus - 1) / cus) * ((double)KT * 1.16 + (KT <= kPersistentBlockSteps ? 1.0 : 4.0));
-    if (N % 256 == 0 && KT >= 16 && KT <= 1024) {  // as launch_gemm has it
-        const int64_t tn = N / 256, tiles = tm * tn, rem = tiles % cus;
-        const int64_t cut = rem > 0 && rem * 2 <= cus ? (rem + tm - 1) / tm : 0;
-        const int64_t head = tm * (tn - cut), rounds = (head + cus - 1) / cus;
-        if (head >= cus && head * 5 >= rounds * cus * 4) full = 6.0 + (double)(rounds * KT) * 2.05 + (cut ? 6.0 + (double)KT * 1.16 : 0.0);
+    BlockPlan best{0, ring_plan(kRingBlock, M, N, K, partial_bytes, cus)};
+    if (M <= 64) return best;
+    const double tiles = block_tiles_cost(M, N, K, cus);
+    if (tiles < best.ring.cost) best = {0, {0, 0, 0, tiles}};
+    if (block_splits_rows(M, N, K)) {
+        const int64_t body = M / 256 * 256;
+        RingPlan rest = ring_plan(kRingBlock, M - body, N, K, partial_bytes, cus);
+        rest.cost += block_tiles_cost(body, N, K, cus);
+        if (rest.cost < best.ring.cost) best = {body, rest};
     }
-    if (full >= best.ring.cost) return best;
-    RingPlan rest{0, 0, 0, 0.0};
-    if (M > body) rest = block_rows_plan(M - body, N, K, partial_bytes, cus);
-    if (full + rest.cost < best.ring.cost) best = {body, rest};
     return best;
 }
 size_t block_partial_bytes(int64_t M, int64_t N, int64_t K) {
@@ -3507,8 +3522,7 @@ static int launch_block_best(GemmArgs& p, int out_dtype, hipStream_t st) {
     r.ld_a = p.ld_a; r.ld_w = p.ld_b; r.ld_out = p.ld_out;
     r.sb_stride_n = p.sb_stride_n; r.sb_stride_k = p.sb_stride_k;
     r.M = p.M - (int)plan.body; r.N = p.N; r.K = p.K;
-    // (rows of the rest that launch_gemm takes: it splits them off itself)
-    if (r.M == 0 || !plan.ring.bm || !ring_takes(kRingBlock, r, out_dtype)) return launch_gemm<kBlock>(p, out_dtype, st);
+    if (!plan.ring.bm || !ring_takes(kRingBlock, r, out_dtype)) return launch_gemm<kBlock>(p, out_dtype, st);
     if (plan.body) {
         GemmArgs body = p;
         body.M = (int)plan.body;

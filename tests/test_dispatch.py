@@ -135,6 +135,9 @@ OPERATORS = [
     ("block, a decode batch", (BLK, 24, 18432, 7168), S, ["gemm_ring<block,64,128> slices=1 grid=144"]),
     ("block, full tiles", (BLK, 4096, 18432, 7168), S, ["gemm_block_256 grid=1024", "gemm_block_w8<256,128,block>"]),
     ("block, full tiles and a ring kernel behind them", (BLK, 3000, 4480, 3200), S, ["gemm_block_w8p<256,128,block>", "gemm_ring<block,64,64>"]),
+    ("block, a round of staged tiles on a wide weight", (BLK, 256, 23552, 3200), S, ["gemm_kernel<128,128,2,2,block>"]),
+    ("block, a short K", (BLK, 1024, 9728, 896), S, ["gemm_kernel<128,128,2,2,block>"]),
+    ("block, fewer tiles than CUs and a long K: slices", (BLK, 256, 3584, 18944), S, ["gemm_ring<block,", "ring_reduce"]),
     ("block, some hundred rows on a wide weight: staged tiles", (BLK, 600, 9472, 5248), S, ["gemm_kernel<128,128,2,2,block>"]),
     ("mxfp4, up to four tokens of a short K: as the one-launch linear", (MX, 4, 896, 896), S, ["gemm_mxfp4_gemv_lds"]),
     ("mxfp4, 17 to 128 tokens, a round of strips", (MX, 64, 18944, 3584), S, ["gemm_mxfp4_strip<64> grid=237"]),
