@@ -25,6 +25,7 @@
 // K need not be a multiple of 128: the chunks of the last step that lie beyond K are loaded as zero with the
 // scale byte 127.
 #include <atomic>
+#include <math.h>
 
 #include "cfp8_common.h"
 #include "gemm_internal.h"
@@ -1771,20 +1772,29 @@ static int launch_mx4(Mx4Args p, int out_dtype, hipStream_t st) {
 }  // namespace cfp8
 
 namespace cfp8 {
-// What the tile kernels below the dispatch would take for M > 128 rows, in microseconds: rounds of tiles on the CUs (a
-// partial round costs nearly a whole one) times K steps, fitted to 35 timed shapes for the 256 x 256 tiles and to 39 for the
-// others (3 % off on average).  Infinite where only the register-staged tiles would be left, which the ring kernel beats
-// everywhere.
+// What the tile kernels below the dispatch would take for M > 128 rows, in microseconds: rounds of tiles on the CUs (a last one
+// cheaper the emptier it is) times K steps, beside the operands' way in; fitted to 603 shapes of 129 to 6144 rows (weights of
+// 896 .. 37888 rows, K 896 .. 18944), each timed behind small writes and behind one that left L2 full, to the mean of the two: 2 to
+// 4 % off on average.  Infinite where only the register-staged tiles would be left, which take twice the ring kernel's time and more.
+// (7 % more for the 128 x 512 tiles: of seven shapes of 2000 to 8000 rows where the estimates were level the ring kernel was ahead in all, 4352 x 4992 x
+// 3456 80.5 against 93.4 us, 2088 x 32768 x 2432 166 against 190.)
 static double mx4_tiles_cost(int64_t M, int64_t N, int64_t K, bool aligned256, int cus) {
-    const double kt = (double)((K + 127) / 128);
-    auto rounds = [&](int64_t tiles, double least) {
+    const double kt = (double)((K + 127) / 128), in = (double)N * (double)K * 0.53 + (double)M * (double)K;
+    auto time = [&](int64_t tiles, double step, double load, double ends) {
         const int64_t full = tiles / cus, rem = tiles % cus;
-        return full == 0 ? 1.0 : (double)full + (rem ? least + (1.0 - least) * (double)rem / cus : 0.0);
+        const double part = (double)rem / cus;
+        return (double)full * (kt * step * (1 + load) + ends) + (rem ? kt * step * (1 + load * (full ? part : part * part)) + ends : 0.0);
     };
+    auto beside = [](double us, double us_in) { return sqrt(sqrt(us * us * us * us + us_in * us_in * us_in * us_in)); };
+    if (aligned256 && (M / 256) * (N / 256) >= 128) {
+        const int64_t tm = M / 256, tn = N / 256, rem = (tm * tn) % cus, cut = (rem + tm - 1) / tm;  // as launch_mx4_best has it
+        const bool two = tm * tn > cus && rem > 0 && rem * 2 <= cus && cut < tn;
+        const double us = two ? time(tm * (tn - cut), 1.055, 0.275, 6.1) + time((M + 127) / 128 * cut, 0.588, 0.433, 7.1) : time(tm * tn, 1.055, 0.275, 6.1);
+        return 2.5 + beside(us, in / 1.71e6);
+    }
     const int64_t t256 = (M + 127) / 128 * ((N + 255) / 256), t512 = (M + 127) / 128 * ((N + 511) / 512);
-    if (aligned256 && (M / 256) * (N / 256) >= 128) return 4.0 + rounds((M / 256) * (N / 256), 0.5) * (kt * 1.3 + 3.0);
-    if (t512 >= 256 && (N + 511) / 512 * 512 - N <= N / 8) return 1.1 + rounds(t512, 0.87) * (kt * 1.63 + 6.0);
-    if (t256 >= 64) return 3.0 + rounds(t256, 0.9) * (kt * (0.62 + 0.2 * (t256 < cus ? (double)t256 / cus : 1.0)) + 2.8);
+    if (t512 >= 256 && (N + 511) / 512 * 512 - N <= N / 8) return 1.07 * beside(time(t512, 1.043, 0.433, 8.8), in / 0.65e6);
+    if (t256 >= 64) return 3.2 + beside(time(t256, 0.772, 0.209, 1.6), in / 2.0e6);
     return 1e30;
 }
 
@@ -1822,8 +1832,9 @@ static int gemm_mx4_dense(Mx4Args& p, float* partial, size_t partial_bytes, int 
         if (mx4_streams_cost(p.M, p.N, p.K, cu_count()) <= plan.cost * 1.05) return CFP8_OK;
     } else {
         const bool aligned256 = p.M % 256 == 0 && p.N % 256 == 0 && p.K % 128 == 0 && p.ld_ws % 4 == 0 && (reinterpret_cast<uintptr_t>(p.ws) & 3u) == 0;
-        // (many rounds of ring tiles take about 5 % longer than estimated)
-        if (mx4_tiles_cost(p.M, p.N, p.K, aligned256, cu_count()) <= plan.cost * (p.M > 1000 ? 1.05 : 1.0)) return CFP8_OK;
+        // (within 5 % the tiles: their time depends less on what L2 holds; 4096 x 9728 x 896 45.4 / 52.2 us behind small and large
+        // writes, ring 42.9 / 61.8.  512 x 9728 x 896 11.0 against 12.4 us, but 1629 x 2304 x 9984 58 against 44)
+        if (mx4_tiles_cost(p.M, p.N, p.K, aligned256, cu_count()) <= plan.cost * 1.05) return CFP8_OK;
     }
     taken = true;
     return launch_ring(kRingMx, r, plan, out_dtype, st);

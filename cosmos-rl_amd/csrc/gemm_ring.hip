@@ -595,16 +595,17 @@ static int launch_ring_mode(RingArgs& p, const RingPlan& plan, int out_dtype, hi
 struct RingRates {
     double step[4], load[4], two[4];  // 128 x 128, 64 x 128, 128 x 64, 64 x 64: microseconds a step; what a full GPU adds; what two a CU add
     double launch, ends, partial, bytes, reduce;
+    double fill;  // what rows that do not exist, and are not loaded, save of a tile
 };
 static const RingRates kRates[3] = {
-    {{0.547, 0.353, 0.346, 0.228}, {0.164, 0.110, 0.131, 0.099}, {0.068, 0.771, 0.787, 0.624}, 3.66, 0.78, 5.33, 2.77, 1.86},
-    {{0.782, 0.470, 0.0, 0.323}, {0.064, 0.086, 0.0, 0.122}, {0.0, 0.0, 0.0, 0.405}, 3.24, 0.91, 5.06, 2.66, 2.21},
-    {{0.491, 0.343, 0.294, 0.210}, {0.097, 0.287, 0.213, 0.115}, {0.789, 0.793, 0.894, 1.104}, 3.1, 0.4, 4.7, 3.4, 2.7},
+    {{0.547, 0.353, 0.346, 0.228}, {0.164, 0.110, 0.131, 0.099}, {0.068, 0.771, 0.787, 0.624}, 3.66, 0.78, 5.33, 2.77, 1.86, 0.0},
+    {{0.782, 0.470, 0.0, 0.323}, {0.064, 0.086, 0.0, 0.122}, {0.0, 0.0, 0.0, 0.405}, 3.24, 0.91, 5.06, 2.66, 2.21, 0.0},
+    {{0.541, 0.419, 0.376, 0.247}, {0.080, 0.068, 0.106, 0.081}, {0.637, 0.513, 0.528, 0.626}, 3.13, 0.55, 5.70, 1.77, 3.11, 0.14},
 };
 static const RingRates kFewRates[3] = {
-    {{0.587, 0.418, 0.387, 0.223}, {0.296, 0.465, 0.130, 0.331}, {0.0, 0.845, 0.886, 1.338}, 2.88, 0.34, 4.17, 7.97, 2.26},
-    {{0.658, 0.393, 0.0, 0.263}, {0.100, 0.335, 0.0, 0.283}, {0.0, 0.0, 0.0, 0.362}, 2.3, 1.2, 4.3, 4.9, 2.3},
-    {{0.630, 0.523, 0.447, 0.290}, {0.170, 0.317, 0.0, 0.121}, {0.942, 0.883, 0.965, 1.274}, 2.51, 0.0, 4.22, 5.52, 2.86},
+    {{0.587, 0.418, 0.387, 0.223}, {0.296, 0.465, 0.130, 0.331}, {0.0, 0.845, 0.886, 1.338}, 2.88, 0.34, 4.17, 7.97, 2.26, 0.2},
+    {{0.658, 0.393, 0.0, 0.263}, {0.100, 0.335, 0.0, 0.283}, {0.0, 0.0, 0.0, 0.362}, 2.3, 1.2, 4.3, 4.9, 2.3, 0.0},
+    {{0.630, 0.523, 0.447, 0.290}, {0.170, 0.317, 0.0, 0.121}, {0.942, 0.883, 0.965, 1.274}, 2.51, 0.0, 4.22, 5.52, 2.86, 0.2},
 };
 static const int kTiles[4][2] = {{128, 128}, {64, 128}, {128, 64}, {64, 64}};
 constexpr int kRingMaxSlices = 16;
@@ -636,7 +637,7 @@ RingPlan ring_plan(int mode, int64_t M, int64_t N, int64_t K, size_t partial_byt
             double us = (double)full * (step * (1 + r.load[c] + r.two[c]) + per * r.ends);
             if (part > 1) us += step * (1 + r.load[c] + r.two[c]) + 2 * r.ends;
             else if (rem) us += step * (1 + r.load[c] * (full ? part : part * part)) + r.ends;
-            if (few && mode != kRingBlock) us *= 0.9 + 0.2 * (double)M / (double)((M + bm - 1) / bm * bm);  // rows that do not exist are not loaded
+            us *= 1 + r.fill * ((double)M / (double)((M + bm - 1) / bm * bm) - 0.5);
             us = r.launch + sqrt(sqrt(us * us * us * us + in * in * in * in));
             if (s > 1) us += r.reduce + 8.0 * s * (double)M * (double)N / (r.partial * 1e6);
             if (us < best.cost) best = {bm, bn, (int)s, us};

@@ -148,6 +148,9 @@ OPERATORS = [
     ("mxfp4, a narrow weight and a long K: slices", (MX, 33, 896, 18944), S, ["gemm_ring<mxfp4,64,64>", "ring_reduce"]),
     ("... without memory", (MX, 33, 896, 18944), 0, ["gemm_ring<mxfp4,64,64> slices=1 grid=14"]),
     ("mxfp4, 200 tokens", (MX, 200, 37888, 3584), S, ["gemm_ring<mxfp4,128,128> slices=1 grid=592"]),
+    ("mxfp4, a short K: rounds of tiles", (MX, 512, 9728, 896), S, ["gemm_mxfp4_tile<128,256>"]),
+    ("mxfp4, a short K, more tiles", (MX, 4096, 9728, 896), S, ["gemm_mxfp4_tile<256,256>", "gemm_mxfp4_tile<128,256>"]),
+    ("mxfp4, a narrow weight and a long K", (MX, 1629, 2304, 9984), S, ["gemm_ring<mxfp4,128,128> slices=1"]),
     ("mxfp4, full tiles", (MX, 8192, 18944, 3584), S, ["gemm_mxfp4_tile<256,256>", "gemm_mxfp4_tile<128,256>"]),
     ("mxfp4, K below a step", (MX, 100, 96, 96), S, ["gemm_mxfp4_staged<128,128>"]),
 ]
