@@ -1857,7 +1857,8 @@ static int launch_mx4_best(Mx4Args& p, float* partial, size_t partial_bytes, int
     // 17..128 tokens on a wide weight: the strip kernel (a narrow weight leaves most CUs without a strip)
     if (M <= 128 && !m_indices && K >= 128 && (N + 79) / 80 >= 128) return M <= 64 ? launch_mx4_strip<64>(p, out_dtype, st) : launch_mx4_strip<128>(p, out_dtype, st);
     if (M <= 64 && !m_indices) {
-        // few weight rows: narrow workgroups, so that there are enough of them
+        // few weight rows: narrow workgroups, so that there are enough of them (what the ring kernel does not take: an output aligned
+        // to 8 bytes only, K < 128, pitches of 2 MiB and more)
         const bool narrow = (N + 15) / 16 <= 512;
         if (M <= 32) return narrow ? launch_mx4_skinny<2, 3>(p, out_dtype, st) : launch_mx4_skinny<2, 5>(p, out_dtype, st);
         return narrow ? launch_mx4_skinny<4, 3>(p, out_dtype, st) : launch_mx4_skinny<4, 5>(p, out_dtype, st);

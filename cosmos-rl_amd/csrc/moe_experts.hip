@@ -227,7 +227,8 @@ static void launch_few_down(int ni, dim3 grid, hipStream_t st, const FewArgs& p)
     }
 }
 
-// The few-rows form holds a strip's whole K in registers: up to 8 K steps a wave of four (gate_up), 12 a wave (down).
+// The few-rows form holds a strip's whole K in registers: up to 8 K steps a wave of four (gate_up, 128 registers of weights and 64 of
+// tokens), 12 a wave (down, 96 registers, and two tiles of 16 rows of 1536 bytes in LDS).
 constexpr int64_t kFewMaxHidden = 4096, kFewMaxInter = 1536;
 // Mean rows an expert up to which a form is taken.  The few-rows form reads an expert's rows once for every strip of 16
 // features, the middle one once for every 128 columns but holds 64 rows in a tile; from about two of those tiles on the grouped

@@ -173,7 +173,6 @@ def _rel(got, want):
                                    (2000, 2064, 2880), (1025, 4112, 160), (8192, 272, 128), (130, 16400, 416), (1024, 4096, 3552),
                                    (4000, 4112, 160), (8192, 2544, 416), (4100, 4096, 2880),
                                    (100, 10480, 2880), (128, 16400, 160), (17, 12272, 4256), (65, 10256, 128), (90, 18944, 3584), (40, 20016, 1184),
-                                   # 272 and 320 tiles of 256 x 256: one full round, the last tile-columns as a second launch
                                    (4096, 4352, 256), (2048, 10240, 384)])
 def test_gemm_mxfp4_against_oracle(dev, M, N, K):
     """fp32 output within 1e-4 (relative Frobenius; the fp32 accumulation of the matrix pipe) of the exact sum, bf16 output within 1e-3 of the bf16-rounded
@@ -188,6 +187,50 @@ def test_gemm_mxfp4_against_oracle(dev, M, N, K):
     got16 = ops.gemm_mxfp4((xq.to(dev), sx.to(dev)), (wq.to(dev), ws.to(dev)), torch.bfloat16)
     assert _rel(got16.cpu().float(), want.float().to(torch.bfloat16).double()) <= 1e-3
     assert torch.equal(got.to(torch.bfloat16), got16)          # the two epilogues round the same accumulators
+
+
+# what remains to the tile kernels beside the ring kernel: a ragged last K step, one round of 256 x 256 tiles, and the last tile-columns
+# of a partial round as a second launch
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,took", [(1000, 4112, 160, "gemm_mxfp4_tile<128,256>"), (1000, 4112, 256, "gemm_mxfp4_tile<128,256>"),
+                                        (2000, 8192, 1152, "gemm_mxfp4_tile<128,512>"),
+                                        (1536, 9728, 512, "gemm_mxfp4_tile<256,256>"), (2304, 9728, 1152, "gemm_mxfp4_tile<256,256> + gemm_mxfp4_tile<128,256>")])
+def test_gemm_mxfp4_tile_kernels(dev, M, N, K, took):
+    from cosmos_rl_amd import _lib, ops
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    info = _lib.gemm_dispatch_info(_lib.DISPATCH_MXFP4, M, N, K, cus=cus, flags=_lib.DISPATCH_SPLIT).split("; ")
+    assert " + ".join(i.split(" ")[0] for i in info) == took, info
+    g = torch.Generator().manual_seed(M + N + K)
+    wq, ws = _mx_weights(g, N, K)
+    xq, sx = _fp8_rows(g, M, K)
+    for dt, tol in ((torch.float32, 1e-4), (torch.bfloat16, 1e-3)):
+        got = ops.gemm_mxfp4((xq.to(dev), sx.to(dev)), (wq.to(dev), ws.to(dev)), dt).cpu()
+        rows = torch.unique(torch.cat([torch.arange(0, M, M // 24), torch.arange(M - 130, M)]))   # (all columns of some rows of every tile)
+        want = MX.gemm(xq[rows], sx[rows], wq, ws)
+        want = want if dt == torch.float32 else want.float().to(torch.bfloat16).double()
+        assert _rel(got[rows].float(), want) <= tol
+
+
+# An output that is aligned to 8 bytes and not to 16: the kernels that write four columns a lane - the streamer of 16 tokens, the strips of 64 and 128
+# tokens on wide weights, their narrow forms (two and four tiles of 16 tokens, 3 and 5 of 16 weight rows), the register-staged tiles
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(16, 80, 2880), (31, 176, 6304), (24, 8400, 2880), (64, 320, 4096), (50, 8272, 896), (40, 20016, 1184), (100, 10480, 2880),
+                                   (128, 16400, 160), (80, 272, 896), (300, 528, 416)])
+def test_gemm_mxfp4_output_aligned_to_eight_bytes(dev, M, N, K):
+    from cosmos_rl_amd import _lib, ops
+    g = torch.Generator().manual_seed(M * 13 + N + K)
+    wq, ws = _mx_weights(g, N, K)
+    xq, sx = _fp8_rows(g, M, K)
+    ld = N + 12
+    buf = torch.full((M * ld + 8,), 3.0, dtype=torch.bfloat16, device=dev)
+    out = buf[4:4 + M * ld].view(M, ld)
+    assert out.data_ptr() % 16 == 8
+    x, s, w, e = xq.to(dev), sx.to(dev), wq.to(dev), ws.to(dev)
+    _lib.check(_lib.load().cfp8_gemm_mxfp4(x.data_ptr(), K, s.data_ptr(), w.data_ptr(), K // 2, e.data_ptr(), K // 32, None, 0, out.data_ptr(), ld,
+                                           ops._out_code(torch.bfloat16), M, N, K, torch.cuda.current_stream().cuda_stream))
+    want = MX.gemm(xq, sx, wq, ws).float().to(torch.bfloat16).double()
+    assert _rel(out[:, :N].float().cpu(), want) <= 1e-3
+    assert bool((out[:, N:] == 3.0).all()) and bool((buf[:4] == 3.0).all()) and bool((buf[4 + M * ld:] == 3.0).all())
 
 
 @pytest.mark.gpu
