@@ -1901,9 +1901,9 @@ static EdgePlan edge_plan(int64_t M, int64_t N, int64_t K, int cus) {
     if (best.cost < 1e30) {
         const int64_t tiles = (int64_t)best.tiles_m * best.tiles_n - best.tail, units = 4 * (int64_t)best.tail + best.edge_rows + best.edge_cols;
         const double kt = (double)(K / 128), part = (double)(tiles % cus) / cus;
-        const double us = (double)(tiles / cus) * (kt * 1.39 + 4.8) + (part > 0 ? kt * 1.39 * (0.6 + 0.4 * part) + 4.8 : 0.0) +
-                          (double)((units + cus - 1) / cus) * (kt * (best.edge_rows ? 1.0 : 0.72) + 6.0);
-        best.cost = 4.3 + beside(us, ((double)N * (double)K + (double)M * (double)K) / 2.4e6);
+        const double us = (double)(tiles / cus) * (kt * 1.223 + 4.22) + (part > 0 ? kt * 1.223 * (0.6 + 0.4 * part) + 4.22 : 0.0) +
+                          (double)((units + cus - 1) / cus) * (kt * (best.edge_rows ? 0.88 : 0.634) + 5.28);
+        best.cost = 7.5 + beside(us, ((double)N * (double)K + (double)M * (double)K) / 2.73e6);
     }
     return best;
 }
@@ -2307,9 +2307,8 @@ __global__ __launch_bounds__(256) void linear_gemv_fused_kernel(const uint4* __r
 }
 
 // whether the one-launch kernel above takes the call
-static bool fused_gemv_applies(int64_t M, int64_t K, const void* x, int64_t ld_x) {
-    return M >= 1 && M <= 4 && K <= (M == 1 ? 8192 : 4096) && K % 128 == 0 && aligned16(x) && ld_x % 8 == 0;
-}
+static bool fused_gemv_size(int64_t M, int64_t K) { return M >= 1 && M <= 4 && K <= (M == 1 ? 8192 : 4096) && K % 128 == 0; }
+static bool fused_gemv_applies(int64_t M, int64_t K, const void* x, int64_t ld_x) { return fused_gemv_size(M, K) && aligned16(x) && ld_x % 8 == 0; }
 template <int MR, int NI>
 static void launch_fused_ni(int ni, dim3 grid, size_t lds, hipStream_t st, const void* x, int64_t ld_x, const GemmArgs& p, int out_dtype) {
     if constexpr (NI > 0) {
@@ -3368,21 +3367,23 @@ __global__ __launch_bounds__(256) void bias_rows_kernel(void* out, int64_t ld_ou
     }
 }
 
-// The times of launch_gemm's rowwise kernels in microseconds, for the choice below; fitted to the same shapes behind small and behind
-// large writes as the ring's, to the mean of the two, 2 to 5 % off on average.
+// The times of launch_gemm's rowwise kernels in microseconds, for the choice below; fitted to the same shapes and in the same way as
+// the ring's.
 // Up to 128 tokens, the weight streamers: up to 16 the weights' way in (token rows come from L2 beside them) joined with the
 // chunks of K one after the other, beyond that rounds of strips times K steps.
 static double rowwise_streams_cost(int64_t M, int64_t N, int64_t K, int cus) {
     const double kt = (double)(K / 128), bytes = (double)N * (double)K;
     if (M <= 16) {
         const int64_t steps = (K / 128 + 3) / 4, chunks = (steps + 7) / 8;  // as launch_rowwise_gemv has them
-        const double latency = (double)chunks * (1.25 + 0.137 * (double)((steps + chunks - 1) / chunks) * (1 + 0.045 * (double)M));
-        const double in = bytes * (1 + 0.03 * (double)M) / 5.35e6 + 0.097 * (double)chunks * (double)N / 4096;
-        return 1.9 + sqrt(latency * latency + in * in);
+        const double latency = (double)chunks * (1.23 + 0.135 * (double)((steps + chunks - 1) / chunks) * (1 + 0.045 * (double)M));
+        const double in = bytes * (1 + 0.03 * (double)M) / 5.44e6 + 0.095 * (double)chunks * (double)N / 4096;
+        return 3.43 + sqrt(latency * latency + in * in);
     }
     const bool narrow = (N + 79) / 80 < 128;  // as launch_rowwise_strip has it
     const int64_t strips = (N + (narrow ? 31 : 79)) / (narrow ? 32 : 80);
-    return 1.5 + (double)((strips + cus - 1) / cus) * (1.5 + kt * (M <= 64 ? (narrow ? 0.215 : 0.451) : (narrow ? 0.32 : 0.626))) + bytes / 30e6;
+    const double rounds = (double)((strips + cus - 1) / cus);
+    if (M <= 64) return narrow ? 2.74 + rounds * (1.46 + kt * 0.209) + bytes / 30.9e6 : 4.42 + rounds * (1.29 + kt * 0.389) + bytes / 34.8e6;
+    return narrow ? 3.77 + rounds * (1.31 + kt * 0.280) + bytes / 34.3e6 : 4.12 + rounds * (1.37 + kt * 0.572) + bytes / 32.8e6;
 }
 // Beyond that: rounds of tiles, a last one cheaper the emptier it is, beside the operands' way in; a remainder of rows is a
 // problem of its own.
@@ -3396,21 +3397,21 @@ static double rowwise_tiles_cost(int64_t M, int64_t N, int64_t K, int cus) {
     };
     if (M % 256 == 0 && N % 128 == 0) {
         const int64_t t256 = M / 256 * ((N + 255) / 256), rem = t256 % cus;
-        if (N % 256 || t256 <= 128) return 4.6 + beside(time(M / 256 * (N / 128), 0.813, 0.207, 0.0), in / 2.65e6);
-        double us = time(t256, 1.159, 0.19, 3.7);
-        if (t256 > cus && rem && rem * 2 <= cus) us = time(t256 - rem, 1.159, 0.19, 3.7) + (double)((4 * rem + cus - 1) / cus) * (kt * 0.731 + 4.7);
-        return 7.1 + beside(us, in / 2.44e6);
+        if (N % 256 || t256 <= 128) return 5.87 + beside(time(M / 256 * (N / 128), 0.754, 0.207, 0.0), in / 2.74e6);
+        if (M > 256) {
+            double us = time(t256, 0.998, 0.19, 3.19);
+            if (t256 > cus && rem && rem * 2 <= cus) us = time(t256 - rem, 0.998, 0.19, 3.19) + (double)((4 * rem + cus - 1) / cus) * (kt * 0.629 + 4.05);
+            return 11.1 + beside(us, in / 5.27e6);
+        }
     }
-    if (M <= 256) return 3.1 + time((N + 127) / 128, 0.846, 0.664, 2.1);
-    if (M > 512 && N % 256 == 0 && M % 256) return rowwise_tiles_cost(M / 256 * 256, N, K, cus) + rowwise_tiles_cost(M % 256, N, K, cus);
-    return 3.6 + beside(time((M + 255) / 256 * ((N + 255) / 256), 1.472, 0.238, 3.8), in / 2.85e6);
+    if (M <= 256) return 3.39 + time((N + 127) / 128, 0.877, 0.664, 2.18);
+    if (M > 512 && N % 256 == 0 && M % 256) return rowwise_tiles_cost(M / 256 * 256, N, K, cus) + rowwise_tiles_cost(M % 256, N, K, cus) - 1.3;
+    if (M <= 512) return 3.57 + beside(time((M + 255) / 256 * ((N + 255) / 256), 1.459, 0.238, 3.77), in / 3.68e6);
+    return 8.91 + beside(time((M + 255) / 256 * ((N + 255) / 256), 1.415, 0.238, 3.65), in / 2.98e6);
 }
 
 // Rowwise product with a bias and memory for partial sums: the form with the least estimated time among the ring kernel
 // (gemm_ring.hip), the walking 256 x 256 tiles with edges, and launch_gemm.
-// Up to 128 tokens launch_gemm's streamers are taken within 8 %, which lose less behind large writes (33 x 18944 x 3584 with the
-// token quantiser 19.9 / 23.7 us behind small and large ones, ring 21.1 / 25.6), and within 25 % beyond 96 tokens, where the ring
-// kernel's second row of tiles of 64 fills up (121 x 3328 x 3328 15.7 / 18.5, ring 16.1 / 21.4).
 // Timed with weights that no cache holds, ring / launch_gemm: 21 x 896 x 17152 11 / 33, 33 x 25344 x 2560 15.0 / 23.6; 33 x 18944 x
 // 3584, one round of strips, 17.3 / 16.4, 64 x 2048 x 1536 7.0 / 6.2, 16 x 1792 x 1792 6.8 / 4.3; 739 x 1024 x 1024 5.8 / 21.7, 152 x 1792
 // x 12672 17 / 88, 1061 x 2560 x 7936 40 / 75, 1024 x 3584 x 3584 with the quantiser 24 / 31; but 2048 x 3584 x 3584, 224 of its tiles of
@@ -3423,7 +3424,8 @@ static int launch_rowwise_best(GemmArgs& p, int out_dtype, hipStream_t st) {
     r.ld_a = p.ld_a; r.ld_w = p.ld_b; r.ld_out = p.ld_out;
     r.M = p.M; r.N = p.N; r.K = p.K;
     RingPlan ring{0, 0, 0, 1e30};
-    if (ring_takes(kRingRow, r, out_dtype)) ring = ring_plan(kRingRow, p.M, p.N, p.K, p.partial_bytes, cus);
+    // (where the linear is one launch the product has its bits, those of the kernel for 16 tokens)
+    if (!fused_gemv_size(p.M, p.K) && ring_takes(kRingRow, r, out_dtype)) ring = ring_plan(kRingRow, p.M, p.N, p.K, p.partial_bytes, cus);
     EdgePlan edge{};
     edge.cost = 1e30;
     if (p.M > 128 && edge_takes(p, out_dtype)) edge = edge_plan(p.M, p.N, p.K, cus);
@@ -3432,7 +3434,6 @@ static int launch_rowwise_best(GemmArgs& p, int out_dtype, hipStream_t st) {
         other = rowwise_tiles_cost(p.M, p.N, p.K, cus);
         // (bias_rows_kernel behind those that take no bias)
         if (p.bias && p.M > 16) other += 4.0 + (p.M > 128 ? 4.0 * p.M * (double)p.N / 4e6 : 0.0);
-        if (p.M <= 128) other /= p.M <= 96 ? 1.08 : 1.25;
     }
     if (ring.cost < 1e30 && ring.cost <= edge.cost && ring.cost <= other) return launch_ring(kRingRow, r, ring, out_dtype, st);
     // (without a bias and without remainders launch_gemm's form of the same tiles is 2 % faster)
@@ -3452,8 +3453,7 @@ static int launch_rowwise_best(GemmArgs& p, int out_dtype, hipStream_t st) {
 }
 
 // The times of launch_gemm's block-scaled kernels for more than 64 rows in microseconds, kernel by kernel as it chooses them; fitted to
-// 905 shapes of 80 to 6144 rows (weights of 896 .. 37888 rows, K 896 .. 18944), each timed behind small writes and behind one
-// that left L2 full, to the mean of the two: 3 % off on average.
+// the same shapes and in the same way as the ring's (gemm_ring.hip: ring_plan).
 static bool block_splits_rows(int64_t M, int64_t N, int64_t K) {  // into full tiles and the rest, as launch_gemm does
     return M >= 768 && M % 256 != 0 && N % 128 == 0 && M / 256 * (N / 128) >= 384 && K / 128 <= kMaxTileWeightScales;
 }
@@ -3468,19 +3468,19 @@ static double block_tiles_cost(int64_t M, int64_t N, int64_t K, int cus) {
         else if (rem) us += kt * step * (1 + load * (full ? part : part * part)) + ends;
         return us;
     };
-    if (M <= 64) return 6.0 + kt * 0.3;
-    if (block_splits_rows(M, N, K)) return block_tiles_cost(M / 256 * 256, N, K, cus) + block_tiles_cost(M % 256, N, K, cus);
+    if (M <= 64) return 24.1 + kt * 0.356;
+    if (block_splits_rows(M, N, K)) return block_tiles_cost(M / 256 * 256, N, K, cus) + block_tiles_cost(M % 256, N, K, cus) + 1.4;
     if (M % 256 == 0 && N % 256 == 0 && KT >= 16 && KT <= 1024) {
         const int64_t tm = M / 256, tn = N / 256, tiles = tm * tn, rem = tiles % cus;
         const int64_t cut = rem > 0 && rem * 2 <= cus ? (rem + tm - 1) / tm : 0;
         const int64_t head = tm * (tn - cut), rounds = (head + cus - 1) / cus;
         if (head >= cus && head * 5 >= rounds * cus * 4)
-            return 2.0 + beside(time(head, 1, 1.42, 0.196, 0.0, 7.8) + (cut ? kt * 0.755 + 8.2 : 0.0), in / 2.17e6);
+            return -1.53 + beside(time(head, 1, 1.359, 0.196, 0.0, 7.46) + (cut ? kt * 0.723 + 7.85 : 0.0), in / 2.58e6);
     }
     if (M > 512 && M % 256 == 0 && N % 128 == 0 && M / 256 * (N / 128) >= 384 && KT <= kMaxTileWeightScales)
-        return 4.6 + beside(time(M / 256 * (N / 128), 1, 0.797, 0.371, 0.0, KT <= kPersistentBlockSteps ? 1.0 : 4.0), in / 1.77e6);
-    if (M > 512 && (M + 255) / 256 * ((N + 127) / 128) >= 384) return 5.0 + beside(time((M + 255) / 256 * ((N + 127) / 128), 1, 1.025, 0.098, 0.0, 2.0), in / 1.4e6);
-    return 1.9 + beside(time((M + 127) / 128 * ((N + 127) / 128), 2, 0.82, 0.088, 0.445, 1.8), in / 2.58e6);
+        return 5.71 + beside(time(M / 256 * (N / 128), 1, 0.676, 0.371, 0.0, KT <= kPersistentBlockSteps ? 0.85 : 3.39), in / 2.26e6);
+    if (M > 512 && (M + 255) / 256 * ((N + 127) / 128) >= 384) return 4.61 + beside(time((M + 255) / 256 * ((N + 127) / 128), 1, 1.047, 0.098, 0.0, 2.04), in / 2.45e6);
+    return 5.41 + beside(time((M + 127) / 128 * ((N + 127) / 128), 2, 0.791, 0.088, 0.445, 1.74), in / 4.02e6);
 }
 
 // Block-scaled product with memory for partial sums, the form with the least estimated time: the ring kernel (gemm_ring.hip) on

@@ -1773,11 +1773,9 @@ static int launch_mx4(Mx4Args p, int out_dtype, hipStream_t st) {
 
 namespace cfp8 {
 // What the tile kernels below the dispatch would take for M > 128 rows, in microseconds: rounds of tiles on the CUs (a last one
-// cheaper the emptier it is) times K steps, beside the operands' way in; fitted to 603 shapes of 129 to 6144 rows (weights of
-// 896 .. 37888 rows, K 896 .. 18944), each timed behind small writes and behind one that left L2 full, to the mean of the two: 2 to
-// 4 % off on average.  Infinite where only the register-staged tiles would be left, which take twice the ring kernel's time and more.
-// (7 % more for the 128 x 512 tiles: of seven shapes of 2000 to 8000 rows where the estimates were level the ring kernel was ahead in all, 4352 x 4992 x
-// 3456 80.5 against 93.4 us, 2088 x 32768 x 2432 166 against 190.)
+// cheaper the emptier it is) times K steps, beside the operands' way in; fitted to the same shapes and in the
+// same way as the ring's (gemm_ring.hip: ring_plan).  Infinite where only the register-staged tiles would be left, which take twice
+// the ring kernel's time and more.
 static double mx4_tiles_cost(int64_t M, int64_t N, int64_t K, bool aligned256, int cus) {
     const double kt = (double)((K + 127) / 128), in = (double)N * (double)K * 0.53 + (double)M * (double)K;
     auto time = [&](int64_t tiles, double step, double load, double ends) {
@@ -1789,31 +1787,31 @@ static double mx4_tiles_cost(int64_t M, int64_t N, int64_t K, bool aligned256, i
     if (aligned256 && (M / 256) * (N / 256) >= 128) {
         const int64_t tm = M / 256, tn = N / 256, rem = (tm * tn) % cus, cut = (rem + tm - 1) / tm;  // as launch_mx4_best has it
         const bool two = tm * tn > cus && rem > 0 && rem * 2 <= cus && cut < tn;
-        const double us = two ? time(tm * (tn - cut), 1.055, 0.275, 6.1) + time((M + 127) / 128 * cut, 0.588, 0.433, 7.1) : time(tm * tn, 1.055, 0.275, 6.1);
-        return 2.5 + beside(us, in / 1.71e6);
+        const double us = two ? time(tm * (tn - cut), 1.009, 0.275, 5.83) + time((M + 127) / 128 * cut, 0.562, 0.433, 6.79) : time(tm * tn, 1.009, 0.275, 5.83);
+        return 3.79 + beside(us, in / 2.29e6);
     }
     const int64_t t256 = (M + 127) / 128 * ((N + 255) / 256), t512 = (M + 127) / 128 * ((N + 511) / 512);
-    if (t512 >= 256 && (N + 511) / 512 * 512 - N <= N / 8) return 1.07 * beside(time(t512, 1.043, 0.433, 8.8), in / 0.65e6);
-    if (t256 >= 64) return 3.2 + beside(time(t256, 0.772, 0.209, 1.6), in / 2.0e6);
+    if (t512 >= 256 && (N + 511) / 512 * 512 - N <= N / 8) return 16.1 + beside(time(t512, 0.966, 0.433, 8.15), in / 1.69e6);
+    if (t256 >= 64) return 6.58 + beside(time(t256, 0.695, 0.209, 1.44), in / 3.02e6);
     return 1e30;
 }
 
 // The same for up to 128 rows: the kernels that stream the weights - a round of workgroups each 16 rows wide and the chunks of K
-// one after the other up to 16 tokens, rounds of strips times K steps beyond - fitted to 258 shapes of 5 to 128 rows, each timed behind
-// small writes and behind one that left L2 full, to the mean of the two (2 to 4 % off on average).  Infinite for narrow weights of 17 rows
-// and more: the ring kernel is the faster one there without slices too (17 x 1664 x 1664 6.5 us both, 64 x 1536 x 8960 30 against 33).
+// one after the other up to 16 tokens, rounds of strips times K steps beyond.  Infinite for narrow weights of 17 rows and
+// more: the ring kernel is the faster one there without slices too (17 x 1664 x 1664 6.5 us both, 64 x 1536 x 8960 30 against 33).
 static double mx4_streams_cost(int64_t M, int64_t N, int64_t K, int cus) {
     const double codes = (double)N * (double)K;
     const int64_t kt = (K + 127) / 128;
     if (M <= 16) {
         const double chunks = (double)((kt + 4 * kGemvDepth - 1) / (4 * kGemvDepth)), steps = (double)((kt + 3) / 4);
         const double more = (double)(((N + 15) / 16 + cus - 1) / cus - 1);
-        if (mx4_gemv_in_lds(M, K)) return 1.8 + chunks * (1.93 + 0.035 * M + 1.24 * more) + steps * (0.026 + 0.024 * M) + codes * (1 + 0.047 * M) / 13.8e6;
-        return 2.1 + chunks * (2.2 + 2.7 * more) + steps * 0.009 * M + codes * (1 + 0.014 * M) / 19.4e6;
+        if (mx4_gemv_in_lds(M, K)) return 2.60 + chunks * (1.98 + 0.036 * M + 1.27 * more) + steps * (0.027 + 0.0246 * M) + codes * (1 + 0.047 * M) / 13.5e6;
+        return 4.03 + chunks * (2.08 + 2.55 * more) + steps * 0.0085 * M + codes * (1 + 0.014 * M) / 20.5e6;
     }
     const int64_t strips = (N + 79) / 80;
     if (strips < 128) return 1e30;
-    return 1.82 + (double)((strips + cus - 1) / cus) * (2.9 + (double)kt * (M <= 64 ? 0.378 : 0.595)) + codes / 23.7e6;
+    const double rounds = (double)((strips + cus - 1) / cus);
+    return M <= 64 ? 3.35 + rounds * (2.78 + (double)kt * 0.362) + codes / 24.7e6 : 4.48 + rounds * (2.82 + (double)kt * 0.578) + codes / 24.4e6;
 }
 
 // One product, ungrouped, with partial sums' memory or none: the ring kernel or the others.
@@ -1827,14 +1825,13 @@ static int gemm_mx4_dense(Mx4Args& p, float* partial, size_t partial_bytes, int 
     if ((p.M <= 4 && p.K <= 4096) || !ring_takes(kRingMx, r, out_dtype)) return CFP8_OK;
     const RingPlan plan = ring_plan(kRingMx, p.M, p.N, p.K, partial_bytes, cu_count());
     if (p.M <= 128) {
-        // (the ring kernel where it is ahead by more than the estimates are off: 18944 x 3584 at 33 tokens 19.5 against 17.4 us,
-        // 16 x 3584 x 3584 8.2 against 6.2, but 33 x 25344 x 2560 15.3 against 25.3)
-        if (mx4_streams_cost(p.M, p.N, p.K, cu_count()) <= plan.cost * 1.05) return CFP8_OK;
+        // (ring kernel / streamers: 18944 x 3584 at 33 tokens 19.5 / 17.4 us, 16 x 3584 x 3584 8.2 / 6.2, but 33 x 25344 x 2560 15.3 / 25.3)
+        if (mx4_streams_cost(p.M, p.N, p.K, cu_count()) <= plan.cost) return CFP8_OK;
     } else {
         const bool aligned256 = p.M % 256 == 0 && p.N % 256 == 0 && p.K % 128 == 0 && p.ld_ws % 4 == 0 && (reinterpret_cast<uintptr_t>(p.ws) & 3u) == 0;
-        // (within 5 % the tiles: their time depends less on what L2 holds; 4096 x 9728 x 896 45.4 / 52.2 us behind small and large
-        // writes, ring 42.9 / 61.8.  512 x 9728 x 896 11.0 against 12.4 us, but 1629 x 2304 x 9984 58 against 44)
-        if (mx4_tiles_cost(p.M, p.N, p.K, aligned256, cu_count()) <= plan.cost * 1.05) return CFP8_OK;
+        // (ring kernel / tiles, behind small and large writes: 4096 x 9728 x 896 42.9 61.8 / 45.4 52.2 us, 256 x 152064 x 3584 161 175 /
+        // 128 145, but 1629 x 2304 x 9984 44 / 58 behind small ones)
+        if (mx4_tiles_cost(p.M, p.N, p.K, aligned256, cu_count()) <= plan.cost) return CFP8_OK;
     }
     taken = true;
     return launch_ring(kRingMx, r, plan, out_dtype, st);

@@ -589,23 +589,28 @@ static int launch_ring_mode(RingArgs& p, const RingPlan& plan, int out_dtype, hi
 // K steps times the tile's step time (longer the more CUs load at once, and as long as for two everywhere as soon as one CU
 // holds two) plus the tile's ends; joins it with the operands' bytes at the rate they come in, (a^4 + b^4)^(1/4), since neither
 // hides the other near where they meet; and adds a fixed time per launch and, for slices, the reduction's launch and their
-// partial sums' way out and back.  The constants are fitted to all combinations at some hundred shapes a mode (weights of 896 .. 37888
-// rows, K 896 .. 18944; kFewRates: 5 .. 128 rows, block scaling 5 .. 64, kRates: the others up to 6144), each timed behind small writes and behind one that left L2
-// full, to the mean of the two: 4 to 6 % off on average, the choice within 1 % of the best combination, 15 to 20 % at worst.
+// partial sums' way out and back.  The constants are fitted to all combinations at some thousand shapes a mode (weights of 896 .. 37888
+// rows, K 896 .. 18944, and up to 160000 rows with K up to 5120; kFewRates: 5 .. 128 rows, block scaling 5 .. 64, kRates: the others up to 6144), each timed behind small writes
+// and behind one that left L2 full, to the mean of the two and to what the choice loses by them, together with the estimates of the
+// other kernels: 2 to 4 % off on average.  Of shapes that the fit had not seen, the choice is within 0.3 (block scaling) to 0.5 % of the
+// best combination on average, more than 5 % behind it for 1 to 3 in a hundred, 30 % at worst.
+// (With one time for the ends of all tiles, long products of 128 x 128 tiles were 20 % quicker than estimated, short ones slower:
+// 4688 x 1536 x 12800 took 112 us on other tiles, 84 on these.)
 struct RingRates {
-    double step[4], load[4], two[4];  // 128 x 128, 64 x 128, 128 x 64, 64 x 64: microseconds a step; what a full GPU adds; what two a CU add
-    double launch, ends, partial, bytes, reduce;
-    double fill;  // what rows that do not exist, and are not loaded, save of a tile
+    double step[4], load[4], two[4], ends[4];  // 128 x 128, 64 x 128, 128 x 64, 64 x 64: microseconds a step; what a full GPU adds; what two a CU add
+    double launch, partial, bytes, reduce, slice;
+    double fill;   // what rows that do not exist, and are not loaded, save of a tile
+    double again;  // what of its ends a round of tiles still takes behind another
 };
 static const RingRates kRates[3] = {
-    {{0.547, 0.353, 0.346, 0.228}, {0.164, 0.110, 0.131, 0.099}, {0.068, 0.771, 0.787, 0.624}, 3.66, 0.78, 5.33, 2.77, 1.86, 0.0},
-    {{0.782, 0.470, 0.0, 0.323}, {0.064, 0.086, 0.0, 0.122}, {0.0, 0.0, 0.0, 0.405}, 3.24, 0.91, 5.06, 2.66, 2.21, 0.0},
-    {{0.541, 0.419, 0.376, 0.247}, {0.080, 0.068, 0.106, 0.081}, {0.637, 0.513, 0.528, 0.626}, 3.13, 0.55, 5.70, 1.77, 3.11, 0.14},
+    {{0.335, 0.336, 0.266, 0.265}, {0.373, 0.311, 0.457, 0.0}, {0.033, 0.753, 0.764, 0.736}, {4.06, 1.54, 1.65, 0.92}, 3.37, 6.79, 2.61, 2.89, -0.020, 0.042, 1.0},
+    {{0.585, 0.436, 0.0, 0.246}, {0.043, 0.0, 0.0, 0.396}, {0.068, 0.0, 0.0, 0.586}, {4.63, 3.28, 0.0, 1.73}, 3.04, 7.78, 3.29, 2.20, 0.134, 0.173, 0.625},
+    {{0.414, 0.300, 0.315, 0.231}, {0.244, 0.504, 0.133, 0.089}, {0.857, 0.817, 0.811, 0.968}, {1.71, 1.20, 1.04, 0.63}, 4.40, 7.61, 2.57, 2.97, 0.102, 0.140, 0.638},
 };
 static const RingRates kFewRates[3] = {
-    {{0.587, 0.418, 0.387, 0.223}, {0.296, 0.465, 0.130, 0.331}, {0.0, 0.845, 0.886, 1.338}, 2.88, 0.34, 4.17, 7.97, 2.26, 0.2},
-    {{0.658, 0.393, 0.0, 0.263}, {0.100, 0.335, 0.0, 0.283}, {0.0, 0.0, 0.0, 0.362}, 2.3, 1.2, 4.3, 4.9, 2.3, 0.0},
-    {{0.630, 0.523, 0.447, 0.290}, {0.170, 0.317, 0.0, 0.121}, {0.942, 0.883, 0.965, 1.274}, 2.51, 0.0, 4.22, 5.52, 2.86, 0.2},
+    {{0.551, 0.423, 0.302, 0.231}, {0.055, 0.277, 0.309, 0.066}, {0.043, 1.176, 1.111, 1.269}, {2.92, 1.03, 1.22, 1.00}, 3.76, 6.25, 8.65, 2.39, 0.039, 0.226, 1.0},
+    {{0.0, 0.343, 0.0, 0.350}, {0.0, 0.382, 0.0, 0.0}, {0.0, 0.270, 0.0, 0.498}, {0.0, 2.53, 0.0, 1.35}, 3.03, 5.00, 7.45, 2.51, 0.053, 0.239, 1.0},
+    {{0.574, 0.457, 0.412, 0.283}, {0.277, 0.449, 0.004, 0.0}, {1.039, 1.480, 0.898, 1.098}, {1.00, 0.43, 1.15, 1.17}, 3.18, 5.98, 12.0, 2.41, 0.114, 0.232, 1.0},
 };
 static const int kTiles[4][2] = {{128, 128}, {64, 128}, {128, 64}, {64, 64}};
 constexpr int kRingMaxSlices = 16;
@@ -634,12 +639,12 @@ RingPlan ring_plan(int mode, int64_t M, int64_t N, int64_t K, size_t partial_byt
             if (mode == kRingBlock && !ring_scales_fit(bm, bn, steps)) continue;
             const uint32_t full = tiles * s / slots, rem = tiles * s - full * slots;
             const double part = (double)rem / cus, step = (double)steps * r.step[c];
-            double us = (double)full * (step * (1 + r.load[c] + r.two[c]) + per * r.ends);
-            if (part > 1) us += step * (1 + r.load[c] + r.two[c]) + 2 * r.ends;
-            else if (rem) us += step * (1 + r.load[c] * (full ? part : part * part)) + r.ends;
+            double us = full ? (double)full * (step * (1 + r.load[c] + r.two[c]) + per * r.ends[c] * r.again) + per * r.ends[c] * (1 - r.again) : 0.0;
+            if (part > 1) us += step * (1 + r.load[c] + r.two[c]) + 2 * r.ends[c];
+            else if (rem) us += step * (1 + r.load[c] * (full ? part : sqrt(part))) + r.ends[c];
             us *= 1 + r.fill * ((double)M / (double)((M + bm - 1) / bm * bm) - 0.5);
             us = r.launch + sqrt(sqrt(us * us * us * us + in * in * in * in));
-            if (s > 1) us += r.reduce + 8.0 * s * (double)M * (double)N / (r.partial * 1e6);
+            if (s > 1) us += r.reduce + r.slice * s + 8.0 * s * (double)M * (double)N / (r.partial * 1e6);
             if (us < best.cost) best = {bm, bn, (int)s, us};
         }
     }

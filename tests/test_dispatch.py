@@ -114,7 +114,7 @@ OPERATORS = [
     ("... a round of 256 x 256", (ROW, 4096, 3584, 18944), S, ["gemm_rowwise_256 grid=224"]),
     ("... a short K", (ROW, 512, 9728, 896), S, ["gemm_rowwise_256x128 grid=152"]),
     ("... too few of them: ring tiles", (ROW, 1024, 3584, 3584), S, ["gemm_ring<rowwise,128,128> slices=1 grid=224"]),
-    ("... with a bias, which they do not take", (ROW, 2048, 4608, 3584), S | BIAS, ["gemm_ring<rowwise,128,64> slices=1"]),
+    ("... with a bias, which they do not take", (ROW, 2048, 4608, 3584), S | BIAS, ["gemm_ring<rowwise,128,128> slices=1 grid=576"]),
     ("1111 tokens, down: a round of ring tiles", (ROW, 1111, 3584, 18944), S, ["gemm_ring<rowwise,128,128> slices=1 grid=252"]),
     ("full tiles without a bias: the walking form", (ROW, 8192, 4608, 3584), S, ["gemm_rowwise_256p tail=64"]),
     ("full tiles with a bias: the edge form, which adds it", (ROW, 8192, 4608, 3584), S | BIAS, ["gemm_rowwise_edge tail=64 edges=0"]),
@@ -124,13 +124,18 @@ OPERATORS = [
     ("17 to 128 tokens, a round of strips", (ROW, 33, 18944, 3584), S, ["gemm_rowwise_strip<64,5> grid=237"]),
     ("... which has no bias of its own", (ROW, 33, 18944, 3584), S | BIAS, ["gemm_ring<rowwise,64,128> slices=1 grid=148"]),
     ("... 64 tokens", (ROW, 64, 18944, 3584), S, ["gemm_rowwise_strip<64,5> grid=237"]),
-    ("... a narrow weight", (ROW, 33, 4608, 3584), S, ["gemm_rowwise_strip<64,2> grid=144"]),
+    ("... a narrow weight", (ROW, 64, 4608, 3584), S, ["gemm_rowwise_strip<64,2> grid=144"]),
+    ("... fewer tokens on it: slices", (ROW, 33, 4608, 3584), S, ["gemm_ring<rowwise,64,64> slices=3 grid=216", "ring_reduce"]),
     ("two rounds of strips and a little: ring tiles", (ROW, 33, 25344, 2560), S, ["gemm_ring<rowwise,64,128> slices=1"]),
     ("65 to 96 tokens: tiles of 64 rows or of 128", (ROW, 80, 2944, 2432), S, ["gemm_ring<rowwise,64,64> slices=1"]),
     ("... a wide weight", (ROW, 80, 32768, 2560), S, ["gemm_ring<rowwise,128,128> slices=1"]),
-    ("128 tokens on the widest weight: two rounds of strips", (ROW, 128, 37888, 3584), S, ["gemm_rowwise_strip<128,5>"]),
+    ("128 tokens: a round of strips", (ROW, 128, 18944, 3584), S, ["gemm_rowwise_strip<128,5> grid=237"]),
+    ("... on the widest weight", (ROW, 128, 37888, 3584), S, ["gemm_ring<rowwise,128,64> slices=1 grid=592"]),
+    ("256 tokens on more than 32768 rows: staged tiles", (ROW, 256, 152064, 3584), S, ["gemm_kernel<256,128,4,2,rowwise>"]),
     ("33 tokens, down: slices", (ROW, 33, 3584, 18944), S, ["gemm_ring<rowwise,64,64> slices=4", "ring_reduce"]),
     ("16 tokens on a small weight", (ROW, 16, 1792, 1792), S, ["gemm_rowwise_gemv"]),
+    ("up to 4 tokens, where the linear is one launch: its bits", (ROW, 4, 37888, 3584), S, ["gemm_rowwise_gemv"]),
+    ("... one token up to K = 8192", (ROW, 1, 37888, 8192), S, ["gemm_rowwise_gemv"]),
     ("16 tokens on a wide weight", (ROW, 16, 37888, 3584), S, ["gemm_ring<rowwise,64,64> slices=1"]),
     ("block, a decode batch", (BLK, 24, 18432, 7168), S, ["gemm_ring<block,64,128> slices=1 grid=144"]),
     ("block, full tiles", (BLK, 4096, 18432, 7168), S, ["gemm_block_256 grid=1024", "gemm_block_w8<256,128,block>"]),

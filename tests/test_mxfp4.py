@@ -193,7 +193,7 @@ def test_gemm_mxfp4_against_oracle(dev, M, N, K):
 # of a partial round as a second launch
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,took", [(1000, 4112, 160, "gemm_mxfp4_tile<128,256>"), (1000, 4112, 256, "gemm_mxfp4_tile<128,256>"),
-                                        (2000, 8192, 1152, "gemm_mxfp4_tile<128,512>"),
+                                        (1500, 20480, 2176, "gemm_mxfp4_tile<128,512>"),
                                         (1536, 9728, 512, "gemm_mxfp4_tile<256,256>"), (2304, 9728, 1152, "gemm_mxfp4_tile<256,256> + gemm_mxfp4_tile<128,256>")])
 def test_gemm_mxfp4_tile_kernels(dev, M, N, K, took):
     from cosmos_rl_amd import _lib, ops
