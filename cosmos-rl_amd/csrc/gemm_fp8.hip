@@ -1872,8 +1872,8 @@ static int launch_rowwise_256p(GemmArgs& p, int out_dtype, hipStream_t st) {
 // tiles.  Between divisions the choice weighs, in microseconds a K step, a whole tile on every CU 1.35, a quarter tile 0.5, or 1.0 for
 // quarters of a row remainder, which read all of the weight again (8192 x 18944 x 3584, nine rounds and one of quarters, 405
 // us; 1111 x 37888 x 3584 180 us with 87 rows as quarters, 2.3 rounds of tiles and 2.4 of quarters).  `cost` is the time
-// of the division taken, fitted to 198 shapes behind small and behind large writes, 2 % off on average: a last round of whole tiles
-// costs 0.6 of a full one and more the fuller it is.
+// of the division taken, fitted with the other estimates (gemm_ring.hip: ring_plan): a last round of whole tiles costs 0.6 of a full
+// one and more the fuller it is.
 static double beside(double us, double in) { return sqrt(sqrt(us * us * us * us + in * in * in * in)); }  // neither hides the other where they meet
 struct EdgePlan {
     int tiles_m, tiles_n, tail, edge_rows, edge_cols;
@@ -3490,7 +3490,7 @@ static double block_tiles_cost(int64_t M, int64_t N, int64_t K, int cus) {
 // Timed with weights that no cache holds, launch_gemm / ring: 22 x 9600 x 4608 35 / 24 us, 8 x 2176 x 4352 26.5 / 13.5, 123 x 1792 x
 // 5120 43 / 16, 256 x 3584 x 18944 126 / 41, 171 x 16000 x 2560 28.8 / 29.4; but 256 x 23552 x 3200 41.6 / 47.1, 600 x 9472 x 5248 67 / 78, 1024 x 9728 x 896
 // 21.8 / 25.2, 2816 x 3328 x 1280 26.3 / 29.8; full tiles with a ring kernel behind them 3000 x 4480 x 3200 86 / 76.  The choice is within
-// 1 % of the best on average, 9 % at worst.
+// 0.3 % of the best on average, 17 % at worst.
 struct BlockPlan {
     int64_t body;   // rows of the full tiles
     RingPlan ring;  // the others (bm == 0: launch_gemm)

@@ -165,6 +165,60 @@ def test_block(dev, M, N, K, kn):
             _check(out, want, M, N, dtype, 0.0)
 
 
+# every tile of the ring kernel for every weight format, with slices of K and without, with weights loaded as a stream (one row of tiles, and
+# what else ring_once names) and cacheably, some with a last step of 64: the smallest products with remainders of rows and columns that
+# the choice takes there
+FORMS = [("block", 64, 64, False, 67, 208, 384), ("block", 64, 64, False, 5, 208, 384), ("block", 64, 64, True, 67, 208, 2176),
+         ("block", 64, 64, True, 5, 208, 2176), ("block", 64, 128, False, 67, 9232, 384), ("block", 64, 128, False, 5, 18448, 384),
+         ("block", 64, 128, True, 67, 2832, 5248), ("block", 64, 128, True, 5, 5648, 2432), ("block", 128, 128, False, 67, 18448, 384),
+         ("block", 128, 128, True, 67, 5648, 7296), ("mxfp4", 64, 64, False, 131, 208, 384), ("mxfp4", 64, 64, False, 19, 208, 640),
+         ("mxfp4", 64, 64, True, 150, 208, 2432), ("mxfp4", 64, 64, True, 5, 208, 9344), ("mxfp4", 64, 128, False, 131, 9232, 384),
+         ("mxfp4", 64, 128, False, 5, 208, 384), ("mxfp4", 64, 128, True, 131, 2064, 7296), ("mxfp4", 64, 128, True, 19, 208, 2176),
+         ("mxfp4", 128, 64, False, 131, 5648, 384), ("mxfp4", 128, 64, False, 67, 9232, 640), ("mxfp4", 128, 64, True, 131, 1808, 5248),
+         ("mxfp4", 128, 64, True, 67, 2832, 2944), ("mxfp4", 128, 64, False, 131, 5648, 448), ("mxfp4", 128, 64, False, 67, 9232, 448),
+         ("mxfp4", 128, 128, False, 131, 11792, 384), ("mxfp4", 128, 128, False, 67, 18448, 384), ("mxfp4", 128, 128, True, 131, 2832, 7296),
+         ("mxfp4", 128, 128, True, 67, 5648, 7296), ("mxfp4", 128, 128, True, 131, 2832, 7360), ("mxfp4", 128, 128, True, 67, 5648, 5312),
+         ("rowwise", 64, 64, False, 67, 208, 384), ("rowwise", 64, 64, False, 5, 14864, 384), ("rowwise", 64, 64, True, 67, 208, 2176),
+         ("rowwise", 64, 64, True, 5, 208, 7296), ("rowwise", 64, 128, False, 131, 9232, 384), ("rowwise", 64, 128, False, 5, 23568, 384),
+         ("rowwise", 64, 128, True, 131, 1808, 5248), ("rowwise", 64, 128, True, 5, 5648, 7296), ("rowwise", 64, 128, True, 131, 1808, 5312),
+         ("rowwise", 64, 128, True, 5, 5648, 3776), ("rowwise", 128, 64, False, 131, 5648, 384), ("rowwise", 128, 64, False, 67, 9232, 384),
+         ("rowwise", 128, 64, True, 1500, 208, 5248), ("rowwise", 128, 64, True, 67, 2832, 3712), ("rowwise", 128, 64, True, 1031, 208, 7360),
+         ("rowwise", 128, 64, True, 67, 2832, 3776), ("rowwise", 128, 128, False, 515, 3600, 640), ("rowwise", 128, 128, False, 67, 23568, 640),
+         ("rowwise", 128, 128, True, 131, 2832, 9344), ("rowwise", 128, 128, True, 67, 9232, 5248), ("rowwise", 128, 128, False, 131, 11792, 704),
+         ("rowwise", 128, 128, False, 67, 18448, 448)]
+
+
+@pytest.mark.parametrize("mode,bm,bn,sliced,M,N,K", FORMS)
+def test_every_form(dev, mode, bm, bn, sliced, M, N, K):
+    from oracle import mxfp4_oracle as MX
+    kind = {"rowwise": _lib.DISPATCH_ROWWISE, "block": _lib.DISPATCH_BLOCK, "mxfp4": _lib.DISPATCH_MXFP4}[mode]
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    took = _lib.gemm_dispatch_info(kind, M, N, K, cus=cus, flags=_lib.DISPATCH_SPLIT).split("; ")
+    assert took[0].startswith(f"gemm_ring<{mode},{bm},{bn}>") and ("slices=1 " not in took[0]) == sliced and len(took) == 1 + sliced, took
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g, device=dev).to(torch.bfloat16)
+    w = torch.randn(N, K, generator=g, device=dev) * 0.05
+    if mode == "rowwise":
+        a, b = ops.quant_rowwise(x), ops.quant_rowwise(w.to(torch.bfloat16))
+        want = _rowwise_want(*a, *b, None)
+        run = lambda dtype: ops.scaled_mm(a[0], b[0].t(), a[1], b[1].reshape(1, N), out_dtype=dtype)
+    elif mode == "block":
+        a = ops.groupwise_activation_quant(x)
+        b = w.to(torch.float8_e4m3fn), torch.rand(-(-N // 128), K // 128, generator=g, device=dev) + 0.5
+        want = ((a[0].double() * a[1].double().repeat_interleave(128, 1)) @
+                (b[0].double() * b[1].double().repeat_interleave(128, 0)[:N].repeat_interleave(128, 1)).t()).cpu()
+        run = lambda dtype: ops.gemm_fp8_fp8_bf16_nt(a, b, torch.empty(M, N, device=dev, dtype=dtype))
+    else:
+        a, b = ops.quant_rowwise(x), ops.quant_mxfp4(w.to(torch.bfloat16))
+        want = MX.gemm(a[0].cpu(), a[1].cpu().reshape(-1), b[0].cpu(), b[1].cpu()).double()
+        run = lambda dtype: ops.gemm_mxfp4(a, b, dtype)
+    for dtype in (torch.float32, torch.bfloat16):
+        ref = want if dtype == torch.float32 else want.float().to(torch.bfloat16).double()
+        got = run(dtype).double().cpu()
+        assert float((got - ref).norm() / ref.norm()) <= (1e-4 if dtype == torch.float32 else 1e-3)
+        assert float((got - ref).abs().max()) <= (1e-3 if dtype == torch.float32 else 2.0 ** -7) * float(ref.abs().max())
+
+
 def test_a_bias_that_torch_follows(dev):
     """the epilogue adds a bias only where nothing else would see the addition"""
     x = torch.randn(33, 256, device=dev).to(torch.bfloat16)
