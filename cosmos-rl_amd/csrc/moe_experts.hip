@@ -16,6 +16,7 @@
 //               64 rows would hold one or two.  A workgroup takes a strip of ONE expert's weight rows, requests all of its
 //               K into registers before anything else, and then walks the expert's rows in tiles of 16
 //               (few_gate_up_kernel, few_down_kernel).
+#include "gemm_internal.h"
 #include "gemm_ring.h"
 
 namespace cfp8 {
@@ -357,11 +358,13 @@ extern "C" int cfp8_moe_experts(const void* x, int64_t ld_x, int64_t tokens, int
     } else {
         if (int rc = cfp8_scatter_quant_group128(x, ld_x, tokens, hidden, i32(p.row_map), topk, i32(p.row_tokens), p.rows, ws + p.xq, hidden, f32(p.xs), stream))
             return rc;
-        if (int rc = cfp8_gemm_grouped_swiglu_quant(ws + p.xq, hidden, f32(p.xs), gate_up, gate_up_scales, i32(p.row_experts), ws + p.hq, inter,
-                                                    f32(p.hs), p.rows, inter, hidden, experts, stream))
+        // (p.rows is a bound: 639 tiles of rows for 8192 tokens, top 8 of 128 experts, of which some 566 hold rows)
+        const int32_t* const rows_end = i32(p.m_offsets) + experts - 1;
+        if (int rc = grouped_swiglu_quant(ws + p.xq, hidden, f32(p.xs), gate_up, gate_up_scales, i32(p.row_experts), rows_end, ws + p.hq, inter,
+                                          f32(p.hs), p.rows, inter, hidden, experts, stream))
             return rc;
-        if (int rc = cfp8_gemm_grouped_block128(ws + p.hq, inter, f32(p.hs), down, down_scales, i32(p.row_experts), ws + p.out, hidden, CFP8_OUT_BF16,
-                                                p.rows, hidden, inter, experts, stream))
+        if (int rc = grouped_block128(ws + p.hq, inter, f32(p.hs), down, down_scales, i32(p.row_experts), rows_end, ws + p.out, hidden, CFP8_OUT_BF16,
+                                      p.rows, hidden, inter, experts, stream))
             return rc;
     }
     return cfp8_combine_rows(ws + p.out, hidden, p.rows, i32(p.row_map), ws + p.weights, CFP8_IN_BF16, tokens, topk, hidden,

@@ -66,6 +66,24 @@ def test_one_call_experts_uneven(dev, T, E, topk, H, I):
     assert not bool(y[~mask].any())
 
 
+# experts of many rows, of which the products learn on the device how many there are: far fewer tiles of rows than the bound, fewer and
+# more than CUs (with and without whole rows of tiles in the down product), none at all
+@pytest.mark.parametrize("T,E,topk,H,I,keep", [(9000, 16, 8, 1024, 768, 0.3), (9000, 16, 8, 512, 640, 0.6), (6000, 20, 6, 1024, 1024, 0.1), (6000, 9, 6, 256, 768, 0.0),
+                                               (2000, 5, 3, 896, 768, 0.9)])
+def test_one_call_experts_many_rows(dev, T, E, topk, H, I, keep):
+    from cosmos_rl_amd.policy.kernel.moe.moe import grouped_experts_forward
+    strategy, module = _module(dev, E, H, I, T)
+    g = torch.Generator(device=dev).manual_seed(T + 3)
+    x = torch.randn(T, H, generator=g, device=dev).to(torch.bfloat16)
+    idx = torch.rand(T, E, generator=g, device=dev).topk(topk, dim=1).indices
+    w = torch.rand(T, topk, generator=g, device=dev).to(torch.bfloat16)
+    mask = torch.rand(T, generator=g, device=dev) < keep
+    y = grouped_experts_forward(x, mask, w, idx, strategy, module, E)
+    want = _chain(x, mask, w, idx, strategy, module, E)
+    assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+    assert not bool(y[~mask].any())
+
+
 def test_one_call_experts_refuses_a_small_workspace(dev):
     t = torch.zeros(256, 256, device=dev, dtype=torch.bfloat16)
     need = _lib.load().cfp8_moe_experts_workspace_bytes(4, 2, 2, 256, 128)
