@@ -281,8 +281,8 @@ __global__ __launch_bounds__(256) void gemm_grouped_xres_kernel(const GemmArgs p
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const f32x4 v = acc[2 * m + h][j];
-                __builtin_amdgcn_raw_buffer_store_b128(u32x4{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])}, ro_p,
-                                                       ((keep_p >> j) & 1u) ? off_p : kDropped, (uint32_t)(j * 16) * ld_out_b + (uint32_t)(2 * m + h) * 64u, 0);
+                buffer_store16(u32x4{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])}, ro_p,
+                               ((keep_p >> j) & 1u) ? off_p : kDropped, (uint32_t)(j * 16) * ld_out_b + (uint32_t)(2 * m + h) * 64u);
             }
     };
     // bf16: the waiting tile, packed: Pk[j][i] = the lane's four columns of w tile i in row j * 16 + lrow
@@ -309,8 +309,8 @@ __global__ __launch_bounds__(256) void gemm_grouped_xres_kernel(const GemmArgs p
         for (int r = 0; r < 4; ++r) Rd[r] = *reinterpret_cast<const i32x4*>(ebuf + (r * 4 + rd_row) * EST + rd_chunk * 16);
     };
     auto turn_store = [&](int j, int r) {
-        __builtin_amdgcn_raw_buffer_store_b128(u32x4{(u32)Rd[r][0], (u32)Rd[r][1], (u32)Rd[r][2], (u32)Rd[r][3]}, ro_p,
-                                               ((keep_p >> (j * 4 + r)) & 1u) ? off_p : kDropped, (uint32_t)(j * 16 + r * 4) * ld_out_b, 0);
+        buffer_store16(u32x4{(u32)Rd[r][0], (u32)Rd[r][1], (u32)Rd[r][2], (u32)Rd[r][3]}, ro_p, ((keep_p >> (j * 4 + r)) & 1u) ? off_p : kDropped,
+                       (uint32_t)(j * 16 + r * 4) * ld_out_b);
     };
     // A step's vector-memory operations are, in this order, its stores (first half) and its eight weight loads (second
     // half, behind the barrier); the stage a step's barrier needs was requested two steps earlier, so what may still be

@@ -95,6 +95,15 @@ bool grouped_xres_pays(const GemmArgs& p);  // enough of the CUs' tile slots wou
 // including the direct-to-LDS loads that are meant to stay in flight across the barrier.
 #define CFP8_WAIT_BARRIER(vm) asm volatile("s_waitcnt vmcnt(" #vm ") lgkmcnt(0)\n\ts_barrier" ::: "memory")
 
+// A 16-byte buffer store with a scalar offset.  The store reads its data registers a while after it has been issued, and a VALU
+// instruction right behind it that writes one of them reaches memory in its place for some of the lanes (seen on gfx950
+// where L2 was full of lines to write back: lanes 12 .. 15 of every 16 stored the result of the next instruction).  One
+// instruction in between is enough; the compiler keeps that distance for stores without a scalar offset only.
+__device__ __forceinline__ void buffer_store16(u32x4 v, __amdgpu_buffer_rsrc_t r, uint32_t lane_offset, uint32_t offset) {
+    __builtin_amdgcn_raw_buffer_store_b128(v, r, lane_offset, offset, 0);
+    asm volatile("s_nop 1" ::"v"(v));
+}
+
 // One int of a table that the kernel does not write, by a scalar load.  Behind the first store of a kernel the compiler turns
 // such a read into a vector load, and then waits for every load in flight, the direct-to-LDS ones included.
 __device__ __forceinline__ int scalar_table_load(const int32_t* table, int index) {
