@@ -88,6 +88,12 @@ struct Divider {
         finite = (__float_as_uint(scale) & 0x7F800000u) != 0x7F800000u;
         r = 1.0f / scale;
     }
+    // the reciprocal is known
+    __device__ __forceinline__ Divider(float scale, float reciprocal) {
+        s = scale;
+        finite = (__float_as_uint(scale) & 0x7F800000u) != 0x7F800000u;
+        r = reciprocal;
+    }
     // The correctly rounded quotient x / s for finite x when `finite`, for the callers of this library: s is the
     // amax / 448 (amax floored at 1e-12) of a set that x belongs to, so |x / s| <= 448 * (1 + 2^-22) - the quotient
     // of the largest element is 448 or the fp32 value next to it - which is below 464 and which the conversion to
@@ -204,6 +210,16 @@ __device__ __forceinline__ uint2 cast8(const uint4& v, const Divider& d) {
         }
     }
     return make_uint2(o[0], o[1]);
+}
+
+// four bf16 (two packed words, element order preserved) -> four fp8 bytes
+__device__ __forceinline__ u32 cast4(u32 w0, u32 w1, const Divider& d) {
+    if (d.finite) {
+        const u32 lo = cvt2<false>(d.fast(bf16_lo(w0)), d.fast(bf16_hi(w0)), 0u);
+        return cvt2<true>(d.fast(bf16_lo(w1)), d.fast(bf16_hi(w1)), lo);
+    }
+    return slow_byte(bf16_lo(w0), d.s) | (slow_byte(bf16_hi(w0), d.s) << 8) | (slow_byte(bf16_lo(w1), d.s) << 16) |
+           (slow_byte(bf16_hi(w1), d.s) << 24);
 }
 
 // cast8 for a scale that need not come from the data's own maximum: the quotient saturates at +-448 before the

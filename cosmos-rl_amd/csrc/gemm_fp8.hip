@@ -48,29 +48,6 @@ __device__ __forceinline__ i32x8 lds_frag(const uint8_t* tile, int row, int quar
     return r;
 }
 
-// Workgroup id -> (tile_m, tile_n).  Consecutive workgroup ids are dealt round
-// robin to the 8 XCDs, each with its own L2: give every XCD one contiguous range
-// of tiles, and walk a range in bands of GM tile-rows so that co-resident
-// workgroups share activation rows and weight rows in that L2.
-// GM: tile-rows per band.  8 for the dense problems; the grouped kernels take kGroupedBandRows = 4, about the
-// tile-rows of one expert at the MoE shapes served here (an expert's weight tile is then shared by the
-// workgroups of one band: FETCH_SIZE of the K = 768 down projection of 128 experts falls from 1.34 to 1.10
-// times its operand bytes, run time unchanged).
-constexpr int kGroupedBandRows = 4;
-template <int GM = 8>
-__device__ __forceinline__ void tile_of_block(int pid, int tiles_m, int tiles_n, int& tm, int& tn) {
-    const int total = tiles_m * tiles_n;
-    const int xcd = pid & 7, local = pid >> 3;
-    const int base = total >> 3, rem = total & 7;
-    const int lin = xcd * base + (xcd < rem ? xcd : rem) + local;
-    const int band = GM * tiles_n;
-    const int g = lin / band, first = g * GM;
-    const int gsz = (tiles_m - first) < GM ? (tiles_m - first) : GM;
-    const int in = lin - g * band;
-    tm = first + in % gsz;
-    tn = in / gsz;
-}
-
 // KTAIL (rowwise only): K is a multiple of 16 but not of 128.  The last K step then ends inside its 128 bytes: lanes
 // whose 16-byte chunk lies past K fetch chunk 0 of their row instead (nothing is read outside a row) and store zeros
 // to LDS, for both operands, so the step's products are those of the K that exists.
@@ -1160,16 +1137,6 @@ __device__ __forceinline__ u32 quarters_max(u32 v) {  // max over the four lanes
     const u32x2s b = __builtin_amdgcn_permlane16_swap(v, v, false, false);
     return umax(b[0], b[1]);
 }
-// four bf16 (two packed words, element order preserved) -> four fp8 bytes
-__device__ __forceinline__ u32 cast4(u32 w0, u32 w1, const Divider& d) {
-    if (d.finite) {
-        const u32 lo = cvt2<false>(d.fast(bf16_lo(w0)), d.fast(bf16_hi(w0)), 0u);
-        return cvt2<true>(d.fast(bf16_lo(w1)), d.fast(bf16_hi(w1)), lo);
-    }
-    return slow_byte(bf16_lo(w0), d.s) | (slow_byte(bf16_hi(w0), d.s) << 8) | (slow_byte(bf16_lo(w1), d.s) << 16) |
-           (slow_byte(bf16_hi(w1), d.s) << 24);
-}
-
 // acc: [weight tile][token tile] of the wave's 64 x 64 block; row_keep[j]: the wave's token row j * 16 + lrow belongs to
 // the tile's expert; rq / rh: buffer descriptors of the tile's first row of the fp8 output and of its scales
 __device__ __forceinline__ void swiglu_quant_epilogue(const f32x4 (&acc)[4][4], uint8_t* xch, int wm, int wn, int lrow, int quarter,

@@ -3,11 +3,12 @@
 //
 // Three forms, by the mean number of rows an expert gets:
 //
-//   many rows   Every expert's rows are padded to tiles of 128 (experts without a row get none), the tokens quantised into
-//               that layout (cfp8_scatter_quant_group128) and multiplied by the grouped GEMMs of the training path.  A
-//               group's rows of padding are zeros all the way: a walking GEMM carries a row's last products into the first
-//               step of its next tile with a scale of zero, so what multiplies there must be finite.  Rows past the last
-//               group are not touched.
+//   many rows   Every expert's rows are padded to tiles of 128 (experts without a row get none).  The tokens are quantised
+//               where they lie and gemm_gate_up_kernel gathers its rows from them; hidden sizes that it does not take are
+//               quantised into the padded layout (cfp8_scatter_quant_group128) for the grouped GEMM of the training path.
+//               Rows of padding are zeros all the way: a walking GEMM carries a row's last products into the first step of
+//               its next tile with a scale of zero, so what multiplies there must be finite.  Rows past the last group are
+//               not touched.
 //   middle      A chunk of prefill: all experts' weights are read, for less than a tile of 128 rows each.  Rows lie one
 //               behind the other without padding; the ring kernel takes tiles of 64 of one expert's rows (gemm_ring.hip:
 //               kRingGateUp reads them from the quantised tokens and ends in SwiGLU, kRingDown), two workgroups a CU.  The
@@ -249,6 +250,7 @@ struct ExpertsPlan {
     Form form;
     int64_t rows;   // rows of the expert-grouped layout (their bound)
     int64_t slots;  // experts that can have a row
+    bool gathers;   // many rows: the gate_up product reads its rows from the quantised tokens
     size_t row_tokens, row_experts, row_map, weights, m_sizes, m_offsets, route, xq, xs, h, hq, hs, out, bytes;
 };
 
@@ -274,7 +276,8 @@ static ExpertsPlan experts_plan(int64_t tokens, int topk, int experts, int64_t h
     p.m_sizes = take((size_t)experts * 4);
     p.m_offsets = take((size_t)experts * 4);
     p.route = take(cfp8_route_tokens_workspace_bytes(tokens, topk, experts));
-    const size_t xrows = (size_t)(many ? p.rows : tokens);
+    p.gathers = many && gate_up_takes(tokens, hidden, inter);
+    const size_t xrows = (size_t)(many && !p.gathers ? p.rows : tokens);
     p.xq = take(xrows * (size_t)hidden);
     p.xs = take(xrows * (size_t)(hidden / 128) * 4);
     p.h = take(many ? 0 : (size_t)p.rows * (size_t)inter * 2);
@@ -356,13 +359,23 @@ extern "C" int cfp8_moe_experts(const void* x, int64_t ld_x, int64_t tokens, int
         launch_few_down<(int)(kFewMaxInter / 128)>((int)(inter / 128), dim3((unsigned)(hidden / 128), (unsigned)p.slots), st, f);
         if (int rc = check_launch("moe_experts")) return rc;
     } else {
-        if (int rc = cfp8_scatter_quant_group128(x, ld_x, tokens, hidden, i32(p.row_map), topk, i32(p.row_tokens), p.rows, ws + p.xq, hidden, f32(p.xs), stream))
-            return rc;
         // (p.rows is a bound: 639 tiles of rows for 8192 tokens, top 8 of 128 experts, of which some 566 hold rows)
         const int32_t* const rows_end = i32(p.m_offsets) + experts - 1;
-        if (int rc = grouped_swiglu_quant(ws + p.xq, hidden, f32(p.xs), gate_up, gate_up_scales, i32(p.row_experts), rows_end, ws + p.hq, inter,
-                                          f32(p.hs), p.rows, inter, hidden, experts, stream))
-            return rc;
+        if (p.gathers) {
+            if (int rc = cfp8_quant_group128(x, tokens, hidden, ld_x, ws + p.xq, hidden, f32(p.xs), CFP8_GROUP_MODE_DIV, stream)) return rc;
+            GateUpArgs g{};
+            g.x = ws + p.xq; g.xs = f32(p.xs); g.w = static_cast<const uint8_t*>(gate_up); g.ws = gate_up_scales;
+            g.row_tokens = i32(p.row_tokens); g.row_experts = i32(p.row_experts); g.rows_end = rows_end;
+            g.h = ws + p.hq; g.hs = f32(p.hs);
+            g.tokens = (int)tokens; g.N = (int)(2 * inter); g.K = (int)hidden;
+            if (int rc = launch_gate_up(g, p.rows, st)) return rc;
+        } else {
+            if (int rc = cfp8_scatter_quant_group128(x, ld_x, tokens, hidden, i32(p.row_map), topk, i32(p.row_tokens), p.rows, ws + p.xq, hidden, f32(p.xs), stream))
+                return rc;
+            if (int rc = grouped_swiglu_quant(ws + p.xq, hidden, f32(p.xs), gate_up, gate_up_scales, i32(p.row_experts), rows_end, ws + p.hq, inter,
+                                              f32(p.hs), p.rows, inter, hidden, experts, stream))
+                return rc;
+        }
         if (int rc = grouped_block128(ws + p.hq, inter, f32(p.hs), down, down_scales, i32(p.row_experts), rows_end, ws + p.out, hidden, CFP8_OUT_BF16,
                                       p.rows, hidden, inter, experts, stream))
             return rc;
