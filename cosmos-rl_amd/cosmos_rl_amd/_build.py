@@ -18,7 +18,7 @@ LIB_DIR = PKG_DIR / "lib"
 LIB_PATH = LIB_DIR / "libcosmosfp8.so"
 OBJ_DIR = CSRC_DIR / "build"
 
-SOURCES = ["api.hip", "quant_rowwise.hip", "quant_tensorwise.hip", "quant_block.hip", "gemm_fp8.hip", "gemm_grouped_xres.hip", "gemm_gate_up.hip", "moe_indices.hip", "moe_route.hip", "moe_experts.hip",
+SOURCES = ["api.hip", "quant_rowwise.hip", "quant_tensorwise.hip", "quant_block.hip", "gemm_fp8.hip", "gemm_grouped_xres.hip", "gemm_experts.hip", "moe_indices.hip", "moe_route.hip", "moe_experts.hip",
            "quant_mxfp4.hip", "gemm_mxfp4.hip", "gemm_ring.hip"]
 
 # Per-file flags.  gemm_grouped_xres.hip: matrix instructions write ordinary vector registers (see the file's header).

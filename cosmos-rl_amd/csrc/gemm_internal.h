@@ -54,21 +54,24 @@ int grouped_swiglu_quant(const void* a, int64_t ld_a, const float* sa, const voi
                          void* q, int64_t ld_q, float* scales, int64_t M, int64_t I, int64_t K, int64_t E, void* stream);
 size_t block_partial_bytes(int64_t M, int64_t N, int64_t K);                      // of the block-scaled product's slices of K
 
-// ---- gemm_gate_up.hip
-struct GateUpArgs {
-    const uint8_t* x;            // [tokens, K] fp8
-    const float* xs;             // [tokens, K / 128]
-    const uint8_t* w;            // [experts, N, K], gate and up rows in turn, 16 at a time
+// ---- gemm_experts.hip
+struct ExpertsArgs {
+    const uint8_t* x;            // fp8: gate_up the tokens [tokens, K], down the rows [rows, K]
+    const float* xs;             // [tokens or rows, K / 128]
+    const uint8_t* w;            // [experts, N, K], gate_up: gate and up rows in turn, 16 at a time
     const float* ws;             // [experts, N / 128, K / 128]
-    const int32_t* row_tokens;   // [rows], negative: a row of padding
+    const int32_t* row_tokens;   // gate_up: [rows], negative: a row of padding
     const int32_t* row_experts;  // [rows]
     const int32_t* rows_end;     // rows that the groups take
-    uint8_t* h;                  // [rows, N / 2] fp8
-    float* hs;                   // [rows, N / 256]
+    uint8_t* h;                  // gate_up: [rows, N / 2] fp8
+    float* hs;                   // gate_up: [rows, N / 256]
+    uint16_t* out;               // down: [rows, N] bf16
     int tokens, N, K, tiles_m, tiles_n;
 };
-bool gate_up_takes(int64_t tokens, int64_t hidden, int64_t inter);
-int launch_gate_up(GateUpArgs& p, int64_t rows, hipStream_t st);
+bool experts_gate_up_takes(int64_t tokens, int64_t hidden, int64_t inter);
+bool experts_down_takes(int64_t hidden, int64_t inter);
+int launch_experts_gate_up(ExpertsArgs& p, int64_t rows, hipStream_t st);
+int launch_experts_down(ExpertsArgs& p, int64_t rows, hipStream_t st);
 
 // ---- units of the kernels in which a workgroup walks rows of tiles ----------
 // The schedule for tiles_m tile rows of tiles_n tiles on `cus` workgroups: one workgroup per CU.  Tile rows beyond the

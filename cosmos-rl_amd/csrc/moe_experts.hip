@@ -4,7 +4,7 @@
 // Three forms, by the mean number of rows an expert gets:
 //
 //   many rows   Every expert's rows are padded to tiles of 128 (experts without a row get none).  The tokens are quantised
-//               where they lie and gemm_gate_up_kernel gathers its rows from them; hidden sizes that it does not take are
+//               where they lie and gemm_experts_kernel gathers its rows from them; hidden sizes that it does not take are
 //               quantised into the padded layout (cfp8_scatter_quant_group128) for the grouped GEMM of the training path.
 //               Rows of padding are zeros all the way: a walking GEMM carries a row's last products into the first step of
 //               its next tile with a scale of zero, so what multiplies there must be finite.  Rows past the last group are
@@ -276,7 +276,7 @@ static ExpertsPlan experts_plan(int64_t tokens, int topk, int experts, int64_t h
     p.m_sizes = take((size_t)experts * 4);
     p.m_offsets = take((size_t)experts * 4);
     p.route = take(cfp8_route_tokens_workspace_bytes(tokens, topk, experts));
-    p.gathers = many && gate_up_takes(tokens, hidden, inter);
+    p.gathers = many && experts_gate_up_takes(tokens, hidden, inter);
     const size_t xrows = (size_t)(many && !p.gathers ? p.rows : tokens);
     p.xq = take(xrows * (size_t)hidden);
     p.xs = take(xrows * (size_t)(hidden / 128) * 4);
@@ -363,12 +363,12 @@ extern "C" int cfp8_moe_experts(const void* x, int64_t ld_x, int64_t tokens, int
         const int32_t* const rows_end = i32(p.m_offsets) + experts - 1;
         if (p.gathers) {
             if (int rc = cfp8_quant_group128(x, tokens, hidden, ld_x, ws + p.xq, hidden, f32(p.xs), CFP8_GROUP_MODE_DIV, stream)) return rc;
-            GateUpArgs g{};
+            ExpertsArgs g{};
             g.x = ws + p.xq; g.xs = f32(p.xs); g.w = static_cast<const uint8_t*>(gate_up); g.ws = gate_up_scales;
             g.row_tokens = i32(p.row_tokens); g.row_experts = i32(p.row_experts); g.rows_end = rows_end;
             g.h = ws + p.hq; g.hs = f32(p.hs);
             g.tokens = (int)tokens; g.N = (int)(2 * inter); g.K = (int)hidden;
-            if (int rc = launch_gate_up(g, p.rows, st)) return rc;
+            if (int rc = launch_experts_gate_up(g, p.rows, st)) return rc;
         } else {
             if (int rc = cfp8_scatter_quant_group128(x, ld_x, tokens, hidden, i32(p.row_map), topk, i32(p.row_tokens), p.rows, ws + p.xq, hidden, f32(p.xs), stream))
                 return rc;
@@ -376,9 +376,17 @@ extern "C" int cfp8_moe_experts(const void* x, int64_t ld_x, int64_t tokens, int
                                               f32(p.hs), p.rows, inter, hidden, experts, stream))
                 return rc;
         }
-        if (int rc = grouped_block128(ws + p.hq, inter, f32(p.hs), down, down_scales, i32(p.row_experts), rows_end, ws + p.out, hidden, CFP8_OUT_BF16,
-                                      p.rows, hidden, inter, experts, stream))
-            return rc;
+        if (experts_down_takes(hidden, inter)) {
+            ExpertsArgs d{};
+            d.x = ws + p.hq; d.xs = f32(p.hs); d.w = static_cast<const uint8_t*>(down); d.ws = down_scales;
+            d.row_experts = i32(p.row_experts); d.rows_end = rows_end; d.out = reinterpret_cast<uint16_t*>(ws + p.out);
+            d.N = (int)hidden; d.K = (int)inter;
+            if (int rc = launch_experts_down(d, p.rows, st)) return rc;
+        } else {
+            if (int rc = grouped_block128(ws + p.hq, inter, f32(p.hs), down, down_scales, i32(p.row_experts), rows_end, ws + p.out, hidden, CFP8_OUT_BF16,
+                                          p.rows, hidden, inter, experts, stream))
+                return rc;
+        }
     }
     return cfp8_combine_rows(ws + p.out, hidden, p.rows, i32(p.row_map), ws + p.weights, CFP8_IN_BF16, tokens, topk, hidden,
                              CFP8_COMBINE_BF16_STEPS, y, ld_y, stream);
