@@ -1,6 +1,8 @@
-// The gate_up product of a MoE layer's experts with many rows, from the quantised tokens to the quantised hidden activation:
+// The two products of a MoE layer's experts with many rows:
 //
-//   h[r, c] = bf16(bf16(silu(gate)) * up) of row r's token and expert, requantised 1x128
+//   gate_up  from the quantised tokens to the quantised hidden activation: h[r, c] = bf16(bf16(silu(gate)) * up) of row r's token
+//            and expert, requantised 1x128
+//   down     from that to bf16 rows
 //
 // Rows lie expert by expert, every group padded to 128 of them (row_tokens < 0: padding, whose operands arrive as zeros); the
 // weight's gate and up rows alternate in units of 16 (one MFMA tile), so that a 128 x 256 tile holds both halves of one 1x128 group
@@ -25,6 +27,10 @@
 // choices by scalar selects: the last three steps, which load the next tile, are code of their own; no detour of the scales
 // through registers), and MFMAs follow the barrier at once, since no product waits for an addition to free its registers.
 // Gathering the rows saves the padded copy of the tokens: 28 us of 38 for a quantiser that writes each token eight times.
+// The down product (165 us, 268 MB written) is bound by its stores among the loads: 119 us without the stores, 113 without the loads, 105
+// without either; neither their cache policy, nor tiles that are contiguous in memory, nor stores behind the next loads change that.
+//
+// A wave whose 64 rows are all padding only loads and keeps the barriers (48 rows an expert: 178 -> 167 us a call).
 #include <atomic>
 #include <type_traits>
 
@@ -57,7 +63,8 @@ __device__ __forceinline__ void quarters_transpose(u32 (&v)[4]) {
     }
 }
 
-template <bool DOWN>
+// ONCE: the weights are loaded as a stream
+template <bool DOWN, bool ONCE>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void gemm_experts_kernel(const ExpertsArgs p) {
     constexpr int XS = kExXS, STAGE = kExStage;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -69,7 +76,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
     if (pid >= ntiles) return;
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int wm = wave & 1, wn = wave >> 1;
+    const int wm = wave >> 2, wn = wave & 3;  // (a SIMD has a wave of either half of the rows)
     const int lrow = lane & 15, quarter = lane >> 4;
     const int KT = p.K >> 7;
     __builtin_assume(KT >= 4 && KT <= 32);
@@ -94,12 +101,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
         vx[i] = token >= 0 ? (uint32_t)token * (uint32_t)p.K + chunk : kExOutside;
         vxs[i] = token >= 0 ? (uint32_t)(token * KT + (lane & 7)) * 4u : kExOutside;
     };
-    auto place = [&](int id, int& m0, int& n0, __amdgpu_buffer_rsrc_t& rw, int& expert) {
+    // `idle`: this wave's 64 rows are all padding (a group's padding follows its rows)
+    auto place = [&](int id, int& m0, int& n0, __amdgpu_buffer_rsrc_t& rw, int& expert, bool& idle) {
         int tm, tn;
         tile_of_block<kGroupedBandRows>(id, tiles_m, p.tiles_n, tm, tn);
         m0 = tm * kExBM;
         n0 = tn * kExBN;
-        expert = scalar_table_load(p.row_experts, m0);  // (a group's rows begin on a multiple of 128)
+        const int32_t *const at = p.row_experts + m0, *const half = p.row_tokens + m0 + 64;  // (a group's rows begin on a multiple of 128)
+        int token;
+        asm volatile("s_load_dword %0, %2, 0x0\n\ts_load_dword %1, %3, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=&s"(expert), "=&s"(token) : "s"(at), "s"(half) : "memory");
+        idle = wm == 1 && token < 0;
         // (down: weight rows beyond N, where N is an odd multiple of 128, arrive as zeros)
         rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.w) + ((int64_t)expert * p.N + n0) * p.K, 0,
                                                (p.N - n0 < kExBN ? p.N - n0 : kExBN) * p.K, 0x00020000);
@@ -108,7 +119,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
         __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)(smem + stage + (wave + 8 * i) * 1024), 16, vx[i], (uint32_t)kt << 7, 0, 0);
     };
     auto dma_w = [&](__amdgpu_buffer_rsrc_t r, int kt, int stage, int i) {
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)(smem + stage + XS + (wave + 8 * i) * 1024), 16, vw[i], (uint32_t)kt << 7, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)(smem + stage + XS + (wave + 8 * i) * 1024), 16, vw[i], (uint32_t)kt << 7, 0, ONCE ? 2 : 0);
     };
     auto dma_scales = [&](__amdgpu_buffer_rsrc_t r, int group, int buf) {  // (steps beyond K: the next token's, never used)
 #pragma unroll
@@ -143,8 +154,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
     };
 
     int m0, n0, expert;
+    bool idle;
     __amdgpu_buffer_rsrc_t rw;
-    place(pid, m0, n0, rw, expert);
+    place(pid, m0, n0, rw, expert, idle);
     __amdgpu_buffer_rsrc_t rx = x_rsrc(m0), rxs = xs_rsrc(m0);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -161,12 +173,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
         for (int i = 0; i < 4; ++i) dma_w(rw, k, k * STAGE, i);
     }
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-#pragma unroll
-    for (int i = 0; i < 4; ++i) W[i] = frag(w_at, i);
-    X[0] = frag(x_at, 0);
-    X[1] = frag(x_at, 1);
-    read_scales(0, 0, 0);
-    CFP8_PHASE_END();
 
     f32x4 acc[4][4], P[4][4];  // [w tile][x tile]
     float sc2[2], sc3[2];      // scales of x tiles 2 and 3 (gate, up) that go with the products waiting in P
@@ -188,10 +194,56 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
         const int pid_n = pid + (int)gridDim.x;
         const bool has_next = pid_n < ntiles;
         int m0n, n0n, expert_n;
+        bool idle_n;
         __amdgpu_buffer_rsrc_t rwn;
-        place(has_next ? pid_n : pid, m0n, n0n, rwn, expert_n);  // (no next tile: this one's first steps are fetched once more)
+        place(has_next ? pid_n : pid, m0n, n0n, rwn, expert_n, idle_n);  // (no next tile: this one's first steps are fetched once more)
         const __amdgpu_buffer_rsrc_t rxn = x_rsrc(m0n), rxsn = xs_rsrc(m0n);
 
+        // what a step loads beside its tile, in front of it: the next barrier waits for it
+        auto beside = [&](int kt, auto first_c, auto left_c) {
+            constexpr bool first = decltype(first_c)::value;
+            constexpr int left = decltype(left_c)::value;
+            if constexpr (first && !DOWN) {
+                if (wave < 2) {
+                    const __amdgpu_buffer_rsrc_t rt = __builtin_amdgcn_make_buffer_rsrc(const_cast<int32_t*>(p.row_tokens) + m0n + wave * 64, 0, 256, 0x00020000);
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rt, (lds_void*)(smem + kExTokens + wave * 256), 4, (uint32_t)lane * 4u, 0, 0, 0);
+                }
+            } else if constexpr (left == 3) {
+                if ((kt & 7) == 4 && kt < 8 * (G - 1)) dma_scales(rxs, (kt >> 3) + 1, buffer_of((kt >> 3) + 1));
+            } else if constexpr (left == 2) {
+                if constexpr (!DOWN) {
+                    const int32_t* const tok = reinterpret_cast<const int32_t*>(smem + kExTokens) + wave * 8 + (lane >> 3);
+                    set_rows(0, tok[0]);
+                    set_rows(1, tok[64]);
+                }
+                dma_scales(rxsn, 0, buffer_of(G));
+                if (wave == 0) dma_weight_scales(expert_n, n0n, par ^ 1);
+            }
+        };
+        // tile kt + 1 has landed when at most the six loads of the step before are outstanding, and the stores of the tile before:
+        // gate_up three behind the loads of its last step, down eight in front of those of this tile's third
+        auto wait = [&](auto first_c) {
+            if constexpr (decltype(first_c)::value && DOWN) CFP8_WAIT_BARRIER(14);
+            else if constexpr (decltype(first_c)::value) CFP8_WAIT_BARRIER(9);
+            else CFP8_WAIT_BARRIER(6);
+        };
+        // a step of a wave without rows: it loads as the others do
+        auto step_idle = [&](int kt, auto first_c, auto left_c) {
+            constexpr int left = decltype(left_c)::value;
+            const int kl = left == 3 ? kt + 3 : 2 - left;
+            wait(first_c);
+            CFP8_PHASE_END();
+            beside(kt, first_c, left_c);
+            CFP8_PHASE_END();
+            if constexpr (!DOWN || left > 0) {
+                dma_x(left == 3 ? rx : rxn, kl, stage, 0);
+                dma_x(left == 3 ? rx : rxn, kl, stage, 1);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) dma_w(left == 3 ? rw : rwn, kl, stage, i);
+            }
+            CFP8_PHASE_END();
+            stage = stage == 2 * STAGE ? 0 : stage + STAGE;
+        };
         // LEFT: K steps behind this one, 3 for all but the last three
         auto step = [&](int kt, auto first_c, auto left_c) {
             constexpr bool first = decltype(first_c)::value;
@@ -216,11 +268,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
                 if (!first) add(i, 3, sc3[i & 1], false);
                 CFP8_PHASE_END();
             }
-            // tile kt + 1 has landed when at most the six loads of the step before are outstanding, and the stores of the tile before:
-            // gate_up three behind the loads of its last step, down eight in front of those of this tile's third
-            if constexpr (first && DOWN) CFP8_WAIT_BARRIER(14);
-            else if constexpr (first) CFP8_WAIT_BARRIER(9);
-            else CFP8_WAIT_BARRIER(6);
+            wait(first_c);
             CFP8_PHASE_END();
             CFP8_PRODUCT(0, 2);
             CFP8_PRODUCT(0, 3);
@@ -234,26 +282,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
                 sc2[u] = sm[2] * s;
                 sc3[u] = sm[3] * s;
             }
-            // what this step loads beside its tile comes first: the next barrier waits for it
-            if constexpr (first && !DOWN) {
-                if (wave < 2) {
-                    const __amdgpu_buffer_rsrc_t rt = __builtin_amdgcn_make_buffer_rsrc(const_cast<int32_t*>(p.row_tokens) + m0n + wave * 64, 0, 256, 0x00020000);
-                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rt, (lds_void*)(smem + kExTokens + wave * 256), 4, (uint32_t)lane * 4u, 0, 0, 0);
-                }
-            } else if constexpr (left == 3) {
-                if ((kt & 7) == 4 && kt < 8 * (G - 1)) dma_scales(rxs, (kt >> 3) + 1, buffer_of((kt >> 3) + 1));
-            } else if constexpr (left == 2) {
-                if constexpr (!DOWN) {
-                    const int32_t* const tok = reinterpret_cast<const int32_t*>(smem + kExTokens) + wave * 8 + (lane >> 3);
-                    set_rows(0, tok[0]);
-                    set_rows(1, tok[64]);
-                }
-                dma_scales(rxsn, 0, buffer_of(G));
-                if (wave == 0) dma_weight_scales(expert_n, n0n, par ^ 1);
-            }
+            beside(kt, first_c, left_c);
             CFP8_PHASE_END();
-            W[0] = frag(wn_, 0);
-            X[0] = frag(xn, 0);
+            if (left > 0) {
+                W[0] = frag(wn_, 0);
+                X[0] = frag(xn, 0);
+            }
             if (loads) dma_x(ra, kl, stage, 0);
             CFP8_PHASE_END();
 #pragma unroll
@@ -263,12 +297,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
                 if (i < 3) CFP8_PRODUCT(i + 1, 3);
                 add(i, 1, sc1[i & 1], first);
                 CFP8_PHASE_END();
-                if (i < 3) W[i + 1] = frag(wn_, i + 1);
+                if (i < 3 && left > 0) W[i + 1] = frag(wn_, i + 1);
                 if (i == 0) {
-                    X[1] = frag(xn, 1);
+                    if (left > 0) X[1] = frag(xn, 1);
                     if (loads) dma_x(ra, kl, stage, 1);
                 }
-                if (i == 1) read_scales(left == 0 ? buffer_of(G) : buffer_of((kt + 1) >> 3), left == 0 ? par ^ 1 : par, left == 0 ? 0 : kt + 1);
+                if (i == 1 && left > 0) read_scales(buffer_of((kt + 1) >> 3), par, kt + 1);
                 if (loads) dma_w(r, kl, stage, i);
                 CFP8_PHASE_END();
             }
@@ -276,18 +310,38 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
         };
         using yes = std::integral_constant<bool, true>;
         using no = std::integral_constant<bool, false>;
-        step(0, yes{}, std::integral_constant<int, 3>{});
-        // x tiles 2 and 3 of a tile's first step are added in its second
+        auto tile = [&](auto& one) {
+            one(0, yes{}, std::integral_constant<int, 3>{});
+            for (int kt = 1; kt < KT - 3; ++kt) one(kt, no{}, std::integral_constant<int, 3>{});
+            one(KT - 3, no{}, std::integral_constant<int, 2>{});
+            one(KT - 2, no{}, std::integral_constant<int, 1>{});
+            one(KT - 1, no{}, std::integral_constant<int, 0>{});
+        };
+        if (idle) {
+            tile(step_idle);
+            // (or the accumulators of the tile before would have to be kept for the way past this branch)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc[i][2] = acc[i][3] = f32x4{0.f, 0.f, 0.f, 0.f};
-        for (int kt = 1; kt < KT - 3; ++kt) step(kt, no{}, std::integral_constant<int, 3>{});
-        step(KT - 3, no{}, std::integral_constant<int, 2>{});
-        step(KT - 2, no{}, std::integral_constant<int, 1>{});
-        step(KT - 1, no{}, std::integral_constant<int, 0>{});
+            for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            add(i, 2, sc2[i & 1], false);
-            add(i, 3, sc3[i & 1], false);
+                for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        } else {
+            // the first fragments landed before the last barrier of the tile before (read there already, they would have to live through its
+            // epilogue and through tiles without rows)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) W[i] = frag(w_at + stage, i);
+            X[0] = frag(x_at + stage, 0);
+            X[1] = frag(x_at + stage, 1);
+            read_scales(buffer_of(0), par, 0);
+            CFP8_PHASE_END();
+            // x tiles 2 and 3 of a tile's first step are added in its second
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[i][2] = acc[i][3] = f32x4{0.f, 0.f, 0.f, 0.f};
+            tile(step);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                add(i, 2, sc2[i & 1], false);
+                add(i, 3, sc3[i & 1], false);
+            }
         }
 
         if constexpr (DOWN) {
@@ -302,12 +356,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
             uint8_t* const own = smem + prev + wave * 1024;
             const uint32_t turn = (uint32_t) reinterpret_cast<uintptr_t>((lds_void*)(own + (lr >> 3) * 8192 + (lr & 7) * 128 + (lq & 1) * 8));
             const uint8_t* const back = own + (le >> 3) * 128 + (((le & 7) ^ (le >> 3)) << 4);
-            const uint32_t at = n0 + wn * 64 < p.N ? (uint32_t)((le >> 3) * p.N + n0 + wn * 64 + (le & 7) * 8) * 2u : kExOutside;
+            const uint32_t at = n0 + wn * 64 < p.N && !idle ? (uint32_t)((le >> 3) * p.N + n0 + wn * 64 + (le & 7) * 8) * 2u : kExOutside;
             // (LDS is written by instructions written out: in front of a store it knows of, the compiler waits for every load in flight)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
+                for (int i = 0; i < 4 && !idle; ++i) {
                     const f32x4 v = acc[i][j];
                     const uint64_t two = (uint64_t)pack_bf16x2(v[0], v[1]) | ((uint64_t)pack_bf16x2(v[2], v[3]) << 32);
                     asm volatile("ds_write_b64 %0, %1 offset:%2" ::"v"(turn + (uint32_t)(((2 * i + (lq >> 1)) ^ (lr & 7)) << 4)), "v"(two), "n"((j & 1) * 16384) : "memory");
@@ -330,49 +384,58 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
             // has both values of an element; both are rounded to bf16 first, as the product would be in memory.  A wave has 32 of the
             // 128 columns of the group: the four that share rows exchange their maxima.  Behind that a lane looks after one row (x tile
             // `quarter`, row lrow): its scale, and the 16 bytes of it that the four quarters hold a word of each.
-            u32 h[2][4][2], mx[4];  // [pair][x tile][two words of two bf16]
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                u32 m = 0;
-#pragma unroll
-                for (int pp = 0; pp < 2; ++pp) {
-                    const f32x4 g = acc[2 * pp][j], u = acc[2 * pp + 1][j];
-                    swiglu_quad(pack_bf16x2(g[0], g[1]), pack_bf16x2(g[2], g[3]), pack_bf16x2(u[0], u[1]), pack_bf16x2(u[2], u[3]), h[pp][j][0], h[pp][j][1]);
-                    m = pk_absmax(pk_absmax(m, h[pp][j][0]), h[pp][j][1]);
-                }
-                mx[j] = pk_fold(m);
-            }
-            quarters_transpose(mx);  // the four quarters' maxima of row lrow of x tile `quarter`
-            const u32 mine = umax(umax(mx[0], mx[1]), umax(mx[2], mx[3]));
+            // A wave without rows stores zeros and their scale.
+            u32 h[2][4][2];  // [pair][x tile][two words of two bf16]
             int le = lane;  // (addresses derived here: kept across the K loop they would cost registers)
             asm volatile("" : "+v"(le));
             const int row = wm * 64 + le;  // x tile `quarter`, row lrow
             const uint32_t xch = (uint32_t) reinterpret_cast<uintptr_t>((lds_void*)(smem + kExExchange + row * 16));
-            // (LDS by instructions written out: in front of a store it knows of, the compiler waits for every load in flight)
-            asm volatile("ds_write_b32 %0, %1" ::"v"(xch + wn * 4), "v"(mine) : "memory");
-            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            u32x4 all;
-            asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(all) : "v"(xch) : "memory");
-            const float scale = scale_from_amax(amax_from_bits(umax(umax(all[0], all[1]), umax(all[2], all[3]))));
-            const Divider own(scale);
-            u32 s4[4], r4[4];
+            if (!idle) {
+                u32 mx[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                s4[j] = __float_as_uint(own.s);
-                r4[j] = __float_as_uint(own.r);
+                for (int j = 0; j < 4; ++j) {
+                    u32 m = 0;
+#pragma unroll
+                    for (int pp = 0; pp < 2; ++pp) {
+                        const f32x4 g = acc[2 * pp][j], u = acc[2 * pp + 1][j];
+                        swiglu_quad(pack_bf16x2(g[0], g[1]), pack_bf16x2(g[2], g[3]), pack_bf16x2(u[0], u[1]), pack_bf16x2(u[2], u[3]), h[pp][j][0], h[pp][j][1]);
+                        m = pk_absmax(pk_absmax(m, h[pp][j][0]), h[pp][j][1]);
+                    }
+                    mx[j] = pk_fold(m);
+                }
+                quarters_transpose(mx);  // the four quarters' maxima of row lrow of x tile `quarter`
+                // (LDS by instructions written out: in front of a store it knows of, the compiler waits for every load in flight)
+                asm volatile("ds_write_b32 %0, %1" ::"v"(xch + wn * 4), "v"(umax(umax(mx[0], mx[1]), umax(mx[2], mx[3]))) : "memory");
             }
-            quarters_transpose(s4);  // those of row lrow of x tile j
-            quarters_transpose(r4);
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            u32x4 bytes[2] = {u32x4{0u, 0u, 0u, 0u}, u32x4{0u, 0u, 0u, 0u}};
+            float scale = scale_from_amax(0.f);
+            if (!idle) {
+                u32x4 all;
+                asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(all) : "v"(xch) : "memory");
+                scale = scale_from_amax(amax_from_bits(umax(umax(all[0], all[1]), umax(all[2], all[3]))));
+                const Divider own(scale);
+                u32 s4[4], r4[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    s4[j] = __float_as_uint(own.s);
+                    r4[j] = __float_as_uint(own.r);
+                }
+                quarters_transpose(s4);  // those of row lrow of x tile j
+                quarters_transpose(r4);
+#pragma unroll
+                for (int pp = 0; pp < 2; ++pp) {
+                    u32 q[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) q[j] = cast4(h[pp][j][0], h[pp][j][1], Divider(__uint_as_float(s4[j]), __uint_as_float(r4[j])));
+                    quarters_transpose(q);
+                    bytes[pp] = u32x4{q[0], q[1], q[2], q[3]};
+                }
+            }
             const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(p.h + (int64_t)m0 * (p.N >> 1), 0, 0x80000000u, 0x00020000);
             const __amdgpu_buffer_rsrc_t rh = __builtin_amdgcn_make_buffer_rsrc(p.hs + (int64_t)m0 * (p.N >> 8), 0, 0x80000000u, 0x00020000);
 #pragma unroll
-            for (int pp = 0; pp < 2; ++pp) {
-                u32 q[4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) q[j] = cast4(h[pp][j][0], h[pp][j][1], Divider(__uint_as_float(s4[j]), __uint_as_float(r4[j])));
-                quarters_transpose(q);
-                buffer_store16(u32x4{q[0], q[1], q[2], q[3]}, rq, (uint32_t)(row * (p.N >> 1)), (uint32_t)((n0 >> 1) + wn * 32 + pp * 16));
-            }
+            for (int pp = 0; pp < 2; ++pp) buffer_store16(bytes[pp], rq, (uint32_t)(row * (p.N >> 1)), (uint32_t)((n0 >> 1) + wn * 32 + pp * 16));
             __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(scale), rh, wn == 0 ? (uint32_t)(row * (p.N >> 8) * 4) : kExOutside, (uint32_t)((n0 >> 8) * 4), 0);
         }
 
@@ -381,6 +444,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
         m0 = m0n;
         n0 = n0n;
         rw = rwn;
+        idle = idle_n;
         rx = rxn;
         rxs = rxsn;
         expert = expert_n;
@@ -401,7 +465,7 @@ bool experts_down_takes(int64_t hidden, int64_t inter) {
     return hidden % 128 == 0 && inter % 128 == 0 && inter / 128 >= 4 && inter / 128 <= 32 && hidden < (1 << 21);
 }
 
-template <bool DOWN>
+template <bool DOWN, bool ONCE>
 static int launch_experts(ExpertsArgs& p, int64_t rows, hipStream_t st) {
     p.tiles_m = (int)(rows / kExBM);
     p.tiles_n = (p.N + kExBN - 1) / kExBN;
@@ -411,13 +475,14 @@ static int launch_experts(ExpertsArgs& p, int64_t rows, hipStream_t st) {
     static std::atomic<bool> raised[65];  // zero-initialised
     const int slot = device_slot();
     if (slot == 64) raised[64].store(false, std::memory_order_relaxed);
-    if (int rc = raise_lds_limit(reinterpret_cast<const void*>(gemm_experts_kernel<DOWN>), kExLds, raised[slot])) return rc;
+    if (int rc = raise_lds_limit(reinterpret_cast<const void*>(gemm_experts_kernel<DOWN, ONCE>), kExLds, raised[slot])) return rc;
     const unsigned blocks = (unsigned)(tiles < cus ? tiles : cus);
     if (!note_launch(DOWN ? "gemm_experts<down>" : "gemm_experts<gate_up>", blocks, 512, kExLds)) return CFP8_OK;
-    hipLaunchKernelGGL(gemm_experts_kernel<DOWN>, dim3(blocks), dim3(512), kExLds, st, p);
+    hipLaunchKernelGGL((gemm_experts_kernel<DOWN, ONCE>), dim3(blocks), dim3(512), kExLds, st, p);
     return check_launch("gemm");
 }
-int launch_experts_gate_up(ExpertsArgs& p, int64_t rows, hipStream_t st) { return launch_experts<false>(p, rows, st); }
-int launch_experts_down(ExpertsArgs& p, int64_t rows, hipStream_t st) { return launch_experts<true>(p, rows, st); }
+// `once`: hardly an expert has a second tile of rows
+int launch_experts_gate_up(ExpertsArgs& p, int64_t rows, bool once, hipStream_t st) { return once ? launch_experts<false, true>(p, rows, st) : launch_experts<false, false>(p, rows, st); }
+int launch_experts_down(ExpertsArgs& p, int64_t rows, bool once, hipStream_t st) { return once ? launch_experts<true, true>(p, rows, st) : launch_experts<true, false>(p, rows, st); }
 
 }  // namespace cfp8

@@ -60,7 +60,7 @@ struct ExpertsArgs {
     const float* xs;             // [tokens or rows, K / 128]
     const uint8_t* w;            // [experts, N, K], gate_up: gate and up rows in turn, 16 at a time
     const float* ws;             // [experts, N / 128, K / 128]
-    const int32_t* row_tokens;   // gate_up: [rows], negative: a row of padding
+    const int32_t* row_tokens;   // [rows], negative: a row of padding
     const int32_t* row_experts;  // [rows]
     const int32_t* rows_end;     // rows that the groups take
     uint8_t* h;                  // gate_up: [rows, N / 2] fp8
@@ -70,8 +70,8 @@ struct ExpertsArgs {
 };
 bool experts_gate_up_takes(int64_t tokens, int64_t hidden, int64_t inter);
 bool experts_down_takes(int64_t hidden, int64_t inter);
-int launch_experts_gate_up(ExpertsArgs& p, int64_t rows, hipStream_t st);
-int launch_experts_down(ExpertsArgs& p, int64_t rows, hipStream_t st);
+int launch_experts_gate_up(ExpertsArgs& p, int64_t rows, bool once, hipStream_t st);
+int launch_experts_down(ExpertsArgs& p, int64_t rows, bool once, hipStream_t st);
 
 // ---- units of the kernels in which a workgroup walks rows of tiles ----------
 // The schedule for tiles_m tile rows of tiles_n tiles on `cus` workgroups: one workgroup per CU.  Tile rows beyond the

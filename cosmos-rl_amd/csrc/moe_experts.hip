@@ -233,12 +233,19 @@ static void launch_few_down(int ni, dim3 grid, hipStream_t st, const FewArgs& p)
 // tokens), 12 a wave (down, 96 registers, and two tiles of 16 rows of 1536 bytes in LDS).
 constexpr int64_t kFewMaxHidden = 4096, kFewMaxInter = 1536;
 // Mean rows an expert up to which a form is taken.  The few-rows form reads an expert's rows once for every strip of 16
-// features, the middle one once for every 128 columns but holds 64 rows in a tile; from about two of those tiles on the grouped
-// GEMMs' larger tiles need fewer loads a product.  Whole calls, few / middle / many rows, us: 128 experts of 2048 x 768, top 8:
-// 8 rows an expert 136 / 146 / 214, 16: 160 / 151 / 212, 49: 241 / 166 / 231, 96: 370 / 233 / 246, 128: 455 / 266 / 256; 32 of
-// 3584 x 1536, top 4: 8: 128 / 130 / 162, 16: 152 / 133 / 161, 97: 363 / 190 / 212, 128: 438 / 225 / 209; 64 of 1024 x 512, top 6:
-// 12: 42 / 44 / 71, 24: 50 / 47 / 74, 96: 88 / 62 / 77, 144: 112 / 76 / 92.
-constexpr int64_t kFewRowsPerExpert = 10, kMiddleRowsPerExpert = 112;
+// features, the middle one once for every 128 columns but holds 64 rows in a tile; from about one of those tiles on the larger
+// tiles of gemm_experts_kernel, whose waves without rows only load, need fewer loads a product and no quantiser in between.
+// Whole calls, few / middle, us: 128 experts of 2048 x 768, top 8: 8 rows an expert 136 / 146, 16: 160 / 151; 32 of 3584 x 1536, top 4:
+// 8: 128 / 130, 16: 152 / 133; 64 of 1024 x 512, top 6: 12: 42 / 44, 24: 50 / 47.  Middle / many: 128 of 2048 x 768: 30: 153 / 158,
+// 40: 160 / 159, 48: 176 / 161, 69: 212 / 172, 156: 312 / 239; 32 of 3584 x 1536: 40: 130 / 145, 50: 140 / 146, 100: 195 / 159; 64 of 1024 x 512:
+// 28: 56 / 54, 56: 68 / 56.
+// Where gemm_experts_kernel does not take both products, against the other grouped GEMMs: 128 of 2048 x 768: 96: 233 / 246, 128: 266 / 256.
+constexpr int64_t kFewRowsPerExpert = 10, kMiddleRowsPerExpert = 44, kMiddleRowsElsewhere = 112;
+// Many rows: up to here an expert has a second tile of 128 rows seldom enough for streaming loads of the weights to pay, if they are
+// more than the memory-side cache holds (those that it holds it keeps from call to call, if loads are cacheable).  Cacheable and
+// streaming, us: 128 experts of 2048 x 768 (604 MB) 48 rows an expert 167 / 161, 69: 179 / 172, 94: 185 / 180, 156: 239 / 288; 64 of 2048 x 1024 (403 MB)
+// 100: 131 / 128; 64 of 2048 x 640 (252 MB) 94: 107 / 107; 64 of 1024 x 512 (101 MB) 56: 56 / 59, 112: 73 / 76.
+constexpr int64_t kTileOnceRowsPerExpert = 100, kMemorySideCache = (int64_t)256 << 20;
 // Up to here the weights of the middle form are loaded as a stream: an expert seldom has a second tile of 64 rows, which reads
 // them again.  128 experts of 2048 x 768, rows an expert, the whole call cacheable and streaming, us: 12.5 148.8 / 137.9, 25
 // 155.6 / 146.5, 49 168.4 / 163.0, 62 194.9 / 203.8, 88 232.6 / 274.3; 32 experts of 3584 x 1536: 32 134.4 / 123.4, 75
@@ -257,8 +264,9 @@ struct ExpertsPlan {
 static ExpertsPlan experts_plan(int64_t tokens, int topk, int experts, int64_t hidden, int64_t inter) {
     ExpertsPlan p{};
     const int64_t pairs = tokens * topk;
+    p.gathers = experts_gate_up_takes(tokens, hidden, inter);
     if (pairs <= kFewRowsPerExpert * experts && hidden <= kFewMaxHidden && inter <= kFewMaxInter) p.form = Form::kFew;
-    else if (pairs <= kMiddleRowsPerExpert * experts && ring_grouped_takes(hidden) && ring_grouped_takes(inter) && tokens * hidden < (int64_t)1 << 31) p.form = Form::kMiddle;
+    else if (pairs <= (p.gathers && experts_down_takes(hidden, inter) ? kMiddleRowsPerExpert : kMiddleRowsElsewhere) * experts && ring_grouped_takes(hidden) && ring_grouped_takes(inter) && tokens * hidden < (int64_t)1 << 31) p.form = Form::kMiddle;
     else p.form = Form::kMany;
     const bool many = p.form == Form::kMany;
     p.slots = pairs < experts ? pairs : experts;
@@ -276,7 +284,7 @@ static ExpertsPlan experts_plan(int64_t tokens, int topk, int experts, int64_t h
     p.m_sizes = take((size_t)experts * 4);
     p.m_offsets = take((size_t)experts * 4);
     p.route = take(cfp8_route_tokens_workspace_bytes(tokens, topk, experts));
-    p.gathers = many && experts_gate_up_takes(tokens, hidden, inter);
+    p.gathers = p.gathers && many;
     const size_t xrows = (size_t)(many && !p.gathers ? p.rows : tokens);
     p.xq = take(xrows * (size_t)hidden);
     p.xs = take(xrows * (size_t)(hidden / 128) * 4);
@@ -361,6 +369,7 @@ extern "C" int cfp8_moe_experts(const void* x, int64_t ld_x, int64_t tokens, int
     } else {
         // (p.rows is a bound: 639 tiles of rows for 8192 tokens, top 8 of 128 experts, of which some 566 hold rows)
         const int32_t* const rows_end = i32(p.m_offsets) + experts - 1;
+        const bool once = tokens * topk <= kTileOnceRowsPerExpert * experts && (int64_t)experts * 3 * hidden * inter > kMemorySideCache;
         if (p.gathers) {
             if (int rc = cfp8_quant_group128(x, tokens, hidden, ld_x, ws + p.xq, hidden, f32(p.xs), CFP8_GROUP_MODE_DIV, stream)) return rc;
             ExpertsArgs g{};
@@ -368,7 +377,7 @@ extern "C" int cfp8_moe_experts(const void* x, int64_t ld_x, int64_t tokens, int
             g.row_tokens = i32(p.row_tokens); g.row_experts = i32(p.row_experts); g.rows_end = rows_end;
             g.h = ws + p.hq; g.hs = f32(p.hs);
             g.tokens = (int)tokens; g.N = (int)(2 * inter); g.K = (int)hidden;
-            if (int rc = launch_experts_gate_up(g, p.rows, st)) return rc;
+            if (int rc = launch_experts_gate_up(g, p.rows, once, st)) return rc;
         } else {
             if (int rc = cfp8_scatter_quant_group128(x, ld_x, tokens, hidden, i32(p.row_map), topk, i32(p.row_tokens), p.rows, ws + p.xq, hidden, f32(p.xs), stream))
                 return rc;
@@ -379,9 +388,9 @@ extern "C" int cfp8_moe_experts(const void* x, int64_t ld_x, int64_t tokens, int
         if (experts_down_takes(hidden, inter)) {
             ExpertsArgs d{};
             d.x = ws + p.hq; d.xs = f32(p.hs); d.w = static_cast<const uint8_t*>(down); d.ws = down_scales;
-            d.row_experts = i32(p.row_experts); d.rows_end = rows_end; d.out = reinterpret_cast<uint16_t*>(ws + p.out);
+            d.row_tokens = i32(p.row_tokens); d.row_experts = i32(p.row_experts); d.rows_end = rows_end; d.out = reinterpret_cast<uint16_t*>(ws + p.out);
             d.N = (int)hidden; d.K = (int)inter;
-            if (int rc = launch_experts_down(d, p.rows, st)) return rc;
+            if (int rc = launch_experts_down(d, p.rows, once, st)) return rc;
         } else {
             if (int rc = grouped_block128(ws + p.hq, inter, f32(p.hs), down, down_scales, i32(p.row_experts), rows_end, ws + p.out, hidden, CFP8_OUT_BF16,
                                           p.rows, hidden, inter, experts, stream))

@@ -64,3 +64,10 @@ def test_no_store_is_overtaken():
     with ThreadPoolExecutor(max_workers=8) as pool:
         found = {src: overwritten(lines) for src, lines in zip(_build.SOURCES, pool.map(_listing, _build.SOURCES))}
     assert not any(found.values()), {src: hits[:3] for src, hits in found.items() if hits}
+
+
+def test_experts_kernel_stays_in_registers():
+    """gemm_experts_kernel counts its vector-memory operations by hand: a spilled register would be one more of them."""
+    lines = _listing("gemm_experts.hip")
+    assert sum(line.strip().startswith("buffer_load_dwordx4") and " lds" in line for line in lines) > 0
+    assert not any(line.strip().startswith("scratch_") for line in lines)
