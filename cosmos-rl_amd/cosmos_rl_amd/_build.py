@@ -5,9 +5,11 @@ travels with the source checkout; it is never installed into site-packages.
 """
 from __future__ import annotations
 
+import importlib.util
 import os
 import shutil
 import subprocess
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -16,6 +18,7 @@ CSRC_DIR = PKG_DIR.parent / "csrc"
 INCLUDE_DIR = PKG_DIR.parent.parent / "include"
 LIB_DIR = PKG_DIR / "lib"
 LIB_PATH = LIB_DIR / "libcosmosfp8.so"
+CALLS_PATH = LIB_DIR / "_torch_calls.so"  # the operators' native host path (csrc/torch_calls.cpp), host code only
 OBJ_DIR = CSRC_DIR / "build"
 
 SOURCES = ["api.hip", "quant_rowwise.hip", "quant_tensorwise.hip", "quant_block.hip", "gemm_fp8.hip", "gemm_grouped_xres.hip", "gemm_experts.hip", "moe_indices.hip", "moe_route.hip", "moe_experts.hip",
@@ -51,6 +54,21 @@ def _compile(src: str) -> Path:
     return obj
 
 
+def _build_calls() -> None:
+    """The torch extension beside the library, with the host compiler; it is linked to the library that ctypes loads."""
+    torch_dir = Path(importlib.util.find_spec("torch").origin).parent
+    inc, lib = torch_dir / "include", torch_dir / "lib"
+    tmp = CALLS_PATH.with_suffix(".so.tmp")
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+           f"-I{inc}", f"-I{inc / 'torch/csrc/api/include'}", "-I/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}", f"-I{INCLUDE_DIR}",
+           str(CSRC_DIR / "torch_calls.cpp"), "-o", str(tmp), f"-L{lib}", "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip",
+           f"-L{LIB_DIR}", f"-l:{LIB_PATH.name}", "-Wl,-rpath,$ORIGIN"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed on torch_calls.cpp:\n{res.stdout}\n{res.stderr}")
+    os.replace(tmp, CALLS_PATH)
+
+
 def build(verbose: bool = False) -> Path:
     OBJ_DIR.mkdir(parents=True, exist_ok=True)
     LIB_DIR.mkdir(parents=True, exist_ok=True)
@@ -62,6 +80,7 @@ def build(verbose: bool = False) -> Path:
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stdout}\n{res.stderr}")
     os.replace(tmp, LIB_PATH)
+    _build_calls()
     if verbose:
         print(f"built {LIB_PATH}")
     return LIB_PATH

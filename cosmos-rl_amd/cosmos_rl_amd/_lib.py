@@ -6,10 +6,12 @@ exception is raised.  Loading the library needs no GPU; calling into it does.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 from ctypes import c_char_p, c_float, c_int, c_int32, c_int64, c_size_t, c_void_p, POINTER
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libcosmosfp8.so"
+CALLS_PATH = LIB_PATH.parent / "_torch_calls.so"
 
 OUT_BF16 = 0
 OUT_F32 = 1
@@ -117,6 +119,17 @@ def load() -> ctypes.CDLL:
         fn.argtypes = args
     _lib = lib
     return lib
+
+
+def torch_calls():
+    """The operators' native host path (csrc/torch_calls.cpp), or None where it is not built: they then take the same steps in Python."""
+    load()
+    if not CALLS_PATH.exists():
+        return None
+    spec = importlib.util.spec_from_file_location("_torch_calls", CALLS_PATH)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    return module
 
 
 DISPATCH_ROWWISE, DISPATCH_LINEAR, DISPATCH_BLOCK, DISPATCH_GROUPED, DISPATCH_GROUPED_SWIGLU, DISPATCH_MXFP4 = range(6)

@@ -33,6 +33,17 @@ def _need_gpu(*tensors: torch.Tensor) -> None:
                 f"{t.device}); there is no CPU path")
 
 
+_torch_calls = None
+
+
+def _native(name: str):
+    """An operator's native form: takes what is given in ordinary use and returns None for everything else."""
+    global _torch_calls
+    if _torch_calls is None:
+        _torch_calls = _lib.torch_calls() or False
+    return getattr(_torch_calls, name) if _torch_calls else lambda *args: None
+
+
 def _ptr(t: Optional[torch.Tensor]) -> int:
     return 0 if t is None else t.data_ptr()
 
@@ -396,6 +407,9 @@ def linear_mxfp4(x: torch.Tensor, weight: Tuple[torch.Tensor, torch.Tensor],
     """x [..., K] bf16 times MXFP4 weights (codes [N, K/2], scales [N, K/32]): per-token dynamic FP8
     quantisation of x (as in ``fp8_linear``) and ``gemm_mxfp4``, one launch for up to 4 tokens."""
     w, ws = weight
+    out = (_mxfp4_call or _find_mxfp4_call())(x, w, ws, out_dtype or torch.bfloat16)
+    if out is not None:
+        return out
     _need_gpu(x, w, ws)
     K = x.shape[-1]
     if x.dtype != torch.bfloat16 or w.dtype != torch.uint8 or ws.dtype != torch.uint8 or w.dim() != 2:
@@ -530,6 +544,21 @@ def _fused_bias(bias: Optional[torch.Tensor], n: int, device: torch.device) -> O
         return None
 
 
+_linear_call = _mxfp4_call = None
+
+
+def _find_linear_call():
+    global _linear_call
+    _linear_call = _native("fp8_linear")
+    return _linear_call
+
+
+def _find_mxfp4_call():
+    global _mxfp4_call
+    _mxfp4_call = _native("linear_mxfp4")
+    return _mxfp4_call
+
+
 def fp8_linear(x: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor,
                bias: Optional[torch.Tensor] = None, out_dtype: torch.dtype = torch.bfloat16,
                workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -538,6 +567,10 @@ def fp8_linear(x: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor
 
     weight: fp8 [K, N] column-major, i.e. ``qweight.t()`` as the reference stores it;
     weight_scale [N, 1]; x bf16 [..., K].  Returns [..., N]."""
+    if workspace is None:
+        out = (_linear_call or _find_linear_call())(x, weight, weight_scale, bias, out_dtype)
+        if out is not None:
+            return out
     _need_gpu(x, weight, weight_scale)
     if x.dtype != torch.bfloat16:
         raise ValueError(f"fp8_linear takes bfloat16 activations, got {x.dtype}")
