@@ -8,6 +8,7 @@
 //   * rows of up to 32768 elements: one workgroup per row, cross-wave max
 //     through LDS.
 //   * longer rows: one workgroup per row, second sweep re-reads the row.
+//   * few rows of 513 to 32768 elements: one workgroup per row with a thread for every 8 to 32 elements.
 //
 // The source may also be fp16 or fp32 (the dtype a weight is transferred in): it
 // is rounded to bf16 first, exactly as `recv.to(torch.bfloat16)` would, and the
@@ -127,6 +128,34 @@ __global__ __launch_bounds__(256) void rowwise_block_kernel(const uint8_t* __res
     rowwise_block_body<V, NTS, SRC>(x, blockIdx.x, nvec, ldx, q, ldq, scales, red);
 }
 
+// Few rows (a decode batch's activations): one workgroup of T threads a row, so that a row's vectors are one to four a thread.  With a
+// wave or 256 threads a row, up to ten vectors a lane are cast one behind the other on a chip that is otherwise empty.
+template <int T, int V, bool NTS, int SRC>
+__global__ __launch_bounds__(T) void rowwise_few_kernel(const uint8_t* __restrict__ x, int nvec, int64_t ldx, uint2* __restrict__ q, int64_t ldq,
+                                                        float* __restrict__ scales) {
+    __shared__ u32 red[T / 64];
+    const int t = threadIdx.x;
+    const uint8_t* const xr = x + (int64_t)blockIdx.x * ldx;
+    uint4 v[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) v[i] = t + T * i < nvec ? ld8<SRC, true>(xr, t + T * i) : make_uint4(0, 0, 0, 0);
+    u32 m = 0;
+#pragma unroll
+    for (int i = 0; i < V; ++i) m = absmax8(m, v[i]);
+    m = wave_max(pk_fold(m));
+    if ((t & 63) == 0) red[t >> 6] = m;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < T / 64; ++w) m = umax(m, red[w]);
+    const float scale = scale_from_amax(amax_from_bits(m));
+    if (t == 0) scales[blockIdx.x] = scale;
+    const Divider d(scale);
+    uint2* const qr = q + (int64_t)blockIdx.x * ldq;
+#pragma unroll
+    for (int i = 0; i < V; ++i)
+        if (t + T * i < nvec) st8<NTS>(qr + t + T * i, cast8(v[i], d));
+}
+
 // ---- many weights in one launch --------------------------------------------------------------
 // The weights of one flush group of a weight sync (rollout_control.py:1308-1319 runs the queued
 // completions together) are a few dozen tensors of 13..140 MB: quantised one launch each, every one
@@ -223,11 +252,28 @@ static bool with_row_variant(RowVariant rv, F&& f) {
     return false;
 }
 
+// Rows up to which a workgroup a row is the faster one, wave or 256 threads / this, us: 3584 columns 33 rows 3.6 / 2.7, 512 4.0 / 3.5, 1111
+// 5.9 / 5.4, 2048 7.1 / 7.6; 2304: 64 3.4 / 2.6, 2048 6.0 / 6.4; 896: 64 2.8 / 2.5, 1111 3.2 / 3.0, 2048 3.4 / 3.5; 4864: 33 3.2 / 3.0, 256 3.4 / 3.3, 400
+// 3.8 / 4.0, 2048 7.3 / 10.6; 18944: 33 4.4 / 3.8, 256 6.4 / 6.1, 512 7.6 / 7.6, 777 10.3 / 11.2.
+static bool few_rows(int64_t rows, int64_t nvec) { return nvec > 64 && nvec <= 4096 && rows <= (nvec <= 512 ? 1280 : 256); }
+
 // streaming_out: write the fp8 bytes with non-temporal stores (weights, consumed much
 // later); false keeps them cacheable (activations feeding the GEMM of the same call).
 template <bool NTS, int SRC>
 static void launch_rowwise_variant(const uint8_t* xv, int64_t rows, int64_t nvec, int64_t ldx, uint2* qv, int64_t ldq,
                                    float* scales, hipStream_t st) {
+    if constexpr (!NTS && SRC == kSrcBF16) {
+        if (few_rows(rows, nvec)) {
+            const dim3 grid((unsigned)rows);
+            if (nvec <= 128) hipLaunchKernelGGL((rowwise_few_kernel<128, 1, NTS, SRC>), grid, dim3(128), 0, st, xv, (int)nvec, ldx, qv, ldq, scales);
+            else if (nvec <= 256) hipLaunchKernelGGL((rowwise_few_kernel<256, 1, NTS, SRC>), grid, dim3(256), 0, st, xv, (int)nvec, ldx, qv, ldq, scales);
+            else if (nvec <= 512) hipLaunchKernelGGL((rowwise_few_kernel<512, 1, NTS, SRC>), grid, dim3(512), 0, st, xv, (int)nvec, ldx, qv, ldq, scales);
+            else if (nvec <= 1024) hipLaunchKernelGGL((rowwise_few_kernel<1024, 1, NTS, SRC>), grid, dim3(1024), 0, st, xv, (int)nvec, ldx, qv, ldq, scales);
+            else if (nvec <= 2048) hipLaunchKernelGGL((rowwise_few_kernel<1024, 2, NTS, SRC>), grid, dim3(1024), 0, st, xv, (int)nvec, ldx, qv, ldq, scales);
+            else hipLaunchKernelGGL((rowwise_few_kernel<1024, 4, NTS, SRC>), grid, dim3(1024), 0, st, xv, (int)nvec, ldx, qv, ldq, scales);
+            return;
+        }
+    }
     const bool done = with_row_variant(row_variant(nvec), [&](auto wave, auto v) {
         constexpr int V = decltype(v)::value;
         if constexpr (decltype(wave)::value)
