@@ -18,6 +18,7 @@
 //               K into registers before anything else, and then walks the expert's rows in tiles of 16
 //               (few_gate_up_kernel, few_down_kernel).
 #include "gemm_internal.h"
+#include "moe_route.h"
 #include "gemm_ring.h"
 
 namespace cfp8 {
@@ -325,13 +326,16 @@ extern "C" int cfp8_moe_experts(const void* x, int64_t ld_x, int64_t tokens, int
     auto i32 = [&](size_t at) { return reinterpret_cast<int32_t*>(ws + at); };
     auto f32 = [&](size_t at) { return reinterpret_cast<float*>(ws + at); };
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (int rc = cfp8_route_tokens(indices, index_bytes, token_mask, tokens, topk, experts, p.form == Form::kMany ? 128 : 1, CFP8_ROUTE_END_NOT_PADDING, p.rows,
-                                   i32(p.row_tokens), p.form == Form::kMany ? i32(p.row_experts) : nullptr, i32(p.row_map), nullptr, weights, weights_dtype,
-                                   ws + p.weights, i32(p.m_sizes), i32(p.m_offsets), ws + p.route,
-                                   cfp8_route_tokens_workspace_bytes(tokens, topk, experts), stream))
+    // the tokens quantised as they lie, for the products that pick their rows themselves
+    const bool as_they_lie = p.form != Form::kMany || p.gathers;
+    if (as_they_lie && tokens * (hidden / 128) > kMaxGroups) return set_error(CFP8_EINVAL, "moe_experts: too many groups for one launch");
+    const GroupRows xq = group_rows(x, tokens, hidden, ld_x, ws + p.xq, hidden, f32(p.xs));
+    if (int rc = route_and_quantise(indices, index_bytes, token_mask, tokens, topk, experts, p.form == Form::kMany ? 128 : 1, CFP8_ROUTE_END_NOT_PADDING, p.rows,
+                                    i32(p.row_tokens), p.form == Form::kMany ? i32(p.row_experts) : nullptr, i32(p.row_map), nullptr, weights, weights_dtype,
+                                    ws + p.weights, i32(p.m_sizes), i32(p.m_offsets), ws + p.route, cfp8_route_tokens_workspace_bytes(tokens, topk, experts),
+                                    as_they_lie ? &xq : nullptr, st))
         return rc;
     if (p.form == Form::kMiddle) {
-        if (int rc = cfp8_quant_group128(x, tokens, hidden, ld_x, ws + p.xq, hidden, f32(p.xs), CFP8_GROUP_MODE_DIV, stream)) return rc;
         const int64_t row_tiles = p.slots + p.rows / kRingGroupRows;
         const bool once = p.rows <= kOnceRowsPerExpert * experts;
         RingArgs r{};
@@ -347,7 +351,6 @@ extern "C" int cfp8_moe_experts(const void* x, int64_t ld_x, int64_t tokens, int
         r.M = (int)p.rows; r.N = (int)hidden; r.K = (int)inter;
         if (int rc = launch_ring_grouped(kRingDown, r, row_tiles, once, st)) return rc;
     } else if (p.form == Form::kFew) {
-        if (int rc = cfp8_quant_group128(x, tokens, hidden, ld_x, ws + p.xq, hidden, f32(p.xs), CFP8_GROUP_MODE_DIV, stream)) return rc;
         FewArgs f{};
         f.xq = ws + p.xq;
         f.xs = f32(p.xs);
@@ -371,7 +374,6 @@ extern "C" int cfp8_moe_experts(const void* x, int64_t ld_x, int64_t tokens, int
         const int32_t* const rows_end = i32(p.m_offsets) + experts - 1;
         const bool once = tokens * topk <= kTileOnceRowsPerExpert * experts && (int64_t)experts * 3 * hidden * inter > kMemorySideCache;
         if (p.gathers) {
-            if (int rc = cfp8_quant_group128(x, tokens, hidden, ld_x, ws + p.xq, hidden, f32(p.xs), CFP8_GROUP_MODE_DIV, stream)) return rc;
             ExpertsArgs g{};
             g.x = ws + p.xq; g.xs = f32(p.xs); g.w = static_cast<const uint8_t*>(gate_up); g.ws = gate_up_scales;
             g.row_tokens = i32(p.row_tokens); g.row_experts = i32(p.row_experts); g.rows_end = rows_end;

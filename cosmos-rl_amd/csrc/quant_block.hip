@@ -1,6 +1,6 @@
 // 128x128 block quantisation (weights), 1x128 group quantisation (activations)
 // and the block dequantiser.  All three are HBM-bound streaming kernels.
-#include "cfp8_common.h"
+#include "quant_group.h"
 
 namespace cfp8 {
 
@@ -83,88 +83,10 @@ __global__ __launch_bounds__(256) void block128_kernel(const uint16_t* __restric
     }
 }
 
-// ---------------------------------------------------------------------------
-// 1x128 groups.  16 lanes own one group (one 16-byte vector each), the max runs
-// over the 16-lane DPP row.  Every thread handles 4 groups of 4 consecutive
-// group-rows so that four loads are in flight per lane.
-// ---------------------------------------------------------------------------
-// With GATHER, output row r quantises input row src_rows[r] (a zero row where that is negative): the token
-// gather in front of the grouped GEMM and the quantiser in one pass, without the gathered bf16 matrix.
-// Groups are numbered row-major (row * ngroups + column) in 32 bits; a thread divides once and steps
-// through its four consecutive groups.  Every load is unconditional on a clamped address (what must read
-// as zero is cleared afterwards), so all four are in flight before the first is used.
+// 1x128 groups (group128_four): sixteen threads a group, four groups one after the other a thread.
 template <int MODE, bool GATHER = false>
-__global__ __launch_bounds__(256) void group128_kernel(const uint4* __restrict__ x, int nvec,
-                                                       u32 ngroups, int64_t ldx, uint2* __restrict__ q, int64_t ldq,
-                                                       float* __restrict__ scales, u32 rows, u32 total_groups,
-                                                       const int32_t* __restrict__ src_rows = nullptr) {
-    const int sub = threadIdx.x & 15;
-    const u32 g0 = (blockIdx.x * 16u + (threadIdx.x >> 4)) * 4u;
-    uint4 v[4];
-    u32 row[4], gcol[4];
-    bool ok[4];
-    {
-        u32 r = g0 / ngroups, c = g0 - r * ngroups;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            row[i] = r;
-            gcol[i] = c;
-            if (++c == ngroups) c = 0, ++r;
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int vec = (int)gcol[i] * 16 + sub;
-        ok[i] = g0 + i < total_groups && vec < nvec;
-        const u32 rc = row[i] < rows ? row[i] : rows - 1;
-        const int vc = vec < nvec ? vec : nvec - 1;
-        if (GATHER) {
-            const int32_t src = src_rows[rc];
-            ok[i] = ok[i] && src >= 0;
-            // tokens are read several times (once per expert they go to): leave them in the caches
-            v[i] = ld16<false>(x + (int64_t)(src >= 0 ? src : 0) * ldx + vc);
-        } else {
-            v[i] = ld16<true>(x + (int64_t)rc * ldx + vc);
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        if (!ok[i]) v[i] = make_uint4(0, 0, 0, 0);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const u32 m = row16_max(pk_fold(absmax8(0u, v[i])));
-        const float amax = amax_from_bits(m);
-        uint2 out;
-        float scale;
-        if (MODE == CFP8_GROUP_MODE_DIV) {
-            scale = scale_from_amax(amax);
-            const Divider d(scale);
-            out = cast8(v[i], d);
-        } else {
-            // x * (448 / clamp(amax, 1e-4)) as torch evaluates `448.0 / tensor`:
-            // reciprocal first, then times 448.  No clamp before the cast: the product
-            // exceeds 448 by at most a few fp32 roundings, far below the NaN threshold 464
-            if (amax != amax) {
-                scale = __uint_as_float(kCanonNaN);
-                out = make_uint2(0x7F7F7F7Fu, 0x7F7F7F7Fu);
-            } else {
-                const float a = fmaxf(amax, 1e-4f);
-                const float mul = (1.0f / a) * kE4M3Max;
-                scale = a / kE4M3Max;
-                const u32 w[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
-                u32 o[2];
-#pragma unroll
-                for (int k = 0; k < 2; ++k) {
-                    u32 p = cvt2<false>(bf16_lo(w[2 * k]) * mul, bf16_hi(w[2 * k]) * mul, 0u);
-                    o[k] = cvt2<true>(bf16_lo(w[2 * k + 1]) * mul, bf16_hi(w[2 * k + 1]) * mul, p);
-                }
-                out = make_uint2(o[0], o[1]);
-            }
-        }
-        const int vec = (int)gcol[i] * 16 + sub;
-        if (g0 + i < total_groups && vec < nvec) q[(int64_t)row[i] * ldq + vec] = out;
-        if (sub == 0 && g0 + i < total_groups) scales[g0 + i] = scale;
-    }
+__global__ __launch_bounds__(256) void group128_kernel(const GroupRows p, const int32_t* __restrict__ src_rows = nullptr) {
+    group128_four<MODE, GATHER>(p, (blockIdx.x * 16u + (threadIdx.x >> 4)) * 4u, src_rows);
 }
 
 // ---------------------------------------------------------------------------
@@ -379,22 +301,13 @@ __global__ __launch_bounds__(256) void scatter_group128_kernel(const uint4* __re
 }
 
 // Groups are numbered in 32 bits, and a block's first group index must not wrap.
-constexpr int64_t kMaxGroups = 0xFFFFFF00ll;
-
 int launch_quant_group128(const void* x, int64_t rows, int64_t cols, int64_t ld_x, void* q, int64_t ld_q,
                           float* scales, int mode, hipStream_t st) {
-    const int64_t ngroups = (cols + 127) / 128;
-    const int64_t total = rows * ngroups;
-    if (total > kMaxGroups) return set_error(CFP8_EINVAL, "quant_group128: too many groups for one launch");
-    const unsigned blocks = (unsigned)((total + 63) / 64);
-    const uint4* xv = static_cast<const uint4*>(x);
-    uint2* qv = static_cast<uint2*>(q);
-    if (mode == CFP8_GROUP_MODE_DIV)
-        hipLaunchKernelGGL(group128_kernel<CFP8_GROUP_MODE_DIV>, dim3(blocks), dim3(256), 0, st, xv, (int)(cols / 8),
-                           (u32)ngroups, ld_x / 8, qv, ld_q / 8, scales, (u32)rows, (u32)total, nullptr);
-    else
-        hipLaunchKernelGGL(group128_kernel<CFP8_GROUP_MODE_DEEPEP>, dim3(blocks), dim3(256), 0, st, xv, (int)(cols / 8),
-                           (u32)ngroups, ld_x / 8, qv, ld_q / 8, scales, (u32)rows, (u32)total, nullptr);
+    if (rows * ((cols + 127) / 128) > kMaxGroups) return set_error(CFP8_EINVAL, "quant_group128: too many groups for one launch");
+    const GroupRows p = group_rows(x, rows, cols, ld_x, q, ld_q, scales);
+    const dim3 grid((p.total_groups + 63) / 64), block(256);
+    if (mode == CFP8_GROUP_MODE_DIV) hipLaunchKernelGGL(group128_kernel<CFP8_GROUP_MODE_DIV>, grid, block, 0, st, p, nullptr);
+    else hipLaunchKernelGGL(group128_kernel<CFP8_GROUP_MODE_DEEPEP>, grid, block, 0, st, p, nullptr);
     return check_launch("quant_group128");
 }
 
@@ -449,12 +362,10 @@ extern "C" int cfp8_gather_quant_group128(const void* x, int64_t ld_x, const int
         return set_error(CFP8_EINVAL, "gather_quant_group128: cols=%lld ld_x=%lld ld_q=%lld must be multiples of 8 with ld >= cols",
                          (long long)cols, (long long)ld_x, (long long)ld_q);
     if (!aligned16(x) || (reinterpret_cast<uintptr_t>(q) & 7u)) return set_error(CFP8_EINVAL, "gather_quant_group128: misaligned pointer");
-    const int64_t ngroups = (cols + 127) / 128, total = rows_out * ngroups;
-    if (total > kMaxGroups) return set_error(CFP8_EINVAL, "gather_quant_group128: too many groups for one launch");
+    if (rows_out * ((cols + 127) / 128) > kMaxGroups) return set_error(CFP8_EINVAL, "gather_quant_group128: too many groups for one launch");
     if (int rc = check_device()) return rc;
-    hipLaunchKernelGGL((group128_kernel<CFP8_GROUP_MODE_DIV, true>), dim3((unsigned)((total + 63) / 64)), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), static_cast<const uint4*>(x), (int)(cols / 8), (u32)ngroups, ld_x / 8,
-                       static_cast<uint2*>(q), ld_q / 8, scales, (u32)rows_out, (u32)total, src_rows);
+    const GroupRows p = group_rows(x, rows_out, cols, ld_x, q, ld_q, scales);
+    hipLaunchKernelGGL((group128_kernel<CFP8_GROUP_MODE_DIV, true>), dim3((p.total_groups + 63) / 64), dim3(256), 0, static_cast<hipStream_t>(stream), p, src_rows);
     return check_launch("gather_quant_group128");
 }
 

@@ -88,6 +88,23 @@ def test_one_call_experts_many_rows(dev, T, E, topk, H, I, keep):
     assert not bool(y[~mask].any())
 
 
+# the tokens are quantised by workgroups behind the routing's, 256 groups each, four in turn a thread: one launch up to 1024 pairs, two beyond,
+# of which the first has a quarter of those workgroups; rows of tokens that do not follow each other
+@pytest.mark.parametrize("T,topk,H", [(1, 1, 128), (3, 8, 128), (51, 4, 640), (52, 4, 640), (128, 8, 640), (129, 8, 640), (1025, 1, 128), (410, 3, 1280), (1639, 2, 640)])
+def test_one_call_experts_quantised_beside_the_routing(dev, T, topk, H):
+    from cosmos_rl_amd.policy.kernel.moe.moe import grouped_experts_forward
+    E = 8
+    strategy, module = _module(dev, E, H, 128, T)
+    g = torch.Generator(device=dev).manual_seed(T + 4)
+    x = torch.randn(T, H + 8, generator=g, device=dev).to(torch.bfloat16)[:, :H]
+    idx = torch.rand(T, E, generator=g, device=dev).topk(topk, dim=1).indices
+    w = torch.rand(T, topk, generator=g, device=dev).to(torch.bfloat16)
+    mask = torch.rand(T, generator=g, device=dev) < 0.8
+    y = grouped_experts_forward(x, mask, w, idx, strategy, module, E)
+    want = _chain(x.contiguous(), mask, w, idx, strategy, module, E)
+    assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+
+
 def test_one_call_experts_refuses_a_small_workspace(dev):
     t = torch.zeros(256, 256, device=dev, dtype=torch.bfloat16)
     need = _lib.load().cfp8_moe_experts_workspace_bytes(4, 2, 2, 256, 128)
