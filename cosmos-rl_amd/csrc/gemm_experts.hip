@@ -30,7 +30,8 @@
 // The down product (165 us, 268 MB written) is bound by its stores among the loads: 119 us without the stores, 113 without the loads, 105
 // without either; neither their cache policy, nor tiles that are contiguous in memory, nor stores behind the next loads change that.
 //
-// A wave whose 64 rows are all padding only loads and keeps the barriers (48 rows an expert: 178 -> 167 us a call).
+// A wave whose 64 rows are all padding only loads and keeps the barriers (48 rows an expert: 178 -> 167 us a call), and those rows of
+// h are neither written nor read (152.4 -> 147.1 us).
 #include <atomic>
 #include <type_traits>
 
@@ -84,13 +85,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
 
     // ---- loads.  Load i of a wave: rows (wave + 8 i) * 8 .. + 7 of the tile, 16-byte chunk c of row r at position c ^ f(r).
     const uint32_t chunk = (uint32_t)(((lane & 7) ^ ((wave & 1) * 4 + ((lane >> 4) & 1))) << 4);
-    // gate_up: all tokens, whose rows the lanes pick; down: the tile's rows
-    auto x_rsrc = [&](int m0) {
-        return DOWN ? __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.x) + (int64_t)m0 * p.K, 0, kExBM * p.K, 0x00020000)
+    // gate_up: all tokens, whose rows the lanes pick; down: the tile's first 64 or 128 rows
+    auto x_rsrc = [&](int m0, int rows) {
+        return DOWN ? __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.x) + (int64_t)m0 * p.K, 0, rows * p.K, 0x00020000)
                     : __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.x), 0, (int)((uint32_t)p.tokens * (uint32_t)p.K), 0x00020000);
     };
-    auto xs_rsrc = [&](int m0) {
-        return DOWN ? __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.xs) + (int64_t)m0 * KT, 0, kExBM * KT * 4, 0x00020000)
+    auto xs_rsrc = [&](int m0, int rows) {
+        return DOWN ? __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.xs) + (int64_t)m0 * KT, 0, rows * KT * 4, 0x00020000)
                     : __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.xs), 0, (int)((uint32_t)p.tokens * (uint32_t)KT * 4u), 0x00020000);
     };
     uint32_t vw[4];
@@ -101,8 +102,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
         vx[i] = token >= 0 ? (uint32_t)token * (uint32_t)p.K + chunk : kExOutside;
         vxs[i] = token >= 0 ? (uint32_t)(token * KT + (lane & 7)) * 4u : kExOutside;
     };
-    // `idle`: this wave's 64 rows are all padding (a group's padding follows its rows)
-    auto place = [&](int id, int& m0, int& n0, __amdgpu_buffer_rsrc_t& rw, int& expert, bool& idle) {
+    // `rows`: 64 where the second half of the tile is padding, whose rows are neither written by gate_up nor read by down (a group's
+    // padding follows its rows)
+    auto place = [&](int id, int& m0, int& n0, __amdgpu_buffer_rsrc_t& rw, int& expert, int& rows) {
         int tm, tn;
         tile_of_block<kGroupedBandRows>(id, tiles_m, p.tiles_n, tm, tn);
         m0 = tm * kExBM;
@@ -110,7 +112,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
         const int32_t *const at = p.row_experts + m0, *const half = p.row_tokens + m0 + 64;  // (a group's rows begin on a multiple of 128)
         int token;
         asm volatile("s_load_dword %0, %2, 0x0\n\ts_load_dword %1, %3, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=&s"(expert), "=&s"(token) : "s"(at), "s"(half) : "memory");
-        idle = wm == 1 && token < 0;
+        rows = token < 0 ? 64 : kExBM;
         // (down: weight rows beyond N, where N is an odd multiple of 128, arrive as zeros)
         rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.w) + ((int64_t)expert * p.N + n0) * p.K, 0,
                                                (p.N - n0 < kExBN ? p.N - n0 : kExBN) * p.K, 0x00020000);
@@ -153,11 +155,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
         else sn = *reinterpret_cast<const u32x2*>(smem + kExWeightScales + par * 256 + kt * 8);
     };
 
-    int m0, n0, expert;
-    bool idle;
+    int m0, n0, expert, rows;
     __amdgpu_buffer_rsrc_t rw;
-    place(pid, m0, n0, rw, expert, idle);
-    __amdgpu_buffer_rsrc_t rx = x_rsrc(m0), rxs = xs_rsrc(m0);
+    place(pid, m0, n0, rw, expert, rows);
+    __amdgpu_buffer_rsrc_t rx = x_rsrc(m0, rows), rxs = xs_rsrc(m0, rows);
+    bool idle = wm == 1 && rows < kExBM;  // this wave has no rows
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int row = (wave + 8 * i) * 8 + (lane >> 3);
@@ -193,11 +195,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
     for (;;) {
         const int pid_n = pid + (int)gridDim.x;
         const bool has_next = pid_n < ntiles;
-        int m0n, n0n, expert_n;
-        bool idle_n;
+        int m0n, n0n, expert_n, rows_n;
         __amdgpu_buffer_rsrc_t rwn;
-        place(has_next ? pid_n : pid, m0n, n0n, rwn, expert_n, idle_n);  // (no next tile: this one's first steps are fetched once more)
-        const __amdgpu_buffer_rsrc_t rxn = x_rsrc(m0n), rxsn = xs_rsrc(m0n);
+        place(has_next ? pid_n : pid, m0n, n0n, rwn, expert_n, rows_n);  // (no next tile: this one's first steps are fetched once more)
+        const __amdgpu_buffer_rsrc_t rxn = x_rsrc(m0n, rows_n), rxsn = xs_rsrc(m0n, rows_n);
 
         // what a step loads beside its tile, in front of it: the next barrier waits for it
         auto beside = [&](int kt, auto first_c, auto left_c) {
@@ -384,7 +385,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
             // has both values of an element; both are rounded to bf16 first, as the product would be in memory.  A wave has 32 of the
             // 128 columns of the group: the four that share rows exchange their maxima.  Behind that a lane looks after one row (x tile
             // `quarter`, row lrow): its scale, and the 16 bytes of it that the four quarters hold a word of each.
-            // A wave without rows stores zeros and their scale.
+            // A wave without rows stores nothing.
             u32 h[2][4][2];  // [pair][x tile][two words of two bf16]
             int le = lane;  // (addresses derived here: kept across the K loop they would cost registers)
             asm volatile("" : "+v"(le));
@@ -435,8 +436,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
             const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(p.h + (int64_t)m0 * (p.N >> 1), 0, 0x80000000u, 0x00020000);
             const __amdgpu_buffer_rsrc_t rh = __builtin_amdgcn_make_buffer_rsrc(p.hs + (int64_t)m0 * (p.N >> 8), 0, 0x80000000u, 0x00020000);
 #pragma unroll
-            for (int pp = 0; pp < 2; ++pp) buffer_store16(bytes[pp], rq, (uint32_t)(row * (p.N >> 1)), (uint32_t)((n0 >> 1) + wn * 32 + pp * 16));
-            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(scale), rh, wn == 0 ? (uint32_t)(row * (p.N >> 8) * 4) : kExOutside, (uint32_t)((n0 >> 8) * 4), 0);
+            for (int pp = 0; pp < 2; ++pp) buffer_store16(bytes[pp], rq, idle ? kExOutside : (uint32_t)(row * (p.N >> 1)), (uint32_t)((n0 >> 1) + wn * 32 + pp * 16));
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(scale), rh, wn == 0 && !idle ? (uint32_t)(row * (p.N >> 8) * 4) : kExOutside, (uint32_t)((n0 >> 8) * 4), 0);
         }
 
         if (!has_next) break;
@@ -444,7 +445,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
         m0 = m0n;
         n0 = n0n;
         rw = rwn;
-        idle = idle_n;
+        idle = wm == 1 && rows_n < kExBM;
         rx = rxn;
         rxs = rxsn;
         expert = expert_n;
