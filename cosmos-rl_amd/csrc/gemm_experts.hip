@@ -31,7 +31,7 @@
 // without either; neither their cache policy, nor tiles that are contiguous in memory, nor stores behind the next loads change that.
 //
 // A wave whose 64 rows are all padding only loads and keeps the barriers (48 rows an expert: 178 -> 167 us a call), and those rows of
-// h are neither written nor read (152.4 -> 147.1 us).
+// h are neither written nor read (152.4 -> 147.1 us), unless the down product is another kernel's (ExpertsArgs::whole_tiles).
 #include <atomic>
 #include <type_traits>
 
@@ -102,8 +102,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
         vx[i] = token >= 0 ? (uint32_t)token * (uint32_t)p.K + chunk : kExOutside;
         vxs[i] = token >= 0 ? (uint32_t)(token * KT + (lane & 7)) * 4u : kExOutside;
     };
-    // `rows`: 64 where the second half of the tile is padding, whose rows are neither written by gate_up nor read by down (a group's
-    // padding follows its rows)
+    // `rows`: 64 where the second half of the tile is padding, whose rows down does not read (a group's padding follows its rows)
     auto place = [&](int id, int& m0, int& n0, __amdgpu_buffer_rsrc_t& rw, int& expert, int& rows) {
         int tm, tn;
         tile_of_block<kGroupedBandRows>(id, tiles_m, p.tiles_n, tm, tn);
@@ -385,7 +384,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
             // has both values of an element; both are rounded to bf16 first, as the product would be in memory.  A wave has 32 of the
             // 128 columns of the group: the four that share rows exchange their maxima.  Behind that a lane looks after one row (x tile
             // `quarter`, row lrow): its scale, and the 16 bytes of it that the four quarters hold a word of each.
-            // A wave without rows stores nothing.
+            // A wave without rows stores nothing, or zeros and their scale for a down product that reads them.
             u32 h[2][4][2];  // [pair][x tile][two words of two bf16]
             int le = lane;  // (addresses derived here: kept across the K loop they would cost registers)
             asm volatile("" : "+v"(le));
@@ -435,9 +434,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
             }
             const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(p.h + (int64_t)m0 * (p.N >> 1), 0, 0x80000000u, 0x00020000);
             const __amdgpu_buffer_rsrc_t rh = __builtin_amdgcn_make_buffer_rsrc(p.hs + (int64_t)m0 * (p.N >> 8), 0, 0x80000000u, 0x00020000);
+            const bool stores = !idle || p.whole_tiles;
 #pragma unroll
-            for (int pp = 0; pp < 2; ++pp) buffer_store16(bytes[pp], rq, idle ? kExOutside : (uint32_t)(row * (p.N >> 1)), (uint32_t)((n0 >> 1) + wn * 32 + pp * 16));
-            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(scale), rh, wn == 0 && !idle ? (uint32_t)(row * (p.N >> 8) * 4) : kExOutside, (uint32_t)((n0 >> 8) * 4), 0);
+            for (int pp = 0; pp < 2; ++pp) buffer_store16(bytes[pp], rq, stores ? (uint32_t)(row * (p.N >> 1)) : kExOutside, (uint32_t)((n0 >> 1) + wn * 32 + pp * 16));
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(scale), rh, wn == 0 && stores ? (uint32_t)(row * (p.N >> 8) * 4) : kExOutside, (uint32_t)((n0 >> 8) * 4), 0);
         }
 
         if (!has_next) break;

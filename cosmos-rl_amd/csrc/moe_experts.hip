@@ -379,6 +379,7 @@ extern "C" int cfp8_moe_experts(const void* x, int64_t ld_x, int64_t tokens, int
             g.row_tokens = i32(p.row_tokens); g.row_experts = i32(p.row_experts); g.rows_end = rows_end;
             g.h = ws + p.hq; g.hs = f32(p.hs);
             g.tokens = (int)tokens; g.N = (int)(2 * inter); g.K = (int)hidden;
+            g.whole_tiles = !experts_down_takes(hidden, inter);
             if (int rc = launch_experts_gate_up(g, p.rows, once, st)) return rc;
         } else {
             if (int rc = cfp8_scatter_quant_group128(x, ld_x, tokens, hidden, i32(p.row_map), topk, i32(p.row_tokens), p.rows, ws + p.xq, hidden, f32(p.xs), stream))
