@@ -30,6 +30,8 @@ constexpr int kRouteMaxBlocks = 128;
 // Of the tokens' quantisation beside two launches of routing, the quarters that go with the first.  8192 tokens of 2048, the launches by themselves:
 // none 4.7 + 13.6 us, one 7.0 + 13.0, two 8.7 + 12.4.
 constexpr int kRouteEarlyQuarters = 1;
+// Groups up to which a quantising thread takes one, not four: 777 tokens of 2048 (12432 groups) 147.7 -> 145.3 us a call; 8192 tokens (131072) 492 -> 494.
+constexpr u32 kRouteFewGroups = 1u << 15;
 
 struct RouteArgs {
     const void* indices;      // [tokens, topk] int32 or int64
@@ -82,8 +84,12 @@ __device__ __forceinline__ RoutePair route_pair(const RouteArgs& p, u32 pair, bo
     return r;
 }
 
-// The workgroups behind the routing's own quantise the tokens, which it does not read: four groups a thread of sixteen.
-__device__ __forceinline__ void route_quantise(const GroupRows& q, u32 block) { group128_four<CFP8_GROUP_MODE_DIV>(q, (block * (kRouteThreads / 16) + (threadIdx.x >> 4)) * 4u); }
+// The workgroups behind the routing's own quantise the tokens, which it does not read.
+__device__ __forceinline__ void route_quantise(const GroupRows& q, u32 block) {
+    const u32 at = block * (kRouteThreads / 16) + (threadIdx.x >> 4);
+    if (q.total_groups <= kRouteFewGroups) group128_some<CFP8_GROUP_MODE_DIV, 1>(q, at);
+    else group128_some<CFP8_GROUP_MODE_DIV, 4>(q, at * 4u);
+}
 
 __global__ __launch_bounds__(kRouteThreads) void route_count_kernel(const RouteArgs p, const GroupRows q) {
     __shared__ int hist[kRouteMaxExperts];
@@ -280,8 +286,8 @@ int route_and_quantise(const void* indices, int index_bytes, const uint8_t* toke
     p.chunk = (p.pairs + blocks - 1) / blocks;
     p.chunk = (p.chunk + kRouteThreads - 1) / kRouteThreads * kRouteThreads;
     p.blocks = (int)blocks;
-    // the quantiser's blocks of 1024 threads, 256 groups each
-    const u32 groups = tokens_q ? tokens_q->total_groups : 0, q_blocks = groups / 256 + (groups % 256 != 0);
+    const u32 groups = tokens_q ? tokens_q->total_groups : 0, per = (kRouteThreads / 16) * (groups <= kRouteFewGroups ? 1 : 4);  // groups a block
+    const u32 q_blocks = groups / per + (groups % per != 0);
     const GroupRows q = tokens_q ? *tokens_q : GroupRows{};
     if (blocks == 1) {
         hipLaunchKernelGGL(route_place_kernel<true>, dim3(1 + q_blocks), dim3(kRouteThreads), lds, st, p, q, 0u);

@@ -83,10 +83,10 @@ __global__ __launch_bounds__(256) void block128_kernel(const uint16_t* __restric
     }
 }
 
-// 1x128 groups (group128_four): sixteen threads a group, four groups one after the other a thread.
-template <int MODE, bool GATHER = false>
+// 1x128 groups (group128_some): sixteen threads a group, N groups one after the other a thread.
+template <int MODE, int N, bool GATHER = false>
 __global__ __launch_bounds__(256) void group128_kernel(const GroupRows p, const int32_t* __restrict__ src_rows = nullptr) {
-    group128_four<MODE, GATHER>(p, (blockIdx.x * 16u + (threadIdx.x >> 4)) * 4u, src_rows);
+    group128_some<MODE, N, GATHER>(p, (blockIdx.x * 16u + (threadIdx.x >> 4)) * (u32)N, src_rows);
 }
 
 // ---------------------------------------------------------------------------
@@ -300,14 +300,22 @@ __global__ __launch_bounds__(256) void scatter_group128_kernel(const uint4* __re
     }
 }
 
+// Groups up to which a thread takes one, not four.  Four / one, us: 12 groups 2.7 / 1.7, 1344 (24 rows of 7168) 3.0 / 2.0, 11200 3.7 / 3.0, 56000 7.4 / 6.6,
+// 112000 11.5 / 11.2, 131072 (8192 rows of 2048) 12.6 / 12.4, 229376 19.1 / 19.4, 458752 33.7 / 36.7.
+constexpr u32 kFewGroups = 1u << 17;
+
 // Groups are numbered in 32 bits, and a block's first group index must not wrap.
 int launch_quant_group128(const void* x, int64_t rows, int64_t cols, int64_t ld_x, void* q, int64_t ld_q,
                           float* scales, int mode, hipStream_t st) {
     if (rows * ((cols + 127) / 128) > kMaxGroups) return set_error(CFP8_EINVAL, "quant_group128: too many groups for one launch");
     const GroupRows p = group_rows(x, rows, cols, ld_x, q, ld_q, scales);
-    const dim3 grid((p.total_groups + 63) / 64), block(256);
-    if (mode == CFP8_GROUP_MODE_DIV) hipLaunchKernelGGL(group128_kernel<CFP8_GROUP_MODE_DIV>, grid, block, 0, st, p, nullptr);
-    else hipLaunchKernelGGL(group128_kernel<CFP8_GROUP_MODE_DEEPEP>, grid, block, 0, st, p, nullptr);
+    const bool few = p.total_groups <= kFewGroups;
+    const u32 per = few ? 16 : 64;  // groups a workgroup
+    const dim3 grid((p.total_groups - 1) / per + 1), block(256);
+    if (mode == CFP8_GROUP_MODE_DIV && few) hipLaunchKernelGGL((group128_kernel<CFP8_GROUP_MODE_DIV, 1>), grid, block, 0, st, p, nullptr);
+    else if (mode == CFP8_GROUP_MODE_DIV) hipLaunchKernelGGL((group128_kernel<CFP8_GROUP_MODE_DIV, 4>), grid, block, 0, st, p, nullptr);
+    else if (few) hipLaunchKernelGGL((group128_kernel<CFP8_GROUP_MODE_DEEPEP, 1>), grid, block, 0, st, p, nullptr);
+    else hipLaunchKernelGGL((group128_kernel<CFP8_GROUP_MODE_DEEPEP, 4>), grid, block, 0, st, p, nullptr);
     return check_launch("quant_group128");
 }
 
@@ -365,7 +373,7 @@ extern "C" int cfp8_gather_quant_group128(const void* x, int64_t ld_x, const int
     if (rows_out * ((cols + 127) / 128) > kMaxGroups) return set_error(CFP8_EINVAL, "gather_quant_group128: too many groups for one launch");
     if (int rc = check_device()) return rc;
     const GroupRows p = group_rows(x, rows_out, cols, ld_x, q, ld_q, scales);
-    hipLaunchKernelGGL((group128_kernel<CFP8_GROUP_MODE_DIV, true>), dim3((p.total_groups + 63) / 64), dim3(256), 0, static_cast<hipStream_t>(stream), p, src_rows);
+    hipLaunchKernelGGL((group128_kernel<CFP8_GROUP_MODE_DIV, 4, true>), dim3((p.total_groups + 63) / 64), dim3(256), 0, static_cast<hipStream_t>(stream), p, src_rows);
     return check_launch("gather_quant_group128");
 }
 

@@ -22,16 +22,16 @@ inline GroupRows group_rows(const void* x, int64_t rows, int64_t cols, int64_t l
 
 // ---------------------------------------------------------------------------
 // 1x128 groups.  16 lanes own one group (one 16-byte vector each), the max runs
-// over the 16-lane DPP row.  Every thread handles 4 groups of 4 consecutive
-// group-rows so that four loads are in flight per lane.
+// over the 16-lane DPP row.  Every thread handles N groups that follow each other: 4 so that four loads are in flight
+// per lane, 1 where there are so few groups that a thread's casts, one behind the other, are what takes the time.
 // ---------------------------------------------------------------------------
 // With GATHER, output row r quantises input row src_rows[r] (a zero row where that is negative): the token
 // gather in front of the grouped GEMM and the quantiser in one pass, without the gathered bf16 matrix.
 // Groups are numbered row-major (row * ngroups + column) in 32 bits; a thread divides once and steps
-// through its four consecutive groups.  Every load is unconditional on a clamped address (what must read
-// as zero is cleared afterwards), so all four are in flight before the first is used.
-template <int MODE, bool GATHER = false>
-__device__ __forceinline__ void group128_four(const GroupRows& p, u32 g0, const int32_t* __restrict__ src_rows = nullptr) {
+// through its consecutive groups.  Every load is unconditional on a clamped address (what must read
+// as zero is cleared afterwards), so all are in flight before the first is used.
+template <int MODE, int N, bool GATHER = false>
+__device__ __forceinline__ void group128_some(const GroupRows& p, u32 g0, const int32_t* __restrict__ src_rows = nullptr) {
     const int sub = threadIdx.x & 15;
     const u32 ngroups = p.ngroups, rows = p.rows, total_groups = p.total_groups;
     const int nvec = p.nvec;
@@ -39,20 +39,20 @@ __device__ __forceinline__ void group128_four(const GroupRows& p, u32 g0, const 
     const uint4* __restrict__ const x = p.x;
     uint2* __restrict__ const q = p.q;
     float* __restrict__ const scales = p.scales;
-    uint4 v[4];
-    u32 row[4], gcol[4];
-    bool ok[4];
+    uint4 v[N];
+    u32 row[N], gcol[N];
+    bool ok[N];
     {
         u32 r = g0 / ngroups, c = g0 - r * ngroups;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < N; ++i) {
             row[i] = r;
             gcol[i] = c;
             if (++c == ngroups) c = 0, ++r;
         }
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < N; ++i) {
         const int vec = (int)gcol[i] * 16 + sub;
         ok[i] = g0 + i < total_groups && vec < nvec;
         const u32 rc = row[i] < rows ? row[i] : rows - 1;
@@ -67,10 +67,10 @@ __device__ __forceinline__ void group128_four(const GroupRows& p, u32 g0, const 
         }
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < N; ++i)
         if (!ok[i]) v[i] = make_uint4(0, 0, 0, 0);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < N; ++i) {
         const u32 m = row16_max(pk_fold(absmax8(0u, v[i])));
         const float amax = amax_from_bits(m);
         uint2 out;

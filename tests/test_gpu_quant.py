@@ -622,6 +622,17 @@ def test_group128(dev, shape):
     assert_bytes(q, qo, f"group {shape} bytes")
 
 
+# a group a thread of sixteen up to 131072 groups, four beyond; the last workgroup partly filled
+@pytest.mark.parametrize("shape", [(16384, 1024), (16385, 1024), (65537, 200), (13, 1160)])
+def test_group128_groups_a_thread(dev, shape):
+    x = O.make_activation(*shape, seed=5, chan_outlier_frac=0.01, outlier_mul=30.0)
+    x[-1, :8] = 0
+    for op, oracle in ((ops.groupwise_activation_quant, O.quant_group128), (ops.per_token_cast_to_fp8, O.group128_cast_deepep)):
+        (q, s), (qo, so) = op(x.to(dev)), oracle(x)
+        assert_scales(s, so, f"group {shape} scales")
+        assert_bytes(q, qo, f"group {shape} bytes")
+
+
 @pytest.mark.parametrize("shape", [(4, 128), (33, 896), (7, 200), (129, 2048)])
 def test_group128_deepep_formula(dev, shape):
     """per_token_cast_to_fp8 exactly as the reference's tests/test_deepep.py states it."""
