@@ -2083,7 +2083,7 @@ __global__ __launch_bounds__(NTL * 128) void gemm_rowwise_skinny_kernel(const Ge
 
 // ---------------------------------------------------------------------------
 // Rowwise GEMM for M <= 16 (single-token decode): no LDS staging and no barrier
-// in the loop.  A workgroup owns 16 weight rows; its four waves split K (wave w
+// in the loop.  A workgroup owns ROWS weight rows (gemv_rows); its four waves split K (wave w
 // takes K steps w, w + 4, ...), each issuing the loads of a chunk of NI K steps
 // before the first MFMA: all of its steps if they are at most eight, else equal
 // chunks of at most eight (16 KiB of weights per wave).  Loads for steps that do
@@ -2096,16 +2096,19 @@ __global__ __launch_bounds__(NTL * 128) void gemm_rowwise_skinny_kernel(const Ge
 // 28.3 / 24.6 us, against 31.8 / 49.4 us otherwise.  The few activation rows come
 // straight from global memory (they stay in L2), rows >= M repeat row 0.
 // ---------------------------------------------------------------------------
-template <int NI, bool OUT_F32>
+template <int NI, int ROWS, bool OUT_F32>
 __global__ __launch_bounds__(256) void gemm_rowwise_gemv_kernel(const GemmArgs p) {
     __shared__ __attribute__((aligned(16))) float red[3 * 64 * 4];
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int lrow = lane & 15, quarter = lane >> 4;
-    const int n0 = blockIdx.x * 16;
+    const int n0 = blockIdx.x * ROWS;
     const int KT = p.K >> 7;
     const bool xok = lrow < p.M;
     const uint8_t* wptr = p.b + (int64_t)(n0 + lrow) * p.ld_b + quarter * 32;  // N % 16 == 0: the 16 rows are there
+    // ROWS < 16: the other rows of the MFMA tile are past the end of this buffer and arrive as zeros without a fetch
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.b) + (int64_t)n0 * p.ld_b, 0, (int)(ROWS * p.ld_b), 0x00020000);
+    const uint32_t vw = lrow < ROWS ? (uint32_t)lrow * (uint32_t)p.ld_b + (uint32_t)quarter * 32u : 0xF0000000u;
     const uint8_t* xptr = p.a + (int64_t)(xok ? lrow : 0) * p.ld_a + quarter * 32;
     f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int base = wave; base < KT; base += 4 * NI) {
@@ -2115,8 +2118,13 @@ __global__ __launch_bounds__(256) void gemm_rowwise_gemv_kernel(const GemmArgs p
             const int kt = base + 4 * i;
             if (kt >= KT) continue;
             const int64_t off = (int64_t)kt << 7;
-            wl[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wptr + off));
-            wh[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wptr + off + 16));
+            if constexpr (ROWS == 16) {
+                wl[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wptr + off));
+                wh[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wptr + off + 16));
+            } else {
+                wl[i] = __builtin_amdgcn_raw_buffer_load_b128(rw, vw, (uint32_t)off, 2);
+                wh[i] = __builtin_amdgcn_raw_buffer_load_b128(rw, vw + 16u, (uint32_t)off, 2);
+            }
             xl[i] = *reinterpret_cast<const u32x4*>(xptr + off);
             xh[i] = *reinterpret_cast<const u32x4*>(xptr + off + 16);
         }
@@ -2138,7 +2146,7 @@ __global__ __launch_bounds__(256) void gemm_rowwise_gemv_kernel(const GemmArgs p
     __syncthreads();
     if (wave == 0) {
         const int n = n0 + quarter * 4, m = lrow;
-        if (m < p.M) {
+        if (m < p.M && quarter * 4 < ROWS) {
 #pragma unroll
             for (int w = 0; w < 3; ++w) {
                 const f32x4 o = *reinterpret_cast<const f32x4*>(red + (w * 64 + lane) * 4);
@@ -2168,11 +2176,11 @@ __global__ __launch_bounds__(256) void gemm_rowwise_gemv_kernel(const GemmArgs p
 // thread holds at most two (four) 16-byte vectors of a token between the amax and the cast, exactly the
 // arithmetic of the rowwise quantiser - into LDS, from where the MFMA fragments are read.  The
 // quantisation hides behind the weight loads, and the separate launch (3 us plus the gap between two
-// launches) is gone: 896 x 4864 10.2 -> 6.1 us; 18944 x 3584 takes 16.2 us.  At four
+// launches) is gone: 896 x 4864 10.2 -> 6.1 us, 4.6 with ROWS = 4 (gemv_rows); 18944 x 3584 takes 16.2 us.  At four
 // tokens the quantisation in every workgroup costs what the launch would (18944 x 2560 15.9 us either way), beyond
 // that more; and 8192 is what a wave's registers hold.  Results are bit-identical to the two-launch path.
 // ---------------------------------------------------------------------------
-template <int MR, int NI, bool OUT_F32>
+template <int MR, int NI, int ROWS, bool OUT_F32>
 __global__ __launch_bounds__(256) void linear_gemv_fused_kernel(const uint4* __restrict__ x, int64_t ldx, const GemmArgs p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t xq[];  // [M][K] fp8
     __shared__ __attribute__((aligned(16))) float red[3 * 64 * 4];
@@ -2180,18 +2188,26 @@ __global__ __launch_bounds__(256) void linear_gemv_fused_kernel(const uint4* __r
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int lrow = lane & 15, quarter = lane >> 4;
-    const int n0 = blockIdx.x * 16;
+    const int n0 = blockIdx.x * ROWS;
     const int KT = p.K >> 7;  // <= 4 NI: all of a wave's K steps at once
     const bool xok = lrow < p.M;
     const uint8_t* wptr = p.b + (int64_t)(n0 + lrow) * p.ld_b + quarter * 32;
+    // ROWS < 16: the other rows of the MFMA tile are past the end of this buffer and arrive as zeros without a fetch
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.b) + (int64_t)n0 * p.ld_b, 0, (int)(ROWS * p.ld_b), 0x00020000);
+    const uint32_t vw = ROWS == 16 || lrow < ROWS ? (uint32_t)lrow * (uint32_t)p.ld_b + (uint32_t)quarter * 32u : 0xF0000000u;
     u32x4 wl[NI], wh[NI];
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
         // (a wave without this step repeats the last one: under a branch the loads were sunk behind the barriers, 17664 x
         // 2176 17 against 11 us)
         const int kt = wave + 4 * i < KT ? wave + 4 * i : KT - 1;
-        wl[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wptr + ((int64_t)kt << 7)));
-        wh[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wptr + ((int64_t)kt << 7) + 16));
+        if constexpr (ROWS == 16) {
+            wl[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wptr + ((int64_t)kt << 7)));
+            wh[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wptr + ((int64_t)kt << 7) + 16));
+        } else {
+            wl[i] = __builtin_amdgcn_raw_buffer_load_b128(rw, vw, (uint32_t)kt << 7, 2);
+            wh[i] = __builtin_amdgcn_raw_buffer_load_b128(rw, vw + 16u, (uint32_t)kt << 7, 2);
+        }
     }
     // the tokens (MR >= M of them): amax, scale, cast - rows >= M read row 0 and are never used
     const int nvec = p.K >> 3;
@@ -2248,7 +2264,7 @@ __global__ __launch_bounds__(256) void linear_gemv_fused_kernel(const uint4* __r
     __syncthreads();
     if (wave == 0) {
         const int n = n0 + quarter * 4, m = lrow;
-        if (m < p.M) {
+        if (m < p.M && quarter * 4 < ROWS) {
 #pragma unroll
             for (int w = 0; w < 3; ++w) {
                 const f32x4 o = *reinterpret_cast<const f32x4*>(red + (w * 64 + lane) * 4);
@@ -2273,43 +2289,66 @@ __global__ __launch_bounds__(256) void linear_gemv_fused_kernel(const uint4* __r
     }
 }
 
+// Weight rows a workgroup of the two gemv kernels.  With 16 of a narrow weight most CUs have nothing to do and the others are bound by what one
+// CU loads; with fewer each still quantises or reads the whole of the tokens, so there are no more workgroups than CUs.  16 / 8 / 4 rows, us
+// (tokens x rows x K), in one launch with the quantiser: 1 x 896 x 4864 6.5 / 5.0 / 4.6, 1 x 1024 x 8192 8.4 / 6.4 / 5.8, 4 x 896 x 4096 7.4 / 6.5 / 6.3, 2 x 896 x 896
+// 3.5 / 3.3 / 3.4, 1 x 1536 x 8192 8.8 / 7.1 / 7.8, 1 x 2048 x 2048 3.9 / 3.5 / 3.8, 1 x 2560 x 2048 4.1 / 4.2 / 4.2, 4 x 4096 x 2048 5.9 / 6.4 / 7.8. The product alone:
+// 16 x 896 x 4864 7.5 / 6.8 / 6.4, 16 x 1024 x 4096 6.7 / 5.7 / 5.5, 12 x 1152 x 896 3.0 / 2.9 / 3.3, 16 x 896 x 896 3.1 / 3.0 / 3.1, 8 x 2048 x 5632 7.8 / 7.1 / 9.0, 16 x 2048 x 2048
+// 4.4 / 4.1 / 5.4, 16 x 2560 x 2048 4.5 / 5.5 / 6.7.
+static int gemv_rows(const GemmArgs& p) {
+    const int cus = cu_count();
+    if (p.ld_b > (1 << 26)) return 16;  // (32-bit offsets of up to 8 rows)
+    return p.N <= 4 * cus && p.K > 2048 ? 4 : p.N <= 8 * cus ? 8 : 16;
+}
+
 // whether the one-launch kernel above takes the call
 static bool fused_gemv_size(int64_t M, int64_t K) { return M >= 1 && M <= 4 && K <= (M == 1 ? 8192 : 4096) && K % 128 == 0; }
 static bool fused_gemv_applies(int64_t M, int64_t K, const void* x, int64_t ld_x) { return fused_gemv_size(M, K) && aligned16(x) && ld_x % 8 == 0; }
-template <int MR, int NI>
+template <int MR, int NI, int ROWS>
 static void launch_fused_ni(int ni, dim3 grid, size_t lds, hipStream_t st, const void* x, int64_t ld_x, const GemmArgs& p, int out_dtype) {
     if constexpr (NI > 0) {
-        if (ni != NI) return launch_fused_ni<MR, NI - 1>(ni, grid, lds, st, x, ld_x, p, out_dtype);
+        if (ni != NI) return launch_fused_ni<MR, NI - 1, ROWS>(ni, grid, lds, st, x, ld_x, p, out_dtype);
         if (out_dtype == CFP8_OUT_F32)
-            hipLaunchKernelGGL((linear_gemv_fused_kernel<MR, NI, true>), grid, dim3(256), lds, st, static_cast<const uint4*>(x), ld_x / 8, p);
+            hipLaunchKernelGGL((linear_gemv_fused_kernel<MR, NI, ROWS, true>), grid, dim3(256), lds, st, static_cast<const uint4*>(x), ld_x / 8, p);
         else
-            hipLaunchKernelGGL((linear_gemv_fused_kernel<MR, NI, false>), grid, dim3(256), lds, st, static_cast<const uint4*>(x), ld_x / 8, p);
+            hipLaunchKernelGGL((linear_gemv_fused_kernel<MR, NI, ROWS, false>), grid, dim3(256), lds, st, static_cast<const uint4*>(x), ld_x / 8, p);
     }
 }
 static int launch_linear_gemv_fused(const void* x, int64_t ld_x, GemmArgs& p, int out_dtype, hipStream_t st) {
-    const int64_t blocks = (p.N + 15) / 16;
+    const int rows = gemv_rows(p);
+    const int64_t blocks = ((int64_t)p.N + rows - 1) / rows;
     const size_t lds = (size_t)p.M * (size_t)p.K;  // <= 16 KiB
     if (!note_launch("linear_gemv_fused", (unsigned)blocks, 256, lds)) return CFP8_OK;
     const int ni = ((p.K >> 7) + 3) / 4;
-    if (p.M == 1) launch_fused_ni<1, 16>(ni, dim3((unsigned)blocks), lds, st, x, ld_x, p, out_dtype);
-    else if (p.M == 2) launch_fused_ni<2, 8>(ni, dim3((unsigned)blocks), lds, st, x, ld_x, p, out_dtype);
-    else launch_fused_ni<4, 8>(ni, dim3((unsigned)blocks), lds, st, x, ld_x, p, out_dtype);
+    auto launch = [&](auto r) {
+        constexpr int ROWS = decltype(r)::value;
+        if (p.M == 1) launch_fused_ni<1, 16, ROWS>(ni, dim3((unsigned)blocks), lds, st, x, ld_x, p, out_dtype);
+        else if (p.M == 2) launch_fused_ni<2, 8, ROWS>(ni, dim3((unsigned)blocks), lds, st, x, ld_x, p, out_dtype);
+        else launch_fused_ni<4, 8, ROWS>(ni, dim3((unsigned)blocks), lds, st, x, ld_x, p, out_dtype);
+    };
+    if (rows == 4) launch(std::integral_constant<int, 4>{});
+    else if (rows == 8) launch(std::integral_constant<int, 8>{});
+    else launch(std::integral_constant<int, 16>{});
     return check_launch("linear");
 }
 
-template <int NI>
+template <int NI, int ROWS>
 static void launch_gemv_ni(int ni, dim3 grid, hipStream_t st, const GemmArgs& p, int out_dtype) {
     if constexpr (NI > 0) {
-        if (ni != NI) return launch_gemv_ni<NI - 1>(ni, grid, st, p, out_dtype);
-        if (out_dtype == CFP8_OUT_F32) hipLaunchKernelGGL((gemm_rowwise_gemv_kernel<NI, true>), grid, dim3(256), 0, st, p);
-        else hipLaunchKernelGGL((gemm_rowwise_gemv_kernel<NI, false>), grid, dim3(256), 0, st, p);
+        if (ni != NI) return launch_gemv_ni<NI - 1, ROWS>(ni, grid, st, p, out_dtype);
+        if (out_dtype == CFP8_OUT_F32) hipLaunchKernelGGL((gemm_rowwise_gemv_kernel<NI, ROWS, true>), grid, dim3(256), 0, st, p);
+        else hipLaunchKernelGGL((gemm_rowwise_gemv_kernel<NI, ROWS, false>), grid, dim3(256), 0, st, p);
     }
 }
 static int launch_rowwise_gemv(GemmArgs& p, int out_dtype, hipStream_t st) {
-    const int64_t blocks = (p.N + 15) / 16;
+    const int rows = gemv_rows(p);
+    const int64_t blocks = ((int64_t)p.N + rows - 1) / rows;
     if (!note_launch("gemm_rowwise_gemv", (unsigned)blocks, 256, 0)) return CFP8_OK;
     const int steps = ((p.K >> 7) + 3) / 4, chunks = (steps + 7) / 8;
-    launch_gemv_ni<8>((steps + chunks - 1) / chunks, dim3((unsigned)blocks), st, p, out_dtype);
+    const int ni = (steps + chunks - 1) / chunks;
+    if (rows == 4) launch_gemv_ni<8, 4>(ni, dim3((unsigned)blocks), st, p, out_dtype);
+    else if (rows == 8) launch_gemv_ni<8, 8>(ni, dim3((unsigned)blocks), st, p, out_dtype);
+    else launch_gemv_ni<8, 16>(ni, dim3((unsigned)blocks), st, p, out_dtype);
     return check_launch("gemm");
 }
 
@@ -3337,7 +3376,7 @@ __global__ __launch_bounds__(256) void bias_rows_kernel(void* out, int64_t ld_ou
 
 // The times of launch_gemm's rowwise kernels in microseconds, for the choice below; fitted to the same shapes and in the same way as
 // the ring's.
-// Up to 128 tokens, the weight streamers: up to 16 the weights' way in (token rows come from L2 beside them) joined with the
+// Up to 128 tokens, the weight streamers: up to 16, in the form with 16 weight rows a workgroup, the weights' way in (token rows come from L2 beside them) joined with the
 // chunks of K one after the other, beyond that rounds of strips times K steps.
 static double rowwise_streams_cost(int64_t M, int64_t N, int64_t K, int cus) {
     const double kt = (double)(K / 128), bytes = (double)N * (double)K;

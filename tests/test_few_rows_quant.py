@@ -3,7 +3,7 @@ bits of the weights' quantiser in front of the scaled product."""
 import pytest
 import torch
 
-from cosmos_rl_amd import ops
+from cosmos_rl_amd import _lib, ops
 from oracle import fp8_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -24,3 +24,44 @@ def test_linear_has_the_bits_of_the_two_steps(dev, K, rows):
         for y in (x, wide[:, :K]):
             got = ops.fp8_linear(y, q.t(), s, out_dtype=torch.float32)
             assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(7.0), want.nan_to_num(7.0)), M
+
+
+# one launch for up to 4 tokens: 4, 8 or 16 weight rows a workgroup, by 1024 and 2048 rows and 2048 columns, beside the two steps
+@pytest.mark.parametrize("N,K", [(16, 128), (16, 2176), (1008, 2048), (1024, 2176), (1024, 4096), (1040, 4096), (2048, 896), (2064, 2176), (896, 4864), (2048, 8192), (1040, 8192)])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_one_launch_linear(dev, N, K, dt):
+    w = O.make_weight((N, K), seed=4).to(dev)
+    q, s = ops.quant_rowwise(w)
+    spread = torch.zeros(N, K + 128, dtype=torch.uint8, device=dev)   # rows that do not follow each other
+    spread[:, :K] = q.view(torch.uint8)
+    apart = spread.view(torch.float8_e4m3fn)[:, :K]
+    bias = torch.randn(N, device=dev).to(torch.bfloat16)
+    for M in (1, 2, 3, 4) if K <= 4096 else (1,):
+        x = O.make_activation(M, K, seed=M, chan_outlier_frac=0.005, outlier_mul=30.0).to(dev)
+        qx, sx = ops.quant_rowwise(x)
+        for weight in (q, apart):
+            for b in (None, bias):
+                assert torch.equal(ops.fp8_linear(x, weight.t(), s, bias=b, out_dtype=dt), ops.scaled_mm(qx, q.t(), sx, s, bias=b, out_dtype=dt)), M
+
+
+# up to 16 tokens: 4, 8 or 16 weight rows a workgroup, one and several chunks of K; a column's bits do not depend on how many rows lie beside it
+@pytest.mark.parametrize("K", [128, 896, 2048, 2176, 4864, 8192])
+@pytest.mark.parametrize("M", [1, 2, 5, 16])
+def test_product_of_few_tokens(dev, M, K):
+    q, s = ops.quant_rowwise(O.make_weight((4096, K), seed=6).to(dev))
+    x = O.make_activation(M, K, seed=M)
+    qx, sx = ops.quant_rowwise(x.to(dev))
+    call = _lib.load().cfp8_scaled_mm_rowwise   # (the kernel for 16 tokens whatever the shape)
+
+    def product(rows, dt):
+        out = torch.zeros(M, rows, dtype=dt, device=dev)
+        _lib.check(call(qx.data_ptr(), K, sx.data_ptr(), q.data_ptr(), K, s.data_ptr(), out.data_ptr(), rows, _lib.OUT_F32 if dt == torch.float32 else _lib.OUT_BF16,
+                        M, rows, K, torch.cuda.current_stream().cuda_stream))
+        return out
+    for dt in (torch.bfloat16, torch.float32):
+        whole = product(4096, dt)
+        for rows in (16, 1008, 1024, 1040, 2048, 2064):
+            assert torch.equal(product(rows, dt), whole[:, :rows])
+    want = O.fp8_linear_rowwise(x, q.view(torch.uint8).cpu()[:1040], s.cpu()[:1040], accum=torch.float64)
+    # (fp32 sums of K products against 64 bits)
+    assert O.rel_frobenius(product(1040, torch.float32).cpu(), want) < 1e-3
