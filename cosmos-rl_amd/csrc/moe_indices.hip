@@ -10,6 +10,8 @@
 //      its source rank (walk over at most num_ranks blocks) and writes the source row, or -1
 //      for a padding row.
 // Integer work, launch-bound at real sizes (a few hundred counts, ~10^5 rows).
+#include <type_traits>
+
 #include "cfp8_common.h"
 
 namespace cfp8 {
@@ -115,14 +117,15 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const uint4* __restric
 //   STEPS: every product and every partial sum is rounded to bf16, the arithmetic of
 //          `y.scatter_add_(0, idx, expert_out * weights[idx, top, None])` on bf16 tensors;
 //   else:  fp32 accumulator acc = fma(row, weight, acc), rounded to bf16 once.
-template <bool STEPS, bool W32>
+//   DEPTH: slots requested at once.  Bound by latency while the chip holds all wavefronts at once, by HBM beyond.
+template <bool STEPS, bool W32, int DEPTH>
 __global__ __launch_bounds__(256) void combine_rows_kernel(const uint4* __restrict__ rows, int64_t ldr,
                                                            int64_t num_rows, const int32_t* __restrict__ row_map,
                                                            const void* __restrict__ weights, int64_t tokens, int topk, int nvec, int chunks,
                                                            uint4* __restrict__ out, int64_t ldo) {
-    const int64_t unit = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int64_t unit = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (unit >= tokens * chunks) return;  // whole wavefronts leave
-    const int64_t t = unit / chunks;
+    const int64_t t = unit >> 32 ? unit / chunks : (int64_t)((u32)unit / (u32)chunks);
     const int lane = threadIdx.x & 63;
     const int v = (int)(unit - t * chunks) * 64 + lane;
     const int vv = v < nvec ? v : nvec - 1;  // lanes past the row end re-read its last vector and store nothing
@@ -139,25 +142,38 @@ __global__ __launch_bounds__(256) void combine_rows_kernel(const uint4* __restri
     }
     u32 y[4] = {0u, 0u, 0u, 0u};
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-    for (int s = 0; s < topk; ++s) {
-        const int32_t r = __builtin_amdgcn_readlane(src, s);
-        const float ws = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), s));
-        uint4 d = ld16<true>(rows + (int64_t)(r < 0 ? 0 : r) * ldr + vv);
-        if (r < 0) d = make_uint4(0, 0, 0, 0);
-        const u32 x[4] = {d.x, d.y, d.z, d.w};
+    auto walk = [&](auto n_c, int s0) {
+        constexpr int N = decltype(n_c)::value;
+        uint4 d[N];
+        int32_t r[N];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float lo = __uint_as_float(x[e] << 16), hi = __uint_as_float(x[e] & 0xFFFF0000u);
-            if (STEPS) {
-                const u32 p = pack_bf16x2(lo * ws, hi * ws);
-                y[e] = pack_bf16x2(__uint_as_float(y[e] << 16) + __uint_as_float(p << 16),
-                                   __uint_as_float(y[e] & 0xFFFF0000u) + __uint_as_float(p & 0xFFFF0000u));
-            } else {
-                acc[2 * e] = __builtin_fmaf(lo, ws, acc[2 * e]);
-                acc[2 * e + 1] = __builtin_fmaf(hi, ws, acc[2 * e + 1]);
+        for (int i = 0; i < N; ++i) {
+            r[i] = __builtin_amdgcn_readlane(src, s0 + i);  // (lanes past topk: no row; s0 + i <= 63)
+            d[i] = ld16<true>(rows + (int64_t)(r[i] < 0 ? 0 : r[i]) * ldr + vv);
+        }
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            if (s0 + i >= topk) break;
+            const float ws = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), s0 + i));
+            if (r[i] < 0) d[i] = make_uint4(0, 0, 0, 0);
+            const u32 x[4] = {d[i].x, d[i].y, d[i].z, d[i].w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float lo = __uint_as_float(x[e] << 16), hi = __uint_as_float(x[e] & 0xFFFF0000u);
+                if (STEPS) {
+                    const u32 p = pack_bf16x2(lo * ws, hi * ws);
+                    y[e] = pack_bf16x2(__uint_as_float(y[e] << 16) + __uint_as_float(p << 16),
+                                       __uint_as_float(y[e] & 0xFFFF0000u) + __uint_as_float(p & 0xFFFF0000u));
+                } else {
+                    acc[2 * e] = __builtin_fmaf(lo, ws, acc[2 * e]);
+                    acc[2 * e + 1] = __builtin_fmaf(hi, ws, acc[2 * e + 1]);
+                }
             }
         }
+    };
+    for (int s0 = 0; s0 < topk; s0 += DEPTH) {
+        if (DEPTH == 4 || topk - s0 > 4) walk(std::integral_constant<int, DEPTH>{}, s0);
+        else walk(std::integral_constant<int, 4>{}, s0);
     }
     if (!STEPS) {
 #pragma unroll
@@ -237,11 +253,18 @@ extern "C" int cfp8_combine_rows(const void* rows, int64_t ld_rows, int64_t num_
     hipStream_t st = static_cast<hipStream_t>(stream);
     const uint4* r = static_cast<const uint4*>(rows);
     uint4* o = static_cast<uint4*>(out);
-    if (mode == CFP8_COMBINE_BF16_STEPS)
-        hipLaunchKernelGGL((combine_rows_kernel<true, false>), grid, block, 0, st, r, ld_rows / 8, num_rows, row_map, weights, tokens, topk, (int)nvec, (int)chunks, o, ld_out / 8);
-    else if (weights_dtype == CFP8_IN_F32)
-        hipLaunchKernelGGL((combine_rows_kernel<false, true>), grid, block, 0, st, r, ld_rows / 8, num_rows, row_map, weights, tokens, topk, (int)nvec, (int)chunks, o, ld_out / 8);
-    else
-        hipLaunchKernelGGL((combine_rows_kernel<false, false>), grid, block, 0, st, r, ld_rows / 8, num_rows, row_map, weights, tokens, topk, (int)nvec, (int)chunks, o, ld_out / 8);
+    // Wavefronts up to which eight slots are requested at once: what 256 CUs hold.  Four / eight, us (tokens x slots x columns): 16 x 8 x 2048 3.9 / 2.9, 200 x
+    // 6 x 2048 5.5 / 4.2, 777 x 8 x 2048 (3108) 9.8 / 8.3, 2000 x 4 x 1536 (6000) 8.1 / 8.2, 8192 x 8 x 2048 (32768) 54.2 / 56.6.
+    constexpr int64_t kDeepWaves = 8192;
+    auto launch = [&](auto steps, auto w32) {
+        constexpr bool S = decltype(steps)::value, W = decltype(w32)::value;
+        if (tokens * chunks <= kDeepWaves)
+            hipLaunchKernelGGL((combine_rows_kernel<S, W, 8>), grid, block, 0, st, r, ld_rows / 8, num_rows, row_map, weights, tokens, topk, (int)nvec, (int)chunks, o, ld_out / 8);
+        else
+            hipLaunchKernelGGL((combine_rows_kernel<S, W, 4>), grid, block, 0, st, r, ld_rows / 8, num_rows, row_map, weights, tokens, topk, (int)nvec, (int)chunks, o, ld_out / 8);
+    };
+    if (mode == CFP8_COMBINE_BF16_STEPS) launch(std::true_type{}, std::false_type{});
+    else if (weights_dtype == CFP8_IN_F32) launch(std::false_type{}, std::true_type{});
+    else launch(std::false_type{}, std::false_type{});
     return check_launch("combine_rows");
 }

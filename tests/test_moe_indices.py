@@ -274,6 +274,29 @@ def test_combine_rows_slot_limits(dev):
     assert not bool(out.any())
 
 
+# eight slots at once up to 8192 wavefronts (one a token here), four beyond; rests of one to eight slots
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", [1, 3, 4, 5, 8, 9, 12, 13, 64])
+def test_combine_rows_slots_at_once(dev, K):
+    from cosmos_rl_amd.policy.kernel.moe.moe import TokenRouting, combine_expert_outputs
+    from oracle import c_oracle as CO
+    g = torch.Generator().manual_seed(K)
+    T, H, R = 8193, 72, 300
+    rows = torch.randn(R, H, generator=g).to(torch.bfloat16)
+    rows[3], rows[7, 5], rows[9] = float("-inf"), float("nan"), 0.0
+    row_map = torch.randint(-1, R, (T, K), generator=g, dtype=torch.int32)
+    w = torch.randn(T, K, generator=g).to(torch.bfloat16)
+    order = torch.arange(K).expand(T, K).contiguous()
+    for mode, name in ((0, "steps"), (1, "fp32")):
+        def combine(n):
+            routing = TokenRouting(None, row_map[:n].contiguous().to(dev), order[:n].contiguous().to(dev), None, None)
+            return combine_expert_outputs(rows.to(dev), routing, w[:n].contiguous().to(dev), **({"accumulate": name} if mode else {}))
+        few, many = combine(T - 1), combine(T)
+        want = CO.combine_rows(rows.view(torch.int16).numpy().view("uint16"), row_map[:40].numpy(), w[:40].view(torch.int16).numpy().view("uint16"), mode)
+        assert _same_bf16(few[:40], torch.from_numpy(want.view("int16")).view(torch.bfloat16))
+        assert torch.equal(few.view(torch.int16), many[: T - 1].view(torch.int16))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("T,H,R", [(300, 2048, 1000), (50, 264, 333), (8, 128, 1), (1000, 7168, 513)])
 def test_permute_quantize_tokens_is_gather_then_quant(dev, T, H, R):
