@@ -13,7 +13,7 @@
 // waits for another: a thread's own pair, its weight, its token's other slots and the mask are requested together, before the
 // histograms are, and the mask decides afterwards.  The tokens' 1x128 quantisation, which needs nothing of the routing, runs in workgroups
 // behind its own instead of in a launch behind it.  Routing and quantising, top 8 of 128 experts of 2048: 16 tokens 7.8 + 4.8 us in two
-// launches, 6.5 in one; 777 tokens 4.7 + 8.8 + 5.1 in three, 5.8 + 9.2 in two; 8192 tokens 4.7 + 11.8 + 11.9, 7.0 + 13.0.
+// launches, 6.5 in one; 777 tokens 4.7 + 8.8 + 5.1 in three, 4.9 + 8.2 in two; 8192 tokens 4.7 + 11.8 + 11.9, 7.0 + 13.0.
 // The same layout built from library calls (a stable argsort, a scatter-add for the counts, a sort along the slots,
 // gathers, comparisons and fills, each over 10^2 .. 10^5 elements) is some thirty launches of 2 .. 45 us each:
 // 230-250 us at every size from 16 to 8192 tokens.
