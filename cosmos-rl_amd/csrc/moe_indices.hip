@@ -117,15 +117,18 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const uint4* __restric
 //   STEPS: every product and every partial sum is rounded to bf16, the arithmetic of
 //          `y.scatter_add_(0, idx, expert_out * weights[idx, top, None])` on bf16 tensors;
 //   else:  fp32 accumulator acc = fma(row, weight, acc), rounded to bf16 once.
-//   DEPTH: slots requested at once.  Bound by latency while the chip holds all wavefronts at once, by HBM beyond.
-template <bool STEPS, bool W32, int DEPTH>
+//   DEEP: up to eight slots are requested at once, exactly those that are left, in straight-line code for each count: what takes the time
+//         is latency, while the chip is far from full (combine_is_deep).  Otherwise one slot behind the other: the wavefronts hide each
+//         other's latency, and HBM bounds what is left (5.0 TB/s at 8192 tokens, top 8, 2048 columns).
+template <bool STEPS, bool W32, bool DEEP>
 __global__ __launch_bounds__(256) void combine_rows_kernel(const uint4* __restrict__ rows, int64_t ldr,
                                                            int64_t num_rows, const int32_t* __restrict__ row_map,
                                                            const void* __restrict__ weights, int64_t tokens, int topk, int nvec, int chunks,
                                                            uint4* __restrict__ out, int64_t ldo) {
-    const int64_t unit = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave = DEEP ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
+    const int64_t unit = (int64_t)blockIdx.x * 4 + wave;
     if (unit >= tokens * chunks) return;  // whole wavefronts leave
-    const int64_t t = unit >> 32 ? unit / chunks : (int64_t)((u32)unit / (u32)chunks);
+    const int64_t t = DEEP ? (int64_t)((u32)unit / (u32)chunks) : unit / chunks;
     const int lane = threadIdx.x & 63;
     const int v = (int)(unit - t * chunks) * 64 + lane;
     const int vv = v < nvec ? v : nvec - 1;  // lanes past the row end re-read its last vector and store nothing
@@ -142,38 +145,49 @@ __global__ __launch_bounds__(256) void combine_rows_kernel(const uint4* __restri
     }
     u32 y[4] = {0u, 0u, 0u, 0u};
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    auto walk = [&](auto n_c, int s0) {
-        constexpr int N = decltype(n_c)::value;
-        uint4 d[N];
-        int32_t r[N];
+    auto request = [&](int s) {
+        const int32_t r = __builtin_amdgcn_readlane(src, s);
+        return ld16<true>(rows + (int64_t)(r < 0 ? 0 : r) * ldr + vv);
+    };
+    auto add = [&](uint4 d, int s) {
+        const float ws = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), s));
+        if (__builtin_amdgcn_readlane(src, s) < 0) d = make_uint4(0, 0, 0, 0);
+        const u32 x[4] = {d.x, d.y, d.z, d.w};
 #pragma unroll
-        for (int i = 0; i < N; ++i) {
-            r[i] = __builtin_amdgcn_readlane(src, s0 + i);  // (lanes past topk: no row; s0 + i <= 63)
-            d[i] = ld16<true>(rows + (int64_t)(r[i] < 0 ? 0 : r[i]) * ldr + vv);
-        }
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-            if (s0 + i >= topk) break;
-            const float ws = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), s0 + i));
-            if (r[i] < 0) d[i] = make_uint4(0, 0, 0, 0);
-            const u32 x[4] = {d[i].x, d[i].y, d[i].z, d[i].w};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float lo = __uint_as_float(x[e] << 16), hi = __uint_as_float(x[e] & 0xFFFF0000u);
-                if (STEPS) {
-                    const u32 p = pack_bf16x2(lo * ws, hi * ws);
-                    y[e] = pack_bf16x2(__uint_as_float(y[e] << 16) + __uint_as_float(p << 16),
-                                       __uint_as_float(y[e] & 0xFFFF0000u) + __uint_as_float(p & 0xFFFF0000u));
-                } else {
-                    acc[2 * e] = __builtin_fmaf(lo, ws, acc[2 * e]);
-                    acc[2 * e + 1] = __builtin_fmaf(hi, ws, acc[2 * e + 1]);
-                }
+        for (int e = 0; e < 4; ++e) {
+            const float lo = __uint_as_float(x[e] << 16), hi = __uint_as_float(x[e] & 0xFFFF0000u);
+            if (STEPS) {
+                const u32 p = pack_bf16x2(lo * ws, hi * ws);
+                y[e] = pack_bf16x2(__uint_as_float(y[e] << 16) + __uint_as_float(p << 16),
+                                   __uint_as_float(y[e] & 0xFFFF0000u) + __uint_as_float(p & 0xFFFF0000u));
+            } else {
+                acc[2 * e] = __builtin_fmaf(lo, ws, acc[2 * e]);
+                acc[2 * e + 1] = __builtin_fmaf(hi, ws, acc[2 * e + 1]);
             }
         }
     };
-    for (int s0 = 0; s0 < topk; s0 += DEPTH) {
-        if (DEPTH == 4 || topk - s0 > 4) walk(std::integral_constant<int, DEPTH>{}, s0);
-        else walk(std::integral_constant<int, 4>{}, s0);
+    if constexpr (DEEP) {
+        auto walk = [&](auto n, int s0) {
+            constexpr int N = decltype(n)::value;
+            uint4 d[N];
+#pragma unroll
+            for (int i = 0; i < N; ++i) d[i] = request(s0 + i);
+#pragma unroll
+            for (int i = 0; i < N; ++i) add(d[i], s0 + i);
+        };
+        int s0 = 0;
+        for (; topk - s0 >= 8; s0 += 8) walk(std::integral_constant<int, 8>{}, s0);
+        switch (topk - s0) {
+            case 7: walk(std::integral_constant<int, 7>{}, s0); break;
+            case 6: walk(std::integral_constant<int, 6>{}, s0); break;
+            case 5: walk(std::integral_constant<int, 5>{}, s0); break;
+            case 4: walk(std::integral_constant<int, 4>{}, s0); break;
+            case 3: walk(std::integral_constant<int, 3>{}, s0); break;
+            case 2: walk(std::integral_constant<int, 2>{}, s0); break;
+            case 1: walk(std::integral_constant<int, 1>{}, s0); break;
+        }
+    } else {
+        for (int s = 0; s < topk; ++s) add(request(s), s);
     }
     if (!STEPS) {
 #pragma unroll
@@ -181,6 +195,12 @@ __global__ __launch_bounds__(256) void combine_rows_kernel(const uint4* __restri
     }
     if (v < nvec) st16<true>(out + t * ldo + v, make_uint4(y[0], y[1], y[2], y[3]));
 }
+
+// Where requesting eight slots at once is the faster form: up to 22 wavefronts a CU, two slots and more.  One behind the other / eight at once, us (tokens
+// x slots x columns, rows from HBM): 16 x 8 x 2048 5.9 / 3.3, 200 x 6 x 2048 5.5 / 3.4, 777 x 2 x 2048 4.0 / 3.8, 777 x 8 x 2048 9.9 / 7.8, 1280 x 4 x 2048
+// 7.5 / 6.9, 1400 x 4 x 2048 (5600 wavefronts) 7.8 / 7.7, 1600 x 4 x 2048 (6400) 8.3 / 8.6, 2048 x 4 x 2048 9.4 / 10.1, 8192 x 8 x 2048 54.3 / 55.1; one
+// slot: 16 x 2048 2.0 / 2.1, 777 x 2048 3.1 / 3.2.
+static bool combine_is_deep(int64_t waves, int topk) { return waves <= 5632 && topk >= 2; }
 
 }  // namespace cfp8
 
@@ -253,15 +273,12 @@ extern "C" int cfp8_combine_rows(const void* rows, int64_t ld_rows, int64_t num_
     hipStream_t st = static_cast<hipStream_t>(stream);
     const uint4* r = static_cast<const uint4*>(rows);
     uint4* o = static_cast<uint4*>(out);
-    // Wavefronts up to which eight slots are requested at once: what 256 CUs hold.  Four / eight, us (tokens x slots x columns): 16 x 8 x 2048 3.9 / 2.9, 200 x
-    // 6 x 2048 5.5 / 4.2, 777 x 8 x 2048 (3108) 9.8 / 8.3, 2000 x 4 x 1536 (6000) 8.1 / 8.2, 8192 x 8 x 2048 (32768) 54.2 / 56.6.
-    constexpr int64_t kDeepWaves = 8192;
     auto launch = [&](auto steps, auto w32) {
         constexpr bool S = decltype(steps)::value, W = decltype(w32)::value;
-        if (tokens * chunks <= kDeepWaves)
-            hipLaunchKernelGGL((combine_rows_kernel<S, W, 8>), grid, block, 0, st, r, ld_rows / 8, num_rows, row_map, weights, tokens, topk, (int)nvec, (int)chunks, o, ld_out / 8);
+        if (combine_is_deep(tokens * chunks, topk))
+            hipLaunchKernelGGL((combine_rows_kernel<S, W, true>), grid, block, 0, st, r, ld_rows / 8, num_rows, row_map, weights, tokens, topk, (int)nvec, (int)chunks, o, ld_out / 8);
         else
-            hipLaunchKernelGGL((combine_rows_kernel<S, W, 4>), grid, block, 0, st, r, ld_rows / 8, num_rows, row_map, weights, tokens, topk, (int)nvec, (int)chunks, o, ld_out / 8);
+            hipLaunchKernelGGL((combine_rows_kernel<S, W, false>), grid, block, 0, st, r, ld_rows / 8, num_rows, row_map, weights, tokens, topk, (int)nvec, (int)chunks, o, ld_out / 8);
     };
     if (mode == CFP8_COMBINE_BF16_STEPS) launch(std::true_type{}, std::false_type{});
     else if (weights_dtype == CFP8_IN_F32) launch(std::false_type{}, std::true_type{});
