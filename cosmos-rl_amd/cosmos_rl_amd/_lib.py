@@ -7,6 +7,8 @@ from __future__ import annotations
 
 import ctypes
 import importlib.util
+import sys
+import warnings
 from ctypes import c_char_p, c_float, c_int, c_int32, c_int64, c_size_t, c_void_p, POINTER
 from pathlib import Path
 
@@ -122,13 +124,22 @@ def load() -> ctypes.CDLL:
 
 
 def torch_calls():
-    """The operators' native host path (csrc/torch_calls.cpp), or None where it is not built: they then take the same steps in Python."""
+    """The operators' native host path (csrc/torch_calls.cpp), or None where it is not built or, with a warning, where it is not for this
+    torch and Python: the operators then take the same steps in Python."""
+    import torch
     load()
     if not CALLS_PATH.exists():
         return None
     spec = importlib.util.spec_from_file_location("_torch_calls", CALLS_PATH)
-    module = importlib.util.module_from_spec(spec)
-    spec.loader.exec_module(module)
+    try:
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        here = f"torch {torch.__version__.split('+')[0]}, Python {sys.version_info[0]}.{sys.version_info[1]}"
+        if module.BUILT_FOR != here:
+            raise ImportError(f"built for {module.BUILT_FOR}, not for {here}")
+    except (ImportError, OSError, SystemError, AttributeError) as e:
+        warnings.warn(f"{CALLS_PATH} does not load ({e}): operators of few tokens take the host longer; build it with `python -m cosmos_rl_amd._build`", RuntimeWarning)
+        return None
     return module
 
 

@@ -19,6 +19,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
+#include <torch/version.h>
 
 #include "cosmos_fp8.h"
 
@@ -121,4 +122,15 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_torch_calls", nullptr, -1, kMeth
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__torch_calls() { return PyModule_Create(&kModule); }
+#define CFP8_TEXT_OF(x) #x
+#define CFP8_TEXT(x) CFP8_TEXT_OF(x)
+
+PyMODINIT_FUNC PyInit__torch_calls() {
+    PyObject* const module = PyModule_Create(&kModule);
+    // (tensors are laid out as this torch has them: another one may load this file and read them wrongly)
+    if (module && PyModule_AddStringConstant(module, "BUILT_FOR", "torch " TORCH_VERSION ", Python " CFP8_TEXT(PY_MAJOR_VERSION) "." CFP8_TEXT(PY_MINOR_VERSION)) < 0) {
+        Py_DECREF(module);
+        return nullptr;
+    }
+    return module;
+}

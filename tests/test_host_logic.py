@@ -326,3 +326,31 @@ def test_create_indices_from_offsets():
     # a row bound instead of the exact count: rows past the last group are padding (-1), nothing is read back
     cap = ops.create_indices_from_offsets_nosync(offs, 640, n_experts=3)
     assert torch.equal(cap[:384], idx) and bool((cap[384:] == -1).all())
+
+
+@pytest.mark.parametrize("state", ["built", "missing", "no library", "another torch"])
+def test_native_host_path_that_does_not_load(state, monkeypatch, tmp_path):
+    """Where the operators' native host path cannot be had, they take the steps in Python - which refuse host tensors in their own words -,
+    with one warning if there is a file that does not load."""
+    import warnings
+
+    from cosmos_rl_amd import _lib
+    for name in ("_torch_calls", "_linear_call", "_mxfp4_call"):
+        monkeypatch.setattr(ops, name, None)
+    if state in ("missing", "no library"):
+        path = tmp_path / "_torch_calls.so"
+        if state == "no library":
+            path.write_bytes(b"\x7fELF and no more")
+        monkeypatch.setattr(_lib, "CALLS_PATH", path)
+    elif state == "another torch":
+        monkeypatch.setattr(torch, "__version__", "2.0.1+rocm7.0")
+    x, w, s = torch.zeros(2, 128, dtype=torch.bfloat16), torch.zeros(128, 16).to(torch.float8_e4m3fn), torch.ones(16, 1)
+    codes = (torch.zeros(16, 64, dtype=torch.uint8), torch.zeros(16, 4, dtype=torch.uint8))
+    with warnings.catch_warnings(record=True) as seen:
+        warnings.simplefilter("always")
+        for _ in range(2):
+            for call in (lambda: ops.fp8_linear(x, w, s), lambda: ops.linear_mxfp4(x, codes)):
+                with pytest.raises(RuntimeError, match="on the GPU only"):
+                    call()
+    assert bool(ops._torch_calls) == (state == "built" and _lib.CALLS_PATH.exists())
+    assert len([m for m in seen if "_torch_calls.so" in str(m.message)]) == (state in ("no library", "another torch"))
