@@ -5,11 +5,11 @@ travels with the source checkout; it is never installed into site-packages.
 """
 from __future__ import annotations
 
-import importlib.util
 import os
 import shutil
 import subprocess
 import sysconfig
+import warnings
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -55,18 +55,26 @@ def _compile(src: str) -> Path:
 
 
 def _build_calls() -> None:
-    """The torch extension beside the library, with the host compiler; it is linked to the library that ctypes loads."""
-    torch_dir = Path(importlib.util.find_spec("torch").origin).parent
-    inc, lib = torch_dir / "include", torch_dir / "lib"
+    """The torch extension beside the library, with the host compiler; it is linked to the library that ctypes loads.  The library does
+    without it: where torch, its headers or a compiler for it are missing, the file is left out and a warning says why."""
+    CALLS_PATH.unlink(missing_ok=True)  # (an old one is not for the library just built)
     tmp = CALLS_PATH.with_suffix(".so.tmp")
-    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
-           f"-I{inc}", f"-I{inc / 'torch/csrc/api/include'}", "-I/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}", f"-I{INCLUDE_DIR}",
-           str(CSRC_DIR / "torch_calls.cpp"), "-o", str(tmp), f"-L{lib}", "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip",
-           f"-L{LIB_DIR}", f"-l:{LIB_PATH.name}", "-Wl,-rpath,$ORIGIN"]
-    res = subprocess.run(cmd, capture_output=True, text=True)
-    if res.returncode != 0:
-        raise RuntimeError(f"g++ failed on torch_calls.cpp:\n{res.stdout}\n{res.stderr}")
-    os.replace(tmp, CALLS_PATH)
+    try:
+        import torch
+        torch_dir = Path(torch.__file__).parent
+        inc, lib = torch_dir / "include", torch_dir / "lib"
+        cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+               f"-I{inc}", f"-I{inc / 'torch/csrc/api/include'}", "-I/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}", f"-I{INCLUDE_DIR}",
+               str(CSRC_DIR / "torch_calls.cpp"), "-o", str(tmp), f"-L{lib}", "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip",
+               f"-L{LIB_DIR}", f"-l:{LIB_PATH.name}", "-Wl,-rpath,$ORIGIN"]
+        res = subprocess.run(cmd, capture_output=True, text=True)
+        why = f"g++ failed on torch_calls.cpp:\n{res.stdout}\n{res.stderr}" if res.returncode else ""
+    except (ImportError, OSError) as e:  # no torch, no g++
+        why = str(e)
+    if why:
+        warnings.warn(f"{CALLS_PATH.name} is not built, operators of few tokens take the host longer: {why}", RuntimeWarning)
+    else:
+        os.replace(tmp, CALLS_PATH)
 
 
 def build(verbose: bool = False) -> Path:

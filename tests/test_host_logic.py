@@ -354,3 +354,35 @@ def test_native_host_path_that_does_not_load(state, monkeypatch, tmp_path):
                     call()
     assert bool(ops._torch_calls) == (state == "built" and _lib.CALLS_PATH.exists())
     assert len([m for m in seen if "_torch_calls.so" in str(m.message)]) == (state in ("no library", "another torch"))
+
+
+@pytest.mark.parametrize("lack", ["torch", "compiler", "headers"])
+def test_build_without_the_native_host_path(lack, monkeypatch, tmp_path):
+    """The C library is built and stays in place where the torch extension cannot be, an extension of an earlier build does not."""
+    import sys
+
+    from cosmos_rl_amd import _build
+    monkeypatch.setattr(_build, "LIB_DIR", tmp_path)
+    monkeypatch.setattr(_build, "OBJ_DIR", tmp_path)
+    monkeypatch.setattr(_build, "LIB_PATH", tmp_path / "libcosmosfp8.so")
+    monkeypatch.setattr(_build, "CALLS_PATH", tmp_path / "_torch_calls.so")
+    monkeypatch.setattr(_build, "_compile", lambda src: tmp_path / src)
+    linked = []
+
+    def run(cmd, **kwargs):
+        if cmd[0] == "g++":
+            if lack == "compiler":
+                raise FileNotFoundError("g++")
+            return SimpleNamespace(returncode=1, stdout="", stderr="Python.h: No such file or directory")
+        out = cmd[cmd.index("-o") + 1]
+        open(out, "w").close()
+        linked.append(out)
+        return SimpleNamespace(returncode=0, stdout="", stderr="")
+    monkeypatch.setattr(_build.subprocess, "run", run)
+    monkeypatch.setattr(_build, "hipcc", lambda: "hipcc")
+    if lack == "torch":
+        monkeypatch.setitem(sys.modules, "torch", None)
+    (tmp_path / "_torch_calls.so").write_bytes(b"of an earlier build")
+    with pytest.warns(RuntimeWarning, match="is not built"):
+        assert _build.build() == tmp_path / "libcosmosfp8.so"
+    assert linked and (tmp_path / "libcosmosfp8.so").exists() and not (tmp_path / "_torch_calls.so").exists()
