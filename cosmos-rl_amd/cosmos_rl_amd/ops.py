@@ -566,7 +566,7 @@ def fp8_linear(x: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor
     per-token dynamic quantisation of x, then the rowwise scaled mm.
 
     weight: fp8 [K, N] column-major, i.e. ``qweight.t()`` as the reference stores it;
-    weight_scale [N, 1]; x bf16 [..., K].  Returns [..., N]."""
+    weight_scale [N, 1] or one value; x bf16 [..., K].  Returns [..., N]."""
     if workspace is None:
         out = (_linear_call or _find_linear_call())(x, weight, weight_scale, bias, out_dtype)
         if out is not None:
@@ -577,6 +577,10 @@ def fp8_linear(x: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor
     K, N = weight.shape
     if weight.stride(0) != 1 and K > 1:
         raise ValueError("weight must be the transposed view of a contiguous [N, K] fp8 tensor")
+    if weight.dtype not in (FP8_DTYPE, torch.uint8):
+        raise ValueError(f"weight must be float8_e4m3fn (or its bytes), got {weight.dtype}")
+    if weight_scale.numel() < N and weight_scale.numel() != 1:
+        raise ValueError(f"fp8_linear needs one scale a weight row ({N}) or one for all, got {weight_scale.numel()}")
     # (A product of few tokens is shorter than the calls around it: no view is made of what has the shape already.
     # Four such linears of one token, with the stream's handle as it is taken above: 57.5 -> 40.0 us.)
     flat = x.dim() == 2 and x.shape[1] == K
@@ -593,6 +597,8 @@ def fp8_linear(x: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor
     sw = weight_scale
     if sw.dtype != torch.float32 or not sw.is_contiguous():
         sw = sw.reshape(-1).contiguous().float()
+    if sw.numel() < N:  # one for all: the kernels read one a row
+        sw = sw.reshape(1).expand(N).contiguous()
     out = torch.empty((M, N), dtype=out_dtype, device=x.device)
     ld_x = x2.stride(0) if M > 1 else K
     ld_w = weight.stride(1) if N > 1 else K

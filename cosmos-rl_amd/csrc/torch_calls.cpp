@@ -64,6 +64,7 @@ PyObject* fp8_linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (x->dim() != 2 || w->dim() != 2 || x->scalar_type() != at::kBFloat16 || s->scalar_type() != at::kFloat || !s->is_contiguous()) Py_RETURN_NONE;
     const int64_t M = x->size(0), K = w->size(0), N = w->size(1);
     if (M < 1 || N < 1 || K < 2 || x->size(1) != K || x->stride(1) != 1 || w->stride(0) != 1) Py_RETURN_NONE;
+    if (s->numel() < N || (w->scalar_type() != at::kFloat8_e4m3fn && w->scalar_type() != at::kByte)) Py_RETURN_NONE;
     if (args[3] != Py_None) {
         // what the GEMMs add themselves: one bf16 value a column that torch does not follow
         if (!plain(args[3], b) || b->scalar_type() != at::kBFloat16 || b->dim() != 1 || b->size(0) != N || b->stride(0) != 1 || b->device() != x->device()) Py_RETURN_NONE;

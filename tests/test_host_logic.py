@@ -1,6 +1,7 @@
 """Host-side mirror of the reference's Python callers, on the CPU.  The HIP operators are
 GPU-only, so these tests stand an oracle-backed stub in for ``ops.scaled_fp8_quant`` - the same
 move the reference's own worker tests make with mocks - and check the protocol around it."""
+import ctypes
 from types import SimpleNamespace
 
 import pytest
@@ -386,3 +387,37 @@ def test_build_without_the_native_host_path(lack, monkeypatch, tmp_path):
     with pytest.warns(RuntimeWarning, match="is not built"):
         assert _build.build() == tmp_path / "libcosmosfp8.so"
     assert linked and (tmp_path / "libcosmosfp8.so").exists() and not (tmp_path / "_torch_calls.so").exists()
+
+
+def test_fp8_linear_scales_and_weight_type(monkeypatch):
+    """The library reads one scale a weight row and one byte an element of the weight: fewer scales than rows and wider weights are refused
+    before a call, one scale for all is spread (as in scaled_mm)."""
+    M, N, K = 3, 32, 128
+    seen = []
+
+    class Library:
+        def cfp8_linear_workspace_bytes(self, *args):
+            return 256
+
+        def cfp8_gemm_partial_bytes(self, *args):
+            return 0
+
+        def cfp8_linear_rowwise_split(self, x, ldx, w, ldw, scales, *args):
+            seen.append(list((ctypes.c_float * N).from_address(scales)))
+            return 0
+    monkeypatch.setattr(ops, "_need_gpu", lambda *tensors: None)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(ops, "_linear_call", lambda *args: None)
+    monkeypatch.setattr(ops._lib, "load", lambda: Library())
+    x, w = torch.zeros(M, K, dtype=torch.bfloat16), torch.zeros(N, K).to(torch.float8_e4m3fn).t()
+    whole = torch.arange(N, dtype=torch.float32)
+    for scale, want in ((whole[:, None], whole), (whole.double(), whole), (torch.arange(N + 8.0), whole), (torch.tensor([3.0]), torch.full((N,), 3.0)),
+                        (torch.tensor(3.0, dtype=torch.bfloat16), torch.full((N,), 3.0))):
+        assert ops.fp8_linear(x, w, scale).shape == (M, N) and seen.pop() == want.tolist()
+    ops.fp8_linear(x, w.t().view(torch.uint8).t(), whole)
+    seen.clear()
+    for bad in ((w, whole[:N - 1]), (w, whole[:0]), (torch.zeros(N, K, dtype=torch.bfloat16).t(), whole), (torch.zeros(N, K).t(), whole),
+                (torch.zeros(N, K).to(torch.float8_e5m2).t(), whole)):
+        with pytest.raises(ValueError):
+            ops.fp8_linear(x, *bad)
+    assert not seen

@@ -70,7 +70,7 @@ def test_linear_left_to_the_steps(dev, monkeypatch):
 
     for call in (lambda: ops.fp8_linear(x.reshape(1, M, K), w, s), lambda: ops.fp8_linear(x.t().contiguous().t(), w, s), lambda: ops.fp8_linear(x, w, s.double()),
                  lambda: ops.fp8_linear(x, w, s, bias=b.float()), lambda: ops.fp8_linear(x, w, s, bias=torch.nn.Parameter(b)),
-                 lambda: ops.fp8_linear(x.as_subclass(Sub), w, s).as_subclass(torch.Tensor), lambda: ops.fp8_linear(x[:0], w, s), seen):
+                 lambda: ops.fp8_linear(x.as_subclass(Sub), w, s).as_subclass(torch.Tensor), lambda: ops.fp8_linear(x[:0], w, s), lambda: ops.fp8_linear(x, w, s[:1]), seen):
         one, two, took = _both(call, monkeypatch)
         assert not took
         assert one.shape == two.shape and torch.equal(one, two) and one.requires_grad == two.requires_grad
@@ -91,7 +91,8 @@ def test_refusals(dev, monkeypatch):
     x, w, s, b = _operands(dev, 5, 256, 512)
     pitched = torch.zeros(5, 515, device=dev, dtype=torch.bfloat16)[:, :512]   # rows that are not 16-byte aligned
     for call in (lambda: ops.fp8_linear(pitched, w, s), lambda: ops.fp8_linear(x.half(), w, s), lambda: ops.fp8_linear(x, w, s, out_dtype=torch.float16),
-                 lambda: ops.fp8_linear(x.cpu(), w, s), lambda: ops.fp8_linear(x, w.t(), s)):
+                 lambda: ops.fp8_linear(x.cpu(), w, s), lambda: ops.fp8_linear(x, w.t(), s), lambda: ops.fp8_linear(x, w, s[:-1]),
+                 lambda: ops.fp8_linear(x, torch.zeros(256, 512, device=dev, dtype=torch.bfloat16).t(), s)):
         said = []
         for native in (ops._native("fp8_linear"), lambda *args: None):
             monkeypatch.setattr(ops, "_linear_call", native)
