@@ -236,12 +236,14 @@ constexpr int64_t kFewMaxHidden = 4096, kFewMaxInter = 1536;
 // Mean rows an expert up to which a form is taken.  The few-rows form reads an expert's rows once for every strip of 16
 // features, the middle one once for every 128 columns but holds 64 rows in a tile; from about one of those tiles on the larger
 // tiles of gemm_experts_kernel, whose waves without rows only load, need fewer loads a product and no quantiser in between.
-// Whole calls, few / middle, us: 128 experts of 2048 x 768, top 8: 8 rows an expert 136 / 146, 16: 160 / 151; 32 of 3584 x 1536, top 4:
-// 8: 128 / 130, 16: 152 / 133; 64 of 1024 x 512, top 6: 12: 42 / 44, 24: 50 / 47.  Middle / many: 128 of 2048 x 768: 30: 153 / 158,
-// 40: 160 / 159, 48: 176 / 161, 69: 212 / 172, 156: 312 / 239; 32 of 3584 x 1536: 40: 130 / 145, 50: 140 / 146, 100: 195 / 159; 64 of 1024 x 512:
-// 28: 56 / 54, 56: 68 / 56.
+// Whole calls, few / middle, us: 128 experts of 2048 x 768, top 8: 8 rows an expert 136 / 146, 16: 159 / 139; 32 of 3584 x 1536, top 4:
+// 8: 128 / 130, 24: 175 / 116; 64 of 1024 x 512, top 6: 12: 38.7 / 37.5, 24: 49 / 44.  Middle / many: 128 of 2048 x 768: 30: 146.9 / 145.7,
+// 44: 156 / 145, 48: 163 / 147, 80: 224 / 165; 64 of 2048 x 1024: 40: 101.1 / 102.3, 50: 115 / 104; 64 of 1024 x 512: 34: 45.4 / 45.6, 40: 46.7 / 45.8, 50: 57 / 47.
+// The large tiles are one a CU, in rounds: where the last ones leave many CUs idle, the small ones, two a CU, stay ahead up to where
+// experts come to have a second tile of 64 rows (many_idles): 32 of 3584 x 1536: 45: 121.6 / 129.7, 50: 133.2 / 133.0, 55: 146 / 137; 32 of 3584 x 1280: 46: 118.6 / 124.2,
+// 50: 114.6 / 121.4, 52: 124.9 / 124.5; 32 of 2560 x 1280: 46: 94.9 / 100.1, 50: 97.1 / 100.3; 48 of 3584 x 1408: 46: 177 / 182; 24 of 3584 x 1536: 46: 111 / 120.
 // Where gemm_experts_kernel does not take both products, against the other grouped GEMMs: 128 of 2048 x 768: 96: 233 / 246, 128: 266 / 256.
-constexpr int64_t kFewRowsPerExpert = 10, kMiddleRowsPerExpert = 44, kMiddleRowsElsewhere = 112;
+constexpr int64_t kFewRowsPerExpert = 10, kMiddleRowsPerExpert = 44, kMiddleRowsManyIdle = 50, kMiddleRowsElsewhere = 112;
 // Many rows: up to here an expert has a second tile of 128 rows seldom enough for streaming loads of the weights to pay, if they are
 // more than the memory-side cache holds (those that it holds it keeps from call to call, if loads are cacheable).  Cacheable and
 // streaming, us: 128 experts of 2048 x 768 (604 MB) 48 rows an expert 167 / 161, 69: 179 / 172, 94: 185 / 180, 156: 239 / 288; 64 of 2048 x 1024 (403 MB)
@@ -252,6 +254,19 @@ constexpr int64_t kTileOnceRowsPerExpert = 100, kMemorySideCache = (int64_t)256 
 // 155.6 / 146.5, 49 168.4 / 163.0, 62 194.9 / 203.8, 88 232.6 / 274.3; 32 experts of 3584 x 1536: 32 134.4 / 123.4, 75
 // 190.2 / 214.2.
 constexpr int64_t kOnceRowsPerExpert = 52;
+
+// Whether the last rounds of gemm_experts_kernel's tiles leave enough CUs idle for the middle form to be ahead beyond kMiddleRowsPerExpert.
+// An expert is one row of tiles of 256 columns; a product of less than one round takes a tile's time however many CUs it leaves, and weights that the
+// memory-side cache keeps leave nothing to wait for (32 of 2304 x 1152: 46: 83.2 / 82.6).  What the middle form loses instead grows with
+// the rows: middle / many at 46 rows an expert by idle K steps a CU: 32 of 3584 x 1024 (2.0) 92.1 / 91.2, 40 of 3072 x 1280 (11.8) 126.3 / 125.8, 32 of 3584 x 1536
+// (17.0) 121.6 / 130.0, 32 of 2304 x 1536 (19.5) 97.0 / 100.4, 64 of 2816 x 1152 (18.8) 159 / 157, 64 of 2304 x 1152 (20.3) 136.7 / 136.0, 64 of 3584 x 1152 (25.5) 188 / 190.
+// With more columns of h than of x it is behind (32 of 2304 x 2816: 48: 153 / 148).
+static bool many_idles(int64_t pairs, int64_t experts, int64_t hidden, int64_t inter) {
+    const int64_t cus = cu_count();
+    auto idle = [&](int64_t tiles, int64_t k) { return tiles > cus ? ((tiles + cus - 1) / cus * cus - tiles) * (k / 128) : 0; };
+    const int64_t steps = idle(experts * (inter / 128), hidden) + idle(experts * ((hidden + 255) / 256), inter);
+    return inter <= hidden && experts * 3 * hidden * inter > kMemorySideCache && steps * 112 >= pairs * cus;
+}
 
 enum class Form { kFew, kMiddle, kMany };
 struct ExpertsPlan {
@@ -266,8 +281,9 @@ static ExpertsPlan experts_plan(int64_t tokens, int topk, int experts, int64_t h
     ExpertsPlan p{};
     const int64_t pairs = tokens * topk;
     p.gathers = experts_gate_up_takes(tokens, hidden, inter);
+    const int64_t middle = !p.gathers || !experts_down_takes(hidden, inter) ? kMiddleRowsElsewhere : many_idles(pairs, experts, hidden, inter) ? kMiddleRowsManyIdle : kMiddleRowsPerExpert;
     if (pairs <= kFewRowsPerExpert * experts && hidden <= kFewMaxHidden && inter <= kFewMaxInter) p.form = Form::kFew;
-    else if (pairs <= (p.gathers && experts_down_takes(hidden, inter) ? kMiddleRowsPerExpert : kMiddleRowsElsewhere) * experts && ring_grouped_takes(hidden) && ring_grouped_takes(inter) && tokens * hidden < (int64_t)1 << 31) p.form = Form::kMiddle;
+    else if (pairs <= middle * experts && ring_grouped_takes(hidden) && ring_grouped_takes(inter) && tokens * hidden < (int64_t)1 << 31) p.form = Form::kMiddle;
     else p.form = Form::kMany;
     const bool many = p.form == Form::kMany;
     p.slots = pairs < experts ? pairs : experts;

@@ -180,3 +180,16 @@ def test_dispatch_info_rejects_bad_arguments():
     assert lib.cfp8_gemm_dispatch_info(GRP, 128, 256, 128, 0, 256, S, buf, 64) == L.EINVAL      # no partial sums there
     # a short buffer truncates, it does not overflow
     assert lib.cfp8_gemm_dispatch_info(ROW, 8192, 18944, 3584, 0, 256, 0, buf, 16) == 0 and len(buf.value) == 15
+
+
+# hidden, inter, experts, top k, rows an expert up to which tiles of 64 rows are taken: 44, or 50 where the last rounds of the large tiles would leave
+# many CUs idle (behind by 4 to 7 % there), or 112 where gemm_experts_kernel does not take both products
+@pytest.mark.parametrize("H,I,E,topk,rows", [(3584, 1536, 32, 4, 50), (2560, 1280, 32, 8, 50), (3584, 1408, 48, 6, 50), (3584, 1024, 32, 4, 44), (2304, 1152, 32, 4, 44), (2304, 2816, 32, 4, 44),
+                                             (2816, 1152, 64, 4, 44), (2048, 768, 128, 8, 44), (1024, 512, 64, 4, 44), (2048, 384, 64, 4, 112)])
+def test_moe_experts_leave_the_tiles_of_64_rows(H, I, E, topk, rows):
+    """The form is seen in its workspace: rows padded to tiles of 128 take more."""
+    size = lambda T: L.load().cfp8_moe_experts_workspace_bytes(T, topk, E, H, I)
+    first = rows * E // topk
+    tokens = range(12 * E // topk, 120 * E // topk)
+    jumps = [T for T in tokens if size(T + 1) > 1.2 * size(T)]
+    assert jumps == [first]
