@@ -70,6 +70,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
     constexpr int XS = kExXS, STAGE = kExStage;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     typedef __attribute__((address_space(3))) void lds_void;
+    // (tiles are dealt to the XCDs in contiguous ranges: those of padding behind the last group, up to the bound, would all be the last XCD's)
     const int bound = p.tiles_m, held = scalar_table_load(p.rows_end, 0) >> 7;
     const int tiles_m = held < bound ? held : bound;
     const int ntiles = tiles_m * p.tiles_n;

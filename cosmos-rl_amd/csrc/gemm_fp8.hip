@@ -2718,8 +2718,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
     constexpr int A_IT = BM / 64, B_IT = BN / 64;
     constexpr int NB = BN / 128;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    const int tiles_m = MODE == kGrouped ? grouped_tile_rows(p, p.tiles_m) : p.tiles_m;
-    const int ntiles = tiles_m * p.tiles_n;
+    const int ntiles = p.tiles_m * p.tiles_n;
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wm = wave % WM, wn = wave / WM;
@@ -2737,7 +2736,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
     typedef __attribute__((address_space(3))) void lds_void;
     auto tile_expert = [&](int pid) {  // grouped: the expert of the tile's rows, negative for a tile of padding
         int tm, tn;
-        tile_of_block<MODE == kGrouped ? kGroupedBandRows : 8>(pid, tiles_m, p.tiles_n, tm, tn);
+        tile_of_block<MODE == kGrouped ? kGroupedBandRows : 8>(pid, p.tiles_m, p.tiles_n, tm, tn);
         return scalar_table_load(p.m_indices, tm * BM);  // groups start on multiples of 128 = BM rows
     };
     auto next_tile = [&](int pid) {  // the next tile of this workgroup that is not padding
@@ -2748,7 +2747,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
     };
     auto tile_rsrc = [&](int pid, int& m0, int& n0, int& expert, __amdgpu_buffer_rsrc_t& ra, __amdgpu_buffer_rsrc_t& rb) {
         int tm, tn;
-        tile_of_block<MODE == kGrouped ? kGroupedBandRows : 8>(pid, tiles_m, p.tiles_n, tm, tn);
+        tile_of_block<MODE == kGrouped ? kGroupedBandRows : 8>(pid, p.tiles_m, p.tiles_n, tm, tn);
         m0 = tm * BM;
         n0 = tn * BN;
         expert = MODE == kGrouped ? scalar_table_load(p.m_indices, m0) : 0;
@@ -3814,9 +3813,10 @@ extern "C" int cfp8_gemm_block128_split(const void* a, int64_t ld_a, const float
     return launch_block_best(p, out_dtype, static_cast<hipStream_t>(stream));
 }
 
-namespace cfp8 {
-int grouped_block128(const void* a, int64_t ld_a, const float* sa, const void* b, const float* sb, const int32_t* m_indices, const int32_t* rows_end,
-                     void* out, int64_t ld_out, int out_dtype, int64_t M, int64_t N, int64_t K, int64_t E, void* stream) {
+extern "C" int cfp8_gemm_grouped_block128(const void* a, int64_t ld_a, const float* sa, const void* b,
+                                          const float* sb, const int32_t* m_indices, void* out, int64_t ld_out,
+                                          int out_dtype, int64_t M, int64_t N, int64_t K, int64_t E, void* stream) {
+    using namespace cfp8;
     if (int rc = check_common("gemm_grouped_block128", a, b, sa, sb, out, ld_a, K, ld_out, out_dtype, M, N, K)) return rc;
     if (M == 0 || N == 0) return CFP8_OK;
     if (!m_indices) return set_error(CFP8_EINVAL, "gemm_grouped_block128: null m_indices");
@@ -3830,7 +3830,6 @@ int grouped_block128(const void* a, int64_t ld_a, const float* sa, const void* b
     p.sa = sa;
     p.sb = sb;
     p.m_indices = m_indices;
-    p.rows_end = rows_end;
     p.out = out;
     p.ld_a = ld_a; p.ld_b = K; p.ld_out = ld_out;
     const int64_t nb = (N + 127) / 128, kb = K / 128;
@@ -3839,8 +3838,10 @@ int grouped_block128(const void* a, int64_t ld_a, const float* sa, const void* b
     return launch_gemm<kGrouped>(p, out_dtype, static_cast<hipStream_t>(stream));
 }
 
-int grouped_swiglu_quant(const void* a, int64_t ld_a, const float* sa, const void* b, const float* sb, const int32_t* m_indices, const int32_t* rows_end,
-                         void* q, int64_t ld_q, float* scales, int64_t M, int64_t I, int64_t K, int64_t E, void* stream) {
+extern "C" int cfp8_gemm_grouped_swiglu_quant(const void* a, int64_t ld_a, const float* sa, const void* b, const float* sb,
+                                              const int32_t* m_indices, void* q, int64_t ld_q, float* scales,
+                                              int64_t M, int64_t I, int64_t K, int64_t E, void* stream) {
+    using namespace cfp8;
     if (M < 0 || I < 0 || K < 0) return set_error(CFP8_EINVAL, "gemm_grouped_swiglu_quant: negative shape");
     if (M == 0 || I == 0) return CFP8_OK;
     if (int rc = check_common("gemm_grouped_swiglu_quant", a, b, sa, sb, q, ld_a, K, 2 * I, CFP8_OUT_BF16, M, 2 * I, K)) return rc;
@@ -3858,7 +3859,6 @@ int grouped_swiglu_quant(const void* a, int64_t ld_a, const float* sa, const voi
     p.sa = sa;
     p.sb = sb;
     p.m_indices = m_indices;
-    p.rows_end = rows_end;
     p.out = q;
     p.h_scales = scales;
     p.ld_hs = I / 128;
@@ -3867,17 +3867,4 @@ int grouped_swiglu_quant(const void* a, int64_t ld_a, const float* sa, const voi
     p.sb_stride_n = kb; p.sb_stride_k = 1; p.sb_stride_e = nb * kb;
     p.M = (int)M; p.N = (int)(2 * I); p.K = (int)K;
     return launch_grouped_swiglu(p, static_cast<hipStream_t>(stream));
-}
-}  // namespace cfp8
-
-extern "C" int cfp8_gemm_grouped_block128(const void* a, int64_t ld_a, const float* sa, const void* b,
-                                          const float* sb, const int32_t* m_indices, void* out, int64_t ld_out,
-                                          int out_dtype, int64_t M, int64_t N, int64_t K, int64_t E, void* stream) {
-    return cfp8::grouped_block128(a, ld_a, sa, b, sb, m_indices, nullptr, out, ld_out, out_dtype, M, N, K, E, stream);
-}
-
-extern "C" int cfp8_gemm_grouped_swiglu_quant(const void* a, int64_t ld_a, const float* sa, const void* b, const float* sb,
-                                              const int32_t* m_indices, void* q, int64_t ld_q, float* scales,
-                                              int64_t M, int64_t I, int64_t K, int64_t E, void* stream) {
-    return cfp8::grouped_swiglu_quant(a, ld_a, sa, b, sb, m_indices, nullptr, q, ld_q, scales, M, I, K, E, stream);
 }

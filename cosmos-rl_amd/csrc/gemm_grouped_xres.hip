@@ -12,8 +12,6 @@
 
 namespace cfp8 {
 
-constexpr int kXresUnitCost = 1;  // starting a unit costs about as much as a tile
-
 // ---------------------------------------------------------------------------
 // Grouped block-scaled GEMM for a short K (K / 128 = 5 or 6: the down projection of a MoE expert, K = the
 // intermediate size), 128 x 256 tiles, FOUR wavefronts (one per SIMD, all 512 registers each).  With so few K steps a
@@ -78,14 +76,6 @@ constexpr int xres_allowed(int k) {
     return n;
 }
 
-// unit_plan's choice of `parts` for `rem` tile rows, one count a lane (up to 64), where the rows are known on the device only.
-__device__ __forceinline__ int wave_unit_parts(int rem, int tiles_n, int cus, int lane) {
-    const int q = lane + 1;
-    const u32 rounds = ((u32)(rem * q) + cus - 1) / cus;
-    const u32 cost = q <= tiles_n ? rounds * (u32)((tiles_n + q - 1) / q + kXresUnitCost) : 0xFFFFFFu;
-    return 64 - (int)(wave_max(~((cost < 0xFFFFFFu ? cost : 0xFFFFFFu) << 6 | (u32)lane)) & 63u);
-}
-
 template <int KT, bool OUT_F32>
 __global__ __launch_bounds__(256) void gemm_grouped_xres_kernel(const GemmArgs p) {
     static_assert(KT >= 5 && KT <= 6, "5 or 6 K steps: the activation fragments stay in registers, and a tile leaves in four of the next tile's steps");
@@ -102,11 +92,9 @@ __global__ __launch_bounds__(256) void gemm_grouped_xres_kernel(const GemmArgs p
     const int lrow = lane & 15, quarter = lane >> 4;
     const int tiles_n = p.tiles_n;
     const int G = (int)gridDim.x;
-    const int tiles_m = grouped_tile_rows(p, p.tiles_m);
-    const int big = tiles_m / G * G;  // tile rows that are units of their own
-    // pieces of each of the remaining tile rows
-    const int parts = tiles_m == p.tiles_m ? p.unit_parts : wave_unit_parts(tiles_m - big, tiles_n, G, lane);
-    const int units = big + (tiles_m - big) * parts;
+    const int big = p.tiles_m / G * G;  // tile rows that are units of their own
+    const int parts = p.unit_parts;     // pieces of each of the remaining tile rows
+    const int units = big + (p.tiles_m - big) * parts;
     typedef __attribute__((address_space(3))) void lds_void;
     constexpr int kWaitVm0 = 0x0F70;  // s_waitcnt vmcnt(0), the other counters left alone
 
@@ -497,13 +485,13 @@ __global__ __launch_bounds__(256) void gemm_grouped_xres_kernel(const GemmArgs p
 
 // Worth it from about 60 % of the tile slots filled (8 experts, 131 tile rows of 8 tiles, 45 % filled: 68 us against
 // 62 us on the one-tile-per-workgroup kernel; 286 tile rows, 81 %: 100 against 124 us).
-bool grouped_xres_pays(const GemmArgs& p) { return unit_plan(p.M / 128, p.N / 256, cu_count(), kXresUnitCost).fill >= 0.6; }
+bool grouped_xres_pays(const GemmArgs& p) { return unit_plan(p.M / 128, p.N / 256, cu_count(), 1).fill >= 0.6; }
 
 template <int KT>
 static int launch_grouped_xres_kt(GemmArgs& p, int out_dtype, hipStream_t st) {
     p.tiles_m = p.M / 128;
     p.tiles_n = p.N / 256;
-    const UnitPlan plan = unit_plan(p.tiles_m, p.tiles_n, cu_count(), kXresUnitCost);
+    const UnitPlan plan = unit_plan(p.tiles_m, p.tiles_n, cu_count(), 1);
     const int parts = plan.parts;
     const int64_t blocks = plan.blocks;
     p.unit_parts = parts;

@@ -35,8 +35,6 @@ struct GemmArgs {
     // gemm_rowwise_edge_kernel: bf16 [N] or null; quarter tiles below the last row of tiles and beside their last column
     const uint16_t* bias;
     int edge_rows, edge_cols;
-    // grouped, or null: on the device, how many of the M rows the groups take (a multiple of 128; the rest is padding)
-    const int32_t* rows_end;
 };
 
 // ---- host side (gemm_fp8.hip) ---------------------------------------------
@@ -47,11 +45,6 @@ int device_slot();                                                              
 int cu_count();                                                                   // compute units of the current device
 // what cfp8_gemm_mxfp4 (`split`: cfp8_gemm_mxfp4_split) launches for a problem, with every operand at `any`; while dry_run()
 int mx4_dispatch(const void* any, int64_t M, int64_t N, int64_t K, int out_dtype, bool split, size_t partial_bytes);
-// cfp8_gemm_grouped_block128 and cfp8_gemm_grouped_swiglu_quant for a caller that knows where the groups end (GemmArgs::rows_end)
-int grouped_block128(const void* a, int64_t ld_a, const float* sa, const void* b, const float* sb, const int32_t* m_indices, const int32_t* rows_end,
-                     void* out, int64_t ld_out, int out_dtype, int64_t M, int64_t N, int64_t K, int64_t E, void* stream);
-int grouped_swiglu_quant(const void* a, int64_t ld_a, const float* sa, const void* b, const float* sb, const int32_t* m_indices, const int32_t* rows_end,
-                         void* q, int64_t ld_q, float* scales, int64_t M, int64_t I, int64_t K, int64_t E, void* stream);
 size_t block_partial_bytes(int64_t M, int64_t N, int64_t K);                      // of the block-scaled product's slices of K
 
 // ---- gemm_experts.hip
@@ -154,17 +147,6 @@ __device__ __forceinline__ void tile_of_block(int pid, int tiles_m, int tiles_n,
     const int in = lin - g * band;
     tm = first + in % gsz;
     tn = in / gsz;
-}
-
-// Rows of tiles of a grouped product that hold rows of a group: `bound` where the caller knows no better.  Walking kernels deal
-// tiles to the XCDs in contiguous ranges, so that tiles of padding behind the last group all fall to the last XCD and the
-// others take its share: 8192 tokens, top 8 of 128 experts of 2048 x 768 (566 rows of tiles, the bound is 639) 568.5 us
-// a call by the bound, 536.3 by the count.
-__device__ __forceinline__ int grouped_tile_rows(const GemmArgs& p, int bound) {
-    const int32_t* const end = p.rows_end;
-    if (!end) return bound;
-    const int rows = scalar_table_load(end, 0) >> 7;
-    return rows < bound ? rows : bound;
 }
 
 }  // namespace cfp8

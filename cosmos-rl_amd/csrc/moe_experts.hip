@@ -400,8 +400,8 @@ extern "C" int cfp8_moe_experts(const void* x, int64_t ld_x, int64_t tokens, int
         } else {
             if (int rc = cfp8_scatter_quant_group128(x, ld_x, tokens, hidden, i32(p.row_map), topk, i32(p.row_tokens), p.rows, ws + p.xq, hidden, f32(p.xs), stream))
                 return rc;
-            if (int rc = grouped_swiglu_quant(ws + p.xq, hidden, f32(p.xs), gate_up, gate_up_scales, i32(p.row_experts), rows_end, ws + p.hq, inter,
-                                              f32(p.hs), p.rows, inter, hidden, experts, stream))
+            if (int rc = cfp8_gemm_grouped_swiglu_quant(ws + p.xq, hidden, f32(p.xs), gate_up, gate_up_scales, i32(p.row_experts), ws + p.hq, inter,
+                                                        f32(p.hs), p.rows, inter, hidden, experts, stream))
                 return rc;
         }
         if (experts_down_takes(hidden, inter)) {
@@ -411,8 +411,8 @@ extern "C" int cfp8_moe_experts(const void* x, int64_t ld_x, int64_t tokens, int
             d.N = (int)hidden; d.K = (int)inter;
             if (int rc = launch_experts_down(d, p.rows, once, st)) return rc;
         } else {
-            if (int rc = grouped_block128(ws + p.hq, inter, f32(p.hs), down, down_scales, i32(p.row_experts), rows_end, ws + p.out, hidden, CFP8_OUT_BF16,
-                                          p.rows, hidden, inter, experts, stream))
+            if (int rc = cfp8_gemm_grouped_block128(ws + p.hq, inter, f32(p.hs), down, down_scales, i32(p.row_experts), ws + p.out, hidden, CFP8_OUT_BF16,
+                                                    p.rows, hidden, inter, experts, stream))
                 return rc;
         }
     }
