@@ -300,16 +300,17 @@ __global__ __launch_bounds__(256) void scatter_group128_kernel(const uint4* __re
     }
 }
 
-// Groups up to which a thread takes one, not four.  Four / one, us: 12 groups 2.7 / 1.7, 1344 (24 rows of 7168) 3.0 / 2.0, 11200 3.7 / 3.0, 56000 7.4 / 6.6,
-// 112000 11.5 / 11.2, 131072 (8192 rows of 2048) 12.6 / 12.4, 229376 19.1 / 19.4, 458752 33.7 / 36.7.
-constexpr u32 kFewGroups = 1u << 17;
+// Groups up to which a thread takes one, not four.  Four / one, us (rows from HBM, launches one behind the other): 1 group 2.4 / 1.7, 1344 (24 rows of 7168)
+// 3.1 / 1.9, 28000 5.2 / 4.3, 56000 7.8 / 6.9, 100000 11.5 / 10.9, 120000 12.7 / 12.3, 131072 (8192 rows of 2048) 13.1 / 13.1, 229376 19.1 / 19.4, 458752
+// 33.7 / 36.7.  By reciprocal (fewer instructions a group): 1344 2.8 / 1.9, 56000 7.4 / 6.7, 100000 11.1 / 10.9, 110000 11.6 / 11.4, 120000 12.2 / 12.2, 131072 12.6 / 13.0.
+constexpr u32 few_groups(int mode) { return mode == CFP8_GROUP_MODE_DIV ? 1u << 17 : 7u << 14; }
 
 // Groups are numbered in 32 bits, and a block's first group index must not wrap.
 int launch_quant_group128(const void* x, int64_t rows, int64_t cols, int64_t ld_x, void* q, int64_t ld_q,
                           float* scales, int mode, hipStream_t st) {
     if (rows * ((cols + 127) / 128) > kMaxGroups) return set_error(CFP8_EINVAL, "quant_group128: too many groups for one launch");
     const GroupRows p = group_rows(x, rows, cols, ld_x, q, ld_q, scales);
-    const bool few = p.total_groups <= kFewGroups;
+    const bool few = p.total_groups <= few_groups(mode);
     const u32 per = few ? 16 : 64;  // groups a workgroup
     const dim3 grid((p.total_groups - 1) / per + 1), block(256);
     if (mode == CFP8_GROUP_MODE_DIV && few) hipLaunchKernelGGL((group128_kernel<CFP8_GROUP_MODE_DIV, 1>), grid, block, 0, st, p, nullptr);

@@ -622,8 +622,8 @@ def test_group128(dev, shape):
     assert_bytes(q, qo, f"group {shape} bytes")
 
 
-# a group a thread of sixteen up to 131072 groups, four beyond; the last workgroup partly filled
-@pytest.mark.parametrize("shape", [(16384, 1024), (16385, 1024), (65537, 200), (13, 1160)])
+# a group a thread of sixteen up to 131072 groups (114688 by reciprocal), four beyond; the last workgroup partly filled
+@pytest.mark.parametrize("shape", [(14336, 1024), (14337, 1024), (16384, 1024), (16385, 1024), (65537, 200), (13, 1160)])
 def test_group128_groups_a_thread(dev, shape):
     x = O.make_activation(*shape, seed=5, chan_outlier_frac=0.01, outlier_mul=30.0)
     x[-1, :8] = 0
