@@ -2294,10 +2294,10 @@ __global__ __launch_bounds__(256) void linear_gemv_fused_kernel(const uint4* __r
 // (tokens x rows x K), in one launch with the quantiser: 1 x 896 x 4864 6.5 / 5.0 / 4.6, 1 x 1024 x 8192 8.4 / 6.4 / 5.8, 4 x 896 x 4096 7.4 / 6.5 / 6.3, 2 x 896 x 896
 // 3.5 / 3.3 / 3.4, 1 x 1536 x 8192 8.8 / 7.1 / 7.8, 1 x 2048 x 2048 3.9 / 3.5 / 3.8, 1 x 2560 x 2048 4.1 / 4.2 / 4.2, 4 x 4096 x 2048 5.9 / 6.4 / 7.8. The product alone:
 // 16 x 896 x 4864 7.5 / 6.8 / 6.4, 16 x 1024 x 4096 6.7 / 5.7 / 5.5, 12 x 1152 x 896 3.0 / 2.9 / 3.3, 16 x 896 x 896 3.1 / 3.0 / 3.1, 8 x 2048 x 5632 7.8 / 7.1 / 9.0, 16 x 2048 x 2048
-// 4.4 / 4.1 / 5.4, 16 x 2560 x 2048 4.5 / 5.5 / 6.7.
+// 4.4 / 4.1 / 5.4, 16 x 2560 x 2048 4.5 / 5.5 / 6.7.  With one or two K steps there is nothing to share out: 16 / 8 rows, 1 x 16 x 128 2.0 / 2.2, 4 x 16 x 256 3.4 / 3.6.
 static int gemv_rows(const GemmArgs& p) {
     const int cus = cu_count();
-    if (p.ld_b > (1 << 26)) return 16;  // (32-bit offsets of up to 8 rows)
+    if (p.K <= 256 || p.ld_b > (1 << 26)) return 16;  // (32-bit offsets of up to 8 rows)
     return p.N <= 4 * cus && p.K > 2048 ? 4 : p.N <= 8 * cus ? 8 : 16;
 }
 

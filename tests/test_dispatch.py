@@ -167,6 +167,13 @@ def test_dispatch_of_the_operators(name, args, flags, want):
     assert len(got) == len(want) and all(w in g for w, g in zip(want, got)), got
 
 
+@pytest.mark.parametrize("N,K,rows", [(16, 128, 16), (1024, 256, 16), (16, 384, 8), (2048, 2048, 8), (1024, 2176, 4), (1040, 2176, 8), (2064, 2176, 16)])
+def test_weight_rows_a_workgroup_of_the_gemv_kernels(N, K, rows):
+    """One or two K steps leave nothing to share out among more workgroups (3 to 6 % behind there)."""
+    assert f"grid={N // rows} " in L.gemm_dispatch_info(LIN, 1, N, K)
+    assert f"gemm_rowwise_gemv grid={N // rows} " in L.gemm_dispatch_info(LIN, 16, N, K)
+
+
 def test_dispatch_info_rejects_bad_arguments():
     lib = L.load()
     import ctypes
