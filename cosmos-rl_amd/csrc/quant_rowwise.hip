@@ -252,10 +252,14 @@ static bool with_row_variant(RowVariant rv, F&& f) {
     return false;
 }
 
-// Rows up to which a workgroup a row is the faster one, wave or 256 threads / this, us: 3584 columns 33 rows 3.6 / 2.7, 512 4.0 / 3.5, 1111
-// 5.9 / 5.4, 2048 7.1 / 7.6; 2304: 64 3.4 / 2.6, 2048 6.0 / 6.4; 896: 64 2.8 / 2.5, 1111 3.2 / 3.0, 2048 3.4 / 3.5; 4864: 33 3.2 / 3.0, 256 3.4 / 3.3, 400
-// 3.8 / 4.0, 2048 7.3 / 10.6; 18944: 33 4.4 / 3.8, 256 6.4 / 6.1, 512 7.6 / 7.6, 777 10.3 / 11.2.
-static bool few_rows(int64_t rows, int64_t nvec) { return nvec > 64 && nvec <= 4096 && rows <= (nvec <= 512 ? 1280 : 256); }
+// Rows up to which a workgroup a row is the faster one, wave or 256 threads / this, us (rows from HBM, launches one behind the other): 1024 columns 768 rows
+// 2.73 / 2.72, 1000 2.78 / 2.83, 1280 2.99 / 3.10; 2304: 16 2.9 / 2.3, 700 3.50 / 3.34, 1200 4.58 / 4.50, 1280 4.64 / 4.69; 3584: 512 4.0 / 3.5, 1280 5.8 / 5.3, 2048
+// 7.1 / 7.6; 4096: 1280 6.5 / 5.7; 4864: 120 2.8 / 2.7, 256 3.11 / 3.08, 400 3.8 / 4.0, 2048 7.3 / 10.6; 18944: 100 4.5 / 4.2, 256 5.7 / 5.5, 512 7.6 / 7.6, 777
+// 10.3 / 11.2.  (Between 256 and 320 vectors nearly half of 512 threads have none.)
+static bool few_rows(int64_t rows, int64_t nvec) {
+    const int64_t most = nvec <= 128 ? 768 : nvec <= 256 ? 1280 : nvec < 320 ? 1200 : nvec <= 512 ? 1280 : 256;
+    return nvec > 64 && nvec <= 4096 && rows <= most;
+}
 
 // streaming_out: write the fp8 bytes with non-temporal stores (weights, consumed much
 // later); false keeps them cacheable (activations feeding the GEMM of the same call).

@@ -9,8 +9,8 @@ from oracle import fp8_oracle as O
 pytestmark = pytest.mark.gpu
 
 
-# rows on either side of the line (1280 up to 4096 columns, 256 beyond), one to four vectors a thread, the last of them partly filled
-@pytest.mark.parametrize("K,rows", [(512, (5, 33)), (528, (5, 1280, 1281)), (1040, (7, 100)), (2064, (1280, 1281)), (4096, (64,)), (4112, (5, 256, 257)), (8208, (17, 256, 257)),
+# rows on either side of the line (768 up to 1024 columns, 1200 from 2064 to 2552, 1280 up to 4096, 256 beyond), one to four vectors a thread, the last of them partly filled
+@pytest.mark.parametrize("K,rows", [(512, (5, 33)), (528, (5, 768, 769)), (1040, (7, 1280, 1281)), (2064, (1200, 1201)), (2560, (1280, 1281)), (4096, (64,)), (4112, (5, 256, 257)), (8208, (17, 256, 257)),
                                     (16400, (256,)), (18944, (33, 257)), (32768, (9,)), (32784, (9,))])
 def test_linear_has_the_bits_of_the_two_steps(dev, K, rows):
     q, s = ops.quant_rowwise(O.make_weight((32, K), seed=3).to(dev))
@@ -26,8 +26,8 @@ def test_linear_has_the_bits_of_the_two_steps(dev, K, rows):
             assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(7.0), want.nan_to_num(7.0)), M
 
 
-# one launch for up to 4 tokens: 4, 8 or 16 weight rows a workgroup, by 1024 and 2048 rows and 2048 columns, beside the two steps
-@pytest.mark.parametrize("N,K", [(16, 128), (16, 2176), (1008, 2048), (1024, 2176), (1024, 4096), (1040, 4096), (2048, 896), (2064, 2176), (896, 4864), (2048, 8192), (1040, 8192)])
+# one launch for up to 4 tokens: 4, 8 or 16 weight rows a workgroup, by 1024 and 2048 rows and 256 and 2048 columns, beside the two steps
+@pytest.mark.parametrize("N,K", [(16, 128), (64, 256), (64, 384), (16, 2176), (1008, 2048), (1024, 2176), (1024, 4096), (1040, 4096), (2048, 896), (2064, 2176), (896, 4864), (2048, 8192), (1040, 8192)])
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
 def test_one_launch_linear(dev, N, K, dt):
     w = O.make_weight((N, K), seed=4).to(dev)
@@ -45,7 +45,7 @@ def test_one_launch_linear(dev, N, K, dt):
 
 
 # up to 16 tokens: 4, 8 or 16 weight rows a workgroup, one and several chunks of K; a column's bits do not depend on how many rows lie beside it
-@pytest.mark.parametrize("K", [128, 896, 2048, 2176, 4864, 8192])
+@pytest.mark.parametrize("K", [128, 384, 896, 2048, 2176, 4864, 8192])
 @pytest.mark.parametrize("M", [1, 2, 5, 16])
 def test_product_of_few_tokens(dev, M, K):
     q, s = ops.quant_rowwise(O.make_weight((4096, K), seed=6).to(dev))
