@@ -91,6 +91,27 @@ def test_one_call_experts_many_rows(dev, T, E, topk, H, I, keep):
     assert not bool(y[~mask].any())
 
 
+# infinities and NaN, from a token and from a weight, and products beyond bf16: they stay in their rows, on tiles of which a half is padding as well
+@pytest.mark.parametrize("T,E,topk,H,I", [(700, 16, 4, 640, 512), (300, 5, 2, 1024, 768), (300, 5, 2, 1024, 384)])
+def test_one_call_experts_of_values_that_are_no_numbers(dev, T, E, topk, H, I):
+    from cosmos_rl_amd.policy.kernel.moe.moe import grouped_experts_forward
+    strategy, module = _module(dev, E, H, I, T)
+    g = torch.Generator(device=dev).manual_seed(T + 5)
+    x = torch.randn(T, H, generator=g, device=dev).to(torch.bfloat16)
+    x[1, 3], x[2, 5], x[3, 7], x[4], x[5] = float("inf"), float("nan"), float("-inf"), 3e38, 0.0
+    module.get_parameter("down_proj_scales").data[E - 1, 0, 0] = float("inf")
+    idx = torch.rand(T, E, generator=g, device=dev).topk(topk, dim=1).indices
+    w = torch.rand(T, topk, generator=g, device=dev).to(torch.bfloat16)
+    mask = torch.rand(T, generator=g, device=dev) < 0.9
+    mask[:6] = True
+    y = grouped_experts_forward(x, mask, w, idx, strategy, module, E)
+    want = _chain(x, mask, w, idx, strategy, module, E)
+    assert torch.equal(y.isnan(), want.isnan()) and torch.equal(y.nan_to_num(7.0), want.nan_to_num(7.0))
+    plain = (idx != E - 1).all(1)
+    plain[1:5] = False
+    assert bool(y[2].isnan().all()) and bool(y[plain].isfinite().all()) and not bool(y[~mask].any())
+
+
 # the tokens are quantised by workgroups behind the routing's, 64 groups each, or 256, four in turn a thread, where there are more than 32768: one
 # launch up to 1024 pairs, two beyond, of which the first has a quarter of those workgroups; rows of tokens that do not follow each other
 @pytest.mark.parametrize("T,topk,H", [(1, 1, 128), (3, 8, 128), (51, 4, 640), (52, 4, 640), (128, 8, 640), (129, 8, 640), (1025, 1, 128), (410, 3, 1280), (1639, 2, 640), (4096, 1, 1024), (4097, 1, 1024), (3641, 2, 1152)])

@@ -77,6 +77,51 @@ def test_linear_left_to_the_steps(dev, monkeypatch):
     assert Seen.calls
 
 
+@pytest.mark.filterwarnings("ignore")
+def test_watched_and_wrapped_calls_are_left_to_the_steps(dev, monkeypatch):
+    """A dispatch mode sees the calls, tracing and torch.func's wrappers end as they do step by step (with an error where a wrapped tensor has
+    no memory); tokens with a tangent give the plain result either way."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+    M, N, K = 5, 256, 512
+    x, w, s, _ = _operands(dev, M, N, K)
+    weight = ops.quant_mxfp4(O.make_weight((N, K), seed=2).to(dev))
+    want = {"linear": ops.fp8_linear(x, w, s), "mxfp4": ops.linear_mxfp4(x, weight)}
+
+    class Seen(TorchDispatchMode):
+        calls = 0
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            Seen.calls += 1
+            return func(*args, **(kwargs or {}))
+
+    def watched(op):
+        with Seen():
+            return op(x)
+
+    def dual(op):
+        with torch.autograd.forward_ad.dual_level():
+            out = op(torch.autograd.forward_ad.make_dual(x, torch.ones_like(x)))
+            assert torch.autograd.forward_ad.unpack_dual(out).tangent is None
+            return out
+
+    def ended(call):
+        try:
+            return call()
+        except Exception as e:
+            return type(e)
+
+    for name, op in (("linear", lambda x: ops.fp8_linear(x, w, s)), ("mxfp4", lambda x: ops.linear_mxfp4(x, weight))):
+        before = Seen.calls
+        one, two, took = _both(lambda: watched(op), monkeypatch)
+        assert not took and Seen.calls > before and torch.equal(one, want[name]) and torch.equal(two, want[name])
+        one, two, took = _both(lambda: dual(op), monkeypatch)
+        assert took and torch.equal(one, want[name]) and torch.equal(two, want[name])
+        for call in (lambda: torch.func.vmap(op)(torch.stack([x, x])), lambda: torch.func.jvp(op, (x,), (x,)), lambda: torch.func.vjp(op, x),
+                     lambda: torch.jit.trace(op, (x,), check_trace=False) and None):
+            one, two, took = _both(lambda: ended(call), monkeypatch)
+            assert not took and (one is two or type(one) is type(two))
+
+
 def test_mxfp4(dev, monkeypatch):
     for M, N, K, dt in ((1, 64, 128, None), (4, 256, 2880, torch.float32), (40, 512, 1024, None)):
         x, weight = O.make_activation(M, K, seed=1).to(dev), ops.quant_mxfp4(O.make_weight((N, K), seed=2).to(dev))
