@@ -12,8 +12,8 @@
 // What bounds it: nothing but latency - 65536 pairs are half a megabyte of indices and outputs of the same size.  So no load
 // waits for another: a thread's own pair, its weight, its token's other slots and the mask are requested together, before the
 // histograms are, and the mask decides afterwards.  The tokens' 1x128 quantisation, which needs nothing of the routing, runs in workgroups
-// behind its own instead of in a launch behind it.  Routing and quantising, top 8 of 128 experts of 2048: 16 tokens 7.8 + 4.8 us in two
-// launches, 6.5 in one; 777 tokens 4.7 + 8.8 + 5.1 in three, 4.9 + 8.2 in two; 8192 tokens 4.7 + 11.8 + 11.9, 7.0 + 13.0.
+// behind its own instead of in a launch behind it.  Routing and quantising, top 8 of 128 experts of 2048, in a kernel trace: 16 tokens 7.8 + 4.8 us in two
+// launches, 6.5 in one; 777 tokens 4.7 + 8.8 + 5.1 in three, 4.8 + 8.4 in two; 8192 tokens 4.7 + 11.8 + 11.9, 4.9 + 15.8.
 // The same layout built from library calls (a stable argsort, a scatter-add for the counts, a sort along the slots,
 // gathers, comparisons and fills, each over 10^2 .. 10^5 elements) is some thirty launches of 2 .. 45 us each:
 // 230-250 us at every size from 16 to 8192 tokens.
@@ -27,11 +27,6 @@ constexpr int kRouteMaxExperts = 1024;
 // take 14 us that way and 12 us in two launches.
 constexpr int kRouteOneLaunchPairs = 1024;
 constexpr int kRouteMaxBlocks = 128;
-// Of the tokens' quantisation beside two launches of routing, the quarters that go with the first.  8192 tokens of 2048, the launches by themselves:
-// none 4.7 + 13.6 us, one 7.0 + 13.0, two 8.7 + 12.4.
-constexpr int kRouteEarlyQuarters = 1;
-// Groups up to which a quantising thread takes one, not four: 777 tokens of 2048 (12432 groups) 147.7 -> 145.3 us a call; 8192 tokens (131072) 492 -> 494.
-constexpr u32 kRouteFewGroups = 1u << 15;
 
 struct RouteArgs {
     const void* indices;      // [tokens, topk] int32 or int64
@@ -85,15 +80,14 @@ __device__ __forceinline__ RoutePair route_pair(const RouteArgs& p, u32 pair, bo
 }
 
 // The workgroups behind the routing's own quantise the tokens, which it does not read.
+// (Four groups a thread: one instead changed nothing from 256 to 131072 groups, whose casts run while the routing waits.)
+constexpr u32 kRouteQuantGroups = kRouteThreads / 16 * 4;  // a workgroup's
 __device__ __forceinline__ void route_quantise(const GroupRows& q, u32 block) {
-    const u32 at = block * (kRouteThreads / 16) + (threadIdx.x >> 4);
-    if (q.total_groups <= kRouteFewGroups) group128_some<CFP8_GROUP_MODE_DIV, 1>(q, at);
-    else group128_some<CFP8_GROUP_MODE_DIV, 4>(q, at * 4u);
+    group128_some<CFP8_GROUP_MODE_DIV, 4>(q, block * kRouteQuantGroups + (threadIdx.x >> 4) * 4u);
 }
 
-__global__ __launch_bounds__(kRouteThreads) void route_count_kernel(const RouteArgs p, const GroupRows q) {
+__global__ __launch_bounds__(kRouteThreads) void route_count_kernel(const RouteArgs p) {
     __shared__ int hist[kRouteMaxExperts];
-    if ((int)blockIdx.x >= p.blocks) return route_quantise(q, blockIdx.x - p.blocks);
     const int t = threadIdx.x;
     const int64_t first = (int64_t)blockIdx.x * p.chunk;
     const int64_t last = first + p.chunk < p.pairs ? first + p.chunk : p.pairs;
@@ -107,15 +101,14 @@ __global__ __launch_bounds__(kRouteThreads) void route_count_kernel(const RouteA
     for (int e = t; e < p.experts; e += kRouteThreads) p.hist[(int64_t)blockIdx.x * p.experts + e] = hist[e];
 }
 
-// q_first: the first of the quantiser's blocks that this launch has (the ones in front went beside the counting)
 template <bool ONE>
-__global__ __launch_bounds__(kRouteThreads) void route_place_kernel(const RouteArgs p, const GroupRows q, const u32 q_first) {
+__global__ __launch_bounds__(kRouteThreads) void route_place_kernel(const RouteArgs p, const GroupRows q) {
     __shared__ int total[kRouteMaxExperts];   // pairs of every expert
     __shared__ int base[kRouteMaxExperts];    // next row of every expert for this workgroup
     __shared__ int ends[kRouteMaxExperts];    // inclusive cumulative group ends
     __shared__ int wave_sum[kRouteWaves];
     extern __shared__ uint16_t counts[];      // [wave][experts rounded up to even]
-    if ((int)blockIdx.x >= p.blocks) return route_quantise(q, blockIdx.x - p.blocks + q_first);
+    if ((int)blockIdx.x >= p.blocks) return route_quantise(q, blockIdx.x - p.blocks);
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int E = p.experts, EP = (E + 1) & ~1;
     const int64_t first = (int64_t)blockIdx.x * p.chunk;
@@ -286,15 +279,16 @@ int route_and_quantise(const void* indices, int index_bytes, const uint8_t* toke
     p.chunk = (p.pairs + blocks - 1) / blocks;
     p.chunk = (p.chunk + kRouteThreads - 1) / kRouteThreads * kRouteThreads;
     p.blocks = (int)blocks;
-    const u32 groups = tokens_q ? tokens_q->total_groups : 0, per = (kRouteThreads / 16) * (groups <= kRouteFewGroups ? 1 : 4);  // groups a block
-    const u32 q_blocks = groups / per + (groups % per != 0);
+    const u32 groups = tokens_q ? tokens_q->total_groups : 0;
+    const unsigned all = (unsigned)blocks + groups / kRouteQuantGroups + (groups % kRouteQuantGroups != 0);
     const GroupRows q = tokens_q ? *tokens_q : GroupRows{};
     if (blocks == 1) {
-        hipLaunchKernelGGL(route_place_kernel<true>, dim3(1 + q_blocks), dim3(kRouteThreads), lds, st, p, q, 0u);
+        hipLaunchKernelGGL(route_place_kernel<true>, dim3(all), dim3(kRouteThreads), lds, st, p, q);
     } else {
-        const u32 early = (u32)((uint64_t)q_blocks * kRouteEarlyQuarters / 4);
-        hipLaunchKernelGGL(route_count_kernel, dim3((unsigned)blocks + early), dim3(kRouteThreads), 0, st, p, q);
-        hipLaunchKernelGGL(route_place_kernel<false>, dim3((unsigned)blocks + q_blocks - early), dim3(kRouteThreads), lds, st, p, q, early);
+        // (the quantiser's workgroups all behind the placing: some of them beside the counting, whose end the placing waits for, took 0.4 to 3 us more a call
+        // at 200 to 4096 tokens of 128 x 2048 x 768, 32 x 3584 x 1536 and 64 x 1024 x 512, the same at 8192)
+        hipLaunchKernelGGL(route_count_kernel, dim3((unsigned)blocks), dim3(kRouteThreads), 0, st, p);
+        hipLaunchKernelGGL(route_place_kernel<false>, dim3(all), dim3(kRouteThreads), lds, st, p, q);
     }
     return check_launch("route_tokens");
 }

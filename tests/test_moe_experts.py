@@ -112,8 +112,8 @@ def test_one_call_experts_of_values_that_are_no_numbers(dev, T, E, topk, H, I):
     assert bool(y[2].isnan().all()) and bool(y[plain].isfinite().all()) and not bool(y[~mask].any())
 
 
-# the tokens are quantised by workgroups behind the routing's, 64 groups each, or 256, four in turn a thread, where there are more than 32768: one
-# launch up to 1024 pairs, two beyond, of which the first has a quarter of those workgroups; rows of tokens that do not follow each other
+# the tokens are quantised by workgroups behind the routing's, 256 groups each, four in turn a thread: in the one launch up to 1024 pairs, in the
+# second of two beyond; rows of tokens that do not follow each other
 @pytest.mark.parametrize("T,topk,H", [(1, 1, 128), (3, 8, 128), (51, 4, 640), (52, 4, 640), (128, 8, 640), (129, 8, 640), (1025, 1, 128), (410, 3, 1280), (1639, 2, 640), (4096, 1, 1024), (4097, 1, 1024), (3641, 2, 1152)])
 def test_one_call_experts_quantised_beside_the_routing(dev, T, topk, H):
     from cosmos_rl_amd.policy.kernel.moe.moe import grouped_experts_forward
