@@ -60,7 +60,7 @@ struct ExpertsArgs {
     float* hs;                   // gate_up: [rows, N / 256]
     uint16_t* out;               // down: [rows, N] bf16
     int tokens, N, K, tiles_m, tiles_n;
-    int whole_tiles;             // gate_up: halves of tiles that are padding are written, for a down product that multiplies them
+    int whole_tiles;             // gate_up: halves of tiles that are padding are written, for a down product of another kernel, which reads them
 };
 bool experts_gate_up_takes(int64_t tokens, int64_t hidden, int64_t inter);
 bool experts_down_takes(int64_t hidden, int64_t inter);

@@ -6,9 +6,10 @@
 //   many rows   Every expert's rows are padded to tiles of 128 (experts without a row get none).  The tokens are quantised
 //               where they lie and gemm_experts_kernel gathers its rows from them; hidden sizes that it does not take are
 //               quantised into the padded layout (cfp8_scatter_quant_group128) for the grouped GEMM of the training path.
-//               Rows of padding are zeros all the way: a walking GEMM carries a row's last products into the first step of
-//               its next tile with a scale of zero, so what multiplies there must be finite.  Rows past the last group are
-//               not touched.
+//               Rows of padding: where a tile's second 64 rows are all padding and gemm_experts_kernel makes both products, those
+//               rows of h are neither written nor read and hold what the workspace held (ExpertsArgs::whole_tiles).  All other
+//               rows of padding are zeros all the way, which is what the grouped GEMMs of the training path are given. Rows past the last
+//               group are not touched.
 //   middle      A chunk of prefill: all experts' weights are read, for less than a tile of 128 rows each.  Rows lie one
 //               behind the other without padding; the ring kernel takes tiles of 64 of one expert's rows (gemm_ring.hip:
 //               kRingGateUp reads them from the quantised tokens and ends in SwiGLU, kRingDown), two workgroups a CU.  The
