@@ -577,7 +577,7 @@ def fp8_linear(x: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor
     K, N = weight.shape
     if weight.stride(0) != 1 and K > 1:
         raise ValueError("weight must be the transposed view of a contiguous [N, K] fp8 tensor")
-    if weight.dtype not in (FP8_DTYPE, torch.uint8):
+    if weight.dtype not in (FP8_DTYPE, torch.uint8, torch.int8):
         raise ValueError(f"weight must be float8_e4m3fn (or its bytes), got {weight.dtype}")
     if weight_scale.numel() < N and weight_scale.numel() != 1:
         raise ValueError(f"fp8_linear needs one scale a weight row ({N}) or one for all, got {weight_scale.numel()}")

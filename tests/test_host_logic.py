@@ -414,7 +414,8 @@ def test_fp8_linear_scales_and_weight_type(monkeypatch):
     for scale, want in ((whole[:, None], whole), (whole.double(), whole), (torch.arange(N + 8.0), whole), (torch.tensor([3.0]), torch.full((N,), 3.0)),
                         (torch.tensor(3.0, dtype=torch.bfloat16), torch.full((N,), 3.0))):
         assert ops.fp8_linear(x, w, scale).shape == (M, N) and seen.pop() == want.tolist()
-    ops.fp8_linear(x, w.t().view(torch.uint8).t(), whole)
+    for raw in (torch.uint8, torch.int8):
+        ops.fp8_linear(x, w.t().view(raw).t(), whole)
     seen.clear()
     for bad in ((w, whole[:N - 1]), (w, whole[:0]), (torch.zeros(N, K, dtype=torch.bfloat16).t(), whole), (torch.zeros(N, K).t(), whole),
                 (torch.zeros(N, K).to(torch.float8_e5m2).t(), whole)):
