@@ -28,6 +28,23 @@ constexpr int few_steps(int tm) { return tm <= 8 ? 2 : 1; }
 constexpr int few_chunks(int tm) { return tm <= 4 || tm > 8 ? 3 : 2; }
 constexpr int few_depth(int mode, int tm) { return mode == kRingMx ? (tm <= 2 ? 3 : 2) : tm <= 2 || (tm > 8 && tm <= 13) ? 4 : 3; }
 constexpr int few_stage(int mode) { return 2048 + (mode == kRingMx ? 256 : 0); }
+// Whether 16-byte chunk `chunk` of a row's 128 in a stage of MXFP4 weights that begins with K step kt holds codes below K (or below a slice's end): a
+// stage is two steps, and the codes of an odd last one end in its middle.  Behind them lies the next row or, where rows have a pitch, what may not be mapped.
+__host__ __device__ constexpr bool few_codes_inside(int kt, uint32_t chunk, uint32_t K) { return ((uint32_t)kt << 7) + chunk * 32 < K; }
+constexpr bool few_codes_stay_in_their_rows() {
+    for (uint32_t K = 32; K <= 4096; K += 32) {
+        uint32_t loaded = 0;
+        for (int kt = 0; kt < (int)((K + 127) / 128) + 4; kt += 2)
+            for (uint32_t c = 0; c < 8; ++c)
+                if (few_codes_inside(kt, c, K)) {
+                    if (((uint32_t)kt << 6) + c * 16 + 16 > K / 2) return false;
+                    loaded += 16;
+                }
+        if (loaded != K / 2) return false;
+    }
+    return true;
+}
+static_assert(few_codes_stay_in_their_rows(), "stages of MXFP4 weights read all of a row's codes and nothing behind them");
 template <int MODE, int TM, int WIDTH>
 struct FewShape {
     static constexpr int CH = few_steps(TM), D = few_depth(MODE, TM), STAGE = few_stage(MODE);
@@ -70,14 +87,13 @@ __global__ __launch_bounds__(few_threads(WIDTH)) void gemm_ring_few_kernel(const
     // a load of 8 rows x 128 bytes: row lane >> 3, whose 16-byte chunk c lies at position c ^ f(row) (gemm_ring.hip; the half says rows 8 .. 15 of 16)
     constexpr int F1 = MX ? 1 : 0;
     auto chunk_of = [&](int half) { return (uint32_t)((lane & 7) ^ ((((lane >> 4) & 1) << F1) | (half << 2))); };
-    uint32_t vw[2], vw_tail[2], vx[XL], vx_tail[XL];
+    uint32_t vw[2], vw_tail[2], vx[XL], vx_tail[XL];  // (MXFP4: vw_tail is the load's chunk)
     int xstep[XL], xdst[XL], xbuf[XL];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         const uint32_t c = chunk_of(h);
         vw[h] = (uint32_t)((lane >> 3) + 8 * h) * (uint32_t)p.ld_w + c * 16;
-        // (MXFP4: the first K of the chunk in its stage)
-        vw_tail[h] = MX ? c * 32 : tail && c * 16 >= (uint32_t)tail ? kOutside : vw[h];
+        vw_tail[h] = MX ? c : tail && c * 16 >= (uint32_t)tail ? kOutside : vw[h];
     }
 #pragma unroll
     for (int i = 0; i < XL; ++i) {
@@ -107,7 +123,7 @@ __global__ __launch_bounds__(few_threads(WIDTH)) void gemm_ring_few_kernel(const
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             uint32_t v;
-            if (MX) v = ((uint32_t)kt << 7) + vw_tail[h] < klimit ? vw[h] : kOutside;
+            if (MX) v = few_codes_inside(kt, vw_tail[h], klimit) ? vw[h] : kOutside;
             else v = kt < kend ? (kt == KT - 1 ? vw_tail[h] : vw[h]) : kOutside;
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_void*)(own + st * STAGE + h * 1024), 16, v, (uint32_t)kt << (MX ? 6 : 7), 0, 2);
         }
@@ -311,17 +327,20 @@ __global__ __launch_bounds__(12 * 64) void linear_stream_kernel(const RingArgs p
     const __amdgpu_buffer_rsrc_t rsc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(MX ? p.ws + (uint64_t)nw0 * (uint64_t)p.ld_ws : p.w), 0,
                                                                          MX ? (int)bytes((int64_t)p.N - nw0, p.ld_ws) : 0, 0x00020000);
     constexpr int F1 = MX ? 1 : 0;
-    uint32_t vw[2];
+    uint32_t vw[2], chunk[2];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) vw[h] = (uint32_t)((lane >> 3) + 8 * h) * (uint32_t)p.ld_w + (uint32_t)((lane & 7) ^ ((((lane >> 4) & 1) << F1) | (h << 2))) * 16u;
+    for (int h = 0; h < 2; ++h) {
+        chunk[h] = (uint32_t)((lane & 7) ^ ((((lane >> 4) & 1) << F1) | (h << 2)));
+        vw[h] = (uint32_t)((lane >> 3) + 8 * h) * (uint32_t)p.ld_w + chunk[h] * 16u;
+    }
     const uint32_t xbytes = (uint32_t)KT * 512u;  // tokens: [K step][4][128 bytes], 16-byte chunk c of token r at position c ^ 2 r; their scales behind them
     uint8_t* const own = smem + xbytes + 256 + wave * D * STAGE;
     auto dma_w = [&](int kt, int st) {
         uint8_t* const to = own + st * STAGE;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            // (MXFP4: an odd last step's stage takes the row's bytes behind it as well, which no product reads, or the next row's)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_void*)(to + h * 1024), 16, kt < KT ? vw[h] : kOutside, (uint32_t)kt << (MX ? 6 : 7), 0, 2);
+            const bool in = MX ? few_codes_inside(kt, chunk[h], (uint32_t)p.K) : kt < KT;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_void*)(to + h * 1024), 16, in ? vw[h] : kOutside, (uint32_t)kt << (MX ? 6 : 7), 0, 2);
         }
         if (MX) {
             const int ks = kt + ((lane >> 4) & 1);

@@ -95,3 +95,31 @@ def test_wide_linear_of_one_token_up_to_8192_columns(dev):
     x = torch.randn(1, 8192, generator=g, device=dev).to(torch.bfloat16)
     qx, sx = ops.quant_rowwise(x)
     assert torch.equal(ops.fp8_linear(x, q.t(), s), ops.scaled_mm(qx, q.t(), sx, s, out_dtype=torch.bfloat16))
+
+
+# weights and scales inside rows of their own pitch, whose other bytes are NaN in e4m3, the largest codes and NaN scales; the last row ends with its memory.  Odd numbers of K steps:
+# MXFP4 weights are loaded by two, and an odd last one ends in the middle of a load (which bytes are read is a static_assert in gemm_ring_few.h)
+@pytest.mark.parametrize("N,K", [(8224, 128), (8224, 384), (12304, 640), (8208, 3968), (8208, 4096)])
+@pytest.mark.parametrize("M", [1, 4])
+def test_wide_linear_of_weights_with_a_pitch(dev, M, N, K):
+    g = torch.Generator(device=dev).manual_seed(N + K + M)
+    x = torch.randn(M, K, generator=g, device=dev).to(torch.bfloat16)
+    w = (torch.randn(N, K, generator=g, device=dev) * 0.05).to(torch.bfloat16)
+
+    def pitched(t, more, filler):
+        whole = torch.full((N, t.shape[1] + more), filler, dtype=torch.uint8, device=dev)
+        whole[:, more:] = t.view(torch.uint8)
+        return whole[:, more:]
+
+    (q, s), (mq, ms) = ops.quant_rowwise(w), ops.quant_mxfp4(w)
+    pq, pmq, pms = pitched(q, 48, 0x7F), pitched(mq, 64, 0x77), pitched(ms, 3, 0xFF)
+    lib, st = _lib.load(), torch.cuda.current_stream().cuda_stream
+    work = torch.empty(lib.cfp8_linear_workspace_bytes(M, K), dtype=torch.uint8, device=dev)
+    for dt in (torch.bfloat16, torch.float32):
+        out = torch.full((M, N + 8), 7.0, dtype=dt, device=dev)
+        _lib.check(lib.cfp8_linear_mxfp4(x.data_ptr(), K, pmq.data_ptr(), pmq.stride(0), pms.data_ptr(), pms.stride(0), out.data_ptr(), N + 8, ops._out_code(dt), M, N, K, None, 0, st))
+        assert torch.equal(out[:, :N], ops.linear_mxfp4(x, (mq, ms), dt)) and bool((out[:, N:] == 7.0).all())
+        out.fill_(7.0)
+        _lib.check(lib.cfp8_linear_rowwise_split(x.data_ptr(), K, pq.data_ptr(), pq.stride(0), s.data_ptr(), None, out.data_ptr(), N + 8, ops._out_code(dt), M, N, K,
+                                                 work.data_ptr(), work.numel(), st))
+        assert torch.equal(out[:, :N], ops.fp8_linear(x, q.t(), s, out_dtype=dt)) and bool((out[:, N:] == 7.0).all())
