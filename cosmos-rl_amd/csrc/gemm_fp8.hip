@@ -3429,15 +3429,14 @@ static int launch_rowwise_best(GemmArgs& p, int out_dtype, hipStream_t st) {
     r.partial = p.partial;
     r.ld_a = p.ld_a; r.ld_w = p.ld_b; r.ld_out = p.ld_out;
     r.M = p.M; r.N = p.N; r.K = p.K;
-    RingPlan ring{0, 0, 0, 1e30, false};
+    RingPlan ring{0, 0, 0, 1e30};
     int strips = 0;
     // (where the linear is one launch the product has its bits, those of the kernel for 16 tokens)
     if (!fused_gemv_size(p.M, p.K) && ring_takes(kRingRow, r, out_dtype)) {
-        // (beyond 80 rows the form for few rows is ahead of every other kernel where it is taken; the estimates are those of the tiles)
         strips = ring_few_strips(kRingRow, r);
-        const bool few = strips && p.M > 80;
-        ring = ring_plan(kRingRow, p.M, p.N, p.K, few ? 0 : p.partial_bytes, cus);
-        if (few) ring.cost = 0;
+        // beyond 80 rows the form for few rows is ahead of every other kernel where it is taken
+        if (strips && p.M > 80) return launch_ring_few(kRingRow, r, strips, out_dtype, st);
+        ring = ring_plan(kRingRow, p.M, p.N, p.K, p.partial_bytes, cus);
     }
     EdgePlan edge{};
     edge.cost = 1e30;
@@ -3452,7 +3451,7 @@ static int launch_rowwise_best(GemmArgs& p, int out_dtype, hipStream_t st) {
     // (without a bias and without remainders launch_gemm's form of the same tiles is 2 % faster)
     const bool even = p.M % 256 == 0 && p.N % 256 == 0 && !p.bias;
     // the strips of launch_gemm's own kernel (33 x 18944 x 3584 16.1 -> 14.5 us)
-    if (strips >= 5 && p.M > 16 && other <= edge.cost) return launch_ring(kRingRow, r, RingPlan{p.M <= 64 ? 64 : 128, strips * 16, 1, other, !p.bias}, out_dtype, st);
+    if (strips >= 5 && p.M > 16 && other <= edge.cost) return launch_ring_few(kRingRow, r, strips, out_dtype, st);
     if (edge.cost < 1e30 && edge.cost <= other && !even) return launch_rowwise_edge(p, edge, out_dtype, st);
     float* const partial = p.partial;
     p.partial = nullptr;  // (launch_gemm's own slices are those of cfp8_linear_rowwise)

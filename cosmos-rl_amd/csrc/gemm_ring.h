@@ -31,11 +31,12 @@ struct RingArgs {
 struct RingPlan {
     int bm, bn, slices;
     double cost;           // microseconds, estimated
-    bool strip;            // the form for few rows in place of another file's strip kernel, whose name the launch record keeps
 };
 RingPlan ring_plan(int mode, int64_t M, int64_t N, int64_t K, size_t partial_bytes, int cus);
 bool ring_takes(int mode, const RingArgs& p, int out_dtype);  // whether the operands fit what the kernel assumes
-int ring_few_strips(int mode, const RingArgs& p);  // strips of 16 weight rows a workgroup of the form for few rows, all of K a workgroup; 0: other kernels are ahead
+// the form for few rows, all of K a workgroup: strips of 16 weight rows a workgroup, 0: other kernels are ahead
+int ring_few_strips(int mode, const RingArgs& p);
+int launch_ring_few(int mode, RingArgs& p, int strips, int out_dtype, hipStream_t st);
 // the linear of up to four tokens (K <= 4096, one token 8192, a multiple of 128) as one launch of streams: waves a workgroup, 0: other kernels are ahead
 int linear_stream_waves(int mode, int64_t M, int64_t N, int64_t K);
 int launch_linear_stream(int mode, const RingArgs& p, const void* x, int64_t ld_x, int waves, int out_dtype, hipStream_t st);

@@ -165,36 +165,39 @@ def test_block(dev, M, N, K, kn):
             _check(out, want, M, N, dtype, 0.0)
 
 
-# every tile of the ring kernel for every weight format, with slices of K and without, with weights loaded as a stream (one row of tiles, and
+# the tiles of the ring kernel for every weight format, with slices of K and without, with weights loaded as a stream (one row of tiles, and
 # what else ring_once names) and cacheably, some with a last step of 64: the smallest products with remainders of rows and columns that
 # the choice takes there
 FORMS = [("block", 64, 64, False, 67, 208, 384), ("block", 64, 64, False, 5, 208, 384), ("block", 64, 64, True, 67, 208, 2176),
-         ("block", 64, 64, True, 5, 208, 2176), ("block", 64, 128, False, 67, 9232, 384), ("block", 64, 128, False, 5, 18448, 384),
-         ("block", 64, 128, True, 67, 2832, 5248), ("block", 64, 128, True, 5, 5648, 2432), ("block", 128, 128, False, 67, 18448, 384),
-         ("block", 128, 128, True, 67, 5648, 7296), ("mxfp4", 64, 64, False, 131, 208, 384), ("mxfp4", 64, 64, False, 19, 208, 640),
-         ("mxfp4", 64, 64, True, 150, 208, 2432), ("mxfp4", 64, 64, True, 5, 208, 9344), ("mxfp4", 64, 128, False, 131, 9232, 384),
-         ("mxfp4", 64, 128, False, 5, 208, 384), ("mxfp4", 64, 128, True, 131, 2064, 7296), ("mxfp4", 64, 128, True, 19, 208, 2176),
+         ("block", 64, 128, False, 67, 9232, 384), ("block", 64, 128, True, 67, 2832, 5248), ("block", 128, 128, True, 67, 5648, 7296),
+         ("mxfp4", 64, 64, False, 131, 208, 384), ("mxfp4", 64, 64, False, 19, 208, 640), ("mxfp4", 64, 64, True, 150, 208, 2432),
+         ("mxfp4", 64, 128, False, 131, 9232, 384), ("mxfp4", 64, 128, False, 5, 208, 384), ("mxfp4", 64, 128, True, 131, 2064, 7296),
          ("mxfp4", 128, 64, False, 131, 5648, 384), ("mxfp4", 128, 64, False, 67, 9232, 640), ("mxfp4", 128, 64, True, 131, 1808, 5248),
          ("mxfp4", 128, 64, True, 67, 2832, 2944), ("mxfp4", 128, 64, False, 131, 5648, 448), ("mxfp4", 128, 64, False, 67, 9232, 448),
-         ("mxfp4", 128, 128, False, 131, 11792, 384), ("mxfp4", 128, 128, False, 67, 18448, 384), ("mxfp4", 128, 128, True, 131, 2832, 7296),
-         ("mxfp4", 128, 128, True, 67, 5648, 7296), ("mxfp4", 128, 128, True, 131, 2832, 7360), ("mxfp4", 128, 128, True, 67, 5648, 5312),
-         ("rowwise", 64, 64, False, 67, 208, 384), ("rowwise", 64, 64, False, 5, 14864, 384), ("rowwise", 64, 64, True, 67, 208, 2176),
-         ("rowwise", 64, 64, True, 5, 208, 7296), ("rowwise", 64, 128, False, 131, 9232, 384), ("rowwise", 64, 128, False, 5, 23568, 384),
-         ("rowwise", 64, 128, True, 131, 1808, 5248), ("rowwise", 64, 128, True, 5, 5648, 7296), ("rowwise", 64, 128, True, 131, 1808, 5312),
-         ("rowwise", 64, 128, True, 5, 5648, 3776), ("rowwise", 128, 64, False, 131, 5648, 384), ("rowwise", 128, 64, False, 67, 9232, 384),
-         ("rowwise", 128, 64, True, 1500, 208, 5248), ("rowwise", 128, 64, True, 67, 2832, 3712), ("rowwise", 128, 64, True, 1031, 208, 7360),
-         ("rowwise", 128, 64, True, 67, 2832, 3776), ("rowwise", 128, 128, False, 515, 3600, 640), ("rowwise", 128, 128, False, 67, 23568, 640),
-         ("rowwise", 128, 128, True, 131, 2832, 9344), ("rowwise", 128, 128, True, 67, 9232, 5248), ("rowwise", 128, 128, False, 131, 11792, 704),
-         ("rowwise", 128, 128, False, 67, 18448, 448)]
+         ("mxfp4", 128, 128, False, 131, 11792, 384), ("mxfp4", 128, 128, True, 131, 2832, 7296), ("mxfp4", 128, 128, True, 67, 5648, 7296),
+         ("mxfp4", 128, 128, True, 131, 2832, 7360), ("mxfp4", 128, 128, True, 67, 5648, 5312), ("rowwise", 64, 64, False, 67, 208, 384),
+         ("rowwise", 64, 64, True, 67, 208, 2176), ("rowwise", 64, 128, False, 131, 9232, 384), ("rowwise", 64, 128, True, 131, 1808, 5248),
+         ("rowwise", 64, 128, True, 131, 1808, 5312), ("rowwise", 128, 64, False, 131, 5648, 384),
+         ("rowwise", 128, 64, False, 67, 9232, 384), ("rowwise", 128, 64, True, 1500, 208, 5248),
+         ("rowwise", 128, 64, True, 67, 2832, 3712), ("rowwise", 128, 64, True, 1031, 208, 7360),
+         ("rowwise", 128, 64, True, 67, 2832, 3776), ("rowwise", 128, 128, False, 515, 3600, 640),
+         ("rowwise", 128, 128, True, 131, 2832, 9344), ("rowwise", 128, 128, True, 67, 9232, 5248),
+         ("rowwise", 128, 128, False, 131, 11792, 704)]
+# the same products where the choice takes the form for few rows: tiles of 16 rows, strips of 16 weight rows a workgroup
+FEW_FORMS = [("block", 1, 4, True, 5, 208, 2176), ("block", 1, 5, False, 5, 18448, 384), ("block", 1, 8, True, 5, 5648, 2432),
+             ("block", 5, 5, False, 67, 18448, 384), ("mxfp4", 1, 4, True, 5, 208, 9344), ("mxfp4", 2, 8, True, 19, 208, 2176),
+             ("mxfp4", 5, 5, False, 67, 18448, 384), ("rowwise", 1, 4, False, 5, 14864, 384), ("rowwise", 1, 4, True, 5, 208, 7296),
+             ("rowwise", 1, 6, False, 5, 23568, 384), ("rowwise", 1, 8, True, 5, 5648, 7296), ("rowwise", 1, 8, True, 5, 5648, 3776),
+             ("rowwise", 5, 6, False, 67, 23568, 640), ("rowwise", 5, 5, False, 67, 18448, 448)]
 
 
-@pytest.mark.parametrize("mode,bm,bn,sliced,M,N,K", FORMS)
-def test_every_form(dev, mode, bm, bn, sliced, M, N, K):
+@pytest.mark.parametrize("kernel,mode,bm,bn,sliced,M,N,K", [("gemm_ring", *f) for f in FORMS] + [("gemm_ring_few", *f) for f in FEW_FORMS])
+def test_every_form(dev, kernel, mode, bm, bn, sliced, M, N, K):
     from oracle import mxfp4_oracle as MX
     kind = {"rowwise": _lib.DISPATCH_ROWWISE, "block": _lib.DISPATCH_BLOCK, "mxfp4": _lib.DISPATCH_MXFP4}[mode]
     cus = torch.cuda.get_device_properties(dev).multi_processor_count
     took = _lib.gemm_dispatch_info(kind, M, N, K, cus=cus, flags=_lib.DISPATCH_SPLIT).split("; ")
-    assert took[0].startswith(f"gemm_ring<{mode},{bm},{bn}>") and ("slices=1 " not in took[0]) == sliced and len(took) == 1 + sliced, took
+    assert took[0].startswith(f"{kernel}<{mode},{bm},{bn}>") and ("slices=1 " not in took[0]) == sliced and len(took) == 1 + sliced, took
     g = torch.Generator(device=dev).manual_seed(M + N + K)
     x = torch.randn(M, K, generator=g, device=dev).to(torch.bfloat16)
     w = torch.randn(N, K, generator=g, device=dev) * 0.05
@@ -253,7 +256,7 @@ def test_strips_of_few_rows(dev, mode, strips, M, N, K):
     from oracle import mxfp4_oracle as MX
     kind = {"rowwise": _lib.DISPATCH_ROWWISE, "block": _lib.DISPATCH_BLOCK, "mxfp4": _lib.DISPATCH_MXFP4}[mode]
     took = _lib.gemm_dispatch_info(kind, M, N, K, cus=torch.cuda.get_device_properties(dev).multi_processor_count, flags=_lib.DISPATCH_SPLIT)
-    assert f" grid={-(-N // (16 * strips))} block={64 * strips} " in took and took.startswith(("gemm_ring<", "gemm_rowwise_strip<", "gemm_mxfp4_strip<")), took
+    assert took.startswith(f"gemm_ring_few<{mode},{-(-M // 16)},{strips}>{' ktail' if K % 128 else ''} slices=1 grid={-(-N // (16 * strips))} block={64 * strips} "), took
     g = torch.Generator(device=dev).manual_seed(M + N + K)
     x, w = torch.randn(M, K, generator=g, device=dev), torch.randn(N, K, generator=g, device=dev) * 0.05
     x[0, ::7] = float("inf") if M > 1 else 1.0  # (rows do not reach each other)
