@@ -168,22 +168,23 @@ def test_block(dev, M, N, K, kn):
 # the tiles of the ring kernel for every weight format, with slices of K and without, with weights loaded as a stream (one row of tiles, and
 # what else ring_once names) and cacheably, some with a last step of 64: the smallest products with remainders of rows and columns that
 # the choice takes there
-FORMS = [("block", 64, 64, False, 67, 208, 384), ("block", 64, 64, False, 5, 208, 384), ("block", 64, 64, True, 67, 208, 2176),
-         ("block", 64, 128, False, 67, 9232, 384), ("block", 64, 128, True, 67, 2832, 5248), ("block", 128, 128, True, 67, 5648, 7296),
-         ("mxfp4", 64, 64, False, 131, 208, 384), ("mxfp4", 64, 64, False, 19, 208, 640), ("mxfp4", 64, 64, True, 150, 208, 2432),
-         ("mxfp4", 64, 128, False, 131, 9232, 384), ("mxfp4", 64, 128, False, 5, 208, 384), ("mxfp4", 64, 128, True, 131, 2064, 7296),
-         ("mxfp4", 128, 64, False, 131, 5648, 384), ("mxfp4", 128, 64, False, 67, 9232, 640), ("mxfp4", 128, 64, True, 131, 1808, 5248),
-         ("mxfp4", 128, 64, True, 67, 2832, 2944), ("mxfp4", 128, 64, False, 131, 5648, 448), ("mxfp4", 128, 64, False, 67, 9232, 448),
-         ("mxfp4", 128, 128, False, 131, 11792, 384), ("mxfp4", 128, 128, True, 131, 2832, 7296), ("mxfp4", 128, 128, True, 67, 5648, 7296),
-         ("mxfp4", 128, 128, True, 131, 2832, 7360), ("mxfp4", 128, 128, True, 67, 5648, 5312), ("rowwise", 64, 64, False, 67, 208, 384),
-         ("rowwise", 64, 64, True, 67, 208, 2176), ("rowwise", 64, 128, False, 131, 9232, 384), ("rowwise", 64, 128, True, 131, 1808, 5248),
-         ("rowwise", 64, 128, True, 131, 1808, 5312), ("rowwise", 128, 64, False, 131, 5648, 384),
-         ("rowwise", 128, 64, False, 67, 9232, 384), ("rowwise", 128, 64, True, 1500, 208, 5248),
-         ("rowwise", 128, 64, True, 67, 2832, 3712), ("rowwise", 128, 64, True, 1031, 208, 7360),
-         ("rowwise", 128, 64, True, 67, 2832, 3776), ("rowwise", 128, 128, False, 515, 3600, 640),
-         ("rowwise", 128, 128, True, 131, 2832, 9344), ("rowwise", 128, 128, True, 67, 9232, 5248),
-         ("rowwise", 128, 128, False, 131, 11792, 704)]
-# the same products where the choice takes the form for few rows: tiles of 16 rows, strips of 16 weight rows a workgroup
+FORMS = [("block", 64, 64, False, 67, 208, 384), ("block", 64, 64, False, 5, 208, 384), ("block", 64, 64, True, 67, 208, 2176), ("block", 64, 64, True, 49, 208, 2176),
+         ("block", 64, 128, False, 67, 9232, 384), ("block", 64, 128, False, 5, 52304, 256), ("block", 64, 128, True, 67, 2832, 5248), ("block", 128, 128, False, 138, 10960, 384),
+         ("block", 128, 128, True, 67, 5648, 7296), ("mxfp4", 64, 64, False, 131, 208, 384), ("mxfp4", 64, 64, False, 19, 208, 640), ("mxfp4", 64, 64, True, 150, 208, 2432),
+         ("mxfp4", 64, 64, True, 70, 208, 3584), ("mxfp4", 64, 64, True, 65, 80, 3520), ("mxfp4", 64, 128, False, 131, 9232, 384), ("mxfp4", 64, 128, False, 5, 208, 384),
+         ("mxfp4", 64, 128, True, 131, 2064, 7296), ("mxfp4", 64, 128, True, 66, 208, 1792), ("mxfp4", 64, 128, True, 65, 80, 1728), ("mxfp4", 128, 64, False, 131, 5648, 384),
+         ("mxfp4", 128, 64, False, 67, 9232, 640), ("mxfp4", 128, 64, False, 131, 5648, 448), ("mxfp4", 128, 64, False, 67, 9232, 448), ("mxfp4", 128, 64, True, 131, 1808, 5248),
+         ("mxfp4", 128, 64, True, 67, 2832, 2944), ("mxfp4", 128, 128, False, 131, 11792, 384), ("mxfp4", 128, 128, False, 82, 16848, 256),
+         ("mxfp4", 128, 128, False, 81, 16976, 320), ("mxfp4", 128, 128, True, 131, 2832, 7296), ("mxfp4", 128, 128, True, 67, 5648, 7296),
+         ("mxfp4", 128, 128, True, 131, 2832, 7360), ("mxfp4", 128, 128, True, 67, 5648, 5312), ("rowwise", 64, 64, False, 67, 208, 384), ("rowwise", 64, 64, False, 34, 8656, 256),
+         ("rowwise", 64, 64, False, 5, 80, 320), ("rowwise", 64, 64, True, 67, 208, 2176), ("rowwise", 64, 64, True, 51, 208, 2560), ("rowwise", 64, 64, True, 54, 80, 1728),
+         ("rowwise", 64, 128, False, 131, 9232, 384), ("rowwise", 64, 128, False, 5, 58704, 256), ("rowwise", 64, 128, True, 131, 1808, 5248),
+         ("rowwise", 64, 128, True, 131, 1808, 5312), ("rowwise", 64, 128, True, 17, 8912, 10624), ("rowwise", 64, 128, True, 18, 17424, 5056),
+         ("rowwise", 128, 64, False, 131, 5648, 384), ("rowwise", 128, 64, False, 67, 9232, 384), ("rowwise", 128, 64, True, 1500, 208, 5248),
+         ("rowwise", 128, 64, True, 67, 2832, 3712), ("rowwise", 128, 64, True, 1031, 208, 7360), ("rowwise", 128, 64, True, 67, 2832, 3776),
+         ("rowwise", 128, 128, False, 515, 3600, 640), ("rowwise", 128, 128, False, 131, 11792, 704), ("rowwise", 128, 128, False, 67, 29072, 512),
+         ("rowwise", 128, 128, False, 65, 25424, 704), ("rowwise", 128, 128, True, 131, 2832, 9344), ("rowwise", 128, 128, True, 67, 9232, 5248)]
+# where the choice takes the form for few rows: tiles of 16 rows, strips of 16 weight rows a workgroup
 FEW_FORMS = [("block", 1, 4, True, 5, 208, 2176), ("block", 1, 5, False, 5, 18448, 384), ("block", 1, 8, True, 5, 5648, 2432),
              ("block", 5, 5, False, 67, 18448, 384), ("mxfp4", 1, 4, True, 5, 208, 9344), ("mxfp4", 2, 8, True, 19, 208, 2176),
              ("mxfp4", 5, 5, False, 67, 18448, 384), ("rowwise", 1, 4, False, 5, 14864, 384), ("rowwise", 1, 4, True, 5, 208, 7296),
@@ -244,11 +245,11 @@ def test_a_bias_that_torch_follows(dev):
 
 # few rows, a strip of 16 weight rows a wave: row tiles of 16 up to the last (16, one; 128, eight; 208, thirteen in the shallower ring, 256), 3 to 12 waves, a last
 # workgroup with waves beyond N, strips on both sides of a 128-block's edge, one K step, fewer than the ring is deep, a last step of 16 and of 64
-FEW = [("rowwise", 3, 16, 8208, 128), ("rowwise", 3, 17, 12288, 400), ("rowwise", 4, 32, 16384, 704), ("rowwise", 5, 33, 18944, 384), ("rowwise", 7, 80, 28560, 896), ("rowwise", 10, 81, 37888, 256),
+FEW = [("rowwise", 3, 16, 8208, 128), ("rowwise", 3, 17, 12288, 400), ("rowwise", 4, 32, 16384, 704), ("rowwise", 5, 33, 18944, 384), ("rowwise", 7, 80, 28560, 1792), ("rowwise", 10, 81, 37888, 256),
        ("rowwise", 9, 128, 32784, 128), ("rowwise", 12, 129, 49152, 144), ("rowwise", 10, 208, 37904, 640), ("rowwise", 9, 209, 36864, 448), ("rowwise", 9, 256, 33024, 512),
-       ("mxfp4", 3, 5, 8208, 128), ("mxfp4", 3, 17, 12288, 416), ("mxfp4", 4, 32, 16384, 640), ("mxfp4", 3, 4, 8448, 4256), ("mxfp4", 5, 33, 18944, 256), ("mxfp4", 7, 128, 28560, 896),
+       ("mxfp4", 3, 5, 8208, 128), ("mxfp4", 3, 17, 12288, 416), ("mxfp4", 4, 32, 16384, 640), ("mxfp4", 3, 4, 8448, 4256), ("mxfp4", 5, 33, 18944, 256), ("mxfp4", 5, 113, 16400, 3232), ("mxfp4", 7, 96, 24592, 2592), ("mxfp4", 9, 128, 32784, 352),
        ("mxfp4", 10, 129, 37888, 128), ("mxfp4", 9, 144, 32784, 352), ("mxfp4", 12, 200, 49152, 480), ("mxfp4", 10, 208, 37904, 512),
-       ("block", 3, 1, 12288, 128), ("block", 3, 32, 8208, 1024), ("block", 4, 7, 16256, 640), ("block", 5, 33, 18432, 256), ("block", 5, 65, 16400, 384), ("block", 7, 128, 28544, 640)]
+       ("block", 3, 1, 12288, 128), ("block", 3, 32, 8208, 1024), ("block", 4, 7, 16256, 640), ("block", 5, 33, 18432, 256), ("block", 5, 65, 16400, 384), ("block", 6, 128, 24464, 1536), ("block", 7, 112, 28544, 1408)]
 
 
 @pytest.mark.parametrize("mode,strips,M,N,K", FEW)
