@@ -143,7 +143,7 @@ def torch_calls():
     return module
 
 
-DISPATCH_ROWWISE, DISPATCH_LINEAR, DISPATCH_BLOCK, DISPATCH_GROUPED, DISPATCH_GROUPED_SWIGLU, DISPATCH_MXFP4 = range(6)
+DISPATCH_ROWWISE, DISPATCH_LINEAR, DISPATCH_BLOCK, DISPATCH_GROUPED, DISPATCH_GROUPED_SWIGLU, DISPATCH_MXFP4, DISPATCH_LINEAR_MXFP4 = range(7)
 DISPATCH_LARGE_WORKSPACE, DISPATCH_SPLIT, DISPATCH_NO_MEMORY, DISPATCH_BIAS = 1, 2, 4, 8  # flags of gemm_dispatch_info
 
 

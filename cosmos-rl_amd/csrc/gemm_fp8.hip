@@ -3576,8 +3576,8 @@ extern "C" int cfp8_gemm_dispatch_info(int kind, int64_t M, int64_t N, int64_t K
     using namespace cfp8;
     if (!buf || buf_bytes == 0) return set_error(CFP8_EINVAL, "gemm_dispatch_info: no buffer");
     buf[0] = 0;
-    const bool rowwise_kind = kind == CFP8_DISPATCH_ROWWISE || kind == CFP8_DISPATCH_LINEAR;
-    if (M <= 0 || N <= 0 || K <= 0 || K % (rowwise_kind ? 16 : kind == CFP8_DISPATCH_MXFP4 ? 32 : 128) || N % 16 || M > 0x7FFFFFFFll || N > 0x7FFFFFFFll || K > 0x7FFFFFFFll || cus <= 0)
+    const bool rowwise_kind = kind == CFP8_DISPATCH_ROWWISE || kind == CFP8_DISPATCH_LINEAR, mx_kind = kind == CFP8_DISPATCH_MXFP4 || kind == CFP8_DISPATCH_LINEAR_MXFP4;
+    if (M <= 0 || N <= 0 || K <= 0 || K % (rowwise_kind ? 16 : mx_kind ? 32 : 128) || N % 16 || M > 0x7FFFFFFFll || N > 0x7FFFFFFFll || K > 0x7FFFFFFFll || cus <= 0)
         return set_error(CFP8_EINVAL, "gemm_dispatch_info: bad shape or compute-unit count");
     if (out_dtype != CFP8_OUT_BF16 && out_dtype != CFP8_OUT_F32) return set_error(CFP8_EINVAL, "gemm_dispatch_info: unknown out_dtype %d", out_dtype);
     // operands that pass every alignment test; nothing dereferences them
@@ -3601,7 +3601,7 @@ extern "C" int cfp8_gemm_dispatch_info(int kind, int64_t M, int64_t N, int64_t K
     g_rec.text[0] = 0;
     int rc = CFP8_OK;
     if (split) {
-        const int bytes_of = kind == CFP8_DISPATCH_LINEAR ? CFP8_DISPATCH_ROWWISE : kind;
+        const int bytes_of = kind == CFP8_DISPATCH_LINEAR ? CFP8_DISPATCH_ROWWISE : kind == CFP8_DISPATCH_LINEAR_MXFP4 ? CFP8_DISPATCH_MXFP4 : kind;
         p.partial = reinterpret_cast<float*>(fake);
         p.partial_bytes = flags & CFP8_DISPATCH_NO_MEMORY ? 0 : cfp8_gemm_partial_bytes(bytes_of, M, N, K);
         p.bias = reinterpret_cast<const uint16_t*>(flags & CFP8_DISPATCH_BIAS ? fake : 0);
@@ -3632,7 +3632,8 @@ extern "C" int cfp8_gemm_dispatch_info(int kind, int64_t M, int64_t N, int64_t K
             rc = split ? launch_block_best(p, out_dtype, nullptr) : launch_gemm<kBlock>(p, out_dtype, nullptr);
             break;
         case CFP8_DISPATCH_MXFP4:
-            rc = mx4_dispatch(reinterpret_cast<const void*>(fake), M, N, K, out_dtype, split, p.partial_bytes);
+        case CFP8_DISPATCH_LINEAR_MXFP4:
+            rc = mx4_dispatch(reinterpret_cast<const void*>(fake), M, N, K, out_dtype, split, p.partial_bytes, kind == CFP8_DISPATCH_LINEAR_MXFP4);
             break;
         case CFP8_DISPATCH_GROUPED:
             p.sb_stride_n = kb; p.sb_stride_k = 1; p.sb_stride_e = nb * kb;

@@ -43,8 +43,8 @@ bool note_launch(const char* kernel, unsigned grid, unsigned block, size_t lds);
 int raise_lds_limit(const void* fn, size_t lds, std::atomic<bool>& flag);         // once per (device, function)
 int device_slot();                                                                // 0..63, 64 = not cached
 int cu_count();                                                                   // compute units of the current device
-// what cfp8_gemm_mxfp4 (`split`: cfp8_gemm_mxfp4_split) launches for a problem, with every operand at `any`; while dry_run()
-int mx4_dispatch(const void* any, int64_t M, int64_t N, int64_t K, int out_dtype, bool split, size_t partial_bytes);
+// what cfp8_gemm_mxfp4 (`split`: cfp8_gemm_mxfp4_split; `linear`: cfp8_linear_mxfp4) launches for a problem, with every operand at `any`; while dry_run()
+int mx4_dispatch(const void* any, int64_t M, int64_t N, int64_t K, int out_dtype, bool split, size_t partial_bytes, bool linear);
 size_t block_partial_bytes(int64_t M, int64_t N, int64_t K);                      // of the block-scaled product's slices of K
 
 // ---- gemm_experts.hip

@@ -1723,6 +1723,7 @@ template <int MR>
 static int launch_linear_mx4_fused_mr(const void* x, int64_t ld_x, const Mx4Args& p, int out_dtype, hipStream_t st) {
     const unsigned blocks = (unsigned)((p.N + 15) / 16);
     const size_t lds = (size_t)p.M * ((size_t)((p.K + 127) / 128) * 128 + 16);  // <= 4 x 4112 bytes
+    if (!note_launch("linear_mxfp4_gemv_fused", blocks, 256, lds)) return CFP8_OK;
     if (out_dtype == CFP8_OUT_F32)
         hipLaunchKernelGGL((linear_mxfp4_gemv_fused_kernel<MR, true>), dim3(blocks), dim3(256), lds, st, static_cast<const uint4*>(x), ld_x / 8, p);
     else
@@ -1898,13 +1899,31 @@ static int launch_mx4_best(Mx4Args& p, float* partial, size_t partial_bytes, int
     return launch_mx4<128, 128, 2, 2, 1>(p, out_dtype, st);
 }
 
-int mx4_dispatch(const void* any, int64_t M, int64_t N, int64_t K, int out_dtype, bool split, size_t partial_bytes) {
+// the linear of up to 4 tokens, K <= 4096, in one launch
+static int launch_linear_mx4(const void* x, int64_t ld_x, const Mx4Args& p, int out_dtype, hipStream_t st) {
+    if (const int waves = p.ld_w < (1 << 21) && p.ld_ws < (1 << 21) ? linear_stream_waves(kRingMx, p.M, p.N, p.K) : 0) {
+        RingArgs r{};
+        r.w = p.w; r.ws = p.ws; r.out = p.out;
+        r.ld_w = p.ld_w; r.ld_ws = p.ld_ws; r.ld_out = p.ld_out;
+        r.M = p.M; r.N = p.N; r.K = p.K;
+        return launch_linear_stream(kRingMx, r, x, ld_x, waves, out_dtype, st);
+    }
+    if (p.M == 1) return launch_linear_mx4_fused_mr<1>(x, ld_x, p, out_dtype, st);
+    if (p.M == 2) return launch_linear_mx4_fused_mr<2>(x, ld_x, p, out_dtype, st);
+    return launch_linear_mx4_fused_mr<4>(x, ld_x, p, out_dtype, st);
+}
+
+int mx4_dispatch(const void* any, int64_t M, int64_t N, int64_t K, int out_dtype, bool split, size_t partial_bytes, bool linear) {
     Mx4Args p{};
     p.a = p.w = p.ws = static_cast<const uint8_t*>(any);
     p.sa = static_cast<const float*>(any);
     p.out = const_cast<void*>(any);
     p.ld_a = K; p.ld_w = K / 2; p.ld_ws = K / 32; p.ld_out = N;
     p.M = (int)M; p.N = (int)N; p.K = (int)K;
+    if (linear) {
+        if (M <= 4 && K <= 4096) return launch_linear_mx4(any, K, p, out_dtype, nullptr);
+        note_launch("quant_rowwise", 0, 256, 0);
+    }
     return launch_mx4_best(p, split ? static_cast<float*>(p.out) : nullptr, split ? partial_bytes : 0, out_dtype, nullptr);
 }
 }  // namespace cfp8
@@ -1989,16 +2008,7 @@ extern "C" int cfp8_linear_mxfp4(const void* x, int64_t ld_x, const void* w, int
         p.out = out;
         p.ld_w = ld_w; p.ld_ws = ld_ws; p.ld_out = ld_out;
         p.M = (int)M; p.N = (int)N; p.K = (int)K;
-        if (const int waves = ld_w < (1 << 21) && ld_ws < (1 << 21) ? linear_stream_waves(kRingMx, M, N, K) : 0) {
-            RingArgs r{};
-            r.w = p.w; r.ws = p.ws; r.out = out;
-            r.ld_w = ld_w; r.ld_ws = ld_ws; r.ld_out = ld_out;
-            r.M = p.M; r.N = p.N; r.K = p.K;
-            return launch_linear_stream(kRingMx, r, x, ld_x, waves, out_dtype, st);
-        }
-        if (M == 1) return launch_linear_mx4_fused_mr<1>(x, ld_x, p, out_dtype, st);
-        if (M == 2) return launch_linear_mx4_fused_mr<2>(x, ld_x, p, out_dtype, st);
-        return launch_linear_mx4_fused_mr<4>(x, ld_x, p, out_dtype, st);
+        return launch_linear_mx4(x, ld_x, p, out_dtype, st);
     }
     if (!workspace || workspace_bytes < cfp8_linear_workspace_bytes(M, K))
         return set_error(CFP8_EWORKSPACE, "linear_mxfp4: workspace of %zu bytes needed, %zu given", cfp8_linear_workspace_bytes(M, K), workspace_bytes);

@@ -483,6 +483,7 @@ int cfp8_gemm_grouped_block128(const void* a, int64_t ld_a, const float* sa,
 #define CFP8_DISPATCH_BLOCK 2          /* cfp8_gemm_block128              */
 #define CFP8_DISPATCH_GROUPED 3        /* cfp8_gemm_grouped_block128      */
 #define CFP8_DISPATCH_GROUPED_SWIGLU 4 /* cfp8_gemm_grouped_swiglu_quant  */
+#define CFP8_DISPATCH_LINEAR_MXFP4 6   /* cfp8_linear_mxfp4               */
 #define CFP8_DISPATCH_LARGE_WORKSPACE 1
 #define CFP8_DISPATCH_SPLIT 2
 #define CFP8_DISPATCH_NO_MEMORY 4

@@ -76,7 +76,8 @@ def test_wide_linear_as_streams_has_the_bits_of_the_two_steps(dev, N, K):
     mq, ms = ops.quant_mxfp4(w)
     bias = torch.randn(N, generator=g, device=dev).to(torch.bfloat16)
     for M in (1, 2, 3, 4):
-        assert _lib.gemm_dispatch_info(_lib.DISPATCH_LINEAR, M, N, K, cus=torch.cuda.get_device_properties(dev).multi_processor_count, flags=_lib.DISPATCH_SPLIT).startswith("linear_stream")
+        for kind, name in ((_lib.DISPATCH_LINEAR, "linear_stream"), (_lib.DISPATCH_LINEAR_MXFP4, "linear_mxfp4_stream")):
+            assert _lib.gemm_dispatch_info(kind, M, N, K, cus=torch.cuda.get_device_properties(dev).multi_processor_count, flags=_lib.DISPATCH_SPLIT).startswith(name)
         x = torch.randn(M, K + 16, generator=g, device=dev).to(torch.bfloat16)[:, :K]   # a pitch of its own
         if M == 4:
             x[1, 3], x[2] = float("nan"), 0.0
