@@ -65,6 +65,7 @@ SIGNATURES = {
     "cfp8_route_tokens": (c_int, [c_void_p, c_int, c_void_p, c_int64, c_int, c_int, c_int64, c_int, c_int64, c_void_p, c_void_p, c_void_p, c_void_p,
                                   c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
     "cfp8_moe_experts_workspace_bytes": (c_size_t, [c_int64, c_int, c_int, c_int64, c_int64]),
+    "cfp8_moe_experts_form": (c_int, [c_int64, c_int, c_int, c_int64, c_int64, c_char_p, c_size_t]),
     "cfp8_moe_experts": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p,
                                  c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_size_t, c_void_p]),
     "cfp8_gather_rows": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_void_p]),
@@ -153,6 +154,13 @@ def gemm_dispatch_info(kind: int, M: int, N: int, K: int, out_dtype: int = OUT_B
     DISPATCH_SPLIT in ``flags``: the entry point that the operators in ``ops`` call."""
     buf = ctypes.create_string_buffer(1024)
     check(load().cfp8_gemm_dispatch_info(kind, M, N, K, out_dtype, cus, flags | (DISPATCH_LARGE_WORKSPACE if with_split_workspace else 0), buf, len(buf)))
+    return buf.value.decode()
+
+
+def moe_experts_form(tokens: int, topk: int, experts: int, hidden: int, inter: int) -> str:
+    """The form of its products that ``cfp8_moe_experts`` takes."""
+    buf = ctypes.create_string_buffer(128)
+    check(load().cfp8_moe_experts_form(tokens, topk, experts, hidden, inter, buf, len(buf)))
     return buf.value.decode()
 
 

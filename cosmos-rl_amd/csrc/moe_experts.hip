@@ -19,6 +19,8 @@
 //               64 rows would hold one or two.  A workgroup takes a strip of ONE expert's weight rows, requests all of its
 //               K into registers before anything else, and then walks the expert's rows in tiles of 16
 //               (few_gate_up_kernel, few_down_kernel).
+#include <stdio.h>
+
 #include <atomic>
 
 #include "gemm_internal.h"
@@ -763,12 +765,16 @@ static bool many_idles(int64_t pairs, int64_t experts, int64_t hidden, int64_t i
     return inter <= hidden && experts * 3 * hidden * inter > kMemorySideCache && steps * 112 >= pairs * cus;
 }
 
-// few_stream_kernel in place of the kernels of a strip a workgroup: no more tiles of 16 rows than workgroups, so that a share lies in two, and
-// weights of 32 MiB and more: with less its tables are what takes the time.  Whole calls, us, strips / streams: 1 token of 32 experts of 1024 x 512, top 4 (6 MB) 16.4 / 18.7, 4
-// (25 MB) 18.9 / 20.5; of 128 of 2048 x 768, top 8: 1 (38 MB) 26.5 / 26.3, 4: 44.1 / 42.1, 16: 90.6 / 81.0, 64: 126.7 / 115.6, 150: 145 / 129; 32 of 3584 x 1536, top 4: 8:
-// 89.2 / 74.7, 60: 129 / 102; 30 of 64 of 1024 x 512, top 6: 34.3 / 33.2.
+// few_stream_kernel in place of the kernels of a strip a workgroup: no more tiles of 16 rows than workgroups, so that a share lies in two; some 640 strips of gate_up and more, of
+// which a wave each has enough of the weights in flight; and weights of 32 MiB and more, of 72 where strips are short and experts have a second row, of 80 where not: with less the
+// tables and a strip's ends are what takes the time.  Beyond kFewRowsPerExpert what they stand beside is the middle form, behind which they are nowhere.  Whole calls on weights that no cache holds, us, strips / streams:
+// 1 token of 64 experts of 3584 x 512, top 8 (512 strips, 42 MiB) 24.0 / 27.1, 2 of 8 of 3584 x 1024, top 2 (512, 42) 24.1 / 25.4, 1 of 60 of 2048 x 1408, top 4 (704, 33) 24.9 / 23.5, 1 of 32 of 3584 x 1536,
+// top 4 (768, 63) 31.0 / 28.0; 2 of 128 of 1280 x 1280, top 4 (38 MiB) 26.1 / 24.9; 32 of 1024 x 512, top 4: 8 (48 MiB, a row an expert) 21.2 / 22.8, 32: 24.1 / 25.6, 96 (12 rows; middle) 30.1 / 29.3; 16 of 2048 x
+// 512, top 4 (48): 8: 23.2 / 24.7, 48 (12 rows) 32.0 / 27.6; 32 of 1024 x 768, top 8 (72): 4: 25.4 / 26.9, 16: 30.3 / 29.7, 32: 32.4 / 30.8; 64 of 1024 x 512, top 6: 8 (72) 26.4 / 27.3, 21 (96)
+// 32.6 / 31.7; 128 of 2048 x 768, top 8: 1 (36) 24.6 / 25.1, 4: 42.4 / 41.0, 16: 90.6 / 81.0, 64: 126.7 / 115.6, 150: 145 / 129; 32 of 3584 x 1536, top 4: 8: 89.2 / 74.7, 60: 129 / 102.
 static bool few_streams(int64_t pairs, int64_t slots, int64_t experts, int64_t hidden, int64_t inter) {
-    return experts <= kStreamMostExperts && slots + pairs / 16 <= cu_count() && slots * 3 * hidden * inter >= (int64_t)32 << 20;
+    const int64_t least = pairs > kFewRowsPerExpert * experts || (inter >= 1024 && hidden > 1024) ? 32 : pairs > experts ? 72 : 80;
+    return experts <= kStreamMostExperts && slots + pairs / 16 <= cu_count() && slots * (inter / 8) >= 640 && slots * 3 * hidden * inter >= least << 20;
 }
 
 enum class Form { kFew, kMiddle, kMany };
@@ -777,6 +783,8 @@ struct ExpertsPlan {
     int64_t rows;   // rows of the expert-grouped layout (their bound)
     int64_t slots;  // experts that can have a row
     bool gathers;   // many rows: the gate_up product reads its rows from the quantised tokens
+    bool streams;   // few rows: few_stream_kernel
+    int down_rows;  // middle: rows of a tile of down_stream_kernel, 0: the ring kernel
     size_t row_tokens, row_experts, row_map, weights, m_sizes, m_offsets, route, xq, xs, h, hq, hs, out, bytes;
 };
 
@@ -786,8 +794,10 @@ static ExpertsPlan experts_plan(int64_t tokens, int topk, int experts, int64_t h
     p.gathers = experts_gate_up_takes(tokens, hidden, inter);
     const int64_t middle = !p.gathers || !experts_down_takes(hidden, inter) ? kMiddleRowsElsewhere : many_idles(pairs, experts, hidden, inter) ? kMiddleRowsManyIdle : kMiddleRowsPerExpert;
     p.slots = pairs < experts ? pairs : experts;
-    const bool behind = down_stream_rows(pairs, p.slots, experts, hidden, inter) && ring_grouped_takes(hidden) && ring_grouped_takes(inter) && (int64_t)experts * 3 * hidden * inter > kMemorySideCache;
-    const int64_t few = few_streams(pairs, p.slots, experts, hidden, inter) && !behind ? kStreamRowsPerExpert : kFewRowsPerExpert;
+    p.streams = few_streams(pairs, p.slots, experts, hidden, inter);
+    p.down_rows = down_stream_rows(pairs, p.slots, experts, hidden, inter);
+    const bool behind = p.down_rows && ring_grouped_takes(hidden) && ring_grouped_takes(inter) && (int64_t)experts * 3 * hidden * inter > kMemorySideCache;
+    const int64_t few = p.streams && !behind ? kStreamRowsPerExpert : kFewRowsPerExpert;
     if (pairs <= few * experts && hidden <= kFewMaxHidden && inter <= kFewMaxInter) p.form = Form::kFew;
     else if (pairs <= middle * experts && ring_grouped_takes(hidden) && ring_grouped_takes(inter) && tokens * hidden < (int64_t)1 << 31) p.form = Form::kMiddle;
     else p.form = Form::kMany;
@@ -823,6 +833,20 @@ static ExpertsPlan experts_plan(int64_t tokens, int topk, int experts, int64_t h
 extern "C" size_t cfp8_moe_experts_workspace_bytes(int64_t tokens, int topk, int experts, int64_t hidden, int64_t inter) {
     if (tokens <= 0 || topk <= 0 || experts <= 0 || hidden <= 0 || inter <= 0) return 0;
     return cfp8::experts_plan(tokens, topk, experts, hidden, inter).bytes;
+}
+
+extern "C" int cfp8_moe_experts_form(int64_t tokens, int topk, int experts, int64_t hidden, int64_t inter, char* buf, size_t buf_bytes) {
+    using namespace cfp8;
+    if (!buf || buf_bytes == 0) return set_error(CFP8_EINVAL, "moe_experts_form: no buffer");
+    buf[0] = 0;
+    if (tokens <= 0 || topk <= 0 || topk > 64 || experts <= 0 || hidden <= 0 || inter <= 0 || hidden % 128 || inter % 128 || tokens > 0x7FFFFFFFll / 64)
+        return set_error(CFP8_EINVAL, "moe_experts_form: bad shape");
+    const ExpertsPlan p = experts_plan(tokens, topk, experts, hidden, inter);
+    if (p.form == Form::kFew) snprintf(buf, buf_bytes, "few %s", p.streams ? "streams" : "strips");
+    else if (p.form == Form::kMany) snprintf(buf, buf_bytes, "many gate_up=%s down=%s", p.gathers ? "experts" : "grouped", experts_down_takes(hidden, inter) ? "experts" : "grouped");
+    else if (p.down_rows) snprintf(buf, buf_bytes, "middle down=streams,%d", p.down_rows);
+    else snprintf(buf, buf_bytes, "middle down=ring");
+    return CFP8_OK;
 }
 
 extern "C" int cfp8_moe_experts(const void* x, int64_t ld_x, int64_t tokens, int64_t hidden, const void* indices, int index_bytes,
@@ -867,7 +891,7 @@ extern "C" int cfp8_moe_experts(const void* x, int64_t ld_x, int64_t tokens, int
         r.M = (int)tokens; r.N = (int)(2 * inter); r.K = (int)hidden;
         if (int rc = launch_ring_grouped(kRingGateUp, r, row_tiles, once, st)) return rc;
         if (int rc = cfp8_quant_group128(ws + p.h, p.rows, inter, inter, ws + p.hq, inter, f32(p.hs), CFP8_GROUP_MODE_DIV, stream)) return rc;
-        if (const int tile = down_stream_rows(tokens * topk, p.slots, experts, hidden, inter)) {
+        if (const int tile = p.down_rows) {
             DownArgs d{};
             d.hq = ws + p.hq; d.hs = f32(p.hs); d.w = static_cast<const uint8_t*>(down); d.ws = down_scales;
             d.sizes = i32(p.m_sizes); d.out = reinterpret_cast<uint16_t*>(ws + p.out);
@@ -893,7 +917,7 @@ extern "C" int cfp8_moe_experts(const void* x, int64_t ld_x, int64_t tokens, int
         f.experts = experts;
         f.hidden = (int)hidden;
         f.inter = (int)inter;
-        if (few_streams(tokens * topk, p.slots, experts, hidden, inter)) {
+        if (p.streams) {
             f.tokens = (int)tokens;
             if (int rc = launch_few_stream<false>(f, st)) return rc;
             f.w = static_cast<const uint8_t*>(down);

@@ -300,6 +300,10 @@ int cfp8_combine_rows(const void* rows, int64_t ld_rows, int64_t num_rows, const
  * inter / 128], y bf16 [tokens, hidden] (ld_y): zero rows for tokens that go nowhere.  hidden, inter multiples of 128,
  * topk <= 64, experts <= 1024.  The workspace is 256-byte aligned and belongs to the call until the stream has run it. */
 size_t cfp8_moe_experts_workspace_bytes(int64_t tokens, int topk, int experts, int64_t hidden, int64_t inter);
+/* Which form of its products cfp8_moe_experts takes, on the current device or, without one, 256 compute units: "few strips", "few streams",
+ * "middle down=ring", "middle down=streams,<rows of a tile>" or "many gate_up=<kernel> down=<kernel>".  No counterpart in the reference: for tests,
+ * as cfp8_gemm_dispatch_info. */
+int cfp8_moe_experts_form(int64_t tokens, int topk, int experts, int64_t hidden, int64_t inter, char* buf, size_t buf_bytes);
 int cfp8_moe_experts(const void* x, int64_t ld_x, int64_t tokens, int64_t hidden, const void* indices, int index_bytes,
                      const uint8_t* token_mask, const void* weights, int weights_dtype, int topk, int experts,
                      const void* gate_up, const float* gate_up_scales, const void* down, const float* down_scales, int64_t inter,

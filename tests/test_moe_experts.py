@@ -201,16 +201,24 @@ def test_token_masks_of_other_forms(dev):
             route_tokens(idx, mask, E)
 
 
-# decode batches as streams of strips (32 MiB of weights and more): one K step in either product, more units of a wave than stages and fewer, experts of 16, 17 and
-# more rows, 256 experts, one tile a workgroup and two, tokens of which none is left
-@pytest.mark.parametrize("T,E,topk,H,I", [(20, 64, 4, 4096, 128), (30, 64, 4, 128, 1536), (2, 128, 8, 2048, 768), (16, 1, 1, 4096, 4096), (17, 3, 1, 4096, 1536), (64, 40, 4, 3072, 640),
-                                          (90, 256, 4, 512, 384), (33, 32, 8, 1152, 1408), (1, 9, 9, 4096, 1152), (130, 127, 8, 1664, 256),
-                                          # down as streams behind tiles of 64 rows: tiles of 64 rows and one to six steps of K, 48 and seven or eight, 32 and 9 to 13; as many tiles as CUs
-                                          (500, 70, 4, 4096, 128), (300, 64, 6, 4096, 256), (600, 127, 8, 2944, 384), (400, 33, 3, 3584, 640), (448, 128, 8, 2048, 768), (450, 200, 8, 1536, 128),
-                                          (200, 64, 8, 1280, 896), (250, 64, 8, 1024, 1024), (160, 40, 5, 1152, 1152), (150, 32, 4, 3584, 1536), (170, 9, 1, 4096, 1664)])
+# the forms of a decode batch and of a chunk of prefill, each with the shape that makes the choice: streams of strips with one K step in either product, more units of a wave than stages and fewer, experts of 16
+# rows and more, as many tiles as workgroups have room for, 11 rows an expert of few weights; weights of which a strip a workgroup is read; down as streams behind tiles of 64 rows with one to six steps
+# of K, 48 with seven or eight, 32 with 9 to 13, and by the ring kernel; tokens of which none is left
+EXPERT_FORMS = [("few streams", 20, 64, 4, 4096, 128), ("few streams", 40, 130, 4, 128, 1536), ("few streams", 3, 128, 8, 2048, 768), ("few streams", 12, 4, 1, 4096, 1536),
+                ("few streams", 33, 4, 1, 4096, 1536), ("few streams", 64, 40, 4, 3072, 640), ("few streams", 60, 256, 4, 512, 384), ("few streams", 33, 32, 8, 1152, 1408),
+                ("few streams", 1, 9, 9, 4096, 1152), ("few streams", 130, 127, 8, 1664, 256), ("few streams", 48, 32, 8, 1024, 512), ("few strips", 2, 128, 8, 2048, 768),
+                ("few strips", 30, 64, 4, 128, 1536), ("few strips", 90, 256, 4, 512, 384), ("few strips", 17, 3, 1, 4096, 1536), ("middle down=streams,64", 500, 70, 4, 3968, 128),
+                ("middle down=streams,64", 300, 64, 6, 3968, 256), ("middle down=streams,64", 600, 127, 8, 2944, 384), ("middle down=streams,64", 400, 33, 3, 3584, 640),
+                ("middle down=streams,64", 448, 128, 8, 2048, 768), ("middle down=streams,64", 450, 200, 8, 1536, 128), ("middle down=streams,48", 200, 64, 8, 1280, 896),
+                ("middle down=streams,48", 250, 64, 8, 1024, 1024), ("middle down=streams,32", 160, 40, 5, 1152, 1152), ("middle down=streams,32", 150, 32, 4, 3584, 1536),
+                ("middle down=streams,32", 170, 9, 1, 3968, 1664), ("middle down=ring", 40, 8, 4, 1024, 512), ("middle down=ring", 60, 4, 1, 3968, 3968)]
+
+
+@pytest.mark.parametrize("form,T,E,topk,H,I", EXPERT_FORMS)
 @pytest.mark.parametrize("kept", [1.0, 0.6, 0.0])
-def test_one_call_experts_as_streams(dev, T, E, topk, H, I, kept):
+def test_one_call_experts_forms(dev, form, T, E, topk, H, I, kept):
     from cosmos_rl_amd.policy.kernel.moe.moe import grouped_experts_forward
+    assert _lib.moe_experts_form(T, topk, E, H, I) == form
     strategy, module = _module(dev, E, H, I, T)
     g = torch.Generator(device=dev).manual_seed(T + 5)
     x = torch.randn(T, H, generator=g, device=dev).to(torch.bfloat16)
