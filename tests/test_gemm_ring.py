@@ -280,3 +280,51 @@ def test_strips_of_few_rows(dev, mode, strips, M, N, K):
         assert all(torch.equal(got.nan_to_num(3.0), run(dtype).nan_to_num(3.0)) for _ in range(2))
         first = 1 if M > 1 else 0
         _check(torch.nn.functional.pad(got[first:], (0, 8, 0, 1), value=7.0), want[first:], M - first, N, dtype, 0.0)
+
+
+# the same with a bias, all of K a workgroup and in slices, and operands inside rows of their own pitch, whose other bytes are NaN in e4m3 and the largest codes and scales; the last row ends with its memory
+STRIPS_PITCHED = [("rowwise", 3, 17, 8208, 400), ("rowwise", 5, 33, 18944, 384), ("rowwise", 7, 80, 28560, 1808), ("rowwise", 10, 81, 37888, 256), ("rowwise", 9, 209, 36864, 448), ("rowwise", 4, 24, 2880, 2880),
+                  ("mxfp4", 3, 5, 8208, 160), ("mxfp4", 5, 33, 18944, 384), ("mxfp4", 9, 144, 32784, 352), ("mxfp4", 4, 26, 3200, 2784), ("block", 5, 33, 16400, 384), ("block", 4, 9, 3840, 2176)]
+
+
+@pytest.mark.parametrize("mode,strips,M,N,K", STRIPS_PITCHED)
+def test_strips_of_few_rows_with_pitches_and_a_bias(dev, mode, strips, M, N, K):
+    kind = {"rowwise": _lib.DISPATCH_ROWWISE, "block": _lib.DISPATCH_BLOCK, "mxfp4": _lib.DISPATCH_MXFP4}[mode]
+    took = _lib.gemm_dispatch_info(kind, M, N, K, cus=torch.cuda.get_device_properties(dev).multi_processor_count, flags=_lib.DISPATCH_SPLIT)
+    assert took.startswith(f"gemm_ring_few<{mode},{-(-M // 16)},{strips}>"), took
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g, device=dev).to(torch.bfloat16)
+    w = torch.randn(N, K, generator=g, device=dev) * 0.05
+    bias = torch.randn(N, generator=g, device=dev).to(torch.bfloat16)
+
+    def pitched(t, more, filler):
+        whole = torch.full((t.shape[0], t.shape[1] + more), filler, dtype=torch.uint8, device=dev)
+        whole[:, more:] = t.view(torch.uint8)
+        return whole[:, more:]
+
+    lib, (part, need) = _lib.load(), _partial(kind, M, N, K, dev)
+    if mode == "block":
+        (q, s), b = ops.groupwise_activation_quant(x), (w.to(torch.float8_e4m3fn), torch.rand(-(-N // 128), K // 128, generator=g, device=dev) + 0.5)
+        plain = lambda dtype: ops.gemm_fp8_fp8_bf16_nt((q, s), b, torch.empty(M, N, device=dev, dtype=dtype))
+    elif mode == "mxfp4":
+        (q, s), b = ops.quant_rowwise(x), ops.quant_mxfp4(w.to(torch.bfloat16))
+        plain = lambda dtype: ops.gemm_mxfp4((q, s), b, dtype)
+        scales = pitched(b[1], 3, 0xFF)
+    else:
+        (q, s), b = ops.quant_rowwise(x), ops.quant_rowwise(w.to(torch.bfloat16))
+        plain = lambda dtype: ops.scaled_mm(q, b[0].t(), s, b[1].reshape(1, N), out_dtype=dtype)
+    pq, pw = pitched(q, 32, 0x7F), pitched(b[0], 64 if mode == "mxfp4" else 48, 0x77 if mode == "mxfp4" else 0x7F)
+    for dtype in (torch.float32, torch.bfloat16):
+        for add in (None, bias) if mode == "rowwise" else (None,):
+            out = _out(M, N, dev, dtype)
+            tail = (out.data_ptr(), N + 8, ops._out_code(dtype), M, N, K, part.data_ptr(), need, _stream())
+            if mode == "block":
+                rc = lib.cfp8_gemm_block128_split(pq.data_ptr(), pq.stride(0), s.data_ptr(), pw.data_ptr(), pw.stride(0), b[1].data_ptr(), K // 128, 1, *tail)
+            elif mode == "mxfp4":
+                rc = lib.cfp8_gemm_mxfp4_split(pq.data_ptr(), pq.stride(0), s.data_ptr(), pw.data_ptr(), pw.stride(0), scales.data_ptr(), scales.stride(0), *tail)
+            else:
+                rc = lib.cfp8_scaled_mm_rowwise_split(pq.data_ptr(), pq.stride(0), s.data_ptr(), pw.data_ptr(), pw.stride(0), b[1].data_ptr(), ops._ptr(add), *tail)
+            _lib.check(rc)
+            want = plain(dtype)
+            assert torch.equal(out[:M, :N], want if add is None else want + add)
+            assert bool((out[M:] == 7.0).all()) and bool((out[:, N:] == 7.0).all())
