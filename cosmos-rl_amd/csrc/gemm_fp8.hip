@@ -3430,13 +3430,10 @@ static int launch_rowwise_best(GemmArgs& p, int out_dtype, hipStream_t st) {
     r.ld_a = p.ld_a; r.ld_w = p.ld_b; r.ld_out = p.ld_out;
     r.M = p.M; r.N = p.N; r.K = p.K;
     RingPlan ring{0, 0, 0, 1e30};
-    int strips = 0;
     // (where the linear is one launch the product has its bits, those of the kernel for 16 tokens)
     if (!fused_gemv_size(p.M, p.K) && ring_takes(kRingRow, r, out_dtype)) {
-        strips = ring_few_strips(kRingRow, r);
-        // beyond 80 rows the form for few rows is ahead of every other kernel where it is taken
-        if (strips && p.M > 80) return launch_ring_few(kRingRow, r, strips, out_dtype, st);
         ring = ring_plan(kRingRow, p.M, p.N, p.K, p.partial_bytes, cus);
+        if (const int strips = ring_few_first(kRingRow, r, ring)) return launch_ring_few(kRingRow, r, strips, out_dtype, st);
     }
     EdgePlan edge{};
     edge.cost = 1e30;
@@ -3450,8 +3447,6 @@ static int launch_rowwise_best(GemmArgs& p, int out_dtype, hipStream_t st) {
     if (ring.cost < 1e30 && ring.cost <= edge.cost && ring.cost <= other) return launch_ring(kRingRow, r, ring, out_dtype, st);
     // (without a bias and without remainders launch_gemm's form of the same tiles is 2 % faster)
     const bool even = p.M % 256 == 0 && p.N % 256 == 0 && !p.bias;
-    // the strips of launch_gemm's own kernel (33 x 18944 x 3584 16.1 -> 14.5 us)
-    if (strips >= 5 && p.M > 16 && other <= edge.cost) return launch_ring_few(kRingRow, r, strips, out_dtype, st);
     if (edge.cost < 1e30 && edge.cost <= other && !even) return launch_rowwise_edge(p, edge, out_dtype, st);
     float* const partial = p.partial;
     p.partial = nullptr;  // (launch_gemm's own slices are those of cfp8_linear_rowwise)
@@ -3536,7 +3531,11 @@ static int launch_block_best(GemmArgs& p, int out_dtype, hipStream_t st) {
     r.ld_a = p.ld_a; r.ld_w = p.ld_b; r.ld_out = p.ld_out;
     r.sb_stride_n = p.sb_stride_n; r.sb_stride_k = p.sb_stride_k;
     r.M = p.M - (int)plan.body; r.N = p.N; r.K = p.K;
-    if (!plan.ring.bm || !ring_takes(kRingBlock, r, out_dtype)) return launch_gemm<kBlock>(p, out_dtype, st);
+    const bool takes = ring_takes(kRingBlock, r, out_dtype);
+    if (takes && !plan.body) {
+        if (const int strips = ring_few_first(kRingBlock, r, plan.ring)) return launch_ring_few(kRingBlock, r, strips, out_dtype, st);
+    }
+    if (!plan.ring.bm || !takes) return launch_gemm<kBlock>(p, out_dtype, st);
     if (plan.body) {
         GemmArgs body = p;
         body.M = (int)plan.body;

@@ -1824,12 +1824,11 @@ static int gemm_mx4_dense(Mx4Args& p, float* partial, size_t partial_bytes, int 
     r.M = p.M; r.N = p.N; r.K = p.K;
     // (up to 4 tokens of K <= 4096 cfp8_linear_mxfp4 is one launch, whose bits the kernel for 16 tokens gives)
     if ((p.M <= 4 && p.K <= 4096) || !ring_takes(kRingMx, r, out_dtype)) return CFP8_OK;
-    // the form for few rows is ahead of every other kernel where it is taken
-    if (const int strips = ring_few_strips(kRingMx, r)) {
+    const RingPlan plan = ring_plan(kRingMx, p.M, p.N, p.K, partial_bytes, cu_count());
+    if (const int strips = ring_few_first(kRingMx, r, plan)) {
         taken = true;
         return launch_ring_few(kRingMx, r, strips, out_dtype, st);
     }
-    const RingPlan plan = ring_plan(kRingMx, p.M, p.N, p.K, partial_bytes, cu_count());
     if (p.M <= 128) {
         // (ring kernel / streamers: 18944 x 3584 at 33 tokens 19.5 / 17.4 us, 16 x 3584 x 3584 8.2 / 6.2, but 33 x 25344 x 2560 15.3 / 25.3)
         if (mx4_streams_cost(p.M, p.N, p.K, cu_count()) <= plan.cost) return CFP8_OK;

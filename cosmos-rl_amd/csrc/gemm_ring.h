@@ -34,8 +34,8 @@ struct RingPlan {
 };
 RingPlan ring_plan(int mode, int64_t M, int64_t N, int64_t K, size_t partial_bytes, int cus);
 bool ring_takes(int mode, const RingArgs& p, int out_dtype);  // whether the operands fit what the kernel assumes
-// the form for few rows, all of K a workgroup: strips of 16 weight rows a workgroup, 0: other kernels are ahead
-int ring_few_strips(int mode, const RingArgs& p);
+// the form for few rows, all of K a workgroup, in place of `plan` and of every other file's kernel: strips of 16 weight rows a workgroup, 0: not
+int ring_few_first(int mode, const RingArgs& p, const RingPlan& plan);
 int launch_ring_few(int mode, RingArgs& p, int strips, int out_dtype, hipStream_t st);
 // the linear of up to four tokens (K <= 4096, one token 8192, a multiple of 128) as one launch of streams: waves a workgroup, 0: other kernels are ahead
 int linear_stream_waves(int mode, int64_t M, int64_t N, int64_t K);

@@ -179,7 +179,7 @@ FORMS = [("block", 64, 64, False, 67, 208, 384), ("block", 64, 64, False, 5, 208
          ("mxfp4", 128, 128, True, 131, 2832, 7360), ("mxfp4", 128, 128, True, 67, 5648, 5312), ("rowwise", 64, 64, False, 67, 208, 384), ("rowwise", 64, 64, False, 34, 8656, 256),
          ("rowwise", 64, 64, False, 5, 80, 320), ("rowwise", 64, 64, True, 67, 208, 2176), ("rowwise", 64, 64, True, 51, 208, 2560), ("rowwise", 64, 64, True, 54, 80, 1728),
          ("rowwise", 64, 128, False, 131, 9232, 384), ("rowwise", 64, 128, False, 5, 58704, 256), ("rowwise", 64, 128, True, 131, 1808, 5248),
-         ("rowwise", 64, 128, True, 131, 1808, 5312), ("rowwise", 64, 128, True, 17, 8912, 10624), ("rowwise", 64, 128, True, 18, 17424, 5056),
+         ("rowwise", 64, 128, True, 131, 1808, 5312), ("rowwise", 64, 128, True, 17, 8912, 10624), ("rowwise", 64, 128, True, 17, 8704, 8896),
          ("rowwise", 128, 64, False, 131, 5648, 384), ("rowwise", 128, 64, False, 67, 9232, 384), ("rowwise", 128, 64, True, 1500, 208, 5248),
          ("rowwise", 128, 64, True, 67, 2832, 3712), ("rowwise", 128, 64, True, 1031, 208, 7360), ("rowwise", 128, 64, True, 67, 2832, 3776),
          ("rowwise", 128, 128, False, 515, 3600, 640), ("rowwise", 128, 128, False, 131, 11792, 704), ("rowwise", 128, 128, False, 67, 29072, 512),
