@@ -1,7 +1,7 @@
 // The ring kernel's form for few rows (included by gemm_ring.hip): all rows in one tile, every wave a strip of 16 weight rows of its own.
-// Rowwise up to 256 rows, MXFP4 208, block-scaled 128.
+// Rowwise up to 256 rows, MXFP4 255, block-scaled 128.
 //
-// Bound by the weights' way in, and behind it by the activations that every workgroup loads.  A wave reads its strip, 8 rows x 128 bytes a
+// Bound by the weights' way in, and behind it by the activations, which every workgroup loads and every wave reads from LDS.  A wave reads its strip, 8 rows x 128 bytes a
 // load, into a ring of its own that no barrier guards; the workgroup shares the activations, a chunk of one or two K steps of all
 // rows, and has one barrier a chunk.  So a workgroup can have any number of strips, and the weight is dealt to the CUs evenly, one
 // workgroup each: 2368 strips as 237 workgroups of ten, where tiles of 64 x 64 are 592 on 512 places and load the activations 592 times.
@@ -9,9 +9,9 @@
 // a fragment's own address pattern straight into registers, 16 rows at a time, stops at 5 TB/s where this one reaches 6.2.
 // Products, us, tiles of the ring kernel / this form, weights cold: 5 x 37888 x 3584 26.6 / 22.6, 33: 28.7 / 24.3, 64: 33.1 / 25.9, 128: 43.9 / 31.8,
 // 200: 56.5 / 43.3, 256: 65.0 / 48.3; 33 x 25344 x 2560 15.2 / 14.2; block-scaled 24 x 18432 x 7168 30.3 / 23.5, 64: 35.2 / 29.5, 100: 47.0 / 40.0.
-// MXFP4: 5 x 37888 x 3584 26.2 / 15.7, 33: 30.9 / 18.4, 128: 44.8 / 28.5, 200: 46.3 / 39.5 (256: 40.5 / 44.9, so 208 rows are the limit); 33 x 18944 x 3584 17.3 / 12.3.
-// At 200 rows a step takes 1.4 us, for which 39 products on the fullest SIMD are 0.6; two or three strips a wave, whose fragments are read half or a third as often, take 47 and 76 us
-// with their four to six waves, chunks of two steps and other depths no less.
+// MXFP4: 5 x 37888 x 3584 26.2 / 15.7, 33: 30.9 / 18.4, 128: 44.8 / 28.5, 200: 46.3 / 39.5; 33 x 18944 x 3584 17.3 / 12.3.
+// MXFP4, 200 rows: a step takes 1.4 us.  The 39 products on the fullest SIMD are 0.6 of it; ten waves that each read 26 KiB of activations and 1 of weights from LDS are 0.9 at 128 bytes a cycle.
+// Two or three strips a wave, whose fragments are read half or a third as often, take 47 and 76 us with their four to six waves, chunks of two steps and other depths no less.
 // Sums and scales are taken in the order of K as in the tiles of the ring kernel, and have their bits.
 #pragma once
 

@@ -243,12 +243,12 @@ def test_a_bias_that_torch_follows(dev):
         ops.fp8_linear(x, q.t(), s, bias=bias.cpu())
 
 
-# few rows, a strip of 16 weight rows a wave: row tiles of 16 up to the last (16, one; 128, eight; 208, thirteen in the shallower ring, 256), 3 to 12 waves, a last
+# few rows, a strip of 16 weight rows a wave: row tiles of 16 up to the last (16, one; 128, eight; 208, thirteen in the shallower ring, 255 and 256, sixteen), 3 to 12 waves, a last
 # workgroup with waves beyond N, strips on both sides of a 128-block's edge, one K step, fewer than the ring is deep, a last step of 16 and of 64
 FEW = [("rowwise", 3, 16, 8208, 128), ("rowwise", 3, 17, 12288, 400), ("rowwise", 4, 32, 16384, 704), ("rowwise", 5, 33, 18944, 384), ("rowwise", 7, 80, 28560, 1792), ("rowwise", 10, 81, 37888, 256),
        ("rowwise", 9, 128, 32784, 128), ("rowwise", 12, 129, 49152, 144), ("rowwise", 10, 208, 37904, 640), ("rowwise", 9, 209, 36864, 448), ("rowwise", 9, 256, 33024, 512),
        ("mxfp4", 3, 5, 8208, 128), ("mxfp4", 3, 17, 12288, 416), ("mxfp4", 4, 32, 16384, 640), ("mxfp4", 3, 4, 8448, 4256), ("mxfp4", 5, 33, 18944, 256), ("mxfp4", 5, 113, 16400, 3232), ("mxfp4", 7, 96, 24592, 2592), ("mxfp4", 9, 128, 32784, 352),
-       ("mxfp4", 10, 129, 37888, 128), ("mxfp4", 9, 144, 32784, 352), ("mxfp4", 12, 200, 49152, 480), ("mxfp4", 10, 208, 37904, 512),
+       ("mxfp4", 10, 129, 37888, 128), ("mxfp4", 9, 144, 32784, 352), ("mxfp4", 12, 200, 49152, 480), ("mxfp4", 10, 208, 37904, 512), ("mxfp4", 9, 209, 32784, 416), ("mxfp4", 10, 240, 37904, 256), ("mxfp4", 11, 225, 41008, 2176), ("mxfp4", 9, 255, 33040, 288),
        ("block", 3, 1, 12288, 128), ("block", 3, 32, 8208, 1024), ("block", 4, 7, 16256, 640), ("block", 5, 33, 18432, 256), ("block", 5, 65, 16400, 384), ("block", 6, 128, 24464, 1536), ("block", 7, 112, 28544, 1408)]
 
 
