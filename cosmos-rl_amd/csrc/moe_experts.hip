@@ -16,9 +16,11 @@
 //               down_stream_kernel the down weights strip by strip.  The
 //               hidden activation is quantised in between, since a 1x128 group of it is spread over two workgroups.
 //   few rows    A decode batch: reading the weights of the experts that have a row is all the time there is, and tiles of
-//               64 rows would hold one or two.  A workgroup takes a strip of ONE expert's weight rows, requests all of its
-//               K into registers before anything else, and then walks the expert's rows in tiles of 16
-//               (few_gate_up_kernel, few_down_kernel).
+//               64 rows would hold one or two.  One workgroup a CU, whose eight waves each take strips of 16 weight rows one
+//               behind the other through LDS stages of their own, for tiles of 16 of an expert's rows (few_stream_kernel); with
+//               less to read (few_streams) a workgroup takes a strip of ONE expert's weight rows, requests all of its K into
+//               registers before anything else, and then walks the expert's rows in tiles of 16 (few_gate_up_kernel,
+//               few_down_kernel).
 #include <stdio.h>
 
 #include <atomic>
@@ -29,8 +31,9 @@
 
 namespace cfp8 {
 
-// The few-rows form holds a strip's whole K in registers: up to 8 K steps a wave of four (gate_up, 128 registers of weights and 64 of
-// tokens), 12 a wave (down, 96 registers, and two tiles of 16 rows of 1536 bytes in LDS).
+// few_gate_up_kernel and few_down_kernel hold a strip's whole K in registers: up to 8 K steps a wave of four (gate_up, 128 registers of weights and
+// 64 of tokens), 12 a wave (down, 96 registers, and two tiles of 16 rows of 1536 bytes in LDS).  few_stream_kernel's tables of two tiles fit LDS beside
+// its stages up to there (down 150 KiB), and its threads load one or two weight scales each and one activation scale (the static_asserts beside the loads).
 constexpr int64_t kFewMaxHidden = 4096, kFewMaxInter = 1536;
 
 struct FewArgs {
@@ -736,9 +739,12 @@ static void launch_few_down(int ni, dim3 grid, hipStream_t st, const FewArgs& p)
 // 50: 114.6 / 121.4, 52: 124.9 / 124.5; 32 of 2560 x 1280: 46: 94.9 / 100.1, 50: 97.1 / 100.3; 48 of 3584 x 1408: 46: 177 / 182; 24 of 3584 x 1536: 46: 111 / 120.
 // Streams / middle: 128 experts of 2048 x 768: 11 rows 132.1 / 134.0, 13: 143.1 / 137.1; 32 of 3584 x 1536: 11: 105.3 / 118.5, 13: 112.3 / 116.4; 64 of 1024 x 512: 12: 36.9 / 38.9, 16: 41.9 /
 // 39.4; 64 of 2048 x 1024: 12: 90.8 / 89.9.
-// Where the middle form's down is down_stream_kernel and the weights are more than the memory-side cache holds, the line is at 10 rows again; streams / middle: 128 of 2048 x 768: 10: 118.1 / 119.6,
-// 11: 126.5 / 120.6, 12: 127.6 / 121.3; 128 of 3584 x 640: 10: 176.4 / 170.9, 12: 189.4 / 174.4; 32 of 3584 x 1536: 9: 98.1 / 105.5, 11: 100.1 / 106.8, 12: 114.6 / 107.2; 64 of 2048 x 1024: 10: 81.4 /
-// 82.0, 12: 82.5 / 82.6; 128 of 1280 x 1280: 10: 129.0 / 127.9, 12: 139.7 / 129.5; weights that it holds, 64 of 1024 x 512: 12: 34.3 / 35.1.
+// Where the middle form's down is down_stream_kernel and the weights are more than the memory-side cache holds, the line is at 10 rows again, between crossings that lie from 8 to beyond 12: what streams lose are
+// experts with a second tile of 16 rows, which read their weights again, and how many those are, or leave CUs a second share, is not in the mean.  Weights that no cache holds, streams / middle: 128 of 2048 x 768: 6: 112.9 / 116.3,
+// 8: 122.9 / 118.1, 9: 122.1 / 119.9, 10: 127.2 / 121.6, 12: 130.9 / 122.7, but 100 of them: 10: 98.4 / 105.0, 12: 105.6 / 108.2; 128 of 3584 x 640: 8: 166.8 / 167.4, 9: 173.7 / 171.5, 10: 178.0 / 172.1, 12: 191.8 / 175.2;
+// 64 of 3584 x 1024: 7: 132.8 / 133.0, 8: 133.9 / 129.0, 10: 137.1 / 130.6; 32 of 3584 x 1536: 10: 104.3 / 108.4, 11: 104.0 / 108.4, 12: 117.4 / 109.2; 64 of 2048 x 1024: 9: 80.0 / 83.2, 10: 82.6 / 83.3, 11: 86.9 / 84.2;
+// 128 of 1280 x 1280: 9: 127.5 / 128.5, 10: 130.1 / 129.4, 12: 138.9 / 130.9; 96 of 2560 x 896: 9: 128.6 / 129.9, 10: 132.1 / 130.6, 12: 148.1 / 134.9.  At the line it is up to 5 % either way.  Weights that the cache holds,
+// 64 of 1024 x 512: 12: 37.7 / 38.6.
 // Where gemm_experts_kernel does not take both products, against the other grouped GEMMs: 128 of 2048 x 768: 96: 233 / 246, 128: 266 / 256.
 constexpr int64_t kFewRowsPerExpert = 10, kStreamRowsPerExpert = 12, kMiddleRowsPerExpert = 44, kMiddleRowsManyIdle = 50, kMiddleRowsElsewhere = 112;
 // Many rows: up to here an expert has a second tile of 128 rows seldom enough for streaming loads of the weights to pay, if they are
