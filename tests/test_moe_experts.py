@@ -204,9 +204,9 @@ def test_token_masks_of_other_forms(dev):
 # the forms of a decode batch and of a chunk of prefill, each with the shape that makes the choice: streams of strips with one K step in either product, more units of a wave than stages and fewer, experts of 16
 # rows and more, as many tiles as workgroups have room for, 11 rows an expert of few weights; weights of which a strip a workgroup is read; down as streams behind tiles of 64 rows with one to six steps
 # of K, 48 with seven or eight, 32 with 9 to 13, and by the ring kernel; tokens of which none is left
-EXPERT_FORMS = [("few streams", 20, 64, 4, 4096, 128), ("few streams", 40, 130, 4, 128, 1536), ("few streams", 3, 128, 8, 2048, 768), ("few streams", 12, 4, 1, 4096, 1536),
+EXPERT_FORMS = [("few streams", 20, 64, 4, 4096, 128), ("few streams", 70, 130, 4, 128, 1536), ("few streams", 3, 128, 8, 2048, 768), ("few streams", 12, 4, 1, 4096, 1536),
                 ("few streams", 33, 4, 1, 4096, 1536), ("few streams", 64, 40, 4, 3072, 640), ("few streams", 60, 256, 4, 512, 384), ("few streams", 33, 32, 8, 1152, 1408),
-                ("few streams", 1, 9, 9, 4096, 1152), ("few streams", 130, 127, 8, 1664, 256), ("few streams", 48, 32, 8, 1024, 512), ("few strips", 2, 128, 8, 2048, 768),
+                ("few streams", 1, 9, 9, 4096, 1152), ("few streams", 130, 127, 8, 1664, 256), ("few streams", 48, 32, 8, 1024, 512), ("few strips", 1, 128, 8, 2048, 768),
                 ("few strips", 30, 64, 4, 128, 1536), ("few strips", 90, 256, 4, 512, 384), ("few strips", 17, 3, 1, 4096, 1536), ("middle down=streams,64", 500, 70, 4, 3968, 128),
                 ("middle down=streams,64", 300, 64, 6, 3968, 256), ("middle down=streams,64", 600, 127, 8, 2944, 384), ("middle down=streams,64", 400, 33, 3, 3584, 640),
                 ("middle down=streams,64", 448, 128, 8, 2048, 768), ("middle down=streams,64", 450, 200, 8, 1536, 128), ("middle down=streams,48", 200, 64, 8, 1280, 896),
