@@ -100,9 +100,11 @@ def test_wide_linear_of_one_token_up_to_8192_columns(dev):
 
 # weights and scales inside rows of their own pitch, whose other bytes are NaN in e4m3, the largest codes and NaN scales; the last row ends with its memory.  Odd numbers of K steps:
 # MXFP4 weights are loaded by two, and an odd last one ends in the middle of a load (which bytes are read is a static_assert in gemm_ring_few.h)
-@pytest.mark.parametrize("N,K", [(8224, 128), (8224, 384), (12304, 640), (8208, 3968), (8208, 4096)])
+@pytest.mark.parametrize("N,K", [(8224, 128), (8224, 384), (12304, 640), (12304, 3968), (8208, 4096)])
 @pytest.mark.parametrize("M", [1, 4])
 def test_wide_linear_of_weights_with_a_pitch(dev, M, N, K):
+    took = _lib.gemm_dispatch_info(_lib.DISPATCH_LINEAR_MXFP4, M, N, K, cus=torch.cuda.get_device_properties(dev).multi_processor_count, flags=_lib.DISPATCH_SPLIT)
+    assert took.startswith("linear_mxfp4_stream "), took
     g = torch.Generator(device=dev).manual_seed(N + K + M)
     x = torch.randn(M, K, generator=g, device=dev).to(torch.bfloat16)
     w = (torch.randn(N, K, generator=g, device=dev) * 0.05).to(torch.bfloat16)
