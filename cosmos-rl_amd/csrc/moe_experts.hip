@@ -773,7 +773,7 @@ static bool many_idles(int64_t pairs, int64_t experts, int64_t hidden, int64_t i
 
 // few_stream_kernel in place of the kernels of a strip a workgroup: no more tiles of 16 rows than workgroups, so that a share lies in two; some 640 strips of gate_up and more, of
 // which a wave each has enough of the weights in flight; and weights of 32 MiB and more, where strips are short of 64 from a third row an expert on, of 72 and (a short
-// K of gate_up) 80 with fewer rows: with less the tables and a strip's ends are what takes the time.  Beyond kFewRowsPerExpert what they stand beside is the middle form, behind which they are nowhere.  Whole calls on weights that no cache holds, us, strips / streams:
+// K of gate_up) 80 with fewer rows: with less the tables and a strip's ends are what takes the time.  Beyond kFewRowsPerExpert what they stand beside is the middle form, which they are ahead of nearly everywhere (32 of 1024 x 1024, 12 rows, 39.2 / 37.7).  Whole calls on weights that no cache holds, us, strips / streams:
 // 1 token of 64 experts of 3584 x 512, top 8 (512 strips, 42 MiB) 24.0 / 27.1, 2 of 8 of 3584 x 1024, top 2 (512, 42) 24.1 / 25.4, 1 of 60 of 2048 x 1408, top 4 (704, 33) 24.9 / 23.5, 1 of 32 of 3584 x 1536,
 // top 4 (768, 63) 31.0 / 28.0; 2 of 128 of 1280 x 1280, top 4 (38 MiB) 26.1 / 24.9; 32 of 1024 x 512, top 4: 8 (48 MiB, a row an expert) 21.2 / 22.8, 32: 24.1 / 25.6, 96 (12 rows; middle) 30.1 / 29.3; 16 of 2048 x
 // 512, top 4 (48): 8: 23.2 / 24.7, 48 (12 rows) 32.0 / 27.6; 32 of 1024 x 768, top 8 (72): 4: 25.4 / 26.9, 16: 30.3 / 29.7, 32: 32.4 / 30.8; 32 of 1152 x 640, top 4 (68): 32: 32.2 / 30.6; 2 of 128 of 3328 x 768, top 5 (73) 32.0 / 31.0; 5 of 64 of 1024 x 640, top 8 (75) 28.9 / 29.4; 64 of 1024 x 512, top 6: 8 (72) 26.4 / 27.3, 21 (96)
