@@ -3416,8 +3416,8 @@ static double rowwise_tiles_cost(int64_t M, int64_t N, int64_t K, int cus) {
     return 8.91 + beside(time((M + 255) / 256 * ((N + 255) / 256), 1.415, 0.238, 3.65), in / 2.98e6);
 }
 
-// Rowwise product with a bias and memory for partial sums: the form with the least estimated time among the ring kernel
-// (gemm_ring.hip), the walking 256 x 256 tiles with edges, and launch_gemm.
+// Rowwise product with a bias and memory for partial sums: strips of few rows where they go first (gemm_ring.hip: ring_few_first), else the form with
+// the least estimated time among the ring kernel's tiles, the walking 256 x 256 tiles with edges, and launch_gemm.
 // Timed with weights that no cache holds, ring / launch_gemm: 21 x 896 x 17152 11 / 33, 33 x 25344 x 2560 15.0 / 23.6; 33 x 18944 x
 // 3584, one round of strips, 17.3 / 16.4, 64 x 2048 x 1536 7.0 / 6.2, 16 x 1792 x 1792 6.8 / 4.3; 739 x 1024 x 1024 5.8 / 21.7, 152 x 1792
 // x 12672 17 / 88, 1061 x 2560 x 7936 40 / 75, 1024 x 3584 x 3584 with the quantiser 24 / 31; but 2048 x 3584 x 3584, 224 of its tiles of
@@ -3492,7 +3492,7 @@ static double block_tiles_cost(int64_t M, int64_t N, int64_t K, int cus) {
     return 5.41 + beside(time((M + 127) / 128 * ((N + 127) / 128), 2, 0.791, 0.088, 0.445, 1.74), in / 4.02e6);
 }
 
-// Block-scaled product with memory for partial sums, the form with the least estimated time: the ring kernel (gemm_ring.hip) on
+// Block-scaled product with memory for partial sums: strips of few rows where they go first (gemm_ring.hip: ring_few_first), else the form with the least estimated time: the ring kernel (gemm_ring.hip) on
 // all rows, launch_gemm on all of them, or launch_gemm's full tiles on the first M / 256 * 256 rows and the ring kernel on the
 // rest.  Up to 64 rows the ring kernel's loads, many steps ahead, and its slices win everywhere.  In the middle its four waves are
 // behind the others' eight, which do the scaling of one half of the waves under the other's products.

@@ -1830,7 +1830,7 @@ static int gemm_mx4_dense(Mx4Args& p, float* partial, size_t partial_bytes, int 
         return launch_ring_few(kRingMx, r, strips, out_dtype, st);
     }
     if (p.M <= 128) {
-        // (ring kernel / streamers: 18944 x 3584 at 33 tokens 19.5 / 17.4 us, 16 x 3584 x 3584 8.2 / 6.2, but 33 x 25344 x 2560 15.3 / 25.3)
+        // (ring kernel's tiles / streamers: 18944 x 3584 at 33 tokens, where strips go first, 19.5 / 17.4 us, 16 x 3584 x 3584 8.2 / 6.2, but 33 x 25344 x 2560 15.3 / 25.3)
         if (mx4_streams_cost(p.M, p.N, p.K, cu_count()) <= plan.cost) return CFP8_OK;
     } else {
         const bool aligned256 = p.M % 256 == 0 && p.N % 256 == 0 && p.K % 128 == 0 && p.ld_ws % 4 == 0 && (reinterpret_cast<uintptr_t>(p.ws) & 3u) == 0;
